@@ -20,9 +20,8 @@
 //                   64 columns through all of k, two such workgroups per CU (int4 and fp4 prefill);
 //                   tiles of up to 160 rows, or of up to 32 / 16 rows with small stages (decode batches,
 //                   and the GEMV op's arithmetic on the N-contiguous containers)
-//   gemm_tile       the bf16 container: 4 wavefronts of 64 columns, x through a double-buffered,
-//                   XOR-swizzled LDS tile, weights from registers; tiles of up to 176 rows, or 32 rows
-//                   and several workgroups per CU for decode-sized batches
+//   gemm_tile_bf16  the bf16 container: 8 wavefronts, tiles of up to 224 rows, x and weights by LDS-direct loads into
+//                   two rings
 //
 // MFMA: v_mfma_f32_16x16x32_bf16.  Lane l = 16*q + i holds, for A, row i and
 // k = 8q..8q+7 of the 16x32 block; for B, column i and the same k; for the result,
@@ -37,10 +36,6 @@
 namespace moe {
 
 constexpr int GM_BN = 256;     // columns per workgroup
-constexpr int GM_MT_MAX = 12;  // 16-row blocks per tile the LDS buffers are sized for (192 rows)
-constexpr int GM_THREADS = 256;
-constexpr int GM_SKINNY_BLOCKS = 2;  // decode kernel: tiles of at most 32 rows ...
-constexpr int GM_SKINNY_WAVES = 3;   // ... and at least this many wavefronts per SIMD
 
 struct GemmParams {
     const uint16_t* x;
@@ -137,27 +132,12 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* p, int64_t bytes) {
     const uint32_t n = bytes > 0xffffffffLL ? 0xffffffffu : (uint32_t)bytes;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, n, 0x00020000);
 }
-__device__ __forceinline__ uint32_t ldg_b32(rsrc_t r, int voff, int soff) {
-    return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
-}
-__device__ __forceinline__ u32x2_t ldg_b64(rsrc_t r, int voff, int soff) {
-    return __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
-}
-__device__ __forceinline__ u32x4_t ldg_b128(rsrc_t r, int voff, int soff) {
-    return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-}
-
-// D = A * B + D with the accumulator tied to AGPRs.  Written as inline asm because the
+// D = A * B + D with the accumulator tied in place.  Written as inline asm because the
 // compiler, given many live accumulators, stops accumulating in place and shuttles them
 // through copies, which halves the MFMA rate.  Hazards: A/B come from VALU or waited
 // loads (interlocked); accumulators are only read by other MFMAs until the epilogue,
-// which waits out the MFMA latency first.
-__device__ __forceinline__ void mfma_16x16x32(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {
-    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-}
-
-// Same with the accumulator in ordinary VGPRs.  A kernel that uses no AGPRs at all may use
-// the whole unified register file as VGPRs (otherwise the compiler splits it in two halves).
+// which waits out the MFMA latency first.  (The accumulators are ordinary VGPRs: a kernel that uses no AGPRs at all may
+// use the whole unified register file as VGPRs, otherwise the compiler splits it in two halves.)
 __device__ __forceinline__ void mfma_16x16x32_v(f32x4_t& acc, const u32x4_t& a, const u32x4_t& b) {
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
 }
@@ -166,65 +146,6 @@ __device__ __forceinline__ void mfma_16x16x32_v(f32x4_t& acc, const u32x4_t& a, 
 __device__ __forceinline__ float swiglu(float g, float u) {
     return g * __builtin_amdgcn_rcpf(1.f + __expf(-g)) * u;
 }
-
-// Ties a value to the chain of volatile asm statements (the MFMAs): whatever is computed
-// from the returned value is emitted after every earlier volatile asm, whatever produced the
-// argument before every later one.  Emits no instruction.  Used to pin each decode unit
-// between two MFMAs; sched_barrier alone only constrains the machine scheduler, not the
-// instruction order chosen at selection time.
-template <typename V>
-__device__ __forceinline__ V pinned(V v) {
-    asm volatile("" : "+v"(v));
-    return v;
-}
-
-// Per-lane view of one tile for the weight loaders.
-struct BCtx {
-    rsrc_t rw, rs;       // weight / scale slab of the expert
-    int vw, vs;          // per-lane byte offsets into them (constant over the tile)
-    int K, N, n0;
-    int i, q, w;         // lane & 15, lane >> 4, wavefront (scalar)
-};
-
-// Each weight container provides
-//   Raw        packed registers of one k step
-//   load_sub   global loads of 32-k sub-step s of the step starting at k0
-//   Dq         the decode, cut into units so that it can be interleaved with MFMAs:
-//              prep(raw, c, s) once per sub-step, then unit(raw, c, s, p, t, out) for
-//              p, t in [0,4) writes dword p (k pair) of the fragment of MFMA t
-//   a_chunk    which 16-byte chunk of the x tile row matches the k values of (s, q)
-//   col        output column (relative to n0) of MFMA t in this lane
-template <int FMT>
-struct BTraits;
-
-// ------------------------------------------------------------------ bf16, [N, K]
-// K-contiguous: lane (i, q) loads 32 contiguous bytes, k = k0 + 16q + [0,16); sub-step
-// s uses the half k0 + 16q + 8s + [0,8), so the matching x chunk is 2q + s.
-template <>
-struct BTraits<MOE_FMT_BF16> {
-    static constexpr int BK = 64, NS = 2;
-    static constexpr int MT_MAX = 11;
-    struct Raw {
-        u32x4_t r[4][2];
-    };
-    __device__ static __forceinline__ int a_chunk(int s, int q) { return 2 * q + s; }
-    __device__ static __forceinline__ int col(const BCtx& c, int t) { return 64 * c.w + 16 * t + c.i; }
-    __device__ static __forceinline__ void init(BCtx& c) {
-        c.vw = (64 * c.w + c.i) * c.K * 2 + 32 * c.q;
-        c.vs = 0;
-    }
-    __device__ static __forceinline__ void load_sub(Raw& raw, const BCtx& c, int k0, int s) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) raw.r[t][s] = ldg_b128(c.rw, c.vw, ((c.n0 + 16 * t) * c.K + k0) * 2 + 16 * s);
-    }
-    struct Dq {
-        __device__ __forceinline__ void init_tile(const BCtx&) {}
-        __device__ __forceinline__ void prep(const Raw&, const BCtx&, int) {}
-        __device__ __forceinline__ void unit(const Raw& raw, const BCtx&, int s, int p, int t, u32x4_t out[4]) {
-            out[t][p] = pinned(raw.r[t][s][p]);
-        }
-    };
-};
 
 // ---------------------------------------------------------------------------------
 // x tile: rows x BK bf16 in LDS, 16-byte chunks, chunk c of row r stored at
@@ -244,185 +165,6 @@ __device__ __forceinline__ int a_lds_unit(int row, int c) {
 // SQ_LDS_BANK_CONFLICT at 39 % of the cycles the LDS was active.)
 __device__ __forceinline__ int a_lds_unit32(int row, int c) {
     return row * 4 + (c ^ ((row >> 1) & 3));
-}
-
-// Per-tile context: lane coordinates and the buffer resources of expert g.
-template <int FMT>
-__device__ __forceinline__ void make_ctx(BCtx& c, const GemmParams& P, int g, int n0) {
-    const int tid = threadIdx.x, lane = tid & 63;
-    c.K = P.K; c.N = P.N; c.n0 = n0;
-    c.i = lane & 15; c.q = lane >> 4; c.w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t KN = (int64_t)P.K * P.N;
-    static_assert(FMT == MOE_FMT_BF16, "the 4-wavefront tile routine serves the bf16 container");
-    c.rw = make_rsrc(P.w + g * KN * 2, KN * 2);
-    c.rs = c.rw;
-}
-
-// Epilogue: fp32 -> bf16 (RNE), rows beyond the chunk are dropped.
-template <int FMT, int MT>
-__device__ __forceinline__ void store_tile(const GemmParams& P, const BCtx& c, f32x4_t (&acc)[MT][4], int64_t row0, int rows,
-                                           int n0) {
-    using T = BTraits<FMT>;
-    // through a buffer resource that ends after the tile's last valid row: stores to padded
-    // rows fall outside it and are dropped (the containers of this routine are K-contiguous: a lane's
-    // 4 accumulators of a row are 16 columns apart)
-    if (P.epilogue == MOE_EPILOGUE_SWIGLU) {
-        // weight rows in blocks of 32 = (16 gate rows, 16 up rows): MFMAs (0, 1) and (2, 3); y has N / 2 columns
-        const int NO = P.N >> 1;
-        const rsrc_t ro = make_rsrc(P.y + row0 * (int64_t)NO, (int64_t)rows * NO * 2);
-        const int vo = (4 * c.q * NO + ((n0 + 64 * c.w) >> 1) + c.i) * 2;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int u = 0; u < 2; ++u)
-                    __builtin_amdgcn_raw_buffer_store_b16(
-                        (uint16_t)(pack_bf16_rne(swiglu(acc[mt][2 * u][r], acc[mt][2 * u + 1][r]), 0.f) & 0xffffu), ro,
-                        vo + 32 * u, (16 * mt + r) * NO * 2, 0);
-        return;
-    }
-    const rsrc_t ry = make_rsrc(P.y + row0 * (int64_t)P.N, (int64_t)rows * P.N * 2);
-    const int vy = (4 * c.q * P.N + n0) * 2;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int so = (16 * mt + r) * P.N * 2;
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-                __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(pack_bf16_rne(acc[mt][t][r], 0.f) & 0xffffu), ry,
-                                                      vy + T::col(c, t) * 2, so, 0);
-        }
-}
-
-template <int FMT, int MT, int CAPB>
-__device__ __forceinline__ void gemm_tile(const GemmParams& P, u32x4_t* lds_a, int g, int64_t row0, int rows, int n0) {
-    using T = BTraits<FMT>;
-    constexpr int BK = T::BK, NS = T::NS;
-    constexpr int CPR = BK / 8;               // 16-byte chunks per tile row
-    constexpr int RPP = GM_THREADS / CPR;     // rows loaded per pass
-    constexpr int PASSES = (16 * MT + RPP - 1) / RPP;
-    constexpr int ABUF = 16 * CAPB * CPR;  // units per buffer (CAPB row blocks)
-
-    const int tid = threadIdx.x;
-    BCtx c;
-    make_ctx<FMT>(c, P, g, n0);
-    T::init(c);
-    typename T::Dq dq;
-    dq.init_tile(c);
-
-    // x rows of this tile through a buffer resource that ends after the last valid row:
-    // padded rows read as zeros.  This thread loads chunk ac of rows ar + RPP*p.
-    const int ar = tid / CPR, ac = tid % CPR;
-    const rsrc_t rx = make_rsrc(P.x + row0 * (int64_t)P.K, (int64_t)rows * P.K * 2);
-    const int vx = (ar * P.K + ac * 8) * 2;
-
-    f32x4_t acc[MT][4];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) acc[mt][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-    u32x4_t areg[PASSES];
-    typename T::Raw raw;
-    const int nk = P.K / BK;
-
-    // Every pass is done by all threads: rows past the tile read as zeros (they lie beyond the
-    // buffer resource) and land in LDS rows that exist (the buffers hold 16 * CAPB rows)
-    // but are never read.  No divergent branch, so the loop body stays one scheduling region.
-    static_assert(PASSES * RPP <= 16 * CAPB, "x tile passes overrun the LDS buffer");
-    auto load_a = [&](int kt) {
-#pragma unroll
-        for (int p = 0; p < PASSES; ++p) areg[p] = ldg_b128(rx, vx, (p * RPP * P.K + kt * BK) * 2);
-    };
-    auto store_a = [&](int buf) {
-#pragma unroll
-        for (int p = 0; p < PASSES; ++p) lds_a[buf * ABUF + a_lds_unit<BK>(ar + RPP * p, ac)] = areg[p];
-    };
-
-    // Software pipeline, one barrier per k step (BK = NS sub-steps of 32 k), every
-    // instruction placed by hand (sched_barrier after each MFMA slot):
-    //  * weights: while the MFMAs of sub-step f run, the fragments of sub-step f+1 are
-    //    decoded, one unit (two elements of one column) at a time between MFMAs; as soon as
-    //    a sub-step's packed registers have been decoded they are refilled with the same
-    //    sub-step of the next k step, straight from global memory a full step ahead;
-    //  * x: fragments come from LDS through a ring of 4 register sets, read RING
-    //    fragments ahead of their MFMAs; the x tile of step kt+1 travels through registers
-    //    into the other LDS buffer.
-    // The last steps prefetch past K: buffer loads beyond a slab return 0 and the x rows
-    // read are inside the tensor; neither is used.
-    constexpr int RING = 3, F = NS * MT;
-    constexpr int SLOTS = 4 * MT;   // MFMAs per sub-step
-    constexpr int UNITS = 17;       // prep + 16 decode units per sub-step
-
-    __syncthreads();  // previous tile's readers are done with both buffers
-    load_a(0);
-    store_a(0);
-#pragma unroll
-    for (int s = 0; s < NS; ++s) T::load_sub(raw, c, 0, s);
-    u32x4_t bf[2][4];
-    dq.prep(raw, c, 0);
-#pragma unroll
-    for (int p = 0; p < 4; ++p)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) dq.unit(raw, c, 0, p, t, bf[0]);
-    __syncthreads();
-    // raw[0] <- sub-step 0 of step 1, a full step ahead
-    T::load_sub(raw, c, BK, 0);
-
-    // One k step.  The global loads of the next x tile are issued one per MFMA slot at the start
-    // of the first sub-step, the LDS writes one per slot at the end of the last one, so that
-    // neither sits between the barrier and the first MFMA or between the last MFMA and the barrier.
-    constexpr int NW = PASSES;   // write slots: one per x pass
-    static_assert(NW + 1 <= SLOTS, "not enough MFMA slots to spread the tile transfers over");
-    auto step = [&](int kt) {
-        const u32x4_t* la = lds_a + (kt & 1) * ABUF;
-        u32x4_t afr[4];
-        auto read_a = [&](int f) {
-            afr[f & 3] = la[a_lds_unit<BK>(16 * (f % MT) + c.i, T::a_chunk(f / MT, c.q))];
-        };
-#pragma unroll
-        for (int f = 0; f < (RING < F ? RING : F); ++f) read_a(f);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            const int sn = (s + 1) % NS;                 // sub-step being decoded
-            u32x4_t* bcur = bf[s & 1];
-            u32x4_t* bnxt = bf[(s + 1) & 1];
-#pragma unroll
-            for (int slot = 0; slot < SLOTS; ++slot) {
-                const int mt = slot >> 2, t = slot & 3, f = s * MT + mt;
-                if (t == 0 && f + RING < F) read_a(f + RING);
-                mfma_16x16x32(acc[mt][t], afr[f & 3], bcur[t]);
-                // fetch the x tile of step kt+1
-                if (s == 0 && slot < PASSES) areg[slot] = ldg_b128(rx, vx, (slot * RPP * P.K + (kt + 1) * BK) * 2);
-                // decode units u with floor(u * SLOTS / UNITS) == slot
-#pragma unroll
-                for (int u = (slot * UNITS + SLOTS - 1) / SLOTS; u < ((slot + 1) * UNITS + SLOTS - 1) / SLOTS; ++u) {
-                    if (u == 0)
-                        dq.prep(raw, c, sn);
-                    else
-                        dq.unit(raw, c, sn, (u - 1) >> 2, (u - 1) & 3, bnxt);
-                }
-                if (slot == ((UNITS - 1) * SLOTS) / UNITS) {
-                    // everything of sub-step sn has been decoded: refill its registers
-                    T::load_sub(raw, c, (kt + (sn == 0 ? 2 : 1)) * BK, sn);
-                }
-                if (s == NS - 1 && slot >= SLOTS - NW) {
-                    const int wi = slot - (SLOTS - NW);
-                    lds_a[((kt + 1) & 1) * ABUF + a_lds_unit<BK>(ar + RPP * wi, ac)] = areg[wi];
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        __syncthreads();
-    };
-    for (int kt = 0; kt < nk; ++kt) step(kt);
-    // the accumulators were last written by MFMAs the compiler cannot see: wait out their latency
-    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-
-    store_tile<FMT, MT>(P, c, acc, row0, rows, n0);
 }
 
 // ---------------------------------------------------------------------------------
@@ -501,9 +243,6 @@ __device__ __forceinline__ uint32_t here(uint32_t v) {
 // fetched 16 bytes per row at a time into buffers of their own (see kc_issue_scale).
 // ---------------------------------------------------------------------------------
 // Kernel variants.
-//   GK_GENERAL  4 wavefronts of 64 columns, one workgroup per CU, tiles of up to 176 rows (bf16 only)
-//   GK_SKINNY   the same tile routine with tiles of at most 32 rows and several workgroups per CU
-//               (decode-sized batches are HBM bound: more weight bytes in flight)
 //   GK_PAIR     quantized containers: 8 wavefronts, k range split between the two wavefronts of a SIMD, tiles of
 //               up to 160 rows
 //   GK_PAIR_SMALL  GK_PAIR with tiles of at most 32 rows: x stages of 4 KB leave LDS for a second workgroup per
@@ -516,7 +255,8 @@ __device__ __forceinline__ uint32_t here(uint32_t v) {
 //               of a SIMD belong to different workgroups and work on different tiles: no partial sums to
 //               exchange, a barrier spans 4 wavefronts instead of 8, and while one workgroup is between two tiles
 //               (stores, tile search, first loads) the other has the SIMDs to itself.  (The N-contiguous containers.)
-enum { GK_GENERAL = 0, GK_SKINNY = 1, GK_PAIR = 2, GK_PAIR_EXACT = 3, GK_PAIR_SMALL = 4, GK_PAIR_EXACT16 = 5, GK_QUAD = 6 };
+//   GK_BF16     gemm_tile_bf16
+enum { GK_PAIR = 2, GK_PAIR_EXACT = 3, GK_PAIR_SMALL = 4, GK_PAIR_EXACT16 = 5, GK_QUAD = 6, GK_BF16 = 7 };
 constexpr bool pair_exact(int kind) { return kind == GK_PAIR_EXACT || kind == GK_PAIR_EXACT16; }
 constexpr int pair_waves(int kind) { return kind == GK_QUAD ? 4 : 8; }
 constexpr int pair_bk(int kind) { return kind == GK_QUAD ? 32 : 64; }   // k per step
@@ -1299,15 +1039,158 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
 }
 
 // ---------------------------------------------------------------------------------
+// Tile routine for the bf16 container (weights [N, K], K-contiguous, nothing to decode): 8 wavefronts, one workgroup per
+// CU, tiles of up to 224 rows x 256 columns; wavefront (wr, cw) multiplies half wr of the rows by the 64 columns of
+// group cw.
+//
+// What bounds it: with up to about 200 rows per expert the weights (2 bytes each) are read once from HBM, and the rate
+// follows from how many of their bytes are on their way, i.e. from how much LDS is left for them; with more rows per
+// expert the latency of L2 misses that a step cannot look far enough ahead for.  With all loads taken out the loop runs
+// at 1.5 PFLOP/s, with all of them hitting L2 at 1.3.  Hence one workgroup per CU, so that x is held once (two of 4
+// wavefronts with 144 rows each, three 25 KB stages: no faster than the routine this replaced), and two rings: x, which
+// the neighbouring column tiles read too and L2 usually holds, two or three pairs of steps deep, the weights three or four.
+// A load instruction brings 64 bytes (one 32-k step) of 16 rows; the two halves of a 128-byte line are requested back
+// to back, in pairs of steps: asked for a step apart the line travels from L2 twice (measured: 535 and 480 us).
+// Weights straight into registers, two steps of 64 k ahead, lose: such loads of 16 rows each cost the CU's
+// vector memory path twice the cycles of LDS-direct ones (498 us, and 616 instead of 570 us on the large shape below).
+//
+// 64 experts, K = 7168, N = 2048, 900 / 1021 tokens x 8 rows (the second unevenly routed): 416 / 542 us with the
+// 4-wavefront routine this replaced, now 391 / 489 (5.1 / 4.1 TB/s); 100 tokens: 361 -> 320 us (5.9 TB/s);
+// 8 experts of 512 rows, K = 4096, N = 14336: 554 -> 491 us (979 TFLOP/s).
+//
+// Column t of a lane is 4 i + t, so that a lane stores 4 adjacent columns in one instruction (the rows of the weight
+// may be assigned to MFMAs and lanes freely); with the SwiGLU epilogue the lane takes the two gate rows and the two up
+// rows of two adjacent output columns, which makes its 4 accumulators what the N-contiguous containers have.
+// ---------------------------------------------------------------------------------
+constexpr int BF_MT_MAX = 7;                                   // row blocks of a wavefront: tiles of 224 rows
+constexpr int BF_B_UNITS = GM_BN * 4;                          // 256 weight rows x 32 k
+constexpr int bf_a_units(int mt) { return 32 * mt * 4; }       // 32 mt rows x 32 k
+// pairs of steps in the two rings: what fits into 156 KB
+constexpr int bf_x_pairs(int mt) { return mt == 4 || mt == 5 ? 3 : 2; }
+constexpr int bf_w_pairs(int mt) { return mt > 3 ? 3 : 4; }
+constexpr int bf_lds_units() {
+    int most = 0;
+    for (int mt = 1; mt <= BF_MT_MAX; ++mt) most = max(most, 2 * (bf_x_pairs(mt) * bf_a_units(mt) + bf_w_pairs(mt) * BF_B_UNITS));
+    return most;
+}
+template <int MT>
+__device__ __forceinline__ void gemm_tile_bf16(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk) {
+    constexpr int XP = bf_x_pairs(MT), WP = bf_w_pairs(MT), NW = 8;
+    constexpr int AU = bf_a_units(MT), BU = BF_B_UNITS;   // units of a half step
+    u32x4_t* const lds_w = smem + XP * 2 * AU;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, i = lane & 15, q = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = wv >> 2, cw = wv & 3;
+    const int np = P.K >> 6;
+    const int64_t KN = (int64_t)P.K * P.N;
+    const int k2 = P.K * 2;
+    const bool swi = P.epilogue == MOE_EPILOGUE_SWIGLU;
+    // Load instructions of 16 rows x 64 bytes: lane l brings the 16-byte chunk (l & 3) ^ ((l >> 3) & 3) of row l >> 2 to
+    // position l & 3 (see a_lds_unit32); both 64-byte halves of a row's 128-byte line are requested back to back
+    const int li = lane >> 2, vc = ((lane & 3) ^ ((lane >> 3) & 3)) * 16;
+    const rsrc_t rx = make_rsrc(P.x + row0 * (int64_t)P.K, (int64_t)rows * k2);
+    const int va = li * k2 + vc;
+    const rsrc_t rw = make_rsrc(P.w + g * (KN * 2), KN * 2);
+    const int vb = (swi ? 32 * (li >> 3) + 2 * (li & 7) : 4 * li) * k2 + vc;
+    constexpr int XI = 2 * MT, NA = (XI + NW - 1) / NW, NB = 2;
+    int ca[NA], cb[NB];
+    uint32_t a_at[NA];
+#pragma unroll
+    for (int m = 0; m < NA; ++m) {
+        int j = wv + NW * m;
+        if (NW * NA > XI) j = j % XI;   // repeat a block rather than issue fewer loads
+        a_at[m] = lds_address(smem + j * 64);
+        ca[m] = 16 * j * k2;
+    }
+#pragma unroll
+    for (int e = 0; e < NB; ++e) {
+        const int j = NB * wv + e, t = j & 3;   // rows of MFMA t of column group j >> 2
+        cb[e] = (n0 + 64 * (j >> 2) + (swi ? (t & 1) + 16 * (t >> 1) : t)) * k2;
+    }
+    const uint32_t b_at = lds_address(lds_w + NB * wv * 64);
+    auto issue_x = [&](int m, int p, int slot) {
+        const int h = m & 1, e = m >> 1;
+        lds_load16_at(rx, here(a_at[e]) + slot * (2 * AU * 16) + h * (AU * 16), va, ca[e] + p * 128 + h * 64);
+    };
+    auto issue_w = [&](int m, int p, int slot) {
+        const int h = m & 1, e = m >> 1;
+        lds_load16_at(rw, here(b_at) + slot * (2 * BU * 16) + h * (BU * 16) + e * 1024, vb, cb[e] + p * 128 + h * 64);
+    };
+#pragma unroll
+    for (int p = 0; p < WP - 1; ++p) {   // (in the order of the loop below: x a ring's depth ahead, then the weights)
+        if (p >= WP - XP)
+#pragma unroll
+            for (int m = 0; m < 2 * NA; ++m) issue_x(m, p - (WP - XP), p - (WP - XP));
+#pragma unroll
+        for (int m = 0; m < 2 * NB; ++m) issue_w(m, p, p);
+    }
+    f32x4_t acc[MT][4];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            asm volatile("v_mov_b32 %0, 0\n\tv_mov_b32 %1, 0\n\tv_mov_b32 %2, 0\n\tv_mov_b32 %3, 0"
+                         : "=v"(acc[mt][t][0]), "=v"(acc[mt][t][1]), "=v"(acc[mt][t][2]), "=v"(acc[mt][t][3]));
+    // the next pair's x and weights have landed: of what was requested behind them, one pair's weights (and its x, where
+    // that ring holds three pairs) may be on their way
+    constexpr int WAITN = (XP - 2) * 2 * NA + 2 * NB;
+    auto pair_barrier = [&]() { asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(WAITN) : "memory"); };
+    pair_barrier();
+    const u32x4_t* const xf = smem + a_lds_unit32(16 * MT * wr + i, q);
+    const u32x4_t* const wf = lds_w + a_lds_unit32(64 * cw + i, q);
+    constexpr int NI = 2 * (NA + NB);
+    constexpr int F = 2 * MT, R = 3 < F ? 3 : F;   // x fragments of a pair, read R ahead of their MFMAs
+    for (int p = 0, xs = 0, ws = 0; p < np; ++p) {
+        const int x_to = xs == 0 ? XP - 1 : xs - 1, w_to = ws == 0 ? WP - 1 : ws - 1;
+        const u32x4_t* lx = xf + xs * (2 * AU);
+        const u32x4_t* lw = wf + ws * (2 * BU);
+        u32x4_t bf[2][4], afr[4];
+        auto read_x = [&](int f) { afr[f & 3] = lx[(f / MT) * AU + (f % MT) * 64]; };
+#pragma unroll
+        for (int t = 0; t < 4; ++t) bf[0][t] = lw[t * 64];
+#pragma unroll
+        for (int f = 0; f < R; ++f) read_x(f);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            if (f + R < F) read_x(f + R);
+            if (f == (MT + 1) / 2 - 1)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) bf[1][t] = lw[BU + t * 64];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) mfma_16x16x32_v(acc[f % MT][t], afr[f & 3], bf[f / MT][t]);
+#pragma unroll
+            for (int m = (f * NI + MT - 1) / MT; f < MT && m < ((f + 1) * NI + MT - 1) / MT; ++m) {
+                if (m < 2 * NA)
+                    issue_x(m, p + XP - 1, x_to);
+                else
+                    issue_w(m - 2 * NA, p + WP - 1, w_to);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        pair_barrier();
+        xs = xs == XP - 1 ? 0 : xs + 1;
+        ws = ws == WP - 1 ? 0 : ws + 1;
+    }
+    // the last loads are for pairs past K and never read; wait out the last MFMAs' latency
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15\n\ts_barrier" ::: "memory");
+    pair_finish<MT, false, true>(P, smem, acc, 0, cw, lane, 64 * cw + 4 * i, row0 + 16 * MT * wr, max(rows - 16 * MT * wr, 0), n0, tk);
+}
+
+// ---------------------------------------------------------------------------------
 // Tile scheduler (role of GMMAntiquantProcess::Process,
 // grouped_gemm/op_kernel/grouped_matmul_antiquant.h:241-288).  Expert g with m_g rows
-// has ceil(m_g/16) row blocks, cut into the fewest chunks of <= MT_MAX blocks, as
+// has ceil(m_g/BLOCK) row blocks, cut into the fewest chunks of <= MT_MAX blocks, as
 // even as possible; each chunk has N/256 tiles.  prefix[] (in LDS) is the exclusive
 // scan of the tile counts.
 // ---------------------------------------------------------------------------------
-template <int MT_MAX>
+template <int MT_MAX, int BLOCK>
 __device__ __forceinline__ void expert_chunks(int m, int& chunks, int& bpc) {
-    const int nblk = (m + 15) >> 4;
+    const int nblk = (m + BLOCK - 1) / BLOCK;
     if (nblk <= MT_MAX) {   // the usual case, without the division
         chunks = nblk ? 1 : 0;
         bpc = nblk;
@@ -1320,29 +1203,22 @@ __device__ __forceinline__ void expert_chunks(int m, int& chunks, int& bpc) {
 template <int FMT, int KIND>
 struct KernelCfg {
     static constexpr bool PAIR = KIND == GK_PAIR || KIND == GK_PAIR_SMALL || KIND == GK_QUAD || pair_exact(KIND);
-    static constexpr bool SKINNY = KIND == GK_SKINNY;
-    static_assert(!PAIR || FMT != MOE_FMT_BF16, "the k-split tile routine decodes quantized containers");
-    static constexpr int WAVES = PAIR ? pair_waves(KIND) : 4;
+    static_assert(PAIR == (FMT != MOE_FMT_BF16), "gemm_tile_pair decodes the quantized containers");
+    static constexpr int WAVES = PAIR ? pair_waves(KIND) : 8;
+    static constexpr int BLOCK = PAIR ? 16 : 32;   // rows per row block of a tile routine's template argument
     static constexpr int BN = GM_BN;                                             // columns per tile
     static constexpr int pair_wgs() {
         if constexpr (PAIR) return pair_wg_per_cu<FMT>(KIND); else return 1;
     }
-    static constexpr int WG_PER_CU = SKINNY ? GM_SKINNY_WAVES : pair_wgs();
+    static constexpr int WG_PER_CU = pair_wgs();
     static constexpr int WAVES_PER_SIMD = WG_PER_CU * WAVES / 4;
-    static constexpr int CAPB = SKINNY ? GM_SKINNY_BLOCKS : PAIR ? PAIR_CAPB : GM_MT_MAX;
-    static constexpr int fmt_mt_max() {
-        if constexpr (PAIR)
-            return pair_mt_max(KIND);
-        else
-            return BTraits<FMT>::MT_MAX;
-    }
-    static constexpr int MTM = CAPB < fmt_mt_max() ? CAPB : fmt_mt_max();        // row blocks per tile
+    static constexpr int MTM = PAIR ? pair_mt_max(KIND) : BF_MT_MAX;             // row blocks per tile
     // 16-byte LDS units of the tile routine (the tile prefix array follows them)
     static constexpr int lds_units() {
         if constexpr (PAIR)
             return pair_lds_units<FMT>(KIND);
         else
-            return 2 * 16 * CAPB * (BTraits<FMT>::BK / 8);
+            return bf_lds_units();
     }
 };
 
@@ -1354,9 +1230,9 @@ __device__ __forceinline__ void run_tile(const GemmParams& P, u32x4_t* smem, int
             if (rows <= 8) return gemm_tile_pair<FMT, MT, KIND, true>(P, smem, g, row0, rows, n0, tk);
         }
         gemm_tile_pair<FMT, MT, KIND>(P, smem, g, row0, rows, n0, tk);
+    } else {
+        gemm_tile_bf16<MT>(P, smem, g, row0, rows, n0, tk);
     }
-    else
-        gemm_tile<FMT, MT, C::CAPB>(P, smem, g, row0, rows, n0);
 }
 
 template <int FMT, int KIND>
@@ -1376,7 +1252,7 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
     const int ntile_n = (P.N + C::BN - 1) / C::BN;
     // scan partials (one per wavefront); later part[0] carries the ticket drawn from the queue, part[1] the tile
     // resolved from it, part[2] the tile routine's arrival counter
-    __shared__ int part[THREADS];
+    __shared__ int part[32];
     constexpr int PART_FIXED = 16;   // first whether this workgroup uses the launch's counter, then its number of fixed sweeps
     auto clamp_row = [&](int64_t v) { return (int)min(max(v, (int64_t)0), P.M); };
     auto expert_rows = [&](int g, int& first) {
@@ -1407,7 +1283,7 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         int sum = 0;
         for (int g = g0; g < g1; ++g) {
             int first, chunks, bpc;
-            expert_chunks<MTM>(expert_rows(g, first), chunks, bpc);
+            expert_chunks<MTM, C::BLOCK>(expert_rows(g, first), chunks, bpc);
             sum += chunks * ntile_n;
         }
         // scan over the threads: within a wavefront by shuffles, across wavefronts through their totals in
@@ -1433,7 +1309,7 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         if (P.table_mode) {
             for (int g = g0; g < g1; ++g) {
                 int first, chunks, bpc;
-                expert_chunks<MTM>(expert_rows(g, first), chunks, bpc);
+                expert_chunks<MTM, C::BLOCK>(expert_rows(g, first), chunks, bpc);
                 prefix[g] = run;
                 run += chunks * ntile_n;
             }
@@ -1490,8 +1366,8 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
             T = sw * sweep + ((sw + 1) * sweep > total ? (int)blockIdx.x : vid);
             if (T >= total) break;
         }
-        // from the last tile of the fixed order on, the k-split tile routines draw the next ticket themselves
-        const bool take = C::PAIR && fixed != GM_NO_QUEUE && sw + 1 >= fixed;
+        // from the last tile of the fixed order on, the tile routines draw the next ticket themselves
+        const bool take = fixed != GM_NO_QUEUE && sw + 1 >= fixed;
         const Ticket tk = {take ? q_own : nullptr, part, part + 2};
         have_ticket = take;
         // largest e with prefix[e] <= T (empty experts have prefix[e] == prefix[e+1]): every wavefront looks at 64
@@ -1523,7 +1399,7 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
                 int tiles = 0;
                 if (ge < e_end) {
                     int first, ch, bp;
-                    expert_chunks<MTM>(expert_rows(ge, first), ch, bp);
+                    expert_chunks<MTM, C::BLOCK>(expert_rows(ge, first), ch, bp);
                     tiles = ch * ntile_n;
                 }
                 int incl = tiles;
@@ -1549,13 +1425,13 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         const int m = __builtin_amdgcn_readfirstlane(expert_rows(g, gfirst));
         const int64_t gbeg = gfirst;
         int chunks, bpc;
-        expert_chunks<MTM>(m, chunks, bpc);
+        expert_chunks<MTM, C::BLOCK>(m, chunks, bpc);
         // row chunks innermost: the tiles that share a weight column tile are neighbours in the order, run at
         // the same time on one XCD and pull that slice of the expert's weights into its L2 once
         const int nt = chunks == 1 ? local : local / chunks, chunk = chunks == 1 ? 0 : local % chunks;
-        const int rbeg = chunk * bpc * 16;
-        const int rows = min(m - rbeg, bpc * 16);
-        const int mt = (rows + 15) >> 4;
+        const int rbeg = chunk * bpc * C::BLOCK;
+        const int rows = min(m - rbeg, bpc * C::BLOCK);
+        const int mt = (rows + C::BLOCK - 1) / C::BLOCK;
         const int rlo = __builtin_amdgcn_readfirstlane((int)(uint32_t)(gbeg & 0xffffffffLL));
         const int rhi = __builtin_amdgcn_readfirstlane((int)(gbeg >> 32));
         const int64_t row0 = (((int64_t)rhi << 32) | (uint32_t)rlo) + rbeg;
@@ -1591,12 +1467,6 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
             case 10:
                 if constexpr (MTM >= 10) run_tile<FMT, 10, KIND>(P, smem, g, row0, rows, n0, tk);
                 break;
-            case 11:
-                if constexpr (MTM >= 11) run_tile<FMT, 11, KIND>(P, smem, g, row0, rows, n0, tk);
-                break;
-            case 12:
-                if constexpr (MTM >= 12) run_tile<FMT, 12, KIND>(P, smem, g, row0, rows, n0, tk);
-                break;
             default: have_ticket = false; break;
         }
     }
@@ -1622,7 +1492,7 @@ static int device_cu_count() {
 template <int FMT, int KIND>
 static int launch_gemm_kind(const GemmParams& P, const moe_grouped_args* a, hipStream_t stream) {
     using C = KernelCfg<FMT, KIND>;
-    const size_t lds_max = (160 * 1024 - 2048) / C::WG_PER_CU;
+    const size_t lds_max = (160 * 1024 - 512) / C::WG_PER_CU;
     const size_t table = ((size_t)a->G + 1) * sizeof(int);
     // tile table, and the row bounds next to it where they fit; else the scheduler reads group_list per tile; else,
     // with more experts than LDS holds a table for, it keeps one entry per thread and walks group_list (see
@@ -1638,7 +1508,7 @@ static int launch_gemm_kind(const GemmParams& P, const moe_grouped_args* a, hipS
     if (cus <= 0) return MOE_ERR_NO_DEVICE;
     // persistent grid: as many workgroups as the CUs hold, but no more than an upper bound on the
     // tile count that needs no look at group_list (every expert adds at most one partly filled chunk)
-    const int64_t max_chunks = a->M / (16 * C::MTM) + a->G;
+    const int64_t max_chunks = a->M / (C::BLOCK * C::MTM) + a->G;
     const int64_t max_tiles = max_chunks * ((a->N + C::BN - 1) / C::BN);
     const int64_t want = max_tiles < (int64_t)cus * C::WG_PER_CU ? max_tiles : (int64_t)cus * C::WG_PER_CU;
     // a multiple of 8 so that the XCD-aware order covers every tile index
@@ -1711,11 +1581,7 @@ static int launch_gemm_fmt(const moe_grouped_args* a, hipStream_t stream) {
         }
         return launch_gemm_kind<FMT, GK_PAIR>(P, a, stream);
     } else {
-        // Decode-like batches (on average at most 24 rows per expert; group_list itself stays on the
-        // device) are HBM bound: use the small-tile kernel.  An expert with more than 32 rows then
-        // costs one pass over its weights per 32 rows.
-        if (a->M <= 24 * a->G) return launch_gemm_kind<FMT, GK_SKINNY>(P, a, stream);
-        return launch_gemm_kind<FMT, GK_GENERAL>(P, a, stream);
+        return launch_gemm_kind<FMT, GK_BF16>(P, a, stream);
     }
 }
 

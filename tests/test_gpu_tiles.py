@@ -1,0 +1,52 @@
+"""GPU parity of tile routines at the sizes where they change: row counts on both sides of each row-block boundary, the
+shortest and uneven runs of their rings, against the CPU oracle with the tolerances of helpers.py (what two roundings to
+bf16 of sums in different order give)."""
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+import helpers as H
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+def _swiglu(case):
+    """[M, N/2] of the fused epilogue on the GPU, and what the oracle's accumulators give."""
+    import moe_gfx950 as mg
+
+    dev = H.upload(case)
+    M, K, N, G = case["M"], case["K"], case["N"], case["G"]
+    y = torch.full((M, N // 2), 0x7FC0, dtype=torch.int16, device="cuda")
+    p = lambda t: 0 if t is None else t.data_ptr()
+    mg.grouped_gemm(mg.grouped_args(mg.format_from_compute_type(case["fmt"]), p(dev["x"]), p(dev["weight"]), p(dev["scale"]),
+                                    p(dev["offset"]), p(dev["group_list"]), p(y), M, K, N, G, case["scale_rows"],
+                                    epilogue=mg.EPILOGUE_SWIGLU), torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    _, z = oracle.grouped_gemm(oracle.FMT_BY_NAME[case["fmt"]], case["x"], case["weight"], case["scale"], case["offset"],
+                               case["group_list"], want_f32=True)
+    want = oracle.swiglu_blocked16(z) if case["fmt"] in ("fp4_b32", "fp4_b16", "bf16") else oracle.swiglu_interleaved(z)
+    return y.cpu().numpy().view(np.uint16), want
+
+
+@pytest.mark.parametrize("epilogue", ["none", "swiglu"])
+@pytest.mark.parametrize("K", [64, 128, 192, 448])   # 1, 2, 3 and 7 pairs of steps
+def test_bf16_row_blocks(K, epilogue):
+    """gemm_tile_bf16: every number of 32-row blocks from 1 to 7, the row before and after each, two and three chunks."""
+    counts = [rows for b in (32, 64, 96, 128, 160, 192, 224) for rows in (b - 1, b, b + 1)] + [1, 16, 17, 449]
+    _say(f"bf16 row blocks K={K} epilogue={epilogue}")
+    case = H.make_case("bf16", len(counts), K, 256, np.cumsum(counts), seed=K, extra_rows=3)
+    used = int(case["group_list"][-1])
+    if epilogue == "swiglu":
+        got, want = _swiglu(case)
+    else:
+        got, want = H.run_cabi(case, H.upload(case), "gemm"), H.oracle_out(case)
+    H.assert_close(got, want, rows=slice(0, used), what=f"bf16 K={K} {epilogue}")
+    assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
