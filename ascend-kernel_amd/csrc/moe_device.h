@@ -77,4 +77,9 @@ __device__ __forceinline__ float wave_reduce_sum(float v) {
     return v;
 }
 
+// silu(g) * u on fp32 accumulators: g / (1 + exp(-g)) with the hardware exp and reciprocal.
+__device__ __forceinline__ float swiglu(float g, float u) {
+    return g * __builtin_amdgcn_rcpf(1.f + __expf(-g)) * u;
+}
+
 }  // namespace moe

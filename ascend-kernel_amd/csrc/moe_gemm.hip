@@ -142,11 +142,6 @@ __device__ __forceinline__ void mfma_16x16x32_v(f32x4_t& acc, const u32x4_t& a, 
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
 }
 
-// silu(g) * u on fp32 accumulators: g / (1 + exp(-g)) with the hardware exp and reciprocal.
-__device__ __forceinline__ float swiglu(float g, float u) {
-    return g * __builtin_amdgcn_rcpf(1.f + __expf(-g)) * u;
-}
-
 // ---------------------------------------------------------------------------------
 // x tile: rows x BK bf16 in LDS, 16-byte chunks, chunk c of row r stored at
 // position c ^ (r & 7) so that the 8 lanes a ds_read_b128 serves together hit
@@ -1587,6 +1582,7 @@ static int launch_gemm_fmt(const moe_grouped_args* a, hipStream_t stream) {
 
 int launch_gemm_exact(const moe_grouped_args* a, hipStream_t stream) {
     const GemmParams P = gemm_params(a);
+    if (stream_preferred(a)) return launch_stream(a, stream, false);
     switch (a->format) {
         case MOE_FMT_FP4_REF:
             // decode-like batches (on average at most 12 rows per expert): 16-row tiles, two workgroups per CU; an
@@ -1604,6 +1600,7 @@ int launch_grouped_gemm(const moe_grouped_args* a, hipStream_t stream) {
     // run with this op's arithmetic.
     // (the GEMV kernels have no fused activation: such calls stay on the GEMM kernels)
     if (a->epilogue == MOE_EPILOGUE_NONE && gemv_preferred(a)) return launch_grouped_gemv(a, stream, true);
+    if (stream_preferred(a)) return launch_stream(a, stream, true);
     switch (a->format) {
         case MOE_FMT_FP4_REF: return launch_gemm_fmt<MOE_FMT_FP4_REF>(a, stream);
         case MOE_FMT_FP8_REF: return launch_gemm_fmt<MOE_FMT_FP8_REF>(a, stream);

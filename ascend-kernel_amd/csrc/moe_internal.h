@@ -30,6 +30,9 @@ bool gemv_preferred(const moe_grouped_args* a);
 // op's arithmetic; MOE_ERR_TOO_LARGE when the expert count does not fit its LDS
 int launch_gemm_exact(const moe_grouped_args* a, hipStream_t stream);
 int launch_grouped_gemm(const moe_grouped_args* a, hipStream_t stream);
+// N-contiguous containers, launches too small to fill the chip with tiles that walk all of K (moe_stream.hip)
+bool stream_preferred(const moe_grouped_args* a);
+int launch_stream(const moe_grouped_args* a, hipStream_t stream, bool gemm_rounding);
 // moves the grouped GEMM's launch number (which picks a launch's tile counter and stamp) by delta; returns the new number
 int64_t gemm_shift_launch_number(int64_t delta);
 int launch_prepack_fp4_ref(const moe_prepack_fp4_args* a, hipStream_t stream);
