@@ -219,3 +219,27 @@ def test_route_rejects_bad_arguments():
     with pytest.raises(mg.MoeError) as e:
         mg.route(a)
     assert e.value.status == mg.ERR_NULL_POINTER       # no group_list
+
+
+@pytest.mark.parametrize("T,E,K,topk", [(16, 64, 64, 64), (16, 256, 64, 65), (17, 64, 64, 8), (128, 64, 64, 8), (1, 1024, 8, 1024),
+                                        (16, 1, 64, 1), (15, 65, 8200, 3), (3, 513, 64, 8)])
+def test_route_on_either_side_of_the_one_launch_path(T, E, K, topk):
+    """At most 16 tokens and 1024 choices are routed by one kernel; one block of choices needs no count kernel either."""
+    _say(f"route one launch T={T} E={E} K={K} topk={topk}")
+    rng = np.random.default_rng(T * E + topk)
+    logits = rng.standard_normal((T, E)).astype(np.float32)
+    x = oracle.f32_to_bf16_bits(rng.standard_normal((T, K)).astype(np.float32))
+    ids, w, gl, rt, roc, xs = _route(logits, None, x, T, E, K, topk)
+    ref_ids, ref_w = R.route_topk(logits, topk)
+    assert np.array_equal(ids, ref_ids)
+    assert np.allclose(w, ref_w, rtol=1e-5, atol=1e-9)
+    ref_gl, ref_rt, ref_roc = R.route_sort(ref_ids, E)
+    assert np.array_equal(gl, ref_gl) and np.array_equal(rt, ref_rt) and np.array_equal(roc, ref_roc)
+    assert np.array_equal(xs, x[ref_rt])
+    given = rng.integers(-2, E + 2, (T, topk)).astype(np.int32)     # ids of the caller's, some dropped
+    _, _, gl, rt, roc, xs = _route(None, given, x, T, E, K, topk)
+    ref_gl, ref_rt, ref_roc = R.route_sort(given, E)
+    total = int(ref_gl[-1])
+    assert np.array_equal(gl, ref_gl) and np.array_equal(roc, ref_roc)
+    assert np.array_equal(rt[:total], ref_rt) and (rt[total:] == -5).all()
+    assert np.array_equal(xs[:total], x[ref_rt]) and (xs[total:] == 0x7FC0).all()
