@@ -303,9 +303,10 @@ static __device__ __forceinline__ void stream_rows(const StreamParams& P, float*
 template <int FMT>
 constexpr int stream_line_cols(int T) { return FMT == MOE_FMT_INT4 ? 256 : FMT == MOE_FMT_FP4_REF && T < 8 ? 64 : 128; }
 
-// Grid: groups of strips over `ranks` experts with rows, dealt to the XCDs (workgroup b runs on XCD b mod 8).  Workgroup of
-// rank r takes the r-th expert that owns rows, the (r + ranks)-th and so on (ranks = min(M, G) covers them all at once); every
-// wavefront finds it by itself, 256 experts per look at group_list (64 per look: 4 dependent reads for G = 256).
+// Grid: groups of strips over `ranks` passes (16 rows of an expert), dealt to the XCDs (workgroup b runs on XCD b mod 8).
+// Workgroup of rank r takes the r-th pass, the (r + ranks)-th and so on (the host's `ranks` covers them all at once); every
+// wavefront finds it by itself, 256 experts per look at group_list (64 per look: 4 dependent reads for G = 256).  The passes of
+// an expert run side by side, not one after the other in one workgroup: 192 rows of one expert make 12 of them.
 template <int FMT, bool ROUNDW, int T>
 __global__ __launch_bounds__(64 * ST_WAVES, T == 8 ? 2 : 4) void stream_kernel(StreamParams P, int ranks) {
     extern __shared__ float red[];
@@ -315,7 +316,7 @@ __global__ __launch_bounds__(64 * ST_WAVES, T == 8 ? 2 : 4) void stream_kernel(S
     const int slot = blockIdx.x >> 3, group = (slot / S) * 8 + (blockIdx.x & 7), groups_n = P.N / LINE;
     if (group >= ranks * groups_n) return;
     const int n0 = (group % groups_n) * LINE + (slot % S) * ST_COLS;
-    // the rank-th expert that owns rows, and how many do
+    // expert and first row of the rank-th pass and the end of that expert's rows; how many passes there are
     int g = 0, r0 = 0, r1 = 0;
     auto find = [&](int rank) {
         constexpr int LOOK = 4;
@@ -332,12 +333,29 @@ __global__ __launch_bounds__(64 * ST_WAVES, T == 8 ? 2 : 4) void stream_kernel(S
 #pragma unroll
             for (int c = 0; c < LOOK; ++c) {
                 unsigned long long live = __ballot(hi[c] > lo[c]);
-                const int n = __popcll(live);
+                int n = __popcll(live), at = 0, pass = 0;
+                if (__ballot(hi[c] - lo[c] > ST_ROWS) == 0) {   // a pass each
+                    if (rank >= seen && rank < seen + n) {
+                        for (int k = rank - seen; k > 0; --k) live &= live - 1;
+                        at = __builtin_ctzll(live);
+                    }
+                } else {
+                    const int own = (max(hi[c] - lo[c], 0) + ST_ROWS - 1) / ST_ROWS;
+                    int incl = own;
+#pragma unroll
+                    for (int off = 1; off < 64; off <<= 1) {
+                        const int up = __shfl_up(incl, off, 64);
+                        if (lane >= off) incl += up;
+                    }
+                    n = __builtin_amdgcn_readlane(incl, 63);
+                    if (rank >= seen && rank < seen + n) {
+                        at = __builtin_ctzll(__ballot(incl > rank - seen));
+                        pass = rank - seen - __builtin_amdgcn_readlane(incl - own, at);
+                    }
+                }
                 if (rank >= seen && rank < seen + n) {
-                    for (int k = rank - seen; k > 0; --k) live &= live - 1;
-                    const int at = __builtin_ctzll(live);
                     g = g0 + 64 * c + at;
-                    r0 = __builtin_amdgcn_readlane(lo[c], at);
+                    r0 = __builtin_amdgcn_readlane(lo[c], at) + pass * ST_ROWS;
                     r1 = __builtin_amdgcn_readlane(hi[c], at);
                 }
                 seen += n;
@@ -346,20 +364,20 @@ __global__ __launch_bounds__(64 * ST_WAVES, T == 8 ? 2 : 4) void stream_kernel(S
         return __builtin_amdgcn_readfirstlane(seen);
     };
     int rank = group / groups_n;
-    const int live_experts = find(rank);
-    while (rank < live_experts) {
-        for (int row = r0; row < r1; row += ST_ROWS) {
-            const int mg = min(ST_ROWS, r1 - row);
-            if constexpr (FMT == MOE_FMT_FP4_REF && !ROUNDW) {
-                if (mg <= 8) stream_rows<FMT, ROUNDW, T, true>(P, red, g, row, mg, n0);
-                else stream_rows<FMT, ROUNDW, T, false>(P, red, g, row, mg, n0);
-            } else {
-                stream_rows<FMT, ROUNDW, T, false>(P, red, g, row, mg, n0);
-            }
-            __syncthreads();   // the partial sums are read
+    const int passes = find(rank);
+    while (rank < passes) {
+        const int mg = min(ST_ROWS, r1 - r0);
+        if constexpr (FMT == MOE_FMT_FP4_REF && !ROUNDW) {
+            if (mg <= 8) stream_rows<FMT, ROUNDW, T, true>(P, red, g, r0, mg, n0);
+            else stream_rows<FMT, ROUNDW, T, false>(P, red, g, r0, mg, n0);
+        } else {
+            stream_rows<FMT, ROUNDW, T, false>(P, red, g, r0, mg, n0);
         }
         rank += ranks;
-        if (rank < live_experts) find(rank);
+        if (rank < passes) {
+            __syncthreads();   // the partial sums are read
+            find(rank);
+        }
     }
 }
 
@@ -382,7 +400,8 @@ static int launch_stream_kind(const moe_grouped_args* a, hipStream_t stream) {
     static std::atomic<uint64_t> lds_set{0};
     if (const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&stream_kernel<FMT, ROUNDW, T>), ST_WAVES * ST_ROWS * ST_COLS * (int)sizeof(float), lds_set))
         return rc;
-    const int64_t ranks = min(a->M, a->G), groups = ranks * (a->N / stream_line_cols<FMT>(T));
+    // passes of 16 rows, at most: M rows over min(M, G) experts
+    const int64_t ranks = (a->M + (ST_ROWS - 1) * min(a->M, a->G)) / ST_ROWS, groups = ranks * (a->N / stream_line_cols<FMT>(T));
     const int64_t grid = (groups + 7) / 8 * 8 * (stream_line_cols<FMT>(T) / ST_COLS);
     hipLaunchKernelGGL((stream_kernel<FMT, ROUNDW, T>), dim3((unsigned)grid), dim3(64 * ST_WAVES), lds, stream, P, (int)ranks);
     return hipGetLastError() == hipSuccess ? MOE_OK : MOE_ERR_LAUNCH;
@@ -404,9 +423,10 @@ static int launch_stream_fmt(const moe_grouped_args* a, hipStream_t stream) {
 
 // Up to 128 tiles of 256 columns, i.e. half of the CUs, and decode-like batches: with 32768 columns (16 experts of
 // 7168 x 2048) int4 34 - 36 us here against 49 - 60 with moe_gemm.hip's tiles, fp4 33 / 50, fp8 49 / 72; with 49152 columns
-// those are ahead (int4 63 / 53, fp8 90 / 82), with 65536 by a factor of 1.3.  Every 16 rows of an expert are a pass over
-// its weights: with up to 16384 columns (8 experts of 4096 x 2048) two passes are still ahead.  The experts that own
-// rows are counted by looking through group_list, 256 at a time.
+// those are ahead (int4 63 / 53, fp8 90 / 82), with 65536 by a factor of 1.3.  With up to 16384 columns twice as many rows:
+// 192 rows unevenly owned by 8 experts of 4096 x 2048, tiles / here: int4 65 / 25 us, fp4 58 / 21, fp8 49 / 28, int8 44 / 25;
+// all 192 owned by one expert: int4 66 / 22, int8 45 / 21.  The passes are found by looking through group_list, 256 experts
+// at a time.
 bool stream_preferred(const moe_grouped_args* a) {
     if (a->format != MOE_FMT_FP4_REF && a->format != MOE_FMT_FP8_REF && a->format != MOE_FMT_INT4 && a->format != MOE_FMT_INT8) return false;
     const int64_t columns = stream_columns(a);

@@ -47,3 +47,18 @@ def test_finds_the_experts_that_own_rows(G, owners):
     _say(f"strips experts G={G}")
     H.assert_close(H.run_cabi(case, H.upload(case), "gemv"), H.oracle_out(case, gemv=True), what=f"G={G}")
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("fmt", ["fp4", "int4"])
+def test_passes_of_unevenly_owned_rows(fmt):
+    """Experts of many passes between experts of one and of none, on both sides of a wavefront's 64 experts."""
+    counts = np.zeros(300, dtype=np.int64)
+    counts[[0, 2, 3, 63, 64, 256, 299]] = [33, 1, 16, 17, 38, 1, 20]
+    case = H.make_case(fmt, len(counts), 256, 256, np.cumsum(counts), seed=5, extra_rows=1)
+    used = int(case["group_list"][-1])
+    assert len(case["x"]) * 256 <= 32768   # few enough columns for the kernel
+    for op in ("gemm", "gemv"):
+        _say(f"strips passes {fmt} {op}")
+        got = H.run_cabi(case, H.upload(case), op)
+        H.assert_close(got, H.oracle_out(case, gemv=op == "gemv"), rows=slice(0, used), what=f"{op} {fmt}")
+        assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
