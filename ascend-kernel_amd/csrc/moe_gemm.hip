@@ -1550,9 +1550,6 @@ static GemmParams gemm_params(const moe_grouped_args* a) {
 template <int FMT>
 static int launch_gemm_fmt(const moe_grouped_args* a, hipStream_t stream) {
     const GemmParams P = gemm_params(a);
-    // The N-contiguous containers run on the k-split kernel at every batch size: measured faster than the
-    // small-tile kernel down to decode batches of 1-2 rows per expert (256 experts of 7168 x 2048: int4
-    // 243 vs 344 us at 128 rows, fp4 476 vs 519 us and fp8 610 vs 784 us at 512 rows).
     if constexpr (FMT != MOE_FMT_BF16) {
         // decode-like batches (on average at most 12 rows per expert) on the 4-bit N-contiguous containers: the
         // small-stage kind (at 8 rows per expert int4 409 vs 506 us, fp4 448 vs 474 us; at 24 the large tiles win,
@@ -1597,9 +1594,8 @@ int launch_gemm_exact(const moe_grouped_args* a, hipStream_t stream) {
 
 int launch_grouped_gemm(const moe_grouped_args* a, hipStream_t stream) {
     // Decode-sized batches on the K-contiguous containers go to the weight-streaming GEMV kernels,
-    // run with this op's arithmetic.
-    // (the GEMV kernels have no fused activation: such calls stay on the GEMM kernels)
-    if (a->epilogue == MOE_EPILOGUE_NONE && gemv_preferred(a)) return launch_grouped_gemv(a, stream, true);
+    // run with this op's arithmetic and epilogue.
+    if (gemv_preferred(a)) return launch_grouped_gemv(a, stream, true);
     if (stream_preferred(a)) return launch_stream(a, stream, true);
     switch (a->format) {
         case MOE_FMT_FP4_REF: return launch_gemm_fmt<MOE_FMT_FP4_REF>(a, stream);

@@ -78,7 +78,7 @@ __device__ __forceinline__ int xs_unit(int k8) {
 template <int FMT, int MG>
 __device__ __forceinline__ void gemv_kmajor_rows(const uint8_t* __restrict__ wg, const uint16_t* __restrict__ sg,
                                                  const uint16_t* __restrict__ x, uint16_t* __restrict__ y,
-                                                 u32x4_t* xs, int64_t row0, int n0, int N, int K) {
+                                                 u32x4_t* xs, float* sums, int64_t row0, int n0, int N, int K, int epilogue) {
     constexpr int CH = KMajor<FMT>::CH;
     constexpr int U = CH / 8;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -165,6 +165,27 @@ __device__ __forceinline__ void gemv_kmajor_rows(const uint8_t* __restrict__ wg,
                 }
             }
         }
+        if constexpr (FMT == MOE_FMT_BF16) {
+            if (epilogue == MOE_EPILOGUE_SWIGLU) {
+                // the workgroup's 32 weight rows are 16 gate rows (wavefronts 0, 1) and the 16 up rows that belong to them;
+                // the sums meet in LDS (the barriers ahead of the next pass's x keep its sums from these)
+                static_assert(KMajor<FMT>::NR_WG == 4 * GVK_NRW, "one step of the workgroup's 4 wavefronts");
+#pragma unroll
+                for (int j = 0; j < GVK_NRW; ++j)
+#pragma unroll
+                    for (int r = 0; r < MG; ++r) {
+                        const float v = wave_reduce_sum(acc[j][r]);
+                        if (lane == 0) sums[r * 32 + wave * GVK_NRW + j] = v;
+                    }
+                __syncthreads();
+                if ((int)threadIdx.x < 16 * MG) {
+                    const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
+                    y[(row0 + r) * (int64_t)(N >> 1) + (n0 >> 1) + c] =
+                        (uint16_t)(pack_bf16_rne(swiglu(sums[r * 32 + c], sums[r * 32 + 16 + c]), 0.f) & 0xffffu);
+                }
+                continue;
+            }
+        }
 #pragma unroll
         for (int j = 0; j < GVK_NRW; ++j)
 #pragma unroll
@@ -180,8 +201,9 @@ __global__ __launch_bounds__(256) void gemv_kmajor_kernel(const uint16_t* __rest
                                                           const uint8_t* __restrict__ w,
                                                           const uint16_t* __restrict__ scale,
                                                           const int64_t* __restrict__ gl, uint16_t* __restrict__ y,
-                                                          int64_t M, int K, int N) {
+                                                          int64_t M, int K, int N, int epilogue) {
     extern __shared__ u32x4_t xs[];
+    __shared__ float sums[GV_ROWS * 32];
     const int g = blockIdx.y, n0 = blockIdx.x * KMajor<FMT>::NR_WG;
     int64_t start, end;
     group_rows(gl, g, M, start, end);
@@ -191,10 +213,10 @@ __global__ __launch_bounds__(256) void gemv_kmajor_kernel(const uint16_t* __rest
     for (int64_t row0 = start; row0 < end; row0 += GV_ROWS) {
         const int mg = (int)min((int64_t)GV_ROWS, end - row0);
         switch (mg) {
-            case 1: gemv_kmajor_rows<FMT, 1>(wg, sg, x, y, xs, row0, n0, N, K); break;
-            case 2: gemv_kmajor_rows<FMT, 2>(wg, sg, x, y, xs, row0, n0, N, K); break;
-            case 3: gemv_kmajor_rows<FMT, 3>(wg, sg, x, y, xs, row0, n0, N, K); break;
-            default: gemv_kmajor_rows<FMT, 4>(wg, sg, x, y, xs, row0, n0, N, K); break;
+            case 1: gemv_kmajor_rows<FMT, 1>(wg, sg, x, y, xs, sums, row0, n0, N, K, epilogue); break;
+            case 2: gemv_kmajor_rows<FMT, 2>(wg, sg, x, y, xs, sums, row0, n0, N, K, epilogue); break;
+            case 3: gemv_kmajor_rows<FMT, 3>(wg, sg, x, y, xs, sums, row0, n0, N, K, epilogue); break;
+            default: gemv_kmajor_rows<FMT, 4>(wg, sg, x, y, xs, sums, row0, n0, N, K, epilogue); break;
         }
     }
 }
@@ -259,7 +281,7 @@ __device__ __forceinline__ uint32_t e2m1_pair_bf16(uint32_t word, int sel) {
 template <int MB, bool ROUNDW, int BLK>
 __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ wg, const uint16_t* __restrict__ sg,
                                                    const uint16_t* __restrict__ x, uint16_t* __restrict__ y,
-                                                   u32x4_t* xs, int64_t row0, int mg, int n0, int N, int K) {
+                                                   u32x4_t* xs, int64_t row0, int mg, int n0, int N, int K, int epilogue) {
     constexpr int KC = GF_LDS_UNITS / MB * 8 / GF_KSTEP * GF_KSTEP;   // k per staged chunk: 7168, 3584 or 1536
     constexpr int RS = KC / 8;                  // row stride in 16-byte units
     constexpr int U = GF_U;
@@ -468,6 +490,25 @@ __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ w
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[r] += __shfl_xor(acc[r], 32);
     }
+    if constexpr (ROUNDW) {
+        if (epilogue == MOE_EPILOGUE_SWIGLU) {
+            // blocks of 32 weight rows are 16 gate rows (an even wavefront's) and their 16 up rows (the next wavefront's):
+            // the sums meet in the scale exchange area (the barriers ahead of the next x keep later scales from it)
+            ss[lane] = __builtin_bit_cast(u32x4_t, acc + acc2);
+            __syncthreads();
+            if (!(wave & 1)) {
+                const f32x4_t up = __builtin_bit_cast(f32x4_t, ss[GF_SCALE_UNITS + lane]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int m = 4 * q + r;
+                    if (m < mg && n < N)
+                        y[(row0 + m) * (int64_t)(N >> 1) + ((n0 + wave * 16) >> 1) + i] =
+                            (uint16_t)(pack_bf16_rne(swiglu(acc[r] + acc2[r], up[r]), 0.f) & 0xffffu);
+                }
+            }
+            return;
+        }
+    }
     // lane (i, q) holds column n, rows 4 q .. 4 q + 3
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -482,7 +523,7 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemv_fp4_mfma_kernel(const u
                                                                          const uint16_t* __restrict__ scale,
                                                                          const int64_t* __restrict__ gl,
                                                                          uint16_t* __restrict__ y, int64_t M, int K,
-                                                                         int N) {
+                                                                         int N, int epilogue) {
     extern __shared__ u32x4_t xs[];
     const int g = blockIdx.y, n0 = blockIdx.x * GF_NR_WG;
     int64_t start, end;
@@ -492,9 +533,9 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemv_fp4_mfma_kernel(const u
     const uint16_t* sg = scale + (int64_t)g * N * (K / BLK);
     for (int64_t row0 = start; row0 < end; row0 += GF_ROWS) {
         const int mg = (int)min((int64_t)GF_ROWS, end - row0);
-        if (mg <= 4) gemv_fp4_mfma_rows<4, ROUNDW, BLK>(wg, sg, x, y, xs, row0, mg, n0, N, K);
-        else if (mg <= 8) gemv_fp4_mfma_rows<8, ROUNDW, BLK>(wg, sg, x, y, xs, row0, mg, n0, N, K);
-        else gemv_fp4_mfma_rows<16, ROUNDW, BLK>(wg, sg, x, y, xs, row0, mg, n0, N, K);
+        if (mg <= 4) gemv_fp4_mfma_rows<4, ROUNDW, BLK>(wg, sg, x, y, xs, row0, mg, n0, N, K, epilogue);
+        else if (mg <= 8) gemv_fp4_mfma_rows<8, ROUNDW, BLK>(wg, sg, x, y, xs, row0, mg, n0, N, K, epilogue);
+        else gemv_fp4_mfma_rows<16, ROUNDW, BLK>(wg, sg, x, y, xs, row0, mg, n0, N, K, epilogue);
     }
 }
 
@@ -507,39 +548,40 @@ static int launch_fp4_mfma(const moe_grouped_args* a, hipStream_t stream) {
     hipLaunchKernelGGL((gemv_fp4_mfma_kernel<ROUNDW, BLK>), grid, dim3(64 * GF_WAVES), lds, stream,
                        static_cast<const uint16_t*>(a->x), static_cast<const uint8_t*>(a->weight),
                        static_cast<const uint16_t*>(a->scale), a->group_list, static_cast<uint16_t*>(a->y), a->M,
-                       (int)a->K, (int)a->N);
+                       (int)a->K, (int)a->N, (int)a->epilogue);
     return hipGetLastError() == hipSuccess ? MOE_OK : MOE_ERR_LAUNCH;
 }
 
 template <int FMT>
 static int launch_kmajor(const moe_grouped_args* a, hipStream_t stream) {
-    const int kc = (int)(a->K < GV_KC ? a->K : GV_KC);
     const size_t lds = (size_t)GV_ROWS * GV_KC / 8 * 16;
-    (void)kc;
     dim3 grid((unsigned)((a->N + KMajor<FMT>::NR_WG - 1) / KMajor<FMT>::NR_WG), (unsigned)a->G);
     hipLaunchKernelGGL((gemv_kmajor_kernel<FMT>), grid, dim3(256), lds, stream,
                        static_cast<const uint16_t*>(a->x), static_cast<const uint8_t*>(a->weight),
                        static_cast<const uint16_t*>(a->scale), a->group_list, static_cast<uint16_t*>(a->y), a->M,
-                       (int)a->K, (int)a->N);
+                       (int)a->K, (int)a->N, (int)a->epilogue);
     return hipGetLastError() == hipSuccess ? MOE_OK : MOE_ERR_LAUNCH;
 }
 
 bool gemv_preferred(const moe_grouped_args* a) {
     // Decode-sized batches on the K-contiguous containers are pure weight streaming: these kernels
-    // read every weight row as contiguous runs.  The bf16 vector kernel takes 4 rows of an expert per
-    // pass over its weights (same arithmetic as the GEMM: the weights are bf16 already).  The
-    // matrix-core fp4_b32 kernel takes 16 and has a variant with the GEMM's weight rounding; the
-    // bound is where the k-split GEMM kernel overtakes it (measured at DeepSeek-V3 shapes, 256 experts of
-    // 7168 x 2048: 8 rows per expert 496 vs 631 us, 16 rows 754 vs 651 us).
+    // read every weight row as contiguous runs.  The matrix-core fp4 kernel takes 16 rows of an expert per pass and has a
+    // variant with the GEMM's weight rounding; the bound is where the k-split GEMM kernel overtakes it (measured at
+    // DeepSeek-V3 shapes, 256 experts of 7168 x 2048: 8 rows per expert 496 vs 631 us, 16 rows 754 vs 651 us).  With the
+    // SwiGLU epilogue, fp4_b32: 16 tokens x 8 on 256 experts of 7168 x 4096 306 vs 468 us, 8 rows of 8 experts of
+    // 4096 x 1024 17 vs 36, 8 rows per expert on 256 of 2048 x 1024 95 vs 99; 12 per expert on 8 of 4096 x 2048 39 vs 37.
     if (a->format == MOE_FMT_FP4_B32 || a->format == MOE_FMT_FP4_B16)
-        return a->K % GF_KSTEP == 0 && a->M <= GF_GEMM_ROWS_PER_EXPERT * a->G;
+        return a->K % GF_KSTEP == 0 && a->M <= (a->epilogue == MOE_EPILOGUE_SWIGLU ? 8 : GF_GEMM_ROWS_PER_EXPERT) * a->G;
+    // The bf16 vector kernel takes 4 rows of an expert per pass over its weights (same arithmetic as the GEMM: the weights
+    // are bf16 already).
     if (a->format == MOE_FMT_BF16) return a->M <= 4 * a->G;
     return false;
 }
 
 int launch_grouped_gemv(const moe_grouped_args* a, hipStream_t stream, bool gemm_rounding) {
     switch (a->format) {
-        case MOE_FMT_BF16: return launch_kmajor<MOE_FMT_BF16>(a, stream);
+        case MOE_FMT_BF16:
+            return launch_kmajor<MOE_FMT_BF16>(a, stream);
         case MOE_FMT_FP4_B32:
             // the matrix-core kernel takes K in whole loop iterations
             if (a->K % GF_KSTEP != 0) return gemm_rounding ? MOE_ERR_BAD_SHAPE : launch_kmajor<MOE_FMT_FP4_B32>(a, stream);

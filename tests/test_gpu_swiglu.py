@@ -59,8 +59,8 @@ def test_swiglu_epilogue(fmt, gl):
 @pytest.mark.parametrize("gl", [[2, 3, 4, 40], [130, 130, 143, 300, 301], [0, 7, 7, 8], [0, 200, 200, 200]],
                          ids=["small", "prefill", "decode", "one_big"])
 def test_swiglu_epilogue_k_contiguous(fmt, gl):
-    """K-contiguous containers: gate and up rows interleaved in blocks of 16 (the decode-sized batches stay on
-    the GEMM kernels: the weight-streaming GEMV kernels have no fused activation)."""
+    """K-contiguous containers: gate and up rows interleaved in blocks of 16 (the decode-sized batches run on
+    the weight-streaming GEMV kernels)."""
     _say(f"swiglu fmt={fmt} gl={gl}")
     case = H.make_case(fmt, len(gl), 512, 512, gl, seed=len(gl) * 11 + len(fmt), extra_rows=2)
     if fmt == "bf16":
@@ -125,3 +125,16 @@ def test_swiglu_via_module_and_rejections():
     with pytest.raises(mg.MoeError) as e:
         mg.grouped_gemv(a)
     assert e.value.status == mg.ERR_BAD_FORMAT
+
+
+@pytest.mark.parametrize("fmt", K_CONTIG)
+def test_swiglu_in_the_weight_streaming_kernels(fmt):
+    """Decode-sized batches: row counts on both sides of the kernels' passes (4 and 16 rows) and of their 4 / 8 / 16-row
+    variants, experts without rows, a K of more than one staged chunk of x."""
+    counts = [1, 0, 2, 3, 4, 5, 8, 9, 16, 17] + [0] * 7
+    _say(f"swiglu streaming fmt={fmt}")
+    case = H.make_case(fmt, len(counts), 2048, 256, np.cumsum(counts), seed=len(fmt), extra_rows=1)
+    assert len(case["x"]) <= 4 * len(counts)   # the rule that sends bf16 there; fp4 takes three times as many
+    got, used = _run(case), sum(counts)
+    H.assert_close(got, _expected(case), rows=slice(0, used), what=f"swiglu streaming {fmt}")
+    assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
