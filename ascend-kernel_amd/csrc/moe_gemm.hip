@@ -1577,6 +1577,8 @@ static int launch_gemm_fmt(const moe_grouped_args* a, hipStream_t stream) {
     }
 }
 
+int launch_gemm_bf16(const moe_grouped_args* a, hipStream_t stream) { return launch_gemm_fmt<MOE_FMT_BF16>(a, stream); }
+
 int launch_gemm_exact(const moe_grouped_args* a, hipStream_t stream) {
     const GemmParams P = gemm_params(a);
     if (stream_preferred(a)) return launch_stream(a, stream, false);

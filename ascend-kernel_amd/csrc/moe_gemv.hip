@@ -573,14 +573,22 @@ bool gemv_preferred(const moe_grouped_args* a) {
     if (a->format == MOE_FMT_FP4_B32 || a->format == MOE_FMT_FP4_B16)
         return a->K % GF_KSTEP == 0 && a->M <= (a->epilogue == MOE_EPILOGUE_SWIGLU ? 8 : GF_GEMM_ROWS_PER_EXPERT) * a->G;
     // The bf16 vector kernel takes 4 rows of an expert per pass over its weights (same arithmetic as the GEMM: the weights
-    // are bf16 already).
-    if (a->format == MOE_FMT_BF16) return a->M <= 4 * a->G;
+    // are bf16 already), the tile kernel up to 224, but only a workgroup per 256 columns.  4 rows per expert, here / there:
+    // 64 experts of 7168 x 2048 (512 tiles) 402 / 303 us, 16 of 7168 x 4096 (256) 208 / 162, 64 of 2048 x 1024 (256)
+    // 88 / 65, but 8 of 7168 x 4096 (128) 106 / 129, 8 of 7168 x 512 (16) 50 / 80; 2 rows, 512 tiles: 264 / 262.
+    if (a->format == MOE_FMT_BF16) return a->M <= (min(a->M, a->G) * a->N >= 65536 ? 2 : 4) * a->G;
     return false;
 }
 
 int launch_grouped_gemv(const moe_grouped_args* a, hipStream_t stream, bool gemm_rounding) {
     switch (a->format) {
         case MOE_FMT_BF16:
+            // more rows than the vector kernel is good for, in sizes that the tile kernel takes (see gemv_preferred): the
+            // two compute the same.  64 experts of 7168 x 2048: 16 rows per expert 1225 -> 331 us, 64 rows 4668 -> 405.  Few
+            // columns: 6 rows per expert 77 here / 81 us there on 8 experts of 7168 x 512, 8 rows 93 / 81; 6 rows on 8 of
+            // 4096 x 2048 79 / 71.
+            if (!gemv_preferred(a) && (a->N * a->G >= 16384 || a->M > 6 * a->G) && a->K % 64 == 0 && a->N % 256 == 0)
+                return launch_gemm_bf16(a, stream);
             return launch_kmajor<MOE_FMT_BF16>(a, stream);
         case MOE_FMT_FP4_B32:
             // the matrix-core kernel takes K in whole loop iterations

@@ -29,6 +29,8 @@ bool gemv_preferred(const moe_grouped_args* a);
 // grouped GEMV on the fp4 / int4 N-contiguous containers by the k-split GEMM kernel run with the GEMV
 // op's arithmetic; MOE_ERR_TOO_LARGE when the expert count does not fit its LDS
 int launch_gemm_exact(const moe_grouped_args* a, hipStream_t stream);
+// bf16 container on the tile kernel (K % 64 == 0, N % 256 == 0)
+int launch_gemm_bf16(const moe_grouped_args* a, hipStream_t stream);
 int launch_grouped_gemm(const moe_grouped_args* a, hipStream_t stream);
 // N-contiguous containers, launches too small to fill the chip with tiles that walk all of K (moe_stream.hip)
 bool stream_preferred(const moe_grouped_args* a);

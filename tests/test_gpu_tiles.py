@@ -50,3 +50,14 @@ def test_bf16_row_blocks(K, epilogue):
         got, want = H.run_cabi(case, H.upload(case), "gemm"), H.oracle_out(case)
     H.assert_close(got, want, rows=slice(0, used), what=f"bf16 K={K} {epilogue}")
     assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
+
+
+@pytest.mark.parametrize("K,N", [(192, 256), (160, 256), (128, 257), (128, 1024)])
+def test_bf16_gemv_of_many_rows(K, N):
+    """Sizes that the tile kernel takes over from the vector kernel, and those (K not a multiple of 64, a ragged N) that it does not."""
+    counts = [0, 7, 1, 33, 250, 0, 4]
+    case = H.make_case("bf16", len(counts), K, N, np.cumsum(counts), seed=K + N, extra_rows=2)
+    _say(f"bf16 gemv of many rows K={K} N={N}")
+    got, used = H.run_cabi(case, H.upload(case), "gemv"), sum(counts)
+    H.assert_close(got, H.oracle_out(case, gemv=True), rows=slice(0, used), what=f"bf16 gemv K={K} N={N}")
+    assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
