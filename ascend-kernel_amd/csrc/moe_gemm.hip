@@ -1079,6 +1079,12 @@ __device__ __forceinline__ void gemm_tile_bf16(const GemmParams& P, u32x4_t* sme
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wv >> 2, cw = wv & 3;
     const int np = P.K >> 6;
+    // Where in K a column tile starts (it goes round).  L2's 16 channels take 256 bytes in turn: with weight rows a multiple
+    // of 4 KB apart all rows of all tiles, which run nearly in step, would ask one channel at a time, so each column tile
+    // starts in the next one.  K = 2048, 256 experts of N = 1024, 8 rows each: 239 -> 201 us; 64 of N = 2048, 48 rows:
+    // 139 -> 122.  Other K gain nothing and lose the x rows that neighbouring tiles find in L2 (prefill, K = 7168: 481 -> 491).
+    const int rot = P.K % 2048 ? 0 : (int)((unsigned)(2 * (g * ((P.N + GM_BN - 1) / GM_BN) + n0 / GM_BN)) % (unsigned)np);
+    auto pair_at = [&](int p) { return p + rot < np ? p + rot : p + rot - np; };
     const int64_t KN = (int64_t)P.K * P.N;
     const int k2 = P.K * 2;
     const bool swi = P.epilogue == MOE_EPILOGUE_SWIGLU;
@@ -1117,9 +1123,9 @@ __device__ __forceinline__ void gemm_tile_bf16(const GemmParams& P, u32x4_t* sme
     for (int p = 0; p < WP - 1; ++p) {   // (in the order of the loop below: x a ring's depth ahead, then the weights)
         if (p >= WP - XP)
 #pragma unroll
-            for (int m = 0; m < 2 * NA; ++m) issue_x(m, p - (WP - XP), p - (WP - XP));
+            for (int m = 0; m < 2 * NA; ++m) issue_x(m, pair_at(p - (WP - XP)), p - (WP - XP));
 #pragma unroll
-        for (int m = 0; m < 2 * NB; ++m) issue_w(m, p, p);
+        for (int m = 0; m < 2 * NB; ++m) issue_w(m, pair_at(p), p);
     }
     f32x4_t acc[MT][4];
 #pragma unroll
@@ -1138,6 +1144,7 @@ __device__ __forceinline__ void gemm_tile_bf16(const GemmParams& P, u32x4_t* sme
     constexpr int NI = 2 * (NA + NB);
     constexpr int F = 2 * MT, R = 3 < F ? 3 : F;   // x fragments of a pair, read R ahead of their MFMAs
     for (int p = 0, xs = 0, ws = 0; p < np; ++p) {
+        const int px = pair_at(p + XP - 1), pw = pair_at(p + WP - 1);
         const int x_to = xs == 0 ? XP - 1 : xs - 1, w_to = ws == 0 ? WP - 1 : ws - 1;
         const u32x4_t* lx = xf + xs * (2 * AU);
         const u32x4_t* lw = wf + ws * (2 * BU);
@@ -1160,9 +1167,9 @@ __device__ __forceinline__ void gemm_tile_bf16(const GemmParams& P, u32x4_t* sme
 #pragma unroll
             for (int m = (f * NI + MT - 1) / MT; f < MT && m < ((f + 1) * NI + MT - 1) / MT; ++m) {
                 if (m < 2 * NA)
-                    issue_x(m, p + XP - 1, x_to);
+                    issue_x(m, px, x_to);
                 else
-                    issue_w(m - 2 * NA, p + WP - 1, w_to);
+                    issue_w(m - 2 * NA, pw, w_to);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -1171,7 +1178,7 @@ __device__ __forceinline__ void gemm_tile_bf16(const GemmParams& P, u32x4_t* sme
         xs = xs == XP - 1 ? 0 : xs + 1;
         ws = ws == WP - 1 ? 0 : ws + 1;
     }
-    // the last loads are for pairs past K and never read; wait out the last MFMAs' latency
+    // the last loads are for pairs behind the last one and never read; wait out the last MFMAs' latency
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15\n\ts_barrier" ::: "memory");
     pair_finish<MT, false, true>(P, smem, acc, 0, cw, lane, 64 * cw + 4 * i, row0 + 16 * MT * wr, max(rows - 16 * MT * wr, 0), n0, tk);
 }
