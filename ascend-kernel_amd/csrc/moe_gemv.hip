@@ -10,7 +10,9 @@
 //                         needs (1 + rows) / 2 instructions per 4-bit weight, more than the chip can issue while HBM
 //                         delivers the codes at full rate), wave-private streaming, no workgroup barrier in the k loop
 // The N-contiguous containers (reference fp4 / fp8, int4) run on the k-split matrix-core kernel of moe_gemm.hip with
-// this op's arithmetic (launch_gemm_exact): measured 3 times faster than a vector kernel on that layout.
+// this op's arithmetic (launch_gemm_exact): measured 3 times faster than a vector kernel on that layout.  bf16 calls with
+// more rows per expert than the vector kernel is good for go to that file's tiles too.  Both kernels also have the GEMM op's
+// SwiGLU epilogue, for its decode-sized calls.
 //
 // Numerics (gemv_impl.h:147-199): weights are decode * scale in fp32, NOT rounded
 // to bf16; fp32 accumulation; one RNE to bf16 at the end (grouped_soft_gemv.h:218-233).
