@@ -32,6 +32,7 @@
 
 #include "moe_device.h"
 #include "moe_internal.h"
+#include "scale_group.h"
 
 namespace moe {
 
@@ -53,9 +54,8 @@ struct GemmParams {
     // first tiles only (the row bounds are read from group_list per tile); 0 neither fits: the first tile of every
     // thread's run of experts only, and a tile is found by walking its run (any number of experts)
     int table_mode;
-    // N-contiguous 4-bit containers: the multiplier that turns a 32-k sub-step index into its scale row, i.e.
-    // divides by the sub-steps per scale group (0: identity)
-    uint32_t sub_to_group;
+    // N-contiguous 4-bit containers: turns a 32-k sub-step index into its scale row
+    ScaleRowDivider scale_div;
 };
 
 // Work queue of the persistent grid.  Workgroups do not run at one speed (of two that share a CU the one
@@ -469,9 +469,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     const rsrc_t rs8 = make_rsrc(static_cast<const float*>(P.scale) + (int64_t)g * (P.K >> 7) * (P.N >> 7),
                                  (int64_t)(P.K >> 7) * (P.N >> 7) * 4);
     const int cs8 = ((n0 + 64 * cw) >> 7) * 4;
-    // sub-step -> scale row as a multiply (worked out on the host from the 32-k sub-steps per scale group)
-    const uint32_t gmul = (B8 || KC) ? 0u : P.sub_to_group;
-    auto scale_row = [&](uint32_t sub) { return gmul ? (int)__umulhi(sub, gmul) : (int)sub; };
+    auto scale_row = [&](uint32_t sub) { return (int)moe::scale_row(P.scale_div, sub); };
     // x rows through a buffer resource that ends after the last valid row (padded rows read as
     // zeros).  Load instruction j covers rows 8j + (lane >> 3); position lane & 7 of a row
     // holds chunk (lane & 7) ^ (row & 7), the swizzle a_lds_unit expects.
@@ -1549,8 +1547,7 @@ static GemmParams gemm_params(const moe_grouped_args* a) {
     P.slot = -1;
     P.stamp = 0;
     P.table_mode = 0;
-    const uint32_t per = a->scale_rows > 0 ? (uint32_t)((a->K / a->scale_rows) >> 5) : 1u;
-    P.sub_to_group = per <= 1 ? 0u : 0xffffffffu / per + 1u;
+    P.scale_div = scale_row_divider(a->K, a->scale_rows);
     return P;
 }
 

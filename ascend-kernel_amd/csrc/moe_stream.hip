@@ -21,6 +21,7 @@
 
 #include "moe_device.h"
 #include "moe_internal.h"
+#include "scale_group.h"
 
 namespace moe {
 
@@ -37,7 +38,7 @@ struct StreamParams {
     int64_t M;
     int K, N, G, scale_rows;
     int epilogue;
-    uint32_t sub_to_group;   // int4: scale row of a 32-k step s = high 32 bits of 2 s * this
+    ScaleRowDivider scale_div;   // int4: the scale row of a 32-k step
 };
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
@@ -130,7 +131,7 @@ static __device__ __forceinline__ void stream_rows(const StreamParams& P, float*
                 }
             }
             if constexpr (I4)
-                load_scales(d.s, (int)__umulhi(2u * (uint32_t)s, P.sub_to_group) * (P.N * 2));
+                load_scales(d.s, (int)scale_row(P.scale_div, (uint32_t)s) * (P.N * 2));
             if constexpr (F8) d.s[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, 0, ((s >> 2) * (P.N >> 7) + (n0 >> 7)) * 4, 0);
         }
     };
@@ -393,8 +394,7 @@ static int launch_stream_kind(const moe_grouped_args* a, hipStream_t stream) {
     P.y = static_cast<uint16_t*>(a->y);
     P.M = a->M; P.K = (int)a->K; P.N = (int)a->N; P.G = (int)a->G; P.scale_rows = (int)a->scale_rows;
     P.epilogue = a->epilogue;
-    const uint32_t per = max((uint32_t)((a->K / max(a->scale_rows, (int64_t)1)) >> 5), 1u);   // 32-k steps per scale row
-    P.sub_to_group = (0x80000000u + per - 1) / per;   // 2^31 / per, rounded up: exact for every step of a K below 2^31
+    P.scale_div = scale_row_divider(a->K, a->scale_rows);
     const int rows = (int)min(a->M, (int64_t)ST_ROWS);
     const size_t lds = (size_t)ST_WAVES * ((rows + 3) & ~3) * ST_COLS * sizeof(float);
     static std::atomic<uint64_t> lds_set{0};
