@@ -52,6 +52,25 @@ def test_bf16_row_blocks(K, epilogue):
     assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
 
 
+@pytest.mark.parametrize("epilogue", ["none", "swiglu"])
+@pytest.mark.parametrize("K", [2048, 4096])
+def test_bf16_starts_all_over_k(K, epilogue):
+    """With K a multiple of 2048 a column tile starts at a k pair of its own and goes round: one expert per start, from the
+    first pair to the last two, tiles of one to three row blocks, experts without rows."""
+    pairs = K // 64
+    counts = [(33, 7, 0, 64, 1, 70)[g % 6] for g in range(pairs // 2 + 1)]
+    _say(f"bf16 starts K={K} epilogue={epilogue}")
+    case = H.make_case("bf16", len(counts), K, 256, np.cumsum(counts), seed=K, extra_rows=3)
+    assert H.kernel_of(case, "gemm", swiglu=epilogue == "swiglu") == "tiles_bf16"
+    used = int(case["group_list"][-1])
+    if epilogue == "swiglu":
+        got, want = _swiglu(case)
+    else:
+        got, want = H.run_cabi(case, H.upload(case), "gemm"), H.oracle_out(case)
+    H.assert_close(got, want, rows=slice(0, used), what=f"bf16 starts K={K} {epilogue}")
+    assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
+
+
 @pytest.mark.parametrize("K,N", [(192, 256), (160, 256), (128, 257), (128, 1024)])
 def test_bf16_gemv_of_many_rows(K, N):
     """Sizes that the tile kernel takes over from the vector kernel, and those (K not a multiple of 64, a ragged N) that it does not."""
