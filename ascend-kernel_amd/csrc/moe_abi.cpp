@@ -214,14 +214,19 @@ int moe_grouped_gemm(const moe_grouped_args* a, moe_stream_t stream) {
     int rc = moe_grouped_gemm_validate(a);
     if (rc != MOE_OK) return rc;
     if (a->M == 0) return MOE_OK;
-    return moe::launch_grouped_gemm(a, static_cast<hipStream_t>(stream));
+    return moe::launch_grouped(a, false, static_cast<hipStream_t>(stream));
 }
 
 int moe_grouped_gemv(const moe_grouped_args* a, moe_stream_t stream) {
     int rc = moe_grouped_gemv_validate(a);
     if (rc != MOE_OK) return rc;
     if (a->M == 0) return MOE_OK;
-    return moe::launch_grouped_gemv(a, static_cast<hipStream_t>(stream));
+    return moe::launch_grouped(a, true, static_cast<hipStream_t>(stream));
+}
+
+const char* moe_test_grouped_kernel(const moe_grouped_args* a, int gemv_op) {
+    if ((gemv_op ? moe_grouped_gemv_validate(a) : moe_grouped_gemm_validate(a)) != MOE_OK) return nullptr;
+    return moe::grouped_kernel_name(moe::grouped_kernel(a, gemv_op != 0));
 }
 
 int64_t moe_test_shift_launch_number(int64_t delta) { return moe::gemm_shift_launch_number(delta); }

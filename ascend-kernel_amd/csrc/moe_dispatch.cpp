@@ -1,0 +1,115 @@
+// Which kernel a grouped call gets, from its sizes alone (group_list stays on the device).  Every rule with what it was
+// measured on; the launchers and the tests ask grouped_kernel.
+#include <algorithm>
+
+#include "moe_internal.h"
+
+namespace moe {
+
+// Columns the launch streams, at most: min(M, G) experts own rows
+static int64_t columns(const moe_grouped_args* a) { return std::min(a->M, a->G) * a->N; }
+
+// bf16 [N, K].  The vector kernel takes 4 rows of an expert per pass over its weights, the tile kernel up to 224, but only a
+// workgroup per 256 columns (the two compute the same).  4 rows per expert, vector / tiles:
+// 64 experts of 7168 x 2048 (512 tiles) 402 / 303 us, 16 of 7168 x 4096 (256) 208 / 162, 64 of 2048 x 1024 (256)
+// 88 / 65, but 8 of 7168 x 4096 (128) 106 / 129, 8 of 7168 x 512 (16) 50 / 80; 2 rows, 512 tiles: 264 / 262.
+static bool bf16_vector_preferred(const moe_grouped_args* a) { return a->M <= (columns(a) >= 65536 ? 2 : 4) * a->G; }
+
+static GroupedKernel bf16_kernel(const moe_grouped_args* a, bool gemv_op) {
+    if (bf16_vector_preferred(a)) return GroupedKernel::VECTOR;
+    if (!gemv_op) return GroupedKernel::TILES_BF16;
+    // The GEMV op takes sizes that the tiles do not, and with few columns the vector kernel stays ahead a little longer.
+    // 64 experts of 7168 x 2048: 16 rows per expert 1225 -> 331 us on the tiles, 64 rows 4668 -> 405.  Few
+    // columns: 6 rows per expert 77 / 81 us on 8 experts of 7168 x 512, 8 rows 93 / 81; 6 rows on 8 of 4096 x 2048 79 / 71.
+    const bool fits = a->K % 64 == 0 && a->N % 256 == 0;
+    return fits && (a->N * a->G >= 16384 || a->M > 6 * a->G) ? GroupedKernel::TILES_BF16 : GroupedKernel::VECTOR;
+}
+
+// fp4 [N, K/2].  The matrix-core GEMV kernel reads every weight row as contiguous runs, takes 16 rows of an expert per pass and
+// has a variant with the GEMM's weight rounding; the bound for the GEMM op is where the k-split tiles overtake it (256 experts
+// of 7168 x 2048: 8 rows per expert 496 vs 631 us, 16 rows 754 vs 651 us).  With the
+// SwiGLU epilogue, fp4_b32: 16 tokens x 8 on 256 experts of 7168 x 4096 306 vs 468 us, 8 rows of 8 experts of
+// 4096 x 1024 17 vs 36, 8 rows per expert on 256 of 2048 x 1024 95 vs 99; 12 per expert on 8 of 4096 x 2048 39 vs 37.
+static GroupedKernel fp4_kcontiguous_kernel(const moe_grouped_args* a, bool gemv_op) {
+    const bool whole = a->K % FP4_ROWS_K == 0;
+    if (gemv_op) return whole ? GroupedKernel::FP4_ROWS : GroupedKernel::VECTOR;
+    return whole && a->M <= (a->epilogue == MOE_EPILOGUE_SWIGLU ? 8 : 12) * a->G ? GroupedKernel::FP4_ROWS : GroupedKernel::TILES_PAIR;
+}
+
+// Strips for launches of up to 128 tiles of 256 columns, i.e. half of the CUs, and decode-like batches: with 32768 columns (16
+// experts of 7168 x 2048) int4 34 - 36 us in strips against 49 - 60 in tiles, fp4 33 / 50, fp8 49 / 72; with 49152 columns
+// tiles are ahead (int4 63 / 53, fp8 90 / 82), with 65536 by a factor of 1.3.  With up to 16384 columns twice as many rows:
+// 192 rows unevenly owned by 8 experts of 4096 x 2048, tiles / strips: int4 65 / 25 us, fp4 58 / 21, fp8 49 / 28, int8 44 / 25;
+// all 192 owned by one expert: int4 66 / 22, int8 45 / 21.  The passes are found by looking through group_list, 256 experts
+// at a time.
+static bool strips_preferred(const moe_grouped_args* a) {
+    return a->G <= 1024 && columns(a) <= 32768 && a->M <= (columns(a) <= 16384 ? 24 : 12) * a->G;
+}
+
+// The narrowest strips whose first passes leave every CU at most one workgroup (an expert with more rows than one pass takes
+// has a workgroup per pass and strip, so there may be more).  Measured, 8 experts of K = 7168, 32 / 64 / 128 columns
+// a strip: N = 512 (4096 columns in all) int4 15 / 18 / 27 us, fp8 16 / 21 / 34; N = 2048 (16384) int4 28 / 20 / 28, fp8
+// 46 / 32 / 39; 16 experts of N = 2048 (32768) int4 75 / 49 / 34, fp8 89 / 60 / 49.
+static GroupedKernel strip_width(const moe_grouped_args* a) {
+    return columns(a) <= 8192 ? GroupedKernel::STRIPS_32 : columns(a) <= 16384 ? GroupedKernel::STRIPS_64 : GroupedKernel::STRIPS_128;
+}
+
+static GroupedKernel n_contiguous_kernel(const moe_grouped_args* a, bool gemv_op) {
+    if (strips_preferred(a)) return strip_width(a);
+    // decode-like batches (on average at most 12 rows per expert) on the 4-bit containers: the small-stage kind (at 8 rows per
+    // expert int4 409 vs 506 us, fp4 448 vs 474 us; at 24 the large tiles win, 531 vs 549 us and 512 vs 609 us).  The
+    // one-byte containers gain nothing from it.  GEMV op, fp4: 16-row tiles, two workgroups per CU; an expert with more rows
+    // than that costs a pass over its weights per 16 rows.
+    const bool decode = a->M <= 12 * a->G;
+    if (gemv_op) return decode && a->format == MOE_FMT_FP4_REF ? GroupedKernel::TILES_PAIR_EXACT16 : GroupedKernel::TILES_PAIR_EXACT;
+    const bool four_bit = a->format == MOE_FMT_INT4 || a->format == MOE_FMT_FP4_REF;
+    if (four_bit && decode) return GroupedKernel::TILES_PAIR_SMALL;
+    // prefill: workgroups of 4 wavefronts without the k split, two per CU.  The 4-bit
+    // ones always (256 experts of 128 rows, K = 7168, N = 4096: int4 1792 against 1905 us, fp4 1724 against 1867 us
+    // with the k-split kind).  The one-byte ones, whose tiles move twice the bytes, when an expert has more rows than
+    // one tile takes on average, so that its row chunks share a weight slice in L2: 8 experts of 512 rows, K = 4096,
+    // N = 14336: int8 454 against 476 us, fp8 480 against 495 us; 64 experts of 512 rows at K = 7168, N = 4096: 1755
+    // against 1870 us and 1872 against 1929 us; but with 128 rows per expert, every weight tile read once from HBM,
+    // 1090 - 1110 against 1063 - 1098 us (int8) and 1125 - 1152 against 1088 - 1136 us (fp8) on 128 experts
+    return four_bit || a->M > PAIR_ROWS * a->G ? GroupedKernel::TILES_QUAD : GroupedKernel::TILES_PAIR;
+}
+
+GroupedKernel grouped_kernel(const moe_grouped_args* a, bool gemv_op) {
+    switch (a->format) {
+        case MOE_FMT_BF16: return bf16_kernel(a, gemv_op);
+        case MOE_FMT_FP4_B32:
+        case MOE_FMT_FP4_B16: return fp4_kcontiguous_kernel(a, gemv_op);
+        default: return n_contiguous_kernel(a, gemv_op);
+    }
+}
+
+const char* grouped_kernel_name(GroupedKernel k) {
+    switch (k) {
+        case GroupedKernel::VECTOR: return "vector";
+        case GroupedKernel::FP4_ROWS: return "fp4_rows";
+        case GroupedKernel::STRIPS_32: return "strips_32";
+        case GroupedKernel::STRIPS_64: return "strips_64";
+        case GroupedKernel::STRIPS_128: return "strips_128";
+        case GroupedKernel::TILES_PAIR: return "tiles_pair";
+        case GroupedKernel::TILES_PAIR_EXACT: return "tiles_pair_exact";
+        case GroupedKernel::TILES_PAIR_SMALL: return "tiles_pair_small";
+        case GroupedKernel::TILES_PAIR_EXACT16: return "tiles_pair_exact16";
+        case GroupedKernel::TILES_QUAD: return "tiles_quad";
+        case GroupedKernel::TILES_BF16: return "tiles_bf16";
+    }
+    return nullptr;
+}
+
+int launch_grouped(const moe_grouped_args* a, bool gemv_op, hipStream_t stream) {
+    const GroupedKernel k = grouped_kernel(a, gemv_op);
+    switch (k) {
+        case GroupedKernel::VECTOR: return launch_vector(a, stream);
+        case GroupedKernel::FP4_ROWS: return launch_fp4_rows(a, !gemv_op, stream);
+        case GroupedKernel::STRIPS_32:
+        case GroupedKernel::STRIPS_64:
+        case GroupedKernel::STRIPS_128: return launch_strips(a, k, !gemv_op, stream);
+        default: return launch_tiles(a, k, stream);
+    }
+}
+
+}  // namespace moe

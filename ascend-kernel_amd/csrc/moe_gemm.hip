@@ -256,7 +256,7 @@ constexpr bool pair_exact(int kind) { return kind == GK_PAIR_EXACT || kind == GK
 constexpr int pair_waves(int kind) { return kind == GK_QUAD ? 4 : 8; }
 constexpr int pair_bk(int kind) { return kind == GK_QUAD ? 32 : 64; }   // k per step
 
-constexpr int PAIR_CAPB = 10;                         // x stages hold 160 rows
+constexpr int PAIR_CAPB = PAIR_ROWS / 16;             // x stages hold 160 rows
 constexpr int PAIR_MT_MAX = 10;
 constexpr int PAIR_SMALL_MT_MAX = 2;                  // row blocks per tile of the small-stage kinds
 constexpr bool pair_small(int kind) { return kind != GK_PAIR && kind != GK_QUAD; }
@@ -1063,7 +1063,10 @@ constexpr int bf_x_pairs(int mt) { return mt == 4 || mt == 5 ? 3 : 2; }
 constexpr int bf_w_pairs(int mt) { return mt > 3 ? 3 : 4; }
 constexpr int bf_lds_units() {
     int most = 0;
-    for (int mt = 1; mt <= BF_MT_MAX; ++mt) most = max(most, 2 * (bf_x_pairs(mt) * bf_a_units(mt) + bf_w_pairs(mt) * BF_B_UNITS));
+    for (int mt = 1; mt <= BF_MT_MAX; ++mt) {
+        const int units = 2 * (bf_x_pairs(mt) * bf_a_units(mt) + bf_w_pairs(mt) * BF_B_UNITS);
+        if (units > most) most = units;
+    }
     return most;
 }
 template <int MT>
@@ -1492,15 +1495,15 @@ static int device_cu_count() {
 template <int FMT, int KIND>
 static int launch_gemm_kind(const GemmParams& P, const moe_grouped_args* a, hipStream_t stream) {
     using C = KernelCfg<FMT, KIND>;
-    const size_t lds_max = (160 * 1024 - 512) / C::WG_PER_CU;
+    constexpr size_t lds_max = (160 * 1024 - 512) / C::WG_PER_CU;
     const size_t table = ((size_t)a->G + 1) * sizeof(int);
     // tile table, and the row bounds next to it where they fit; else the scheduler reads group_list per tile; else,
     // with more experts than LDS holds a table for, it keeps one entry per thread and walks group_list (see
     // GemmParams::table_mode)
-    const size_t units = (size_t)C::lds_units() * 16;
+    constexpr size_t units = (size_t)C::lds_units() * 16, thread_table = (size_t)(64 * C::WAVES + 1) * sizeof(int);
+    static_assert(units + thread_table <= lds_max, "any number of experts");
     const int table_mode = units + 2 * table <= lds_max ? 2 : units + table <= lds_max ? 1 : 0;
-    const size_t lds = units + (table_mode ? table_mode * table : (size_t)(64 * C::WAVES + 1) * sizeof(int));
-    if (lds > lds_max) return MOE_ERR_TOO_LARGE;
+    const size_t lds = units + (table_mode ? table_mode * table : thread_table);
     static std::atomic<uint64_t> lds_set{0};
     if (const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&grouped_gemm_kernel<FMT, KIND>), (int)lds_max, lds_set))
         return rc;
@@ -1551,66 +1554,42 @@ static GemmParams gemm_params(const moe_grouped_args* a) {
     return P;
 }
 
-template <int FMT>
-static int launch_gemm_fmt(const moe_grouped_args* a, hipStream_t stream) {
+int launch_tiles(const moe_grouped_args* a, GroupedKernel kind, hipStream_t stream) {
     const GemmParams P = gemm_params(a);
-    if constexpr (FMT != MOE_FMT_BF16) {
-        // decode-like batches (on average at most 12 rows per expert) on the 4-bit N-contiguous containers: the
-        // small-stage kind (at 8 rows per expert int4 409 vs 506 us, fp4 448 vs 474 us; at 24 the large tiles win,
-        // 531 vs 549 us and 512 vs 609 us).  The one-byte containers gain nothing from it.
-        if constexpr (FMT == MOE_FMT_INT4 || FMT == MOE_FMT_FP4_REF)
-            if (a->M <= 12 * a->G) return launch_gemm_kind<FMT, GK_PAIR_SMALL>(P, a, stream);
-        // prefill on the N-contiguous containers: workgroups of 4 wavefronts without the k split, two per CU.  The 4-bit
-        // ones always (256 experts of 128 rows, K = 7168, N = 4096: int4 1792 against 1905 us, fp4 1724 against 1867 us
-        // with the k-split kind).  The one-byte ones, whose tiles move twice the bytes, when an expert has more rows than
-        // one tile takes on average, so that its row chunks share a weight slice in L2: 8 experts of 512 rows, K = 4096,
-        // N = 14336: int8 454 against 476 us, fp8 480 against 495 us; 64 experts of 512 rows at K = 7168, N = 4096: 1755
-        // against 1870 us and 1872 against 1929 us; but with 128 rows per expert, every weight tile read once from HBM,
-        // 1090 - 1110 against 1063 - 1098 us (int8) and 1125 - 1152 against 1088 - 1136 us (fp8) on 128 experts
-        constexpr bool four_bit = FMT == MOE_FMT_INT4 || FMT == MOE_FMT_FP4_REF;
-        constexpr bool one_byte = FMT == MOE_FMT_INT8 || FMT == MOE_FMT_FP8_REF;
-        if constexpr (four_bit || one_byte) {
-            if (four_bit || a->M > (int64_t)(16 * PAIR_CAPB) * a->G) {
-                const int rc = launch_gemm_kind<FMT, GK_QUAD>(P, a, stream);
-                if (rc != MOE_ERR_TOO_LARGE) return rc;
+    switch (kind) {
+        case GroupedKernel::TILES_PAIR:
+            switch (a->format) {
+                case MOE_FMT_FP8_REF: return launch_gemm_kind<MOE_FMT_FP8_REF, GK_PAIR>(P, a, stream);
+                case MOE_FMT_INT8: return launch_gemm_kind<MOE_FMT_INT8, GK_PAIR>(P, a, stream);
+                case MOE_FMT_FP4_B32: return launch_gemm_kind<MOE_FMT_FP4_B32, GK_PAIR>(P, a, stream);
+                case MOE_FMT_FP4_B16: return launch_gemm_kind<MOE_FMT_FP4_B16, GK_PAIR>(P, a, stream);
+                default: return MOE_ERR_BAD_FORMAT;
             }
-        }
-        return launch_gemm_kind<FMT, GK_PAIR>(P, a, stream);
-    } else {
-        return launch_gemm_kind<FMT, GK_BF16>(P, a, stream);
-    }
-}
-
-int launch_gemm_bf16(const moe_grouped_args* a, hipStream_t stream) { return launch_gemm_fmt<MOE_FMT_BF16>(a, stream); }
-
-int launch_gemm_exact(const moe_grouped_args* a, hipStream_t stream) {
-    const GemmParams P = gemm_params(a);
-    if (stream_preferred(a)) return launch_stream(a, stream, false);
-    switch (a->format) {
-        case MOE_FMT_FP4_REF:
-            // decode-like batches (on average at most 12 rows per expert): 16-row tiles, two workgroups per CU; an
-            // expert with more rows than that costs a pass over its weights per 16 rows
-            if (a->M <= 12 * a->G) return launch_gemm_kind<MOE_FMT_FP4_REF, GK_PAIR_EXACT16>(P, a, stream);
-            return launch_gemm_kind<MOE_FMT_FP4_REF, GK_PAIR_EXACT>(P, a, stream);
-        case MOE_FMT_INT4: return launch_gemm_kind<MOE_FMT_INT4, GK_PAIR_EXACT>(P, a, stream);
-        case MOE_FMT_FP8_REF: return launch_gemm_kind<MOE_FMT_FP8_REF, GK_PAIR_EXACT>(P, a, stream);
-        default: return MOE_ERR_BAD_FORMAT;
-    }
-}
-
-int launch_grouped_gemm(const moe_grouped_args* a, hipStream_t stream) {
-    // Decode-sized batches on the K-contiguous containers go to the weight-streaming GEMV kernels,
-    // run with this op's arithmetic and epilogue.
-    if (gemv_preferred(a)) return launch_grouped_gemv(a, stream, true);
-    if (stream_preferred(a)) return launch_stream(a, stream, true);
-    switch (a->format) {
-        case MOE_FMT_FP4_REF: return launch_gemm_fmt<MOE_FMT_FP4_REF>(a, stream);
-        case MOE_FMT_FP8_REF: return launch_gemm_fmt<MOE_FMT_FP8_REF>(a, stream);
-        case MOE_FMT_INT8: return launch_gemm_fmt<MOE_FMT_INT8>(a, stream);
-        case MOE_FMT_INT4: return launch_gemm_fmt<MOE_FMT_INT4>(a, stream);
-        case MOE_FMT_FP4_B32: return launch_gemm_fmt<MOE_FMT_FP4_B32>(a, stream);
-        case MOE_FMT_FP4_B16: return launch_gemm_fmt<MOE_FMT_FP4_B16>(a, stream);
-        case MOE_FMT_BF16: return launch_gemm_fmt<MOE_FMT_BF16>(a, stream);
+        case GroupedKernel::TILES_PAIR_SMALL:
+            switch (a->format) {
+                case MOE_FMT_FP4_REF: return launch_gemm_kind<MOE_FMT_FP4_REF, GK_PAIR_SMALL>(P, a, stream);
+                case MOE_FMT_INT4: return launch_gemm_kind<MOE_FMT_INT4, GK_PAIR_SMALL>(P, a, stream);
+                default: return MOE_ERR_BAD_FORMAT;
+            }
+        case GroupedKernel::TILES_QUAD:
+            switch (a->format) {
+                case MOE_FMT_FP4_REF: return launch_gemm_kind<MOE_FMT_FP4_REF, GK_QUAD>(P, a, stream);
+                case MOE_FMT_FP8_REF: return launch_gemm_kind<MOE_FMT_FP8_REF, GK_QUAD>(P, a, stream);
+                case MOE_FMT_INT8: return launch_gemm_kind<MOE_FMT_INT8, GK_QUAD>(P, a, stream);
+                case MOE_FMT_INT4: return launch_gemm_kind<MOE_FMT_INT4, GK_QUAD>(P, a, stream);
+                default: return MOE_ERR_BAD_FORMAT;
+            }
+        case GroupedKernel::TILES_PAIR_EXACT:
+            switch (a->format) {
+                case MOE_FMT_FP4_REF: return launch_gemm_kind<MOE_FMT_FP4_REF, GK_PAIR_EXACT>(P, a, stream);
+                case MOE_FMT_FP8_REF: return launch_gemm_kind<MOE_FMT_FP8_REF, GK_PAIR_EXACT>(P, a, stream);
+                case MOE_FMT_INT4: return launch_gemm_kind<MOE_FMT_INT4, GK_PAIR_EXACT>(P, a, stream);
+                default: return MOE_ERR_BAD_FORMAT;
+            }
+        case GroupedKernel::TILES_PAIR_EXACT16:
+            return a->format == MOE_FMT_FP4_REF ? launch_gemm_kind<MOE_FMT_FP4_REF, GK_PAIR_EXACT16>(P, a, stream) : MOE_ERR_BAD_FORMAT;
+        case GroupedKernel::TILES_BF16:
+            return a->format == MOE_FMT_BF16 ? launch_gemm_kind<MOE_FMT_BF16, GK_BF16>(P, a, stream) : MOE_ERR_BAD_FORMAT;
         default: return MOE_ERR_BAD_FORMAT;
     }
 }

@@ -9,10 +9,10 @@
 //   gemv_fp4_mfma_kernel  fp4 codes: one v_mfma_f32_16x16x32_bf16 per 32-k block and 16 weight rows (a vector kernel
 //                         needs (1 + rows) / 2 instructions per 4-bit weight, more than the chip can issue while HBM
 //                         delivers the codes at full rate), wave-private streaming, no workgroup barrier in the k loop
-// The N-contiguous containers (reference fp4 / fp8, int4) run on the k-split matrix-core kernel of moe_gemm.hip with
-// this op's arithmetic (launch_gemm_exact): measured 3 times faster than a vector kernel on that layout.  bf16 calls with
-// more rows per expert than the vector kernel is good for go to that file's tiles too.  Both kernels also have the GEMM op's
-// SwiGLU epilogue, for its decode-sized calls.
+// The N-contiguous containers (reference fp4 / fp8, int4) run on the matrix-core kernels of moe_stream.hip and moe_gemm.hip with
+// this op's arithmetic: measured 3 times faster than a vector kernel on that layout.  bf16 calls with
+// more rows per expert than the vector kernel is good for go to the tiles of moe_gemm.hip too (moe_dispatch.cpp).  Both kernels
+// also have the GEMM op's SwiGLU epilogue, for its decode-sized calls.
 //
 // Numerics (gemv_impl.h:147-199): weights are decode * scale in fp32, NOT rounded
 // to bf16; fp32 accumulation; one RNE to bf16 at the end (grouped_soft_gemv.h:218-233).
@@ -257,7 +257,7 @@ constexpr int GF_LDS_UNITS = 3584;        // 56 KiB of x per staged chunk
 constexpr int GF_SCALE_UNITS = 128;       // per wavefront: the 4 q lanes' 2 x 16 bytes of scales for 16 rows
 constexpr int GF_U = 4;                   // 128-k groups (one 16-byte load per lane each) per loop iteration
 constexpr int GF_KSTEP = 128 * GF_U;      // k per loop iteration; K must be a multiple
-constexpr int GF_GEMM_ROWS_PER_EXPERT = 12;// grouped GEMM calls with at most this many rows per expert on average come here
+static_assert(GF_KSTEP == FP4_ROWS_K, "what the dispatch goes by");
 
 __device__ __forceinline__ uint32_t e2m1_pair_bf16(uint32_t word, int sel) {
     switch (sel) {
@@ -565,46 +565,19 @@ static int launch_kmajor(const moe_grouped_args* a, hipStream_t stream) {
     return hipGetLastError() == hipSuccess ? MOE_OK : MOE_ERR_LAUNCH;
 }
 
-bool gemv_preferred(const moe_grouped_args* a) {
-    // Decode-sized batches on the K-contiguous containers are pure weight streaming: these kernels
-    // read every weight row as contiguous runs.  The matrix-core fp4 kernel takes 16 rows of an expert per pass and has a
-    // variant with the GEMM's weight rounding; the bound is where the k-split GEMM kernel overtakes it (measured at
-    // DeepSeek-V3 shapes, 256 experts of 7168 x 2048: 8 rows per expert 496 vs 631 us, 16 rows 754 vs 651 us).  With the
-    // SwiGLU epilogue, fp4_b32: 16 tokens x 8 on 256 experts of 7168 x 4096 306 vs 468 us, 8 rows of 8 experts of
-    // 4096 x 1024 17 vs 36, 8 rows per expert on 256 of 2048 x 1024 95 vs 99; 12 per expert on 8 of 4096 x 2048 39 vs 37.
-    if (a->format == MOE_FMT_FP4_B32 || a->format == MOE_FMT_FP4_B16)
-        return a->K % GF_KSTEP == 0 && a->M <= (a->epilogue == MOE_EPILOGUE_SWIGLU ? 8 : GF_GEMM_ROWS_PER_EXPERT) * a->G;
-    // The bf16 vector kernel takes 4 rows of an expert per pass over its weights (same arithmetic as the GEMM: the weights
-    // are bf16 already), the tile kernel up to 224, but only a workgroup per 256 columns.  4 rows per expert, here / there:
-    // 64 experts of 7168 x 2048 (512 tiles) 402 / 303 us, 16 of 7168 x 4096 (256) 208 / 162, 64 of 2048 x 1024 (256)
-    // 88 / 65, but 8 of 7168 x 4096 (128) 106 / 129, 8 of 7168 x 512 (16) 50 / 80; 2 rows, 512 tiles: 264 / 262.
-    if (a->format == MOE_FMT_BF16) return a->M <= (min(a->M, a->G) * a->N >= 65536 ? 2 : 4) * a->G;
-    return false;
+int launch_vector(const moe_grouped_args* a, hipStream_t stream) {
+    switch (a->format) {
+        case MOE_FMT_BF16: return launch_kmajor<MOE_FMT_BF16>(a, stream);
+        case MOE_FMT_FP4_B32: return launch_kmajor<MOE_FMT_FP4_B32>(a, stream);
+        case MOE_FMT_FP4_B16: return launch_kmajor<MOE_FMT_FP4_B16>(a, stream);
+        default: return MOE_ERR_BAD_FORMAT;
+    }
 }
 
-int launch_grouped_gemv(const moe_grouped_args* a, hipStream_t stream, bool gemm_rounding) {
+int launch_fp4_rows(const moe_grouped_args* a, bool gemm_rounding, hipStream_t stream) {
     switch (a->format) {
-        case MOE_FMT_BF16:
-            // more rows than the vector kernel is good for, in sizes that the tile kernel takes (see gemv_preferred): the
-            // two compute the same.  64 experts of 7168 x 2048: 16 rows per expert 1225 -> 331 us, 64 rows 4668 -> 405.  Few
-            // columns: 6 rows per expert 77 here / 81 us there on 8 experts of 7168 x 512, 8 rows 93 / 81; 6 rows on 8 of
-            // 4096 x 2048 79 / 71.
-            if (!gemv_preferred(a) && (a->N * a->G >= 16384 || a->M > 6 * a->G) && a->K % 64 == 0 && a->N % 256 == 0)
-                return launch_gemm_bf16(a, stream);
-            return launch_kmajor<MOE_FMT_BF16>(a, stream);
-        case MOE_FMT_FP4_B32:
-            // the matrix-core kernel takes K in whole loop iterations
-            if (a->K % GF_KSTEP != 0) return gemm_rounding ? MOE_ERR_BAD_SHAPE : launch_kmajor<MOE_FMT_FP4_B32>(a, stream);
-            return gemm_rounding ? launch_fp4_mfma<true, 32>(a, stream) : launch_fp4_mfma<false, 32>(a, stream);
-        case MOE_FMT_FP4_B16:
-            if (a->K % GF_KSTEP != 0) return gemm_rounding ? MOE_ERR_BAD_SHAPE : launch_kmajor<MOE_FMT_FP4_B16>(a, stream);
-            return gemm_rounding ? launch_fp4_mfma<true, 16>(a, stream) : launch_fp4_mfma<false, 16>(a, stream);
-        case MOE_FMT_FP4_REF:
-        case MOE_FMT_INT4:
-        case MOE_FMT_FP8_REF: {
-            // the matrix-core GEMM kernels run with this op's arithmetic (fp32 weights)
-            return launch_gemm_exact(a, stream);
-        }
+        case MOE_FMT_FP4_B32: return gemm_rounding ? launch_fp4_mfma<true, 32>(a, stream) : launch_fp4_mfma<false, 32>(a, stream);
+        case MOE_FMT_FP4_B16: return gemm_rounding ? launch_fp4_mfma<true, 16>(a, stream) : launch_fp4_mfma<false, 16>(a, stream);
         default: return MOE_ERR_BAD_FORMAT;
     }
 }

@@ -22,19 +22,25 @@ inline int ensure_dynamic_lds(const void* kernel, int bytes, std::atomic<uint64_
 }
 
 int launch_dequant_fp4_bf16(const moe_dequant_args* a, hipStream_t stream);
-// gemm_rounding: use the grouped GEMM's arithmetic (weights rounded to bf16) where the two ops differ.
-int launch_grouped_gemv(const moe_grouped_args* a, hipStream_t stream, bool gemm_rounding = false);
-// True when the GEMV launcher is the faster path for a grouped GEMM call of this shape.
-bool gemv_preferred(const moe_grouped_args* a);
-// grouped GEMV on the fp4 / int4 N-contiguous containers by the k-split GEMM kernel run with the GEMV
-// op's arithmetic; MOE_ERR_TOO_LARGE when the expert count does not fit its LDS
-int launch_gemm_exact(const moe_grouped_args* a, hipStream_t stream);
-// bf16 container on the tile kernel (K % 64 == 0, N % 256 == 0)
-int launch_gemm_bf16(const moe_grouped_args* a, hipStream_t stream);
-int launch_grouped_gemm(const moe_grouped_args* a, hipStream_t stream);
-// N-contiguous containers, launches too small to fill the chip with tiles that walk all of K (moe_stream.hip)
-bool stream_preferred(const moe_grouped_args* a);
-int launch_stream(const moe_grouped_args* a, hipStream_t stream, bool gemm_rounding);
+// The kernels of the two grouped ops.  TILES_PAIR_EXACT and TILES_PAIR_EXACT16 have the GEMV op's arithmetic (weights not
+// rounded to bf16), the other TILES that of the GEMM op; STRIPS and FP4_ROWS come with either.
+enum class GroupedKernel {
+    VECTOR,               // K-contiguous containers without matrix cores (moe_gemv.hip)
+    FP4_ROWS,             // K-contiguous fp4, 16 rows of an expert per pass (moe_gemv.hip)
+    STRIPS_32, STRIPS_64, STRIPS_128,   // N-contiguous containers in strips of that many columns (moe_stream.hip)
+    TILES_PAIR, TILES_PAIR_EXACT, TILES_PAIR_SMALL, TILES_PAIR_EXACT16, TILES_QUAD, TILES_BF16   // kinds of moe_gemm.hip
+};
+constexpr int FP4_ROWS_K = 512;   // K of an FP4_ROWS call is a multiple
+constexpr int PAIR_ROWS = 160;    // rows of the largest tile of the quantized containers
+// the kernel of a valid call, by its sizes, format and epilogue (moe_dispatch.cpp)
+GroupedKernel grouped_kernel(const moe_grouped_args* a, bool gemv_op);
+const char* grouped_kernel_name(GroupedKernel k);
+int launch_grouped(const moe_grouped_args* a, bool gemv_op, hipStream_t stream);
+int launch_vector(const moe_grouped_args* a, hipStream_t stream);
+// gemm_rounding: the arithmetic of the GEMM op
+int launch_fp4_rows(const moe_grouped_args* a, bool gemm_rounding, hipStream_t stream);
+int launch_strips(const moe_grouped_args* a, GroupedKernel width, bool gemm_rounding, hipStream_t stream);
+int launch_tiles(const moe_grouped_args* a, GroupedKernel kind, hipStream_t stream);
 // moves the grouped GEMM's launch number (which picks a launch's tile counter and stamp) by delta; returns the new number
 int64_t gemm_shift_launch_number(int64_t delta);
 int launch_prepack_fp4_ref(const moe_prepack_fp4_args* a, hipStream_t stream);

@@ -407,41 +407,24 @@ static int launch_stream_kind(const moe_grouped_args* a, hipStream_t stream) {
     return hipGetLastError() == hipSuccess ? MOE_OK : MOE_ERR_LAUNCH;
 }
 
-// Columns the launch streams, at most: min(M, G) experts own rows
-static int64_t stream_columns(const moe_grouped_args* a) { return min(a->M, a->G) * a->N; }
-
-// The narrowest strips that still leave every CU at most one workgroup.  Measured, 8 experts of K = 7168, 32 / 64 / 128 columns
-// a strip: N = 512 (4096 columns in all) int4 15 / 18 / 27 us, fp8 16 / 21 / 34; N = 2048 (16384) int4 28 / 20 / 28, fp8
-// 46 / 32 / 39; 16 experts of N = 2048 (32768) int4 75 / 49 / 34, fp8 89 / 60 / 49.
 template <int FMT, bool ROUNDW>
-static int launch_stream_fmt(const moe_grouped_args* a, hipStream_t stream) {
-    const int64_t columns = stream_columns(a);
-    if (columns <= 8192) return launch_stream_kind<FMT, ROUNDW, 2>(a, stream);
-    if (columns <= 16384) return launch_stream_kind<FMT, ROUNDW, 4>(a, stream);
-    return launch_stream_kind<FMT, ROUNDW, 8>(a, stream);
+static int launch_stream_fmt(const moe_grouped_args* a, GroupedKernel width, hipStream_t stream) {
+    switch (width) {
+        case GroupedKernel::STRIPS_32: return launch_stream_kind<FMT, ROUNDW, 2>(a, stream);
+        case GroupedKernel::STRIPS_64: return launch_stream_kind<FMT, ROUNDW, 4>(a, stream);
+        default: return launch_stream_kind<FMT, ROUNDW, 8>(a, stream);
+    }
 }
 
-// Up to 128 tiles of 256 columns, i.e. half of the CUs, and decode-like batches: with 32768 columns (16 experts of
-// 7168 x 2048) int4 34 - 36 us here against 49 - 60 with moe_gemm.hip's tiles, fp4 33 / 50, fp8 49 / 72; with 49152 columns
-// those are ahead (int4 63 / 53, fp8 90 / 82), with 65536 by a factor of 1.3.  With up to 16384 columns twice as many rows:
-// 192 rows unevenly owned by 8 experts of 4096 x 2048, tiles / here: int4 65 / 25 us, fp4 58 / 21, fp8 49 / 28, int8 44 / 25;
-// all 192 owned by one expert: int4 66 / 22, int8 45 / 21.  The passes are found by looking through group_list, 256 experts
-// at a time.
-bool stream_preferred(const moe_grouped_args* a) {
-    if (a->format != MOE_FMT_FP4_REF && a->format != MOE_FMT_FP8_REF && a->format != MOE_FMT_INT4 && a->format != MOE_FMT_INT8) return false;
-    const int64_t columns = stream_columns(a);
-    return a->G <= 1024 && columns <= 32768 && a->M <= (columns <= 16384 ? 24 : 12) * a->G;
-}
-
-int launch_stream(const moe_grouped_args* a, hipStream_t stream, bool gemm_rounding) {
+int launch_strips(const moe_grouped_args* a, GroupedKernel width, bool gemm_rounding, hipStream_t stream) {
     switch (a->format) {
         case MOE_FMT_FP4_REF:
-            return gemm_rounding ? launch_stream_fmt<MOE_FMT_FP4_REF, true>(a, stream) : launch_stream_fmt<MOE_FMT_FP4_REF, false>(a, stream);
+            return gemm_rounding ? launch_stream_fmt<MOE_FMT_FP4_REF, true>(a, width, stream) : launch_stream_fmt<MOE_FMT_FP4_REF, false>(a, width, stream);
         case MOE_FMT_FP8_REF:
-            return gemm_rounding ? launch_stream_fmt<MOE_FMT_FP8_REF, true>(a, stream) : launch_stream_fmt<MOE_FMT_FP8_REF, false>(a, stream);
+            return gemm_rounding ? launch_stream_fmt<MOE_FMT_FP8_REF, true>(a, width, stream) : launch_stream_fmt<MOE_FMT_FP8_REF, false>(a, width, stream);
         case MOE_FMT_INT4:
-            return gemm_rounding ? launch_stream_fmt<MOE_FMT_INT4, true>(a, stream) : launch_stream_fmt<MOE_FMT_INT4, false>(a, stream);
-        case MOE_FMT_INT8: return gemm_rounding ? launch_stream_fmt<MOE_FMT_INT8, true>(a, stream) : MOE_ERR_BAD_FORMAT;
+            return gemm_rounding ? launch_stream_fmt<MOE_FMT_INT4, true>(a, width, stream) : launch_stream_fmt<MOE_FMT_INT4, false>(a, width, stream);
+        case MOE_FMT_INT8: return gemm_rounding ? launch_stream_fmt<MOE_FMT_INT8, true>(a, width, stream) : MOE_ERR_BAD_FORMAT;
         default: return MOE_ERR_BAD_FORMAT;
     }
 }

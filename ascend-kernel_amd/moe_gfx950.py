@@ -27,6 +27,7 @@ SYMBOLS = (
     "moe_dequant_fp4_bf16", "moe_grouped_gemm", "moe_grouped_gemv",
     "moe_prepack_fp4_ref_validate", "moe_prepack_fp4_ref_workspace_bytes", "moe_prepack_fp4_ref",
     "moe_route_validate", "moe_route_workspace_bytes", "moe_route", "moe_route_static", "moe_test_shift_launch_number",
+    "moe_test_grouped_kernel",
 )
 
 
@@ -81,6 +82,8 @@ for _n, _t in (("dequant_fp4_bf16", DequantArgs), ("grouped_gemm", GroupedArgs),
 lib.moe_route_static.restype = ctypes.c_int
 lib.moe_test_shift_launch_number.restype = ctypes.c_int64
 lib.moe_test_shift_launch_number.argtypes = [ctypes.c_int64]
+lib.moe_test_grouped_kernel.restype = ctypes.c_char_p
+lib.moe_test_grouped_kernel.argtypes = [ctypes.POINTER(GroupedArgs), ctypes.c_int]
 lib.moe_route_static.argtypes = [ctypes.POINTER(RouteArgs), ctypes.c_void_p]
 ROUTE_STATIC_SCRATCH_BYTES = 2 << 20
 
@@ -118,6 +121,14 @@ def grouped_args(fmt: int, x_ptr: int, w_ptr: int, scale_ptr, offset_ptr, gl_ptr
 
 def grouped_gemm(args: GroupedArgs, stream: int = 0) -> None:
     _check(lib.moe_grouped_gemm(ctypes.byref(args), ctypes.c_void_p(stream)), "moe_grouped_gemm")
+
+
+def grouped_kernel(args: GroupedArgs, op: str) -> str:
+    """Name of the kernel that the op ("gemm" / "gemv") runs for these arguments (test support, host only)."""
+    name = lib.moe_test_grouped_kernel(ctypes.byref(args), int(op == "gemv"))
+    if name is None:
+        raise ValueError(f"not a valid {op} call")
+    return name.decode()
 
 
 def grouped_gemv(args: GroupedArgs, stream: int = 0) -> None:

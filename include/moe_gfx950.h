@@ -259,6 +259,10 @@ int moe_route_static(const moe_route_args *args, moe_stream_t stream);
  * that a test can make a launch find its counter taken over by a later one. */
 int64_t moe_test_shift_launch_number(int64_t delta);
 
+/* Test support: the name of the kernel that moe_grouped_gemm (gemv_op 0) or moe_grouped_gemv (1) runs for these
+ * arguments, NULL if they are not valid.  Host only; the pointers are not followed.  The names may change. */
+const char *moe_test_grouped_kernel(const moe_grouped_args *args, int gemv_op);
+
 #ifdef __cplusplus
 }
 #endif

@@ -94,6 +94,15 @@ def oracle_out(case, gemv: bool = False, row_mask=None) -> np.ndarray:
                                case["offset"], case["group_list"], round_bf16=not gemv, row_mask=row_mask)
 
 
+def kernel_of(case, op: str, swiglu: bool = False) -> str:
+    """Name of the kernel that a call of these sizes runs (host only: the pointers stand for any aligned ones)."""
+    import moe_gfx950 as mg
+
+    p = 0x1000
+    return mg.grouped_kernel(mg.grouped_args(mg.format_from_compute_type(case["fmt"]), p, p, p, p, p, p, case["M"], case["K"], case["N"],
+                                             case["G"], case["scale_rows"], epilogue=mg.EPILOGUE_SWIGLU if swiglu else mg.EPILOGUE_NONE), op)
+
+
 # ----------------------------------------------------------------------------- GPU side
 def to_dev(a, device="cuda"):
     if a is None:

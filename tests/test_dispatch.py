@@ -1,0 +1,61 @@
+"""Which kernel a grouped call gets, on both sides of every rule of the dispatch (host only)."""
+import pytest
+
+import helpers as H
+
+N_CONTIG = ("fp4", "fp8", "int8", "int4")
+
+
+def kernel(fmt, op, M, G, K, N, swiglu=False):
+    scale_rows = {"fp4": K // 16, "int4": K // 32}.get(fmt, 1)
+    return H.kernel_of(dict(fmt=fmt, M=M, K=K, N=N, G=G, scale_rows=scale_rows), op, swiglu)
+
+
+@pytest.mark.parametrize("op", ["gemm", "gemv"])
+@pytest.mark.parametrize("fmt", N_CONTIG)
+def test_strips(fmt, op):
+    if op == "gemv" and fmt == "int8":
+        pytest.skip("the GEMV op has no such container")
+    at = lambda M, G, N: kernel(fmt, op, M, G, 7168, N)   # noqa: E731
+    assert at(8, 256, 512) == "strips_32"                              # a token with 8 experts
+    assert (at(32, 32, 256), at(33, 33, 256)) == ("strips_32", "strips_64")      # 8192 columns
+    assert (at(64, 64, 256), at(65, 65, 256)) == ("strips_64", "strips_128")     # 16384 columns
+    assert at(128, 128, 256) == "strips_128" and at(129, 129, 256).startswith("tiles")   # 32768 columns
+    assert at(24 * 8, 8, 2048) == "strips_64" and at(24 * 8 + 1, 8, 2048).startswith("tiles")
+    assert at(12 * 16, 16, 2048) == "strips_128" and at(12 * 16 + 1, 16, 2048).startswith("tiles")
+    assert at(4, 1024, 256) == "strips_32" and at(4, 1025, 256).startswith("tiles")
+
+
+def test_tiles_of_the_n_contiguous_containers():
+    rows = {r: {f: kernel(f, "gemm", r * 64, 64, 7168, 2048) for f in N_CONTIG} for r in (12, 13, 160, 161)}
+    assert rows[12] == dict(fp4="tiles_pair_small", int4="tiles_pair_small", fp8="tiles_pair", int8="tiles_pair")
+    assert rows[13] == rows[160] == dict(fp4="tiles_quad", int4="tiles_quad", fp8="tiles_pair", int8="tiles_pair")
+    assert rows[161] == dict.fromkeys(N_CONTIG, "tiles_quad")
+    rows = {r: {f: kernel(f, "gemv", r * 64, 64, 7168, 2048) for f in ("fp4", "int4", "fp8")} for r in (12, 13)}
+    assert rows[12] == dict(fp4="tiles_pair_exact16", int4="tiles_pair_exact", fp8="tiles_pair_exact")
+    assert rows[13] == dict.fromkeys(("fp4", "int4", "fp8"), "tiles_pair_exact")
+
+
+@pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
+def test_k_contiguous_fp4(fmt):
+    at = lambda op, r, K, swiglu=False: kernel(fmt, op, r * 64, 64, K, 2048, swiglu)   # noqa: E731
+    assert (at("gemv", 1, 7168), at("gemv", 100, 7168), at("gemv", 1, 7168 + 32)) == ("fp4_rows", "fp4_rows", "vector")
+    assert (at("gemm", 12, 7168), at("gemm", 13, 7168), at("gemm", 1, 7168 + 128)) == ("fp4_rows", "tiles_pair", "tiles_pair")
+    assert (at("gemm", 8, 7168, True), at("gemm", 9, 7168, True)) == ("fp4_rows", "tiles_pair")
+
+
+def test_bf16():
+    at = lambda op, M, G, N, K=7168: kernel("bf16", op, M, G, K, N)   # noqa: E731
+    for op in ("gemm", "gemv"):
+        assert (at(op, 2 * 64, 64, 2048), at(op, 2 * 64 + 1, 64, 2048)) == ("vector", "tiles_bf16")
+    assert (at("gemm", 4 * 8, 8, 4096), at("gemm", 4 * 8 + 1, 8, 4096)) == ("vector", "tiles_bf16")
+    assert (at("gemv", 6 * 8, 8, 512), at("gemv", 6 * 8 + 1, 8, 512)) == ("vector", "tiles_bf16")
+    # sizes that the tiles do not take
+    assert at("gemv", 1000, 8, 2049) == at("gemv", 1000, 8, 2048, K=7168 + 32) == "vector"
+
+
+def test_not_a_valid_call():
+    with pytest.raises(ValueError):
+        kernel("int8", "gemv", 4, 4, 256, 256)
+    with pytest.raises(ValueError):
+        kernel("bf16", "gemm", 4, 4, 256, 100)

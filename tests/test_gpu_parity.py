@@ -145,15 +145,16 @@ def test_gemm_parity_deep_k_and_wide_n(fmt, K, N):
     H.assert_close(got, H.oracle_out(case), what=f"{fmt} K={K} N={N}")
 
 
-@pytest.mark.parametrize("op", ["gemm", "gemv"])
+@pytest.mark.parametrize("op,gl,kernel", [("gemm", [5, 140, 140, 301], "tiles_pair"), ("gemv", [3, 3, 40, 41], "strips_32"),
+                                          ("gemv", [3, 3, 120, 121], "tiles_pair_exact")], ids=["gemm", "gemv", "gemv_tiles"])
 @pytest.mark.parametrize("N", [128, 384, 1408])
-def test_fp8_n_multiple_of_128(N, op):
+def test_fp8_n_multiple_of_128(N, op, gl, kernel):
     """The reference tiles uint8 weights 128 columns wide (grouped_gemm/op_host/grouped_matmul_antiquant_tiling.cpp:616-621,
     grouped_soft_gemv/op_host/grouped_soft_gemv_tiling.cpp:105-128): N need not be a multiple of the 256-column
     tile here.  The half-empty last tile must write nothing past column N (the row's successor starts there)."""
-    _say(f"fp8 N={N} op={op}")
-    gl = [3, 3, 40, 41] if op == "gemv" else [5, 140, 140, 301]
+    _say(f"fp8 N={N} op={op} {kernel}")
     case = H.make_case("fp8", len(gl), 512, N, gl, seed=N, extra_rows=2)
+    assert H.kernel_of(case, op) == kernel
     got = H.run_cabi(case, H.upload(case), op)
     H.assert_close(got, H.oracle_out(case, gemv=op == "gemv"), rows=slice(0, gl[-1]), what=f"fp8 N={N} {op}")
     assert (got[gl[-1]:] == 0x7FC0).all()
@@ -187,13 +188,13 @@ def test_decode_batches_on_the_small_tile_kinds(fmt, shape, op):
     has workgroups."""
     _say(f"{op} small tiles fmt={fmt} {shape}")
     if shape == "row_counts":
-        counts, K, N = [1, 0, 4, 5, 16, 17, 32, 33, 70, 0, 3, 8, 9, 7] + [0] * 8, 1024, 512
+        counts, K, N = [1, 0, 4, 5, 16, 17, 32, 33, 70, 0, 3, 8, 9, 7] + [0] * 8, 1024, 2048   # more columns than strips take
     else:
         rng = np.random.default_rng(zlib.crc32(f"small/{fmt}".encode()))
         counts, K, N = list(rng.choice([0] * 6 + [1, 3, 16, 17, 33, 40], 160)), 256, 2048
     gl = list(np.cumsum(counts))
-    assert gl[-1] <= 12 * len(gl)
     case = H.make_case(fmt, len(gl), K, N, gl, seed=len(gl), extra_rows=2, group=64)
+    assert H.kernel_of(case, op) == ("tiles_pair_small" if op == "gemm" else "tiles_pair_exact16" if fmt == "fp4" else "tiles_pair_exact")
     got = H.run_cabi(case, H.upload(case), op)
     H.assert_close(got, H.oracle_out(case, gemv=op == "gemv"), rows=slice(0, gl[-1]), what=f"small tiles {op} {fmt}/{shape}")
     assert (got[gl[-1]:] == 0x7FC0).all()
@@ -419,14 +420,17 @@ def test_gemv_fp4_b32_row_counts_up_to_and_beyond_16(K, N, fmt):
                                            ("int4", 1024, 256, 128), ("int4", 7168, 512, 128), ("int4", 192, 256, 32),
                                            ("int4", 256, 256, 64), ("fp8", 1024, 256, 128), ("fp8", 7168, 512, 128),
                                            ("fp8", 128, 256, 128)])
-def test_gemv_n_contiguous_row_counts_up_to_and_beyond_32(fmt, K, N, group):
+@pytest.mark.parametrize("more,kernel", [([], "strips_32"), ([110], "tiles_pair_exact")], ids=["strips", "tiles"])
+def test_gemv_n_contiguous_row_counts_up_to_and_beyond_32(fmt, K, N, group, more, kernel):
     """The GEMV op on the reference fp4 / fp8 containers and on int4 runs on the matrix cores with weights
     that are not rounded to bf16 (the codes go through the MFMA, the fp32 scales are applied to its
-    results), in tiles of up to 32 rows of an expert; K = 64 (fp8: 128) is a single scale block."""
-    _say(f"gemv {fmt} rows K={K} N={N} group={group}")
-    counts = [1, 0, 4, 5, 16, 17, 32, 33, 70, 0, 3]
+    results), in strips of few columns, 16 rows a pass, or, with more than 24 rows per expert, in tiles of up to 32 rows of an
+    expert; K = 64 (fp8: 128) is a single scale block."""
+    _say(f"gemv {fmt} rows K={K} N={N} group={group} {kernel}")
+    counts = [1, 0, 4, 5, 16, 17, 32, 33, 70, 0, 3] + more
     gl = list(np.cumsum(counts))
     case = H.make_case(fmt, len(gl), K, N, gl, seed=K + N + group, extra_rows=2, group=group)
+    assert H.kernel_of(case, "gemv") == kernel
     got = H.run_cabi(case, H.upload(case), "gemv")
     H.assert_close(got, H.oracle_out(case, gemv=True), rows=slice(0, gl[-1]), what=f"gemv {fmt} rows K={K} N={N}")
     assert (got[gl[-1]:] == 0x7FC0).all()
@@ -545,17 +549,28 @@ def test_gemv_matches_gemm_on_the_same_inputs():
 
 
 # -------------------------------------------------- error behaviour through the module
-@pytest.mark.parametrize("gl_name,gl", [("decode", [3, 3, 7, 9]), ("prefill", [40, 90, 130, 200])])
-@pytest.mark.parametrize("fmt", ["int4", "fp4", "fp8", "fp4_b32", "fp4_b16"])
-def test_each_op_uses_its_own_weight_rounding(fmt, gl_name, gl):
+_TILES = {"int4": ("tiles_pair_small", "tiles_pair_exact"), "fp4": ("tiles_pair_small", "tiles_pair_exact16"), "fp8": ("tiles_pair", "tiles_pair_exact")}
+_QUAD = {"int4": ("tiles_quad", "tiles_pair_exact"), "fp4": ("tiles_quad", "tiles_pair_exact"), "fp8": ("tiles_pair", "tiles_pair_exact")}
+ROUNDING = ([(f, "decode", [3, 3, 7, 9], 512, ("strips_32", "strips_32")) for f in _TILES]
+            + [(f, "strips_64", [2, 4, 6, 7, 9, 10, 12, 14], 1536, ("strips_64", "strips_64")) for f in _TILES]
+            + [(f, "strips_128", [1, 2, 14, 15, 17, 18, 19, 21, 22], 2560, ("strips_128", "strips_128")) for f in _TILES]
+            + [(f, "decode_tiles", [3] * 9 + [14, 15, 17] + [20] * 8, 2048, k) for f, k in _TILES.items()]
+            + [(f, "prefill", [40, 90, 130, 200], 512, k) for f, k in _QUAD.items()]
+            + [(f, "decode", [3, 3, 7, 9], 512, ("fp4_rows", "fp4_rows")) for f in ("fp4_b32", "fp4_b16")]
+            + [(f, "prefill", [40, 90, 130, 200], 512, ("tiles_pair", "fp4_rows")) for f in ("fp4_b32", "fp4_b16")])
+
+
+@pytest.mark.parametrize("fmt,gl_name,gl,N,kernels", ROUNDING, ids=[f"{c[0]}-{c[1]}" for c in ROUNDING])
+def test_each_op_uses_its_own_weight_rounding(fmt, gl_name, gl, N, kernels):
     """The GEMM op multiplies weights rounded to bf16 (the reference's phase 1), the GEMV op un-rounded fp32
     weights (gemv_impl.h:147-199).  The two differ by about a quarter of an output ulp, far inside the parity
     tolerance, so they are told apart by counting outputs whose bf16 bits differ: against the oracle of its own
     arithmetic an op differs only where the summation order moves a sum across a rounding boundary, against the
-    other arithmetic in a sizeable share of the outputs.  Covers every dispatch: k-split tiles, the matrix-core
-    GEMV kernels run with either rounding, decode and prefill sized batches."""
+    other arithmetic in a sizeable share of the outputs.  Covers every kernel of the quantized containers whose arithmetic
+    could be the other op's: strips of each width, the small and large tiles, the matrix-core GEMV kernels."""
     _say(f"rounding fmt={fmt} gl={gl_name}")
-    case = H.make_case(fmt, len(gl), 2048, 512, gl, seed=len(fmt) + gl[0])
+    case = H.make_case(fmt, len(gl), 2048, N, gl, seed=len(fmt) + gl[0])
+    assert (H.kernel_of(case, "gemm"), H.kernel_of(case, "gemv")) == kernels
     dev = H.upload(case)
     ref = {False: H.oracle_out(case, gemv=False), True: H.oracle_out(case, gemv=True)}
     apart = float(np.mean(ref[False] != ref[True]))

@@ -22,6 +22,7 @@ def test_strips(fmt, width, K):
     case = H.make_case(fmt, len(COUNTS), K, N, np.cumsum(COUNTS), seed=K + width, extra_rows=2)
     used = int(case["group_list"][-1])
     for op in ("gemm",) if fmt == "int8" else ("gemm", "gemv"):
+        assert H.kernel_of(case, op) == f"strips_{width}"
         _say(f"strips {op} {fmt} width={width} K={K}")
         got = H.run_cabi(case, H.upload(case), op)
         H.assert_close(got, H.oracle_out(case, gemv=op == "gemv"), rows=slice(0, used), what=f"{op} {fmt} width={width} K={K}")
@@ -56,7 +57,7 @@ def test_passes_of_unevenly_owned_rows(fmt):
     counts[[0, 2, 3, 63, 64, 256, 299]] = [33, 1, 16, 17, 38, 1, 20]
     case = H.make_case(fmt, len(counts), 256, 256, np.cumsum(counts), seed=5, extra_rows=1)
     used = int(case["group_list"][-1])
-    assert len(case["x"]) * 256 <= 32768   # few enough columns for the kernel
+    assert H.kernel_of(case, "gemm") == H.kernel_of(case, "gemv") == "strips_128"
     for op in ("gemm", "gemv"):
         _say(f"strips passes {fmt} {op}")
         got = H.run_cabi(case, H.upload(case), op)

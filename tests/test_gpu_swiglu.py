@@ -55,6 +55,21 @@ def test_swiglu_epilogue(fmt, gl):
     assert (got[gl[-1]:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
 
 
+@pytest.mark.parametrize("fmt,kernel", [("fp4", "tiles_pair_small"), ("int4", "tiles_pair_small"), ("fp8", "tiles_pair"), ("int8", "tiles_pair")])
+def test_swiglu_decode_batches_on_tiles(fmt, kernel):
+    """Batches of few rows per expert in more columns than strips take: row counts on both sides of the 16-row blocks and of
+    the small kind's tiles of two of them, several tiles per expert, experts without rows."""
+    _say(f"swiglu {fmt} decode on tiles")
+    counts = [1, 0, 4, 5, 16, 17, 32, 33, 70, 0, 3, 8, 9, 7] + [0] * 8
+    case = H.make_case(fmt, len(counts), 256, 2048, np.cumsum(counts), seed=len(fmt), extra_rows=2)
+    assert H.kernel_of(case, "gemm", swiglu=True) == kernel
+    if fmt in ("int4", "int8"):
+        case["x"] = oracle.f32_to_bf16_bits(oracle.bf16_bits_to_f32(case["x"]) * 4.0)
+    got, used = _run(case), sum(counts)
+    H.assert_close(got, _expected(case), rows=slice(0, used), what=f"swiglu {fmt} decode on tiles")
+    assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
+
+
 @pytest.mark.parametrize("fmt", K_CONTIG)
 @pytest.mark.parametrize("gl", [[2, 3, 4, 40], [130, 130, 143, 300, 301], [0, 7, 7, 8], [0, 200, 200, 200]],
                          ids=["small", "prefill", "decode", "one_big"])
