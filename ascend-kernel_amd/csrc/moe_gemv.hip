@@ -80,7 +80,7 @@ __device__ __forceinline__ int xs_unit(int k8) {
 template <int FMT, int MG>
 __device__ __forceinline__ void gemv_kmajor_rows(const uint8_t* __restrict__ wg, const uint16_t* __restrict__ sg,
                                                  const uint16_t* __restrict__ x, uint16_t* __restrict__ y,
-                                                 u32x4_t* xs, float* sums, int64_t row0, int n0, int N, int K, int epilogue) {
+                                                 u32x4_t* xs, int64_t row0, int n0, int N, int K, int epilogue) {
     constexpr int CH = KMajor<FMT>::CH;
     constexpr int U = CH / 8;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -170,8 +170,10 @@ __device__ __forceinline__ void gemv_kmajor_rows(const uint8_t* __restrict__ wg,
         if constexpr (FMT == MOE_FMT_BF16) {
             if (epilogue == MOE_EPILOGUE_SWIGLU) {
                 // the workgroup's 32 weight rows are 16 gate rows (wavefronts 0, 1) and the 16 up rows that belong to them;
-                // the sums meet in LDS (the barriers ahead of the next pass's x keep its sums from these)
+                // the sums meet in LDS, where x was (the barrier ahead of the next pass's x keeps that from these)
                 static_assert(KMajor<FMT>::NR_WG == 4 * GVK_NRW, "one step of the workgroup's 4 wavefronts");
+                float* const sums = reinterpret_cast<float*>(xs);
+                __syncthreads();
 #pragma unroll
                 for (int j = 0; j < GVK_NRW; ++j)
 #pragma unroll
@@ -205,7 +207,6 @@ __global__ __launch_bounds__(256) void gemv_kmajor_kernel(const uint16_t* __rest
                                                           const int64_t* __restrict__ gl, uint16_t* __restrict__ y,
                                                           int64_t M, int K, int N, int epilogue) {
     extern __shared__ u32x4_t xs[];
-    __shared__ float sums[GV_ROWS * 32];
     const int g = blockIdx.y, n0 = blockIdx.x * KMajor<FMT>::NR_WG;
     int64_t start, end;
     group_rows(gl, g, M, start, end);
@@ -215,10 +216,10 @@ __global__ __launch_bounds__(256) void gemv_kmajor_kernel(const uint16_t* __rest
     for (int64_t row0 = start; row0 < end; row0 += GV_ROWS) {
         const int mg = (int)min((int64_t)GV_ROWS, end - row0);
         switch (mg) {
-            case 1: gemv_kmajor_rows<FMT, 1>(wg, sg, x, y, xs, sums, row0, n0, N, K, epilogue); break;
-            case 2: gemv_kmajor_rows<FMT, 2>(wg, sg, x, y, xs, sums, row0, n0, N, K, epilogue); break;
-            case 3: gemv_kmajor_rows<FMT, 3>(wg, sg, x, y, xs, sums, row0, n0, N, K, epilogue); break;
-            default: gemv_kmajor_rows<FMT, 4>(wg, sg, x, y, xs, sums, row0, n0, N, K, epilogue); break;
+            case 1: gemv_kmajor_rows<FMT, 1>(wg, sg, x, y, xs, row0, n0, N, K, epilogue); break;
+            case 2: gemv_kmajor_rows<FMT, 2>(wg, sg, x, y, xs, row0, n0, N, K, epilogue); break;
+            case 3: gemv_kmajor_rows<FMT, 3>(wg, sg, x, y, xs, row0, n0, N, K, epilogue); break;
+            default: gemv_kmajor_rows<FMT, 4>(wg, sg, x, y, xs, row0, n0, N, K, epilogue); break;
         }
     }
 }
@@ -556,7 +557,8 @@ static int launch_fp4_mfma(const moe_grouped_args* a, hipStream_t stream) {
 
 template <int FMT>
 static int launch_kmajor(const moe_grouped_args* a, hipStream_t stream) {
-    const size_t lds = (size_t)GV_ROWS * GV_KC / 8 * 16;
+    constexpr size_t lds = (size_t)GV_ROWS * GV_KC / 8 * 16;
+    static_assert(lds <= 64 * 1024, "what a kernel without static LDS may have unasked");
     dim3 grid((unsigned)((a->N + KMajor<FMT>::NR_WG - 1) / KMajor<FMT>::NR_WG), (unsigned)a->G);
     hipLaunchKernelGGL((gemv_kmajor_kernel<FMT>), grid, dim3(256), lds, stream,
                        static_cast<const uint16_t*>(a->x), static_cast<const uint8_t*>(a->weight),
