@@ -13,7 +13,20 @@ static int64_t columns(const moe_grouped_args* a) { return std::min(a->M, a->G) 
 // workgroup per 256 columns (the two compute the same).  4 rows per expert, vector / tiles:
 // 64 experts of 7168 x 2048 (512 tiles) 402 / 303 us, 16 of 7168 x 4096 (256) 208 / 162, 64 of 2048 x 1024 (256)
 // 88 / 65, but 8 of 7168 x 4096 (128) 106 / 129, 8 of 7168 x 512 (16) 50 / 80; 2 rows, 512 tiles: 264 / 262.
-static bool bf16_vector_preferred(const moe_grouped_args* a) { return a->M <= (columns(a) >= 65536 ? 2 : 4) * a->G; }
+// With the SwiGLU epilogue the line lies lower: an expert's passes are one chain in its workgroups, which is what unevenly
+// routed rows wait for, and where K is a multiple of 2048 the tiles start all over K and are faster.  Routing skew 0.25 / 1
+// (standard deviation of a per-expert bias of the logits), vector kernel against tiles, us: 256 experts of 2048 x 2048,
+// 2 rows per expert on average 344 / 294 against 318 / 179, 1 row 216 / 158 against 233 / 138; 8 of 4096 x 7168, 4 rows 131 / 139
+// against 81 / 81, 1 row 63 / 62 against 75 / 75; other K: 64 of 7168 x 2048, 2 rows 267 / 247 against 300 / 271; 16 of 7168 x 3584, 4 rows
+// 174 / 173 against 142 / 138, 2 rows 114 / 116 against 139 / 134.  Up to 32 rows in all, which are few passes however they are
+// routed, in few columns: 4 rows on 8 of 2048 x 2048 26 / 31 against 29 / 29, 8 of 7168 x 4096 111 / 125 against 130 / 130; but 64
+// rows, 4 on 16 of 3072 x 1024, 42 / 69 against 40 / 40.
+static bool bf16_vector_preferred(const moe_grouped_args* a) {
+    const bool spread = a->K % 2048 == 0;
+    if (a->epilogue != MOE_EPILOGUE_SWIGLU) return a->M <= (columns(a) >= 65536 ? 2 : 4) * a->G;
+    if (a->M <= 32 && columns(a) <= (spread ? 16384 : 32768)) return a->M <= 4 * a->G;
+    return a->M <= (spread ? 1 : 2) * a->G;
+}
 
 static GroupedKernel bf16_kernel(const moe_grouped_args* a, bool gemv_op) {
     if (bf16_vector_preferred(a)) return GroupedKernel::VECTOR;
@@ -27,13 +40,20 @@ static GroupedKernel bf16_kernel(const moe_grouped_args* a, bool gemv_op) {
 
 // fp4 [N, K/2].  The matrix-core GEMV kernel reads every weight row as contiguous runs, takes 16 rows of an expert per pass and
 // has a variant with the GEMM's weight rounding; the bound for the GEMM op is where the k-split tiles overtake it (256 experts
-// of 7168 x 2048: 8 rows per expert 496 vs 631 us, 16 rows 754 vs 651 us).  With the
-// SwiGLU epilogue, fp4_b32: 16 tokens x 8 on 256 experts of 7168 x 4096 306 vs 468 us, 8 rows of 8 experts of
-// 4096 x 1024 17 vs 36, 8 rows per expert on 256 of 2048 x 1024 95 vs 99; 12 per expert on 8 of 4096 x 2048 39 vs 37.
+// of 7168 x 2048: 8 rows per expert 496 vs 631 us, 16 rows 754 vs 651 us).  With the SwiGLU epilogue, fp4_b32, routing skew
+// 0.25 / 1 (see bf16), this kernel against tiles, us: 256 experts of 2048 x 1024, 4 rows per expert on average 63 / 62 against
+// 84 / 59, 5 rows 66 / 77 against 87 / 59, 8 rows 83 / 102 against 91 / 67 (an expert of 109 rows is 7 passes in a row); 256 of
+// 7168 x 4096, 4 rows 809 / 568 against 1145 / 663; 128 of 4096 x 1536, 8 rows 120 / 144 against 132 / 88.  Up to 64 rows in all,
+// four passes at most: 8 of 4096 x 2048, 8 rows 23 / 39 against 36 / 36.
+static bool fp4_rows_preferred(const moe_grouped_args* a) {
+    if (a->epilogue != MOE_EPILOGUE_SWIGLU) return a->M <= 12 * a->G;
+    return a->M <= (a->M <= 64 ? 8 : 5) * a->G;
+}
+
 static GroupedKernel fp4_kcontiguous_kernel(const moe_grouped_args* a, bool gemv_op) {
     const bool whole = a->K % FP4_ROWS_K == 0;
     if (gemv_op) return whole ? GroupedKernel::FP4_ROWS : GroupedKernel::VECTOR;
-    return whole && a->M <= (a->epilogue == MOE_EPILOGUE_SWIGLU ? 8 : 12) * a->G ? GroupedKernel::FP4_ROWS : GroupedKernel::TILES_PAIR;
+    return whole && fp4_rows_preferred(a) ? GroupedKernel::FP4_ROWS : GroupedKernel::TILES_PAIR;
 }
 
 // Strips for launches of up to 128 tiles of 256 columns, i.e. half of the CUs, and decode-like batches: with 32768 columns (16

@@ -41,7 +41,11 @@ def test_k_contiguous_fp4(fmt):
     at = lambda op, r, K, swiglu=False: kernel(fmt, op, r * 64, 64, K, 2048, swiglu)   # noqa: E731
     assert (at("gemv", 1, 7168), at("gemv", 100, 7168), at("gemv", 1, 7168 + 32)) == ("fp4_rows", "fp4_rows", "vector")
     assert (at("gemm", 12, 7168), at("gemm", 13, 7168), at("gemm", 1, 7168 + 128)) == ("fp4_rows", "tiles_pair", "tiles_pair")
-    assert (at("gemm", 8, 7168, True), at("gemm", 9, 7168, True)) == ("fp4_rows", "tiles_pair")
+    # with SwiGLU, 5 rows per expert; 8 with up to 64 rows in all
+    assert (at("gemm", 5, 7168, True), at("gemm", 6, 7168, True)) == ("fp4_rows", "tiles_pair")
+    few = lambda M, G: kernel(fmt, "gemm", M, G, 4096, 2048, True)   # noqa: E731
+    assert (few(64, 8), few(65, 8)) == ("fp4_rows", "tiles_pair")
+    assert (few(32, 4), few(33, 4)) == ("fp4_rows", "tiles_pair")
 
 
 def test_bf16():
@@ -50,6 +54,14 @@ def test_bf16():
         assert (at(op, 2 * 64, 64, 2048), at(op, 2 * 64 + 1, 64, 2048)) == ("vector", "tiles_bf16")
     assert (at("gemm", 4 * 8, 8, 4096), at("gemm", 4 * 8 + 1, 8, 4096)) == ("vector", "tiles_bf16")
     assert (at("gemv", 6 * 8, 8, 512), at("gemv", 6 * 8 + 1, 8, 512)) == ("vector", "tiles_bf16")
+    # with SwiGLU
+    swi = lambda M, G, N, K: kernel("bf16", "gemm", M, G, K, N, True)   # noqa: E731
+    assert (swi(256, 256, 2048, 4096), swi(257, 256, 2048, 4096)) == ("vector", "tiles_bf16")
+    assert (swi(512, 256, 2048, 7168), swi(513, 256, 2048, 7168)) == ("vector", "tiles_bf16")
+    # up to 32 rows
+    assert (swi(32, 8, 2048, 4096), swi(32, 8, 2304, 4096)) == ("vector", "tiles_bf16")
+    assert (swi(32, 8, 4096, 7168), swi(32, 8, 4352, 7168)) == ("vector", "tiles_bf16")
+    assert (swi(28, 7, 2048, 4096), swi(29, 7, 2048, 4096), swi(33, 9, 1024, 4096)) == ("vector", "tiles_bf16", "tiles_bf16")
     # sizes that the tiles do not take
     assert at("gemv", 1000, 8, 2049) == at("gemv", 1000, 8, 2048, K=7168 + 32) == "vector"
 

@@ -85,6 +85,21 @@ def test_swiglu_epilogue_k_contiguous(fmt, gl):
     assert (got[gl[-1]:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
 
 
+@pytest.mark.parametrize("fmt,kernel,gl", [("bf16", "vector", [0, 9, 9, 10]), ("fp4_b32", "fp4_rows", [0, 20, 21, 30]),
+                                           ("fp4_b16", "fp4_rows", [1, 1, 25, 30])])
+def test_swiglu_passes_over_the_weights(fmt, kernel, gl):
+    """An expert with more rows than one pass of the weight-streaming kernels: the sums of one pass lie where the next one
+    puts its x (bf16) or its scales (fp4)."""
+    _say(f"swiglu {fmt} passes")
+    case = H.make_case(fmt, len(gl), 512, 512, gl, seed=len(fmt), extra_rows=2)
+    assert H.kernel_of(case, "gemm", swiglu=True) == kernel
+    if fmt == "bf16":
+        case["x"] = oracle.f32_to_bf16_bits(oracle.bf16_bits_to_f32(case["x"]) * 4.0)
+    got = _run(case)
+    H.assert_close(got, _expected(case), rows=slice(0, gl[-1]), what=f"swiglu {fmt} passes")
+    assert (got[gl[-1]:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
+
+
 def test_swiglu_fp8_half_empty_last_tile():
     _say("swiglu fp8 N=384")
     gl = [5, 140, 140, 301]
