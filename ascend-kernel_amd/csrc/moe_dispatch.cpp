@@ -28,14 +28,25 @@ static bool bf16_vector_preferred(const moe_grouped_args* a) {
     return a->M <= (spread ? 1 : 2) * a->G;
 }
 
+// Tiles of at most 128 rows where tiles of 224, evenly filled, would be no more than half as many as the 256 CUs: an expert's
+// rows then go to two CUs or more, whose workgroups share a weight slice in L2.  us, 176-row tiles of an earlier kernel / 224 / 128:
+// 64 experts of 4096 x 512, 160 rows each (128 tiles) 115 / 117 / 88, unevenly routed (skew 0.5, see above) 114 / 120 / 99; 16 of
+// 4096 x 2048, 160 rows 98 / 101 / 76, unevenly 97 / 100 / 97; 8 of 7168 x 2048, 160 rows 133 / 121 / 96; 8 of 4096 x 1024,
+// 256 rows (64 tiles) 75 / 66 / 54; 75 rows, one tile either way, 116 / 89 / 91.  96 rows are as good with even routing, but unevenly
+// routed they make a few tiles more than there are CUs (64 of 4096 x 512: 134 us); 64 rows lose (143).
+static GroupedKernel bf16_tiles(const moe_grouped_args* a) {
+    const int64_t experts = std::max(std::min(a->M, a->G), (int64_t)1), chunks = (a->M + BF16_ROWS * experts - 1) / (BF16_ROWS * experts);
+    return 2 * experts * chunks * ((a->N + 255) / 256) <= 256 ? GroupedKernel::TILES_BF16_128 : GroupedKernel::TILES_BF16;
+}
+
 static GroupedKernel bf16_kernel(const moe_grouped_args* a, bool gemv_op) {
     if (bf16_vector_preferred(a)) return GroupedKernel::VECTOR;
-    if (!gemv_op) return GroupedKernel::TILES_BF16;
+    if (!gemv_op) return bf16_tiles(a);
     // The GEMV op takes sizes that the tiles do not, and with few columns the vector kernel stays ahead a little longer.
     // 64 experts of 7168 x 2048: 16 rows per expert 1225 -> 331 us on the tiles, 64 rows 4668 -> 405.  Few
     // columns: 6 rows per expert 77 / 81 us on 8 experts of 7168 x 512, 8 rows 93 / 81; 6 rows on 8 of 4096 x 2048 79 / 71.
     const bool fits = a->K % 64 == 0 && a->N % 256 == 0;
-    return fits && (a->N * a->G >= 16384 || a->M > 6 * a->G) ? GroupedKernel::TILES_BF16 : GroupedKernel::VECTOR;
+    return fits && (a->N * a->G >= 16384 || a->M > 6 * a->G) ? bf16_tiles(a) : GroupedKernel::VECTOR;
 }
 
 // fp4 [N, K/2].  The matrix-core GEMV kernel reads every weight row as contiguous runs, takes 16 rows of an expert per pass and
@@ -116,6 +127,7 @@ const char* grouped_kernel_name(GroupedKernel k) {
         case GroupedKernel::TILES_PAIR_EXACT16: return "tiles_pair_exact16";
         case GroupedKernel::TILES_QUAD: return "tiles_quad";
         case GroupedKernel::TILES_BF16: return "tiles_bf16";
+        case GroupedKernel::TILES_BF16_128: return "tiles_bf16_128";
     }
     return nullptr;
 }

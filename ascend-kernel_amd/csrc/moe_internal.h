@@ -28,10 +28,12 @@ enum class GroupedKernel {
     VECTOR,               // K-contiguous containers without matrix cores (moe_gemv.hip)
     FP4_ROWS,             // K-contiguous fp4, 16 rows of an expert per pass (moe_gemv.hip)
     STRIPS_32, STRIPS_64, STRIPS_128,   // N-contiguous containers in strips of that many columns (moe_stream.hip)
-    TILES_PAIR, TILES_PAIR_EXACT, TILES_PAIR_SMALL, TILES_PAIR_EXACT16, TILES_QUAD, TILES_BF16   // kinds of moe_gemm.hip
+    TILES_PAIR, TILES_PAIR_EXACT, TILES_PAIR_SMALL, TILES_PAIR_EXACT16, TILES_QUAD,   // kinds of moe_gemm.hip
+    TILES_BF16, TILES_BF16_128   // tiles of up to BF16_ROWS, of up to 128 rows
 };
 constexpr int FP4_ROWS_K = 512;   // K of an FP4_ROWS call is a multiple
 constexpr int PAIR_ROWS = 160;    // rows of the largest tile of the quantized containers
+constexpr int BF16_ROWS = 224;    // rows of the largest bf16 tile
 // the kernel of a valid call, by its sizes, format and epilogue (moe_dispatch.cpp)
 GroupedKernel grouped_kernel(const moe_grouped_args* a, bool gemv_op);
 const char* grouped_kernel_name(GroupedKernel k);

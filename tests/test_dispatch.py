@@ -52,16 +52,20 @@ def test_bf16():
     at = lambda op, M, G, N, K=7168: kernel("bf16", op, M, G, K, N)   # noqa: E731
     for op in ("gemm", "gemv"):
         assert (at(op, 2 * 64, 64, 2048), at(op, 2 * 64 + 1, 64, 2048)) == ("vector", "tiles_bf16")
-    assert (at("gemm", 4 * 8, 8, 4096), at("gemm", 4 * 8 + 1, 8, 4096)) == ("vector", "tiles_bf16")
-    assert (at("gemv", 6 * 8, 8, 512), at("gemv", 6 * 8 + 1, 8, 512)) == ("vector", "tiles_bf16")
+    assert (at("gemm", 4 * 8, 8, 4096), at("gemm", 4 * 8 + 1, 8, 4096)) == ("vector", "tiles_bf16_128")
+    assert (at("gemv", 6 * 8, 8, 512), at("gemv", 6 * 8 + 1, 8, 512)) == ("vector", "tiles_bf16_128")
+    # up to 128 tiles of 224 rows
+    for op in ("gemm", "gemv"):
+        assert (at(op, 224 * 64, 64, 512), at(op, 224 * 64 + 1, 64, 512)) == ("tiles_bf16_128", "tiles_bf16")
+        assert (at(op, 1000, 64, 512), at(op, 1000, 64, 768), at(op, 1000, 129, 256)) == ("tiles_bf16_128", "tiles_bf16", "tiles_bf16")
     # with SwiGLU
     swi = lambda M, G, N, K: kernel("bf16", "gemm", M, G, K, N, True)   # noqa: E731
     assert (swi(256, 256, 2048, 4096), swi(257, 256, 2048, 4096)) == ("vector", "tiles_bf16")
     assert (swi(512, 256, 2048, 7168), swi(513, 256, 2048, 7168)) == ("vector", "tiles_bf16")
     # up to 32 rows
-    assert (swi(32, 8, 2048, 4096), swi(32, 8, 2304, 4096)) == ("vector", "tiles_bf16")
+    assert (swi(32, 8, 2048, 4096), swi(32, 8, 2304, 4096)) == ("vector", "tiles_bf16_128")
     assert (swi(32, 8, 4096, 7168), swi(32, 8, 4352, 7168)) == ("vector", "tiles_bf16")
-    assert (swi(28, 7, 2048, 4096), swi(29, 7, 2048, 4096), swi(33, 9, 1024, 4096)) == ("vector", "tiles_bf16", "tiles_bf16")
+    assert (swi(28, 7, 2048, 4096), swi(29, 7, 2048, 4096), swi(33, 9, 1024, 4096)) == ("vector", "tiles_bf16_128", "tiles_bf16_128")
     # sizes that the tiles do not take
     assert at("gemv", 1000, 8, 2049) == at("gemv", 1000, 8, 2048, K=7168 + 32) == "vector"
 

@@ -439,10 +439,12 @@ def test_gemv_n_contiguous_row_counts_up_to_and_beyond_32(fmt, K, N, group, more
 @pytest.mark.parametrize("fmt,op,G,style", [
     ("int4", "gemv", 2100, "decode"), ("fp4", "gemv", 2100, "decode"), ("fp8", "gemv", 2100, "decode"),
     ("int4", "gemm", 2100, "decode"), ("int4", "gemm", 2100, "prefill"),
-    # beyond what LDS holds a table for (about 3000 experts next to the small stages, 2700 / 5000 next to the large)
+    # both sides of what LDS holds next to the rings of the bf16 tiles: the row bounds, the tile table
+    ("bf16", "gemm", 447, "prefill"), ("bf16", "gemm", 448, "prefill"), ("bf16", "gemm", 895, "prefill"), ("bf16", "gemm", 896, "prefill"),
+    # beyond what LDS holds a table for (1900 to 5600 experts; next to the fp8 GEMV stages 20000)
     ("int4", "gemv", 6000, "decode"), ("int4", "gemm", 6000, "decode"), ("fp8", "gemv", 6000, "decode"),
     ("int4", "gemm", 6000, "prefill"), ("fp4", "gemm", 6000, "prefill"), ("int8", "gemm", 6000, "prefill"),
-    ("fp4_b32", "gemm", 6000, "prefill"), ("bf16", "gemm", 12000, "decode")])
+    ("fp4_b32", "gemm", 6000, "prefill"), ("bf16", "gemm", 12000, "decode"), ("bf16", "gemm", 3000, "prefill")])
 def test_any_number_of_experts(fmt, op, G, style):
     """The grouped GEMM kernels keep the first tile of every expert in LDS while that fits; with more experts (the
     reference loops over any number, grouped_gemm/op_kernel/grouped_matmul_antiquant.h:241-242) they keep one entry
@@ -459,6 +461,7 @@ def test_any_number_of_experts(fmt, op, G, style):
     gl = list(np.cumsum(counts))
     K, N = (64, 256) if fmt == "bf16" else (128, 256)
     case = H.make_case(fmt, G, K, N, gl, seed=12, group=32 if fmt == "int4" else 128 if fmt == "fp8" else 16, extra_rows=3)
+    assert H.kernel_of(case, op) == "vector" if (fmt, style) == ("bf16", "decode") else H.kernel_of(case, op).startswith("tiles")
     got = H.run_cabi(case, H.upload(case), op)
     H.assert_close(got, H.oracle_out(case, gemv=op == "gemv"), rows=slice(0, gl[-1]), what=f"{op} {fmt} G={G}")
     assert (got[gl[-1]:] == 0x7FC0).all()

@@ -38,11 +38,15 @@ def _swiglu(case):
 
 @pytest.mark.parametrize("epilogue", ["none", "swiglu"])
 @pytest.mark.parametrize("K", [64, 128, 192, 448])   # 1, 2, 3 and 7 pairs of steps
-def test_bf16_row_blocks(K, epilogue):
-    """gemm_tile_bf16: every number of 32-row blocks from 1 to 7, the row before and after each, two and three chunks."""
+@pytest.mark.parametrize("tile", [224, 128])
+def test_bf16_row_blocks(tile, K, epilogue):
+    """gemm_tile_bf16: every number of 32-row blocks from 1 to 7, the row before and after each, two and three chunks; and with
+    so few column tiles that an expert's rows are cut into chunks of 128."""
     counts = [rows for b in (32, 64, 96, 128, 160, 192, 224) for rows in (b - 1, b, b + 1)] + [1, 16, 17, 449]
-    _say(f"bf16 row blocks K={K} epilogue={epilogue}")
+    counts += [0] * (129 - len(counts)) if tile == 224 else [257, 385]
+    _say(f"bf16 row blocks K={K} epilogue={epilogue} tiles of {tile} rows")
     case = H.make_case("bf16", len(counts), K, 256, np.cumsum(counts), seed=K, extra_rows=3)
+    assert H.kernel_of(case, "gemm", swiglu=epilogue == "swiglu") == {224: "tiles_bf16", 128: "tiles_bf16_128"}[tile]
     used = int(case["group_list"][-1])
     if epilogue == "swiglu":
         got, want = _swiglu(case)
@@ -61,7 +65,7 @@ def test_bf16_starts_all_over_k(K, epilogue):
     counts = [(33, 7, 0, 64, 1, 70)[g % 6] for g in range(pairs // 2 + 1)]
     _say(f"bf16 starts K={K} epilogue={epilogue}")
     case = H.make_case("bf16", len(counts), K, 256, np.cumsum(counts), seed=K, extra_rows=3)
-    assert H.kernel_of(case, "gemm", swiglu=epilogue == "swiglu") == "tiles_bf16"
+    assert H.kernel_of(case, "gemm", swiglu=epilogue == "swiglu") == "tiles_bf16_128"
     used = int(case["group_list"][-1])
     if epilogue == "swiglu":
         got, want = _swiglu(case)
