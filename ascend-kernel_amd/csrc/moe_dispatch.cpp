@@ -14,18 +14,17 @@ static int64_t columns(const moe_grouped_args* a) { return std::min(a->M, a->G) 
 // 64 experts of 7168 x 2048 (512 tiles) 402 / 303 us, 16 of 7168 x 4096 (256) 208 / 162, 64 of 2048 x 1024 (256)
 // 88 / 65, but 8 of 7168 x 4096 (128) 106 / 129, 8 of 7168 x 512 (16) 50 / 80; 2 rows, 512 tiles: 264 / 262.
 // With the SwiGLU epilogue the line lies lower: an expert's passes are one chain in its workgroups, which is what unevenly
-// routed rows wait for, and where K is a multiple of 2048 the tiles start all over K and are faster.  Routing skew 0.25 / 1
-// (standard deviation of a per-expert bias of the logits), vector kernel against tiles, us: 256 experts of 2048 x 2048,
-// 2 rows per expert on average 344 / 294 against 318 / 179, 1 row 216 / 158 against 233 / 138; 8 of 4096 x 7168, 4 rows 131 / 139
-// against 81 / 81, 1 row 63 / 62 against 75 / 75; other K: 64 of 7168 x 2048, 2 rows 267 / 247 against 300 / 271; 16 of 7168 x 3584, 4 rows
-// 174 / 173 against 142 / 138, 2 rows 114 / 116 against 139 / 134.  Up to 32 rows in all, which are few passes however they are
-// routed, in few columns: 4 rows on 8 of 2048 x 2048 26 / 31 against 29 / 29, 8 of 7168 x 4096 111 / 125 against 130 / 130; but 64
-// rows, 4 on 16 of 3072 x 1024, 42 / 69 against 40 / 40.
+// routed rows wait for.  Vector / tiles in us at a routing skew (standard deviation of a per-expert bias of the logits) of 0.25
+// and of 1, by rows per expert on average.  2 rows: 64 experts of 7168 x 2048 267 / 300 and 247 / 271, 64 of 2560 x 2048
+// 108 / 128 and 112 / 112, 128 of 3072 x 1536 176 / 199 and 159 / 131; but with short rows of K, 128 of 1536 x 1536 116 / 108 and
+// 108 / 65, 256 of 2048 x 2048 344 / 318 and 294 / 179, and at K = 4096, where the tiles start all over K, 128 of 4096 x 1536
+// 268 / 245 and 221 / 164.  1 row: 256 of 2048 x 2048 216 / 233 and 158 / 138.  Up to 32 rows in all, few passes however
+// they are routed, in few columns, 4 rows: 8 of 2048 x 2048 26 / 29 and 31 / 29, 8 of 7168 x 4096 111 / 130 and 125 / 130,
+// but 8 of 3584 x 4096 63 / 47 and 71 / 47.
 static bool bf16_vector_preferred(const moe_grouped_args* a) {
-    const bool spread = a->K % 2048 == 0;
     if (a->epilogue != MOE_EPILOGUE_SWIGLU) return a->M <= (columns(a) >= 65536 ? 2 : 4) * a->G;
-    if (a->M <= 32 && columns(a) <= (spread ? 16384 : 32768)) return a->M <= 4 * a->G;
-    return a->M <= (spread ? 1 : 2) * a->G;
+    if (a->M <= 32 && a->K >= 2048 && columns(a) <= (a->K >= 6144 ? 32768 : 16384)) return a->M <= 4 * a->G;
+    return a->M <= (a->K <= 2048 || a->K == 4096 ? 1 : 2) * a->G;
 }
 
 // Tiles of at most 128 rows where tiles of 224, evenly filled, would be no more than half as many as the 256 CUs: an expert's

@@ -60,11 +60,13 @@ def test_bf16():
         assert (at(op, 1000, 64, 512), at(op, 1000, 64, 768), at(op, 1000, 129, 256)) == ("tiles_bf16_128", "tiles_bf16", "tiles_bf16")
     # with SwiGLU
     swi = lambda M, G, N, K: kernel("bf16", "gemm", M, G, K, N, True)   # noqa: E731
-    assert (swi(256, 256, 2048, 4096), swi(257, 256, 2048, 4096)) == ("vector", "tiles_bf16")
-    assert (swi(512, 256, 2048, 7168), swi(513, 256, 2048, 7168)) == ("vector", "tiles_bf16")
-    # up to 32 rows
-    assert (swi(32, 8, 2048, 4096), swi(32, 8, 2304, 4096)) == ("vector", "tiles_bf16_128")
-    assert (swi(32, 8, 4096, 7168), swi(32, 8, 4352, 7168)) == ("vector", "tiles_bf16")
+    for K in (1024, 2048, 4096):
+        assert (swi(256, 256, 2048, K), swi(257, 256, 2048, K)) == ("vector", "tiles_bf16")
+    for K in (2112, 3072, 6144, 7168):
+        assert (swi(512, 256, 2048, K), swi(513, 256, 2048, K)) == ("vector", "tiles_bf16")
+    # up to 32 rows in all
+    assert (swi(32, 8, 2048, 2048), swi(32, 8, 2304, 2048), swi(32, 8, 2048, 1984)) == ("vector", "tiles_bf16_128", "tiles_bf16_128")
+    assert (swi(32, 8, 4096, 6144), swi(32, 8, 4352, 6144), swi(32, 8, 4096, 6080)) == ("vector", "tiles_bf16", "tiles_bf16_128")
     assert (swi(28, 7, 2048, 4096), swi(29, 7, 2048, 4096), swi(33, 9, 1024, 4096)) == ("vector", "tiles_bf16_128", "tiles_bf16_128")
     # sizes that the tiles do not take
     assert at("gemv", 1000, 8, 2049) == at("gemv", 1000, 8, 2048, K=7168 + 32) == "vector"

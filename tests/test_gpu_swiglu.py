@@ -85,7 +85,7 @@ def test_swiglu_epilogue_k_contiguous(fmt, gl):
     assert (got[gl[-1]:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
 
 
-@pytest.mark.parametrize("fmt,kernel,gl", [("bf16", "vector", [0, 9, 9, 10]), ("fp4_b32", "fp4_rows", [0, 20, 21, 30]),
+@pytest.mark.parametrize("fmt,kernel,gl", [("bf16", "vector", [1, 10] + [10] * 13 + [11]), ("fp4_b32", "fp4_rows", [0, 20, 21, 30]),
                                            ("fp4_b16", "fp4_rows", [1, 1, 25, 30])])
 def test_swiglu_passes_over_the_weights(fmt, kernel, gl):
     """An expert with more rows than one pass of the weight-streaming kernels: the sums of one pass lie where the next one
