@@ -54,7 +54,6 @@ struct GemmParams {
     // first tiles only (the row bounds are read from group_list per tile); 0 neither fits: the first tile of every
     // thread's run of experts only, and a tile is found by walking its run (any number of experts)
     int table_mode;
-    int row_blocks; // bf16: 32-row blocks of a tile, at most
     // N-contiguous 4-bit containers: turns a 32-k sub-step index into its scale row
     ScaleRowDivider scale_div;
 };
@@ -252,7 +251,8 @@ __device__ __forceinline__ uint32_t here(uint32_t v) {
 //               exchange, a barrier spans 4 wavefronts instead of 8, and while one workgroup is between two tiles
 //               (stores, tile search, first loads) the other has the SIMDs to itself.  (The N-contiguous containers.)
 //   GK_BF16     gemm_tile_bf16
-enum { GK_PAIR = 2, GK_PAIR_EXACT = 3, GK_PAIR_SMALL = 4, GK_PAIR_EXACT16 = 5, GK_QUAD = 6, GK_BF16 = 7 };
+//   GK_BF16_128 the same with tiles of at most 128 rows (a limit read at run time instead costs the small calls of either 1.5 %)
+enum { GK_PAIR = 2, GK_PAIR_EXACT = 3, GK_PAIR_SMALL = 4, GK_PAIR_EXACT16 = 5, GK_QUAD = 6, GK_BF16 = 7, GK_BF16_128 = 8 };
 constexpr bool pair_exact(int kind) { return kind == GK_PAIR_EXACT || kind == GK_PAIR_EXACT16; }
 constexpr int pair_waves(int kind) { return kind == GK_QUAD ? 4 : 8; }
 constexpr int pair_bk(int kind) { return kind == GK_QUAD ? 32 : 64; }   // k per step
@@ -1189,19 +1189,19 @@ __device__ __forceinline__ void gemm_tile_bf16(const GemmParams& P, u32x4_t* sme
 // ---------------------------------------------------------------------------------
 // Tile scheduler (role of GMMAntiquantProcess::Process,
 // grouped_gemm/op_kernel/grouped_matmul_antiquant.h:241-288).  Expert g with m_g rows
-// has ceil(m_g/BLOCK) row blocks, cut into the fewest chunks of <= mt_max blocks, as
+// has ceil(m_g/BLOCK) row blocks, cut into the fewest chunks of <= MT_MAX blocks, as
 // even as possible; each chunk has N/256 tiles.  prefix[] (in LDS) is the exclusive
 // scan of the tile counts.
 // ---------------------------------------------------------------------------------
-template <int BLOCK>
-__device__ __forceinline__ void expert_chunks(int m, int mt_max, int& chunks, int& bpc) {
+template <int MT_MAX, int BLOCK>
+__device__ __forceinline__ void expert_chunks(int m, int& chunks, int& bpc) {
     const int nblk = (m + BLOCK - 1) / BLOCK;
-    if (nblk <= mt_max) {   // the usual case, without the division
+    if (nblk <= MT_MAX) {   // the usual case, without the division
         chunks = nblk ? 1 : 0;
         bpc = nblk;
         return;
     }
-    chunks = (nblk + mt_max - 1) / mt_max;
+    chunks = (nblk + MT_MAX - 1) / MT_MAX;
     bpc = (nblk + chunks - 1) / chunks;
 }
 
@@ -1217,7 +1217,7 @@ struct KernelCfg {
     }
     static constexpr int WG_PER_CU = pair_wgs();
     static constexpr int WAVES_PER_SIMD = WG_PER_CU * WAVES / 4;
-    static constexpr int MTM = PAIR ? pair_mt_max(KIND) : BF_MT_MAX;             // row blocks per tile
+    static constexpr int MTM = PAIR ? pair_mt_max(KIND) : KIND == GK_BF16_128 ? 4 : BF_MT_MAX;             // row blocks per tile
     // 16-byte LDS units of the tile routine (the tile prefix array follows them)
     static constexpr int lds_units() {
         if constexpr (PAIR)
@@ -1247,7 +1247,6 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
     extern __shared__ u32x4_t smem[];
     constexpr int THREADS = 64 * WAVES;
     constexpr int MTM = C::MTM;
-    const int mt_max = C::PAIR ? MTM : P.row_blocks;
     // [G + 1] first tile of every expert; table_mode 0: [THREADS + 1] first tile of every thread's run of experts
     int* prefix = reinterpret_cast<int*>(smem + C::lds_units());
     // [G + 1] row bounds: rowc[g] = group_list[g - 1] clamped to [0, M] (rowc[0] = 0); expert g owns the rows
@@ -1289,7 +1288,7 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         int sum = 0;
         for (int g = g0; g < g1; ++g) {
             int first, chunks, bpc;
-            expert_chunks<C::BLOCK>(expert_rows(g, first), mt_max, chunks, bpc);
+            expert_chunks<MTM, C::BLOCK>(expert_rows(g, first), chunks, bpc);
             sum += chunks * ntile_n;
         }
         // scan over the threads: within a wavefront by shuffles, across wavefronts through their totals in
@@ -1315,7 +1314,7 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         if (P.table_mode) {
             for (int g = g0; g < g1; ++g) {
                 int first, chunks, bpc;
-                expert_chunks<C::BLOCK>(expert_rows(g, first), mt_max, chunks, bpc);
+                expert_chunks<MTM, C::BLOCK>(expert_rows(g, first), chunks, bpc);
                 prefix[g] = run;
                 run += chunks * ntile_n;
             }
@@ -1405,7 +1404,7 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
                 int tiles = 0;
                 if (ge < e_end) {
                     int first, ch, bp;
-                    expert_chunks<C::BLOCK>(expert_rows(ge, first), mt_max, ch, bp);
+                    expert_chunks<MTM, C::BLOCK>(expert_rows(ge, first), ch, bp);
                     tiles = ch * ntile_n;
                 }
                 int incl = tiles;
@@ -1431,7 +1430,7 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         const int m = __builtin_amdgcn_readfirstlane(expert_rows(g, gfirst));
         const int64_t gbeg = gfirst;
         int chunks, bpc;
-        expert_chunks<C::BLOCK>(m, mt_max, chunks, bpc);
+        expert_chunks<MTM, C::BLOCK>(m, chunks, bpc);
         // row chunks innermost: the tiles that share a weight column tile are neighbours in the order, run at
         // the same time on one XCD and pull that slice of the expert's weights into its L2 once
         const int nt = chunks == 1 ? local : local / chunks, chunk = chunks == 1 ? 0 : local % chunks;
@@ -1514,7 +1513,7 @@ static int launch_gemm_kind(const GemmParams& P, const moe_grouped_args* a, hipS
     if (cus <= 0) return MOE_ERR_NO_DEVICE;
     // persistent grid: as many workgroups as the CUs hold, but no more than an upper bound on the
     // tile count that needs no look at group_list (every expert adds at most one partly filled chunk)
-    const int64_t max_chunks = a->M / (C::BLOCK * (C::PAIR ? C::MTM : P.row_blocks)) + a->G;
+    const int64_t max_chunks = a->M / (C::BLOCK * C::MTM) + a->G;
     const int64_t max_tiles = max_chunks * ((a->N + C::BN - 1) / C::BN);
     const int64_t want = max_tiles < (int64_t)cus * C::WG_PER_CU ? max_tiles : (int64_t)cus * C::WG_PER_CU;
     // a multiple of 8 so that the XCD-aware order covers every tile index
@@ -1553,13 +1552,12 @@ static GemmParams gemm_params(const moe_grouped_args* a) {
     P.slot = -1;
     P.stamp = 0;
     P.table_mode = 0;
-    P.row_blocks = 0;
     P.scale_div = scale_row_divider(a->K, a->scale_rows);
     return P;
 }
 
 int launch_tiles(const moe_grouped_args* a, GroupedKernel kind, hipStream_t stream) {
-    GemmParams P = gemm_params(a);
+    const GemmParams P = gemm_params(a);
     switch (kind) {
         case GroupedKernel::TILES_PAIR:
             switch (a->format) {
@@ -1593,9 +1591,9 @@ int launch_tiles(const moe_grouped_args* a, GroupedKernel kind, hipStream_t stre
         case GroupedKernel::TILES_PAIR_EXACT16:
             return a->format == MOE_FMT_FP4_REF ? launch_gemm_kind<MOE_FMT_FP4_REF, GK_PAIR_EXACT16>(P, a, stream) : MOE_ERR_BAD_FORMAT;
         case GroupedKernel::TILES_BF16:
-        case GroupedKernel::TILES_BF16_128:
-            P.row_blocks = kind == GroupedKernel::TILES_BF16 ? BF_MT_MAX : 4;
             return a->format == MOE_FMT_BF16 ? launch_gemm_kind<MOE_FMT_BF16, GK_BF16>(P, a, stream) : MOE_ERR_BAD_FORMAT;
+        case GroupedKernel::TILES_BF16_128:
+            return a->format == MOE_FMT_BF16 ? launch_gemm_kind<MOE_FMT_BF16, GK_BF16_128>(P, a, stream) : MOE_ERR_BAD_FORMAT;
         default: return MOE_ERR_BAD_FORMAT;
     }
 }
