@@ -1084,8 +1084,9 @@ __device__ __forceinline__ void gemm_tile_bf16(const GemmParams& P, u32x4_t* sme
     const int np = P.K >> 6;
     // Where in K a column tile starts (it goes round).  L2's 16 channels take 256 bytes in turn: with weight rows a multiple
     // of 4 KB apart all rows of all tiles, which run nearly in step, would ask one channel at a time, so each column tile
-    // starts in the next one.  K = 2048, 256 experts of N = 1024, 8 rows each: 239 -> 201 us; 64 of N = 2048, 48 rows:
-    // 139 -> 122.  Other K gain nothing and lose the x rows that neighbouring tiles find in L2 (prefill, K = 7168: 481 -> 491).
+    // starts in the next one.  K = 2048, 256 experts of N = 1024, 8 rows each: 239 us without, 201 with (212 with the 4-wavefront
+    // routine this replaced); 64 of N = 2048, 48 rows:
+    // 139 / 122.  Other K gain nothing and lose the x rows that neighbouring tiles find in L2 (prefill, K = 7168: 481 / 491).
     const int rot = P.K % 2048 ? 0 : (int)((unsigned)(2 * (g * ((P.N + GM_BN - 1) / GM_BN) + n0 / GM_BN)) % (unsigned)np);
     auto pair_at = [&](int p) { return p + rot < np ? p + rot : p + rot - np; };
     const int64_t KN = (int64_t)P.K * P.N;

@@ -7,8 +7,8 @@
 // a few 32-k steps ahead, without LDS or barriers, and the partial sums meet once in LDS.  That case (18 MB of fp4 weights and
 // scales): 47.6 -> 11.2 us, int4 48 -> 15, fp8 70 -> 16; two tokens on 256 experts of 7168 x 2048: int4 49 -> 33 us.
 // What bounds it now: the launch, group_list and one step's latency are about 6 us; then what a few wavefronts per SIMD
-// issue (about 1.5 vector instructions per weight, twice that in 32-column strips, where four lanes load a dword of 8 codes
-// and use two of them).
+// issue (about 1.5 vector instructions per weight, 3.2 in 32-column strips, where four lanes load a dword of 8 codes
+// and use two of them; half of a wavefront's time there is waiting for its loads).
 //
 // MFMA: v_mfma_f32_16x16x32_bf16, x rows in A, weights in B.  Lane (i, q) = (lane & 15, lane >> 4) loads, of each of the 8 k
 // rows 8 q + [0, 8) of a step, the dword (T = 8 and bytes: two) with its columns T i + [0, T): the 8 values of one column are
