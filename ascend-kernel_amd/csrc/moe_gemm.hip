@@ -12,14 +12,15 @@
 // grid walks it with an XCD-aware order so that the workgroups of one XCD share the x rows and
 // weight slices of the same experts in that XCD's L2, and takes the last two or three tiles of every
 // workgroup from a work counter (see tile_queue).  Every wavefront owns its columns for ALL
-// rows of the tile, so each weight element is dequantized exactly once per tile.  Two tile routines:
-//   gemm_tile_pair  every quantized container (int4, int8, the K-contiguous fp4 containers, the
-//                   reference's fp4 and fp8); x, packed weights and scales arrive by LDS-direct loads into a
-//                   ring of stages walked by an unrolled k loop.  Either 8 wavefronts, the two of a SIMD
-//                   splitting the k range (int8, fp8, K-contiguous fp4), or 4 wavefronts that each take their
-//                   64 columns through all of k, two such workgroups per CU (int4 and fp4 prefill);
+// rows of the tile, so each weight element is dequantized exactly once per tile.  Three tile routines:
+//   gemm_tile_pair  the N-contiguous containers (int4, int8, the reference's fp4 and fp8); x, packed weights and
+//                   scales arrive by LDS-direct loads into a ring of stages walked by an unrolled k loop.  Either 8
+//                   wavefronts, the two of a SIMD splitting the k range (int8, fp8), or 4 wavefronts that each take
+//                   their 64 columns through all of k, two such workgroups per CU (int4 and fp4 prefill);
 //                   tiles of up to 160 rows, or of up to 32 / 16 rows with small stages (decode batches,
 //                   and the GEMV op's arithmetic on the N-contiguous containers)
+//   gemm_tile_fp4_k the K-contiguous fp4 containers: 4 wavefronts, two workgroups per CU, tiles of up to 160 rows; x in a
+//                   ring of 32-k stages, every wavefront's own weights and scales 128 k at a time
 //   gemm_tile_bf16  the bf16 container: 8 wavefronts, tiles of up to 224 rows, x and weights by LDS-direct loads into
 //                   two rings
 //
@@ -187,7 +188,7 @@ __device__ __forceinline__ uint32_t here(uint32_t v) {
 }
 
 // ---------------------------------------------------------------------------------
-// Tile routine for the quantized containers (int4, int8, reference fp4 / fp8, K-contiguous fp4) with two
+// Tile routine for the N-contiguous containers (int4, int8, reference fp4 / fp8) with two
 // wavefronts per SIMD that split the k range.  Described for int4; what differs for the others follows.
 //
 // A single wavefront issues at most one instruction every ~5 cycles whatever its kind, and an
@@ -232,13 +233,9 @@ __device__ __forceinline__ uint32_t here(uint32_t v) {
 // the bits of the two rounded operations, see i8_one_rounding); fp8 decodes two codes at a time through
 // fp16 (see e4m3_ref_pair_over_256_fp16) and gets the fp32 scale of its 128 x 128 block through the ring,
 // 4 bytes per wavefront and step.
-//
-// K-contiguous fp4 (weight [N, K/2]): a step's tile is 256 weight rows x 32 bytes; MFMA t of a lane takes
-// weight row 64 cw + 16 t + i, whose 8 codes of the sub-step are one dword; the scales [N, K/block] are
-// fetched 16 bytes per row at a time into buffers of their own (see kc_issue_scale).
 // ---------------------------------------------------------------------------------
 // Kernel variants.
-//   GK_PAIR     quantized containers: 8 wavefronts, k range split between the two wavefronts of a SIMD, tiles of
+//   GK_PAIR     N-contiguous containers: 8 wavefronts, k range split between the two wavefronts of a SIMD, tiles of
 //               up to 160 rows
 //   GK_PAIR_SMALL  GK_PAIR with tiles of at most 32 rows: x stages of 4 KB leave LDS for a second workgroup per
 //               CU (decode-sized batches on the 4-bit containers)
@@ -249,10 +246,11 @@ __device__ __forceinline__ uint32_t here(uint32_t v) {
 //               64 columns through the whole k range in steps of 32 k, two workgroups per CU.  The two wavefronts
 //               of a SIMD belong to different workgroups and work on different tiles: no partial sums to
 //               exchange, a barrier spans 4 wavefronts instead of 8, and while one workgroup is between two tiles
-//               (stores, tile search, first loads) the other has the SIMDs to itself.  (The N-contiguous containers.)
+//               (stores, tile search, first loads) the other has the SIMDs to itself.
+//   GK_FP4_K    gemm_tile_fp4_k
 //   GK_BF16     gemm_tile_bf16
 //   GK_BF16_128 the same with tiles of at most 128 rows (a limit read at run time instead costs the small calls of either 1.5 %)
-enum { GK_PAIR = 2, GK_PAIR_EXACT = 3, GK_PAIR_SMALL = 4, GK_PAIR_EXACT16 = 5, GK_QUAD = 6, GK_BF16 = 7, GK_BF16_128 = 8 };
+enum { GK_PAIR = 2, GK_PAIR_EXACT = 3, GK_PAIR_SMALL = 4, GK_PAIR_EXACT16 = 5, GK_QUAD = 6, GK_BF16 = 7, GK_BF16_128 = 8, GK_FP4_K = 9 };
 constexpr bool pair_exact(int kind) { return kind == GK_PAIR_EXACT || kind == GK_PAIR_EXACT16; }
 constexpr int pair_waves(int kind) { return kind == GK_QUAD ? 4 : 8; }
 constexpr int pair_bk(int kind) { return kind == GK_QUAD ? 32 : 64; }   // k per step
@@ -290,13 +288,9 @@ template <int FMT>
 constexpr int pair_sc_units(int kind) {
     return (FMT == MOE_FMT_FP4_REF ? 128 : FMT == MOE_FMT_INT4 ? 64 : FMT == MOE_FMT_FP8_REF ? 8 : 0) * pair_bk(kind) / 64;
 }
-// The K-contiguous fp4 containers keep their scales [N, K/block] outside the stages: 16 bytes (2 or 4 steps'
-// worth) per weight row at a time, three buffers of 256 rows
-template <int FMT>
-constexpr int pair_kc_scale_units() { return (FMT == MOE_FMT_FP4_B32 || FMT == MOE_FMT_FP4_B16) ? 3 * 256 : 0; }
 template <int FMT>
 constexpr int pair_lds_units(int kind) {
-    return pair_stages<FMT>(kind) * (pair_a_units(kind) + pair_b_units<FMT>(kind) + pair_sc_units<FMT>(kind)) + pair_kc_scale_units<FMT>();
+    return pair_stages<FMT>(kind) * (pair_a_units(kind) + pair_b_units<FMT>(kind) + pair_sc_units<FMT>(kind));
 }
 
 // End of a k-split tile.  The two wavefronts of a pair (same columns, the two k halves) hold partial sums of the
@@ -305,17 +299,17 @@ constexpr int pair_lds_units(int kind) {
 // wavefront, the second by h == 1, so both reduce and store at the same time.  Rounds of at most 4 row
 // blocks (8 wavefronts x 4 blocks x 4 KB fit the x stage area, free now).
 // WHOLE: the wavefront holds the whole sums (no k split): it stores all of its row blocks, nothing is exchanged.
-template <int MT, bool KC, bool WHOLE = false>
+template <int MT, bool WHOLE = false>
 __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, f32x4_t (&acc)[MT][4], int h, int cw, int lane,
                                             int col0, int64_t row0, int rows, int n0, const Ticket& tk) {
-    const int i = lane & 15, q = lane >> 4;
+    const int q = lane >> 4;
     const bool takes = tk.counter != nullptr && threadIdx.x == 0;
     unsigned next_tile = 0;
     if (takes) next_tile = queue_draw_raw(tk.counter);
     constexpr int MH = (MT + 1) / 2, RR = MH < 4 ? MH : 4, ROUNDS = (MH + RR - 1) / RR;
     // the last tile of an N that is not a multiple of 256 (the reference's fp8 container: multiples of 128)
     // computes columns past N from whatever follows in the slab: they are not stored
-    const bool live = KC || n0 + col0 < P.N;
+    const bool live = n0 + col0 < P.N;
     const bool swi = P.epilogue == MOE_EPILOGUE_SWIGLU;
     // stores go through a buffer resource that ends after the tile's last valid row: those to padded rows
     // fall outside it and are dropped
@@ -323,18 +317,7 @@ __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, 
     const rsrc_t ry = make_rsrc(P.y + row0 * (int64_t)NO, (int64_t)rows * NO * 2);
     auto store_block = [&](int mt) {
         if (!live) return;
-        if (swi && KC) {
-            // K-contiguous containers: the weight rows come in blocks of 32 = (16 gate rows, 16 up rows), which are
-            // the MFMAs t = (0, 1) and (2, 3) of this lane; y has N / 2 columns
-            const int vo = (4 * q * NO + ((n0 + 64 * cw) >> 1) + i) * 2;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int u = 0; u < 2; ++u)
-                    __builtin_amdgcn_raw_buffer_store_b16(
-                        (uint16_t)(pack_bf16_rne(swiglu(acc[mt][2 * u][r], acc[mt][2 * u + 1][r]), 0.f) & 0xffffu), ry,
-                        vo + 32 * u, (16 * mt + r) * NO * 2, 0);
-        } else if (swi) {
+        if (swi) {
             // this lane's 4 columns are (gate, gate, up, up) of 2 output columns; y has N / 2 columns
             const int vo = (4 * q * NO + ((n0 + col0) >> 1)) * 2;
 #pragma unroll
@@ -342,15 +325,6 @@ __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, 
                 __builtin_amdgcn_raw_buffer_store_b32(
                     pack_bf16_rne(swiglu(acc[mt][0][r], acc[mt][2][r]), swiglu(acc[mt][1][r], acc[mt][3][r])), ry, vo,
                     (16 * mt + r) * NO * 2, 0);
-        } else if (KC) {
-            // K-contiguous containers: MFMA t holds column 64 cw + 16 t + i, one 2-byte store each
-            const int vy = (4 * q * P.N + n0 + 64 * cw + i) * 2;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(pack_bf16_rne(acc[mt][t][r], 0.f) & 0xffffu), ry,
-                                                          vy + 32 * t, (16 * mt + r) * P.N * 2, 0);
         } else {
             const int vy = (4 * q * P.N + n0 + col0) * 2;
 #pragma unroll
@@ -417,20 +391,15 @@ __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, 
 // the multiplies of the general case, and no masking.
 template <int FMT, int MT, int KIND, bool STACK2 = false>
 __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk) {
-    static_assert(FMT != MOE_FMT_BF16, "the k-split tile routine decodes quantized containers");
+    static_assert(FMT == MOE_FMT_INT4 || FMT == MOE_FMT_INT8 || FMT == MOE_FMT_FP4_REF || FMT == MOE_FMT_FP8_REF, "the N-contiguous containers");
     constexpr bool EXACT = pair_exact(KIND);
     static_assert(!STACK2 || (EXACT && FMT == MOE_FMT_FP4_REF && MT == 1), "two scale groups stacked in one MFMA: fp4, at most 8 rows");
     static_assert(!EXACT || FMT == MOE_FMT_INT4 || FMT == MOE_FMT_FP4_REF || FMT == MOE_FMT_FP8_REF,
                   "un-rounded weights: the N-contiguous containers of the GEMV op");
     constexpr bool FP4 = FMT == MOE_FMT_FP4_REF, I8 = FMT == MOE_FMT_INT8, F8 = FMT == MOE_FMT_FP8_REF;
-    // K-contiguous fp4 (weight [N, K/2], scales [N, K/KBLK]): the step's tile is 256 weight rows x 32 bytes
-    constexpr bool KC = FMT == MOE_FMT_FP4_B32 || FMT == MOE_FMT_FP4_B16;
-    constexpr int KBLK = FMT == MOE_FMT_FP4_B32 ? 32 : 16;
     constexpr bool B8 = I8 || F8;   // one byte per weight: tiles of 64 rows x 256 bytes
     // Q4: the kind without the k split (GK_QUAD): 4 wavefronts, steps of 32 k, every wavefront in every step
     constexpr bool Q4 = KIND == GK_QUAD;
-    static_assert(!Q4 || FMT == MOE_FMT_INT4 || FMT == MOE_FMT_INT8 || FMT == MOE_FMT_FP4_REF || FMT == MOE_FMT_FP8_REF,
-                  "the 4-wavefront kind serves the N-contiguous containers");
     constexpr int NW = pair_waves(KIND);
     constexpr int BK = pair_bk(KIND), S = pair_stages<FMT>(KIND), PAIR_SC_UNITS = pair_sc_units<FMT>(KIND);
     constexpr int PAIR_B_UNITS = pair_b_units<FMT>(KIND);
@@ -463,9 +432,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
 
     const int64_t KN = (int64_t)P.K * P.N;
     const rsrc_t rw = B8 ? make_rsrc(P.w + g * KN, KN) : make_rsrc(P.w + g * (KN >> 1), KN >> 1);
-    const rsrc_t rs = KC ? make_rsrc(static_cast<const uint16_t*>(P.scale) + g * (KN / KBLK), (KN / KBLK) * 2)
-                         : make_rsrc(static_cast<const uint16_t*>(P.scale) + (int64_t)g * P.scale_rows * P.N,
-                                     (int64_t)P.scale_rows * P.N * 2);
+    const rsrc_t rs = make_rsrc(static_cast<const uint16_t*>(P.scale) + (int64_t)g * P.scale_rows * P.N, (int64_t)P.scale_rows * P.N * 2);
     // fp8: the expert's fp32 block scales [K/128, N/128]; this wavefront's 128-column block
     const rsrc_t rs8 = make_rsrc(static_cast<const float*>(P.scale) + (int64_t)g * (P.K >> 7) * (P.N >> 7),
                                  (int64_t)(P.K >> 7) * (P.N >> 7) * 4);
@@ -485,17 +452,13 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     // int8 / fp8 (rows of 256 bytes): instruction e of wavefront wv brings rows 8 wv + 4 e + (lane >> 4); the
     // 64-byte quarters of a row are permuted by (row >> 3) & 3 = wv & 3, so that the four q groups read
     // from different quarters of the banks
-    // K-contiguous fp4: LDS unit 64 wv + lane of the stage holds one 16-byte half of weight row
-    // n = 32 wv + (lane >> 1); the halves of the rows with odd (n >> 3) are swapped (bank spread)
-    const int kc_n = 32 * wv + (lane >> 1);
-    const int vb = KC   ? kc_n * (P.K >> 1) + 16 * ((lane & 1) ^ ((kc_n >> 3) & 1))
-                   : B8 ? (lane >> 4) * P.N + (((lane & 15) ^ (4 * (wv & 3))) * 16)
-                        : (lane >> 3) * (P.N >> 1) + (((lane & 7) ^ (4 * (wv & 1))) * 16);
+    const int vb = B8 ? (lane >> 4) * P.N + (((lane & 15) ^ (4 * (wv & 3))) * 16)
+                      : (lane >> 3) * (P.N >> 1) + (((lane & 7) ^ (4 * (wv & 1))) * 16);
     constexpr int XI = Q4 ? MT : 2 * MT;          // x load instructions per step (1 KB each: 16 or 8 rows)
     constexpr int XROWS = Q4 ? 16 : 8;
     constexpr int NA = (XI + NW - 1) / NW;        // ... per wavefront
     constexpr int NB = B8 ? 2 : 1;                // packed-tile instructions
-    constexpr int NI = NA + NB + ((PAIR_SC_UNITS || KC) ? 1 : 0);   // + this wavefront's share of the step's scales
+    constexpr int NI = NA + NB + (PAIR_SC_UNITS ? 1 : 0);   // + this wavefront's share of the step's scales
     int ja[NA], ca[NA];
 #pragma unroll
     for (int m = 0; m < NA; ++m) {
@@ -506,31 +469,16 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     }
     // (Q4 on the reference's fp4 container: the 32 k of a step are the rows [16 hp, +16) and [32 + 16 hp, +16) of the
     // container's 64-row tile, hp = step & 1: wavefront wv brings the 8 rows from 32 (wv >> 1) + 16 hp + 8 (wv & 1) on)
-    const int cb = KC            ? n0 * (P.K >> 1)
-                   : B8          ? 8 * wv * P.N + n0
+    const int cb = B8            ? 8 * wv * P.N + n0
                    : (Q4 && FP4) ? (32 * (wv >> 1) + 8 * (wv & 1)) * (P.N >> 1) + (n0 >> 1)
                                  : 8 * wv * (P.N >> 1) + (n0 >> 1);
-    const int kb_step = KC ? BK / 2 : B8 ? BK * P.N : BK * (P.N >> 1);
+    const int kb_step = B8 ? BK * P.N : BK * (P.N >> 1);
     // byte offset of step kp's packed rows in the expert's slab
     auto b_step_offset = [&](int kp) {
         if constexpr (Q4 && FP4)
             return ((kp >> 1) * 64 + (kp & 1) * 16) * (P.N >> 1);
         else
             return kp * kb_step;
-    };
-    // K-contiguous fp4 scales.  Fetching the 4 or 8 bytes a weight row needs per step costs a request per
-    // row and step (measured: 20 % of the kernel); instead 16 bytes of a row -- the scales of SUP steps --
-    // are fetched at a time: the load slot of step kt brings, for step index kp = kt + KC_D, the rows
-    // [RPS (kp % SUP), + RPS) of super-block kp / SUP (one lane per row, RPW rows per wavefront) into buffer
-    // (kp / SUP) % 3 of 256 rows x 16 bytes behind the stages.  KC_D = SUP + 3: a load issued in step t is
-    // visible after barrier t + 2, and the scales of step s are read during step s - 1.  Three buffers: the
-    // first load into a buffer comes after the last read of its previous occupant.
-    constexpr int SUP = KBLK == 32 ? 4 : 2, KC_D = SUP + 3, RPS = 256 / SUP, RPW = RPS / 8;
-    const int kc_vs = lane * (P.K / KBLK) * 2;
-    auto kc_issue_scale = [&](int kp) {
-        const int sb = kp / SUP, j = kp % SUP, row = RPS * j + RPW * wv;
-        if (lane < RPW)
-            lds_load16(rs, lds_s + (sb % 3) * 256 + row, kc_vs, (n0 + row) * (P.K / KBLK) * 2 + sb * 16);
     };
     // scales of a step: int4 2 rows of 512 bytes, 128 bytes (8 lanes) per wavefront: bytes [128 (wv & 3), +128) of
     // row wv >> 2; fp4 4 rows (one per 16 k), 256 bytes (16 lanes) per wavefront: bytes [256 (wv & 1), +256) of row wv >> 1
@@ -551,8 +499,6 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             const int e = m - NA;
             lds_load16_at(rw, here(b_at) + ST * (PAIR_B_UNITS * 16) + e * 1024, vb,
                           cb + (B8 ? 4 * e * P.N : 0) + b_step_offset(kt + AHEAD));
-        } else if constexpr (KC) {
-            kc_issue_scale(kt + KC_D);
         } else if constexpr (F8) {
             // the block scale of the stage's 128-k block, 4 bytes by lane 0 (past K: reads as 0, unused)
             if (lane == 0)
@@ -645,11 +591,6 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
                      "s_cbranch_scc1 2f\n\ts_sleep 1\n\ts_branch 1b\n2:"
                      : "=&v"(seen_v), "=&s"(seen_s) : "s"(arrivals_at), "s"((uint32_t)NW * steps), "v"(early) : "memory", "scc");
     };
-    if constexpr (KC) {
-        // the scale loads the groups below do not cover (older than all of them: landed by the first barrier)
-#pragma unroll
-        for (int kp = 0; kp < KC_D - AHEAD; ++kp) kc_issue_scale(kp);
-    }
 #pragma unroll
     for (int st0 = 0; st0 < AHEAD; ++st0) issue_group(st0 - AHEAD, st0);
 #pragma unroll
@@ -686,8 +627,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     // this lane's packed dwords and scales of its sub-step of LDS stage st
     uint32_t r[8];
     u32x2_t sc = {0u, 0u}, sc2 = {0u, 0u};   // sc2: with EXACT, the fp4 scales of the second 16 k of the sub-step
-    // (s: the step the stage belongs to)
-    auto read_raw = [&](int st, int s) {
+    auto read_raw = [&](int st) {
         const uint16_t* sc16 = reinterpret_cast<const uint16_t*>(lds_s + st * PAIR_SC_UNITS);
         if constexpr (FP4) {
             // Reference pre-shuffle (grouped_gemm/test/python/test_group_gemm_fp4.py:129-142): the tile row
@@ -708,22 +648,6 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             } else {
                 sc = *reinterpret_cast<const u32x2_t*>(sc16 + 256 * (2 * h + (q >> 1)) + col0);
             }
-        } else if constexpr (KC) {
-            // MFMA t takes weight row n = 64 cw + 16 t + i: its 8 codes k = 32 h + 8 q + [0, 8) are dword q of
-            // the row's half h; the scale of that block
-            const uint32_t* t32 = reinterpret_cast<const uint32_t*>(lds_b + st * PAIR_B_UNITS);
-            // the row's 8 scales of super-block s / SUP; this lane's block among them
-            const uint16_t* sup = reinterpret_cast<const uint16_t*>(lds_s + ((s / SUP) % 3) * 256) +
-                                  (KBLK == 16 ? 4 * (s % SUP) + 2 * h + (q >> 1) : 2 * (s % SUP) + h);
-            uint32_t s4[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int n = 64 * cw + 16 * t + i;
-                r[t] = t32[(2 * n + (h ^ ((i >> 3) & 1))) * 4 + q];
-                s4[t] = sup[8 * n];
-            }
-            sc[0] = s4[0] | (s4[1] << 16);
-            sc[1] = s4[2] | (s4[3] << 16);
         } else if constexpr (B8) {
             // dword 16 cw + i of each of this lane's 8 k rows; the quarter of the row it lies in is
             // permuted by (row >> 3) & 3 = q (see vb)
@@ -738,7 +662,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             sc = *reinterpret_cast<const u32x2_t*>(sc16 + 256 * h + col0);
         }
     };
-    read_raw(0, 0);
+    read_raw(0);
 
     // One data step; st = step mod S is its LDS stage, sn the next one, sl the stage this step's loads
     // go to (wave-uniform).
@@ -754,7 +678,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
         if constexpr (EXACT) {
             m[0] = m[1] = m[2] = m[3] = FP4 ? 1.f : 512.f;
             z[0] = z[1] = z[2] = z[3] = FP4 ? 0.f : -8.f;
-        } else if constexpr (FP4 || KC) {
+        } else if constexpr (FP4) {
             m[0] = s0; m[1] = s1; m[2] = s2; m[3] = s3;
             z[0] = z[1] = z[2] = z[3] = 0.f;
         } else {
@@ -777,20 +701,6 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
                 // first x fragments of the MFMA phase, read under the rest of the decode
 #pragma unroll
                 for (int f = 0; f < R; ++f) afr[f & 3] = la[x_unit(16 * f + xrow)];
-            }
-            if constexpr (KC) {
-                // dword r[t] = 8 consecutive k of MFMA t's weight row: byte p = the k pair p
-#pragma unroll
-                for (int t = p0; t < p0 + 2; ++t) {
-                    const f32x2_t f0 = e2m1_pair_to_f32<0>(r[t]), f1 = e2m1_pair_to_f32<1>(r[t]);
-                    const f32x2_t f2 = e2m1_pair_to_f32<2>(r[t]), f3 = e2m1_pair_to_f32<3>(r[t]);
-                    bf[t][0] = pack_bf16_rne(f0[0] * m[t], f0[1] * m[t]);
-                    bf[t][1] = pack_bf16_rne(f1[0] * m[t], f1[1] * m[t]);
-                    bf[t][2] = pack_bf16_rne(f2[0] * m[t], f2[1] * m[t]);
-                    bf[t][3] = pack_bf16_rne(f3[0] * m[t], f3[1] * m[t]);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                continue;
             }
             if constexpr (F8) {
                 // byte t of the dwords of k rows 2p, 2p+1, decoded as a pair through fp16 (see
@@ -986,7 +896,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             }
 #pragma unroll
             for (int m = (mt * NI + MT - 1) / MT; m < ((mt + 1) * NI + MT - 1) / MT; ++m) issue(m, kt, sl);
-            if (mt == 0) read_raw(sn, kt + 1);
+            if (mt == 0) read_raw(sn);
             __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_s_setprio(0);
@@ -999,21 +909,10 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     // unrolled over the ring, so that every stage number is a constant and the LDS addresses of a step are
     // immediate offsets (with run-time stage numbers a step spent 9 vector and about 25 scalar instructions on
     // them: measured 10 % of the kernel's time at K = 7168); a tile starts at stage 0
-    // (the K-contiguous containers keep run-time stage numbers: their routine has no registers left for the
-    // unrolled form)
-    if constexpr (!KC) {
-        for (int kt0 = 0; kt0 < nk; kt0 += S) {
+    for (int kt0 = 0; kt0 < nk; kt0 += S) {
 #pragma unroll
-            for (int u = 0; u < S; ++u)
-                if (kt0 + u < nk) step(kt0 + u, u, (u + 1) % S, (u + S - 1) % S);
-        }
-    } else {
-        for (int kt = 0, st = 0, sl = S - 1; kt < nk; ++kt) {
-            const int sn = st == S - 1 ? 0 : st + 1;
-            step(kt, st, sn, sl);
-            st = sn;
-            sl = sl == S - 1 ? 0 : sl + 1;
-        }
+        for (int u = 0; u < S; ++u)
+            if (kt0 + u < nk) step(kt0 + u, u, (u + 1) % S, (u + S - 1) % S);
     }
     if constexpr (!SPLIT_BARRIER)
         if (h == 1) ring_barrier();   // barrier nk-1
@@ -1029,7 +928,186 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[0][t][e] += __shfl_xor(acc[0][t][e], 32);
     }
-    pair_finish<MT, KC, Q4>(P, smem, acc, h, cw, lane, col0, row0, rows, n0, tk);
+    pair_finish<MT, Q4>(P, smem, acc, h, cw, lane, col0, row0, rows, n0, tk);
+}
+
+// ---------------------------------------------------------------------------------
+// Tile routine for the K-contiguous fp4 containers (weights [N, K/2], scales [N, K/16 or K/32]): workgroups of 4 wavefronts,
+// two per CU, as GK_QUAD: wavefront cw takes columns 64 cw .. + 63 of the tile through all of k for up to 160 rows.
+//
+// Bound by issue, as the N-contiguous kinds: 2 vector instructions per weight (exact convert, times its scale, rounded to
+// bf16) beside the MFMAs.  Two workgroups per CU hide each other's barriers and the time between tiles, which the 8-wavefront
+// k-split routine that served these containers before did not.
+// 128 experts of 2048 x 7168, 2047 tokens x 8 rows: fp4_b16 FIGURES_B16 (FIGURES_T).
+//
+// The weight rows of a wavefront's columns are read by that wavefront alone, so its weights and scales are its own business:
+// it loads them for 128 k at a time ("a super-step": 64 bytes of 64 rows, four LDS-direct loads; 32-byte pieces would touch
+// twice as many lines), one super-step ahead, into one of two buffers, and waits for nobody.  The scales of a super-step, 16 or
+// 8 bytes a row, come through registers into 1 KB of the wavefront's own LDS once the last of the previous ones is read.  Only x
+// is shared: a ring of four 32-k stages, three steps ahead, one barrier per step.
+//
+// Step j of a super-step reads dword q of 16-byte unit j of every weight row: the 8 codes k = 32 j + 8 q + [0, 8).  Unit j of
+// the row in slot s lies at position j ^ ((s >> 2) & 3), so that the 64 lanes of a read (16 rows x 4 dwords) hit 64 banks.
+// Column t of a lane is 4 i + t (SwiGLU: two gate and two up rows of two adjacent output columns), as in gemm_tile_bf16.
+// ---------------------------------------------------------------------------------
+constexpr int FK_MT_MAX = PAIR_MT_MAX;               // row blocks of 16: tiles of up to 160 rows
+constexpr int FK_XS = 4;                             // x stages
+constexpr int FK_X_UNITS = 16 * FK_MT_MAX * 4;       // 32 k
+constexpr int FK_W_UNITS = GM_BN * 4;                // 256 weight rows x 128 k
+constexpr int FK_S_UNITS = GM_BN;                    // their scales: 16 bytes a row (fp4_b32: 8)
+constexpr int fk_lds_units() { return FK_XS * FK_X_UNITS + 2 * FK_W_UNITS + FK_S_UNITS; }
+template <int FMT, int MT>
+__device__ __forceinline__ void gemm_tile_fp4_k(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk) {
+    constexpr int BLK = FMT == MOE_FMT_FP4_B32 ? 32 : 16, NSC = 128 / BLK;   // scales of a row per super-step
+    constexpr int NW = 4, NA = (MT + NW - 1) / NW, AHEAD = FK_XS - 1;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, i = lane & 15, q = lane >> 4;
+    const int cw = __builtin_amdgcn_readfirstlane(tid >> 6);
+    u32x4_t* const lds_w = smem + FK_XS * FK_X_UNITS + cw * (FK_W_UNITS / 4);   // this wavefront's quarter of the first buffer
+    u32x4_t* const lds_s = smem + FK_XS * FK_X_UNITS + 2 * FK_W_UNITS + cw * (FK_S_UNITS / 4);
+    const int nss = P.K >> 7;
+    const int k2 = P.K * 2, kh = P.K >> 1, ks = P.K / BLK * 2;   // bytes of a row of x, weights, scales
+    const int64_t KN = (int64_t)P.K * P.N;
+    const bool swi = P.epilogue == MOE_EPILOGUE_SWIGLU;
+    // x as in GK_QUAD: load instructions of 16 rows x 64 bytes, see a_lds_unit32
+    const rsrc_t rx = make_rsrc(P.x + row0 * (int64_t)P.K, (int64_t)rows * k2);
+    const int va = (lane >> 2) * k2 + ((lane & 3) ^ ((lane >> 3) & 3)) * 16;
+    int ca[NA];
+    uint32_t a_at[NA];
+#pragma unroll
+    for (int m = 0; m < NA; ++m) {
+        int j = cw + NW * m;
+        if (NW * NA > MT) j = j % MT;   // repeat a block rather than issue fewer loads
+        a_at[m] = lds_address(smem + j * 64);
+        ca[m] = 16 * j * k2;
+    }
+    auto issue_x = [&](int m, int kt, int st) { lds_load16_at(rx, here(a_at[m]) + st * (FK_X_UNITS * 16), va, ca[m] + kt * 64); };
+    // Slot 16 t + i of a wavefront's weights and scales is the weight row that lane i multiplies in MFMA t.  Weights: load
+    // instruction t brings its 16 slots, lane l unit (l & 3) ^ ((l >> 4) & 3) of slot l >> 2 to position l & 3
+    auto lane_row = [&](int l) { return swi ? 32 * (l >> 3) + 2 * (l & 7) : 4 * l; };
+    auto mfma_row = [&](int t) { return swi ? (t & 1) + 16 * (t >> 1) : t; };
+    const rsrc_t rw = make_rsrc(P.w + g * (KN >> 1), KN >> 1);
+    const int vb = lane_row(lane >> 2) * kh + ((lane & 3) ^ (lane >> 4)) * 16;
+    const int cb = (n0 + 64 * cw) * kh;
+    const uint32_t b_at = lds_address(lds_w);
+    auto issue_w = [&](int t, int ss) { lds_load16_at(rw, here(b_at) + (ss & 1) * (FK_W_UNITS * 16) + t * 1024, vb, cb + mfma_row(t) * kh + ss * 64); };
+    const rsrc_t rs = make_rsrc(static_cast<const uint16_t*>(P.scale) + g * (KN / BLK), (KN / BLK) * 2);
+    const int vs = (lane_row(i) + mfma_row(q)) * ks, cs = (n0 + 64 * cw) * ks;
+    u32x4_t sreg = {0u, 0u, 0u, 0u};
+    auto load_scales = [&](int ss) {
+        if constexpr (BLK == 16) {
+            sreg = __builtin_amdgcn_raw_buffer_load_b128(rs, vs, cs + ss * 16, 0);
+        } else {
+            const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(rs, vs, cs + ss * 8, 0);
+            sreg[0] = v[0];
+            sreg[1] = v[1];
+        }
+    };
+    auto put_scales = [&]() {
+        if constexpr (BLK == 16)
+            lds_s[lane] = sreg;
+        else
+            reinterpret_cast<u32x2_t*>(lds_s)[lane] = u32x2_t{sreg[0], sreg[1]};
+    };
+
+    load_scales(0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) issue_w(t, 0);
+#pragma unroll
+    for (int st = 0; st < AHEAD; ++st)
+#pragma unroll
+        for (int m = 0; m < NA; ++m) issue_x(m, st, st);
+    f32x4_t acc[MT][4];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            asm volatile("v_mov_b32 %0, 0\n\tv_mov_b32 %1, 0\n\tv_mov_b32 %2, 0\n\tv_mov_b32 %3, 0"
+                         : "=v"(acc[mt][t][0]), "=v"(acc[mt][t][1]), "=v"(acc[mt][t][2]), "=v"(acc[mt][t][3]));
+    put_scales();
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * NA) : "memory");   // x stage 0 and the weights are there
+
+    uint32_t r[4], sk[4];
+    // this lane's codes and scales of step J of super-step ss
+    auto read_raw = [&](auto J, int ss) {
+        constexpr int j = decltype(J)::value;
+        const uint32_t* t32 = reinterpret_cast<const uint32_t*>(lds_w + (ss & 1) * FK_W_UNITS);
+        const uint16_t* s16 = reinterpret_cast<const uint16_t*>(lds_s);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            r[t] = t32[((16 * t + i) * 4 + (j ^ (i >> 2))) * 4 + q];
+            sk[t] = s16[(16 * t + i) * NSC + (BLK == 16 ? 2 * j + (q >> 1) : j)];
+        }
+    };
+    read_raw(std::integral_constant<int, 0>{}, 0);
+
+    constexpr int R = 3 < MT ? 3 : MT;   // x fragments read ahead of their MFMAs
+    auto step = [&](auto J, int ss) __attribute__((always_inline)) {
+        constexpr int j = decltype(J)::value;
+        const int kt = 4 * ss + j;
+        const u32x4_t* la = smem + j * FK_X_UNITS + a_lds_unit32(i, q);
+        u32x4_t bf[4], afr[4];
+#pragma unroll
+        for (int t0 = 0; t0 < 4; t0 += 2) {
+            if (t0 == 2)
+#pragma unroll
+                for (int f = 0; f < R; ++f) afr[f] = la[f * 64];
+#pragma unroll
+            for (int t = t0; t < t0 + 2; ++t) {
+                const float m = bf16_bits_to_f32(sk[t]);
+                const f32x2_t f0 = e2m1_pair_to_f32<0>(r[t]), f1 = e2m1_pair_to_f32<1>(r[t]);
+                const f32x2_t f2 = e2m1_pair_to_f32<2>(r[t]), f3 = e2m1_pair_to_f32<3>(r[t]);
+                bf[t][0] = pack_bf16_rne(f0[0] * m, f0[1] * m);
+                bf[t][1] = pack_bf16_rne(f1[0] * m, f1[1] * m);
+                bf[t][2] = pack_bf16_rne(f2[0] * m, f2[1] * m);
+                bf[t][3] = pack_bf16_rne(f3[0] * m, f3[1] * m);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_s_setprio(3);
+        // x stage kt + 3 replaces stage kt - 1, which everybody has left at the barrier; the next super-step's weights
+        // and scales are requested in the first step (x first: see the waits below)
+        constexpr int NI = NA + (j == 0 ? 5 : 0);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            if (mt + R < MT) afr[(mt + R) & 3] = la[(mt + R) * 64];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) mfma_16x16x32_v(acc[mt][t], afr[mt & 3], bf[t]);
+#pragma unroll
+            for (int m = (mt * NI + MT - 1) / MT; m < ((mt + 1) * NI + MT - 1) / MT; ++m) {
+                if (m < NA)
+                    issue_x(m, kt + AHEAD, (j + AHEAD) % FK_XS);
+                else if (m < NA + 4)
+                    issue_w(m - NA, ss + 1);
+                else
+                    load_scales(ss + 1);
+            }
+            if (mt == 0) {
+                if constexpr (j == 3) {
+                    put_scales();
+                    read_raw(std::integral_constant<int, 0>{}, ss + 1);
+                } else {
+                    read_raw(std::integral_constant<int, j + 1>{}, ss);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        // x stage kt + 1 (requested in step kt - 2) has landed: behind it are two steps' x and, in steps 0 and 1, the
+        // weights and scales of step 0; after step 2 these have landed too, which step 3 reads
+        constexpr int WAITN = 2 * NA + (j < 2 ? 5 : 0);
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(WAITN) : "memory");
+    };
+    for (int ss = 0; ss < nss; ++ss) {
+        step(std::integral_constant<int, 0>{}, ss);
+        step(std::integral_constant<int, 1>{}, ss);
+        step(std::integral_constant<int, 2>{}, ss);
+        step(std::integral_constant<int, 3>{}, ss);
+    }
+    // the last loads are for steps past K and never read; wait out the last MFMAs' latency
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15\n\ts_barrier" ::: "memory");
+    pair_finish<MT, true>(P, smem, acc, 0, cw, lane, 64 * cw + 4 * i, row0, rows, n0, tk);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1184,7 +1262,7 @@ __device__ __forceinline__ void gemm_tile_bf16(const GemmParams& P, u32x4_t* sme
     }
     // the last loads are for pairs behind the last one and never read; wait out the last MFMAs' latency
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15\n\ts_barrier" ::: "memory");
-    pair_finish<MT, false, true>(P, smem, acc, 0, cw, lane, 64 * cw + 4 * i, row0 + 16 * MT * wr, max(rows - 16 * MT * wr, 0), n0, tk);
+    pair_finish<MT, true>(P, smem, acc, 0, cw, lane, 64 * cw + 4 * i, row0 + 16 * MT * wr, max(rows - 16 * MT * wr, 0), n0, tk);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1209,22 +1287,23 @@ __device__ __forceinline__ void expert_chunks(int m, int& chunks, int& bpc) {
 template <int FMT, int KIND>
 struct KernelCfg {
     static constexpr bool PAIR = KIND == GK_PAIR || KIND == GK_PAIR_SMALL || KIND == GK_QUAD || pair_exact(KIND);
-    static_assert(PAIR == (FMT != MOE_FMT_BF16), "gemm_tile_pair decodes the quantized containers");
-    static constexpr int WAVES = PAIR ? pair_waves(KIND) : 8;
-    static constexpr int BLOCK = PAIR ? 16 : 32;   // rows per row block of a tile routine's template argument
+    static constexpr bool FP4_K = FMT == MOE_FMT_FP4_B32 || FMT == MOE_FMT_FP4_B16;
+    static_assert(FP4_K == (KIND == GK_FP4_K) && PAIR == (FMT != MOE_FMT_BF16 && !FP4_K), "the routine of the container");
+    static constexpr int WAVES = PAIR ? pair_waves(KIND) : FP4_K ? 4 : 8;
+    static constexpr int BLOCK = PAIR || FP4_K ? 16 : 32;   // rows per row block of a tile routine's template argument
     static constexpr int BN = GM_BN;                                             // columns per tile
     static constexpr int pair_wgs() {
-        if constexpr (PAIR) return pair_wg_per_cu<FMT>(KIND); else return 1;
+        if constexpr (PAIR) return pair_wg_per_cu<FMT>(KIND); else return FP4_K ? 2 : 1;
     }
     static constexpr int WG_PER_CU = pair_wgs();
     static constexpr int WAVES_PER_SIMD = WG_PER_CU * WAVES / 4;
-    static constexpr int MTM = PAIR ? pair_mt_max(KIND) : KIND == GK_BF16_128 ? 4 : BF_MT_MAX;             // row blocks per tile
+    static constexpr int MTM = PAIR ? pair_mt_max(KIND) : FP4_K ? FK_MT_MAX : KIND == GK_BF16_128 ? 4 : BF_MT_MAX;   // row blocks per tile
     // 16-byte LDS units of the tile routine (the tile prefix array follows them)
     static constexpr int lds_units() {
         if constexpr (PAIR)
             return pair_lds_units<FMT>(KIND);
         else
-            return bf_lds_units();
+            return FP4_K ? fk_lds_units() : bf_lds_units();
     }
 };
 
@@ -1236,6 +1315,8 @@ __device__ __forceinline__ void run_tile(const GemmParams& P, u32x4_t* smem, int
             if (rows <= 8) return gemm_tile_pair<FMT, MT, KIND, true>(P, smem, g, row0, rows, n0, tk);
         }
         gemm_tile_pair<FMT, MT, KIND>(P, smem, g, row0, rows, n0, tk);
+    } else if constexpr (C::FP4_K) {
+        gemm_tile_fp4_k<FMT, MT>(P, smem, g, row0, rows, n0, tk);
     } else {
         gemm_tile_bf16<MT>(P, smem, g, row0, rows, n0, tk);
     }
@@ -1564,8 +1645,8 @@ int launch_tiles(const moe_grouped_args* a, GroupedKernel kind, hipStream_t stre
             switch (a->format) {
                 case MOE_FMT_FP8_REF: return launch_gemm_kind<MOE_FMT_FP8_REF, GK_PAIR>(P, a, stream);
                 case MOE_FMT_INT8: return launch_gemm_kind<MOE_FMT_INT8, GK_PAIR>(P, a, stream);
-                case MOE_FMT_FP4_B32: return launch_gemm_kind<MOE_FMT_FP4_B32, GK_PAIR>(P, a, stream);
-                case MOE_FMT_FP4_B16: return launch_gemm_kind<MOE_FMT_FP4_B16, GK_PAIR>(P, a, stream);
+                case MOE_FMT_FP4_B32: return launch_gemm_kind<MOE_FMT_FP4_B32, GK_FP4_K>(P, a, stream);
+                case MOE_FMT_FP4_B16: return launch_gemm_kind<MOE_FMT_FP4_B16, GK_FP4_K>(P, a, stream);
                 default: return MOE_ERR_BAD_FORMAT;
             }
         case GroupedKernel::TILES_PAIR_SMALL:

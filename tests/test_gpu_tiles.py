@@ -84,3 +84,22 @@ def test_bf16_gemv_of_many_rows(K, N):
     got, used = H.run_cabi(case, H.upload(case), "gemv"), sum(counts)
     H.assert_close(got, H.oracle_out(case, gemv=True), rows=slice(0, used), what=f"bf16 gemv K={K} N={N}")
     assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
+
+
+@pytest.mark.parametrize("epilogue", ["none", "swiglu"])
+@pytest.mark.parametrize("K", [128, 256, 384, 896])   # 1, 2, 3 and 7 super-steps
+@pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
+def test_fp4_k_contiguous_row_blocks(fmt, K, epilogue):
+    """gemm_tile_fp4_k: every number of 16-row blocks from 1 to 10, the row before and after each, two and three chunks, over
+    two column tiles."""
+    counts = [rows for b in range(16, 161, 16) for rows in (b - 1, b, b + 1)] + [1, 0, 321]
+    _say(f"{fmt} row blocks K={K} epilogue={epilogue}")
+    case = H.make_case(fmt, len(counts), K, 512, np.cumsum(counts), seed=K, extra_rows=3)
+    assert H.kernel_of(case, "gemm", swiglu=epilogue == "swiglu") == "tiles_pair"
+    used = int(case["group_list"][-1])
+    if epilogue == "swiglu":
+        got, want = _swiglu(case)
+    else:
+        got, want = H.run_cabi(case, H.upload(case), "gemm"), H.oracle_out(case)
+    H.assert_close(got, want, rows=slice(0, used), what=f"{fmt} K={K} {epilogue}")
+    assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
