@@ -19,8 +19,8 @@
 //                   their 64 columns through all of k, two such workgroups per CU (int4 and fp4 prefill);
 //                   tiles of up to 160 rows, or of up to 32 / 16 rows with small stages (decode batches,
 //                   and the GEMV op's arithmetic on the N-contiguous containers)
-//   gemm_tile_fp4_k the K-contiguous fp4 containers: 4 wavefronts, two workgroups per CU, tiles of up to 160 rows; x in a
-//                   ring of 32-k stages, every wavefront's own weights and scales 128 k at a time
+//   gemm_tile_fp4_k the K-contiguous fp4 containers: 4 wavefronts, two workgroups per CU, tiles of up to 144 rows; x in a
+//                   ring of 32-k stages, every wavefront's own weights and scales 256 k at a time
 //   gemm_tile_bf16  the bf16 container: 8 wavefronts, tiles of up to 224 rows, x and weights by LDS-direct loads into
 //                   two rings
 //
@@ -933,40 +933,43 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
 
 // ---------------------------------------------------------------------------------
 // Tile routine for the K-contiguous fp4 containers (weights [N, K/2], scales [N, K/16 or K/32]): workgroups of 4 wavefronts,
-// two per CU, as GK_QUAD: wavefront cw takes columns 64 cw .. + 63 of the tile through all of k for up to 160 rows.
+// two per CU, as GK_QUAD: wavefront cw takes columns 64 cw .. + 63 of the tile through all of k for up to 144 rows.
 //
 // Bound by issue, as the N-contiguous kinds: 2 vector instructions per weight (exact convert, times its scale, rounded to
-// bf16) beside the MFMAs.  Two workgroups per CU hide each other's barriers and the time between tiles, which the 8-wavefront
-// k-split routine that served these containers before did not.
-// 128 experts of 2048 x 7168, 2047 tokens x 8 rows: fp4_b16 FIGURES_B16 (FIGURES_T).
+// bf16) beside the MFMAs, and next to that by requests to L2.  Two workgroups per CU hide each other's barriers and the time
+// between tiles, which the 8-wavefront k-split routine that served these containers before did not.
+// us, that routine / this one: 128 experts of 2048 x 7168, 2047 tokens x 8 rows: fp4_b16 686 / 570 (843 TFLOP/s), fp4_b32
+// 635 / 551; 7168 x 2048 the same rows, fp4_b32: 624 / 593; 4608 x 3072, 1245 tokens x 8, unevenly routed, fp4_b16: 490 / 436; 8 of
+// 3968 x 13568, 841 rows each, fp4_b32: 699 / 627.  (The reference's fp4 container on GK_QUAD: 522, 534 on the first and third.)
 //
 // The weight rows of a wavefront's columns are read by that wavefront alone, so its weights and scales are its own business:
-// it loads them for 128 k at a time ("a super-step": 64 bytes of 64 rows, four LDS-direct loads; 32-byte pieces would touch
-// twice as many lines), one super-step ahead, into one of two buffers, and waits for nobody.  The scales of a super-step, 16 or
-// 8 bytes a row, come through registers into 1 KB of the wavefront's own LDS once the last of the previous ones is read.  Only x
-// is shared: a ring of four 32-k stages, three steps ahead, one barrier per step.
+// it loads them for 256 k at a time, whole 128-byte lines of 64 rows, into registers, a period of 8 steps ahead, puts them into
+// its own LDS when the last of the previous period is read, and waits for nobody.  (64 bytes of a row at a time, straight to
+// LDS: the other half of a line was gone from L2 when its turn came, 64 workgroups of 256 lines each on an XCD; 1.6 GB fetched
+// instead of 1.2, by counters, and 635 us instead of 593 at K = 7168.  Both halves back to back but in instructions of 16 rows x
+// 64 bytes: 615 us, twice the requests.)  Only x is shared: a ring of four 32-k stages, three steps ahead, one barrier per step.
 //
-// Step j of a super-step reads dword q of 16-byte unit j of every weight row: the 8 codes k = 32 j + 8 q + [0, 8).  Unit j of
-// the row in slot s lies at position j ^ ((s >> 2) & 3), so that the 64 lanes of a read (16 rows x 4 dwords) hit 64 banks.
+// Step u of a period reads dword q of 16-byte unit u of every weight row: the 8 codes k = 32 u + 8 q + [0, 8).  Unit u of the
+// row in slot s lies at position u ^ ((s >> 1) & 7), so that the 64 lanes of a read (16 rows x 4 dwords) hit 64 banks.
 // Column t of a lane is 4 i + t (SwiGLU: two gate and two up rows of two adjacent output columns), as in gemm_tile_bf16.
 // ---------------------------------------------------------------------------------
-constexpr int FK_MT_MAX = PAIR_MT_MAX;               // row blocks of 16: tiles of up to 160 rows
+constexpr int FK_MT_MAX = 9;                         // row blocks of 16; a tenth leaves no registers for the weights ahead
 constexpr int FK_XS = 4;                             // x stages
 constexpr int FK_X_UNITS = 16 * FK_MT_MAX * 4;       // 32 k
-constexpr int FK_W_UNITS = GM_BN * 4;                // 256 weight rows x 128 k
-constexpr int FK_S_UNITS = GM_BN;                    // their scales: 16 bytes a row (fp4_b32: 8)
-constexpr int fk_lds_units() { return FK_XS * FK_X_UNITS + 2 * FK_W_UNITS + FK_S_UNITS; }
+constexpr int FK_W_UNITS = GM_BN * 8;                // 256 weight rows x 256 k
+constexpr int FK_S_UNITS = GM_BN * 2;                // their scales: 32 bytes a row (fp4_b32: 16)
+constexpr int fk_lds_units() { return FK_XS * FK_X_UNITS + FK_W_UNITS + FK_S_UNITS; }
 template <int FMT, int MT>
 __device__ __forceinline__ void gemm_tile_fp4_k(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk) {
-    constexpr int BLK = FMT == MOE_FMT_FP4_B32 ? 32 : 16, NSC = 128 / BLK;   // scales of a row per super-step
+    constexpr int BLK = FMT == MOE_FMT_FP4_B32 ? 32 : 16, SL = 32 / BLK;   // SL: load instructions of a period's scales
     constexpr int NW = 4, NA = (MT + NW - 1) / NW, AHEAD = FK_XS - 1;
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, i = lane & 15, q = lane >> 4;
     const int cw = __builtin_amdgcn_readfirstlane(tid >> 6);
-    u32x4_t* const lds_w = smem + FK_XS * FK_X_UNITS + cw * (FK_W_UNITS / 4);   // this wavefront's quarter of the first buffer
-    u32x4_t* const lds_s = smem + FK_XS * FK_X_UNITS + 2 * FK_W_UNITS + cw * (FK_S_UNITS / 4);
-    const int nss = P.K >> 7;
+    u32x4_t* const lds_w = smem + FK_XS * FK_X_UNITS + cw * (FK_W_UNITS / 4);   // this wavefront's own
+    u32x4_t* const lds_s = smem + FK_XS * FK_X_UNITS + FK_W_UNITS + cw * (FK_S_UNITS / 4);
+    const int nk = P.K >> 5;                                     // a multiple of 4
     const int k2 = P.K * 2, kh = P.K >> 1, ks = P.K / BLK * 2;   // bytes of a row of x, weights, scales
     const int64_t KN = (int64_t)P.K * P.N;
     const bool swi = P.epilogue == MOE_EPILOGUE_SWIGLU;
@@ -983,37 +986,35 @@ __device__ __forceinline__ void gemm_tile_fp4_k(const GemmParams& P, u32x4_t* sm
         ca[m] = 16 * j * k2;
     }
     auto issue_x = [&](int m, int kt, int st) { lds_load16_at(rx, here(a_at[m]) + st * (FK_X_UNITS * 16), va, ca[m] + kt * 64); };
-    // Slot 16 t + i of a wavefront's weights and scales is the weight row that lane i multiplies in MFMA t.  Weights: load
-    // instruction t brings its 16 slots, lane l unit (l & 3) ^ ((l >> 4) & 3) of slot l >> 2 to position l & 3
-    auto lane_row = [&](int l) { return swi ? 32 * (l >> 3) + 2 * (l & 7) : 4 * l; };
+    // Slot 16 t + i of a wavefront's weights and scales is the weight row that lane i multiplies in MFMA t, row lane_row(i) +
+    // mfma_row(t) of its 64.  Weights: load e brings slots 8 e + (l >> 3), the whole 128 bytes of each
+    const int lane_rows = swi ? 2 : 4;   // lanes i and i + 1 (i + 8: 32 rows, either way)
     auto mfma_row = [&](int t) { return swi ? (t & 1) + 16 * (t >> 1) : t; };
     const rsrc_t rw = make_rsrc(P.w + g * (KN >> 1), KN >> 1);
-    const int vb = lane_row(lane >> 2) * kh + ((lane & 3) ^ (lane >> 4)) * 16;
     const int cb = (n0 + 64 * cw) * kh;
-    const uint32_t b_at = lds_address(lds_w);
-    auto issue_w = [&](int t, int ss) { lds_load16_at(rw, here(b_at) + (ss & 1) * (FK_W_UNITS * 16) + t * 1024, vb, cb + mfma_row(t) * kh + ss * 64); };
-    const rsrc_t rs = make_rsrc(static_cast<const uint16_t*>(P.scale) + g * (KN / BLK), (KN / BLK) * 2);
-    const int vs = (lane_row(i) + mfma_row(q)) * ks, cs = (n0 + 64 * cw) * ks;
-    u32x4_t sreg = {0u, 0u, 0u, 0u};
-    auto load_scales = [&](int ss) {
-        if constexpr (BLK == 16) {
-            sreg = __builtin_amdgcn_raw_buffer_load_b128(rs, vs, cs + ss * 16, 0);
-        } else {
-            const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(rs, vs, cs + ss * 8, 0);
-            sreg[0] = v[0];
-            sreg[1] = v[1];
-        }
+    const int vb0 = (lane >> 3) * lane_rows * kh + ((lane & 7) ^ (lane >> 4)) * 16;
+    const int vb1 = (lane >> 3) * lane_rows * kh + ((lane & 7) ^ (lane >> 4) ^ 4) * 16;
+    u32x4_t wreg[8], sreg[SL];
+    auto load_w = [&](int e, int p) {
+        wreg[e] = __builtin_amdgcn_raw_buffer_load_b128(rw, e & 1 ? vb1 : vb0, cb + (mfma_row(e >> 1) + 32 * (e & 1)) * kh + p * 128, 0);
     };
-    auto put_scales = [&]() {
-        if constexpr (BLK == 16)
-            lds_s[lane] = sreg;
-        else
-            reinterpret_cast<u32x2_t*>(lds_s)[lane] = u32x2_t{sreg[0], sreg[1]};
+    // scales: fp4_b32 the 16 bytes of slot l; fp4_b16 load e the 32 bytes of slots 32 e + (l >> 1)
+    const rsrc_t rs = make_rsrc(static_cast<const uint16_t*>(P.scale) + g * (KN / BLK), (KN / BLK) * 2);
+    const int sl = SL == 1 ? lane : lane >> 1;   // slot
+    const int vs = (32 * ((sl >> 3) & 1) + lane_rows * (sl & 7) + mfma_row(sl >> 4)) * ks + (SL == 1 ? 0 : (lane & 1) * 16);
+    const int cs = (n0 + 64 * cw) * ks;
+    auto load_s = [&](int e, int p) { sreg[e] = __builtin_amdgcn_raw_buffer_load_b128(rs, vs, cs + mfma_row(2) * e * ks + p * (16 * SL), 0); };
+    auto put = [&]() {
+#pragma unroll
+        for (int e = 0; e < SL; ++e) lds_s[e * 64 + lane] = sreg[e];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) lds_w[e * 64 + lane] = wreg[e];
     };
 
-    load_scales(0);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) issue_w(t, 0);
+    for (int e = 0; e < SL; ++e) load_s(e, 0);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) load_w(e, 0);
 #pragma unroll
     for (int st = 0; st < AHEAD; ++st)
 #pragma unroll
@@ -1025,29 +1026,31 @@ __device__ __forceinline__ void gemm_tile_fp4_k(const GemmParams& P, u32x4_t* sm
         for (int t = 0; t < 4; ++t)
             asm volatile("v_mov_b32 %0, 0\n\tv_mov_b32 %1, 0\n\tv_mov_b32 %2, 0\n\tv_mov_b32 %3, 0"
                          : "=v"(acc[mt][t][0]), "=v"(acc[mt][t][1]), "=v"(acc[mt][t][2]), "=v"(acc[mt][t][3]));
-    put_scales();
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * NA) : "memory");   // x stage 0 and the weights are there
+    put();
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * NA) : "memory");   // x stage 0 is there
 
     uint32_t r[4], sk[4];
-    // this lane's codes and scales of step J of super-step ss
-    auto read_raw = [&](auto J, int ss) {
-        constexpr int j = decltype(J)::value;
-        const uint32_t* t32 = reinterpret_cast<const uint32_t*>(lds_w + (ss & 1) * FK_W_UNITS);
-        const uint16_t* s16 = reinterpret_cast<const uint16_t*>(lds_s);
+    // this lane's codes and scales of step u of the period
+    const uint32_t* const t32 = reinterpret_cast<const uint32_t*>(lds_w) + i * 32 + q;
+    const uint16_t* const s16 = reinterpret_cast<const uint16_t*>(lds_s) + i * (8 * SL) + (BLK == 16 ? q >> 1 : 0);
+    auto read_raw = [&](int u) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            r[t] = t32[((16 * t + i) * 4 + (j ^ (i >> 2))) * 4 + q];
-            sk[t] = s16[(16 * t + i) * NSC + (BLK == 16 ? 2 * j + (q >> 1) : j)];
+            r[t] = t32[16 * t * 32 + (u ^ (i >> 1)) * 4];
+            sk[t] = s16[16 * t * (8 * SL) + u * SL];
         }
     };
-    read_raw(std::integral_constant<int, 0>{}, 0);
+    read_raw(0);
 
-    constexpr int R = 3 < MT ? 3 : MT;   // x fragments read ahead of their MFMAs
-    auto step = [&](auto J, int ss) __attribute__((always_inline)) {
-        constexpr int j = decltype(J)::value;
-        const int kt = 4 * ss + j;
-        const u32x4_t* la = smem + j * FK_X_UNITS + a_lds_unit32(i, q);
-        u32x4_t bf[4], afr[4];
+    constexpr int R = MT == 9 ? 2 : MT < 3 ? MT : 3, RB = R + 1;   // x fragments read ahead of their MFMAs (nine blocks: registers)
+    // what step u requests of the next period's weights and scales (0 for u < 0 too)
+    constexpr auto extra = [](int u) { return u >= 0 && u < 4 ? 2 + (u < SL ? 1 : 0) : 0; };
+    // step u of period p; MORE: with requests for the next period (or the counts below would include loads that nothing reads and
+    // that the compiler therefore takes out)
+    auto step = [&](auto U, auto MORE, int p) __attribute__((always_inline)) {
+        constexpr int u = decltype(U)::value, st = u % FK_XS, here_n = MORE ? extra(u) : 0, before_n = MORE ? extra(u - 1) : 0;
+        const u32x4_t* la = smem + st * FK_X_UNITS + a_lds_unit32(i, q);
+        u32x4_t bf[4], afr[RB];
 #pragma unroll
         for (int t0 = 0; t0 < 4; t0 += 2) {
             if (t0 == 2)
@@ -1066,45 +1069,56 @@ __device__ __forceinline__ void gemm_tile_fp4_k(const GemmParams& P, u32x4_t* sm
             __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_s_setprio(3);
-        // x stage kt + 3 replaces stage kt - 1, which everybody has left at the barrier; the next super-step's weights
-        // and scales are requested in the first step (x first: see the waits below)
-        constexpr int NI = NA + (j == 0 ? 5 : 0);
+        // the x stage three steps ahead replaces the one everybody has left at the barrier; a quarter of the next weights
+        constexpr int NI = NA + extra(u);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            if (mt + R < MT) afr[(mt + R) & 3] = la[(mt + R) * 64];
+            if (mt + R < MT) afr[(mt + R) % RB] = la[(mt + R) * 64];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) mfma_16x16x32_v(acc[mt][t], afr[mt & 3], bf[t]);
+            for (int t = 0; t < 4; ++t) {
+                if constexpr (MT == 1)   // (few enough for the compiler, which moves them to other registers behind the loop)
+                    acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, afr[0]), __builtin_bit_cast(bf16x8_t, bf[t]), acc[0][t], 0, 0, 0);
+                else
+                    mfma_16x16x32_v(acc[mt][t], afr[mt % RB], bf[t]);
+            }
 #pragma unroll
             for (int m = (mt * NI + MT - 1) / MT; m < ((mt + 1) * NI + MT - 1) / MT; ++m) {
                 if (m < NA)
-                    issue_x(m, kt + AHEAD, (j + AHEAD) % FK_XS);
-                else if (m < NA + 4)
-                    issue_w(m - NA, ss + 1);
+                    issue_x(m, 8 * p + u + AHEAD, (u + AHEAD) % FK_XS);
+                else if (!MORE)
+                    break;
+                else if (m < NA + 2)
+                    load_w(2 * u + m - NA, p + 1);
                 else
-                    load_scales(ss + 1);
+                    load_s(u, p + 1);
             }
             if (mt == 0) {
-                if constexpr (j == 3) {
-                    put_scales();
-                    read_raw(std::integral_constant<int, 0>{}, ss + 1);
-                } else {
-                    read_raw(std::integral_constant<int, j + 1>{}, ss);
-                }
+                if constexpr (u == 7) put();
+                read_raw((u + 1) & 7);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_s_setprio(0);
-        // x stage kt + 1 (requested in step kt - 2) has landed: behind it are two steps' x and, in steps 0 and 1, the
-        // weights and scales of step 0; after step 2 these have landed too, which step 3 reads
-        constexpr int WAITN = 2 * NA + (j < 2 ? 5 : 0);
+        // x of the next step (requested two steps ago) has landed: behind it are all requests of the last step and this one
+        // (whole steps: within a step the compiler may order the requests as it likes)
+        constexpr int WAITN = 2 * NA + before_n + here_n;
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(WAITN) : "memory");
     };
-    for (int ss = 0; ss < nss; ++ss) {
-        step(std::integral_constant<int, 0>{}, ss);
-        step(std::integral_constant<int, 1>{}, ss);
-        step(std::integral_constant<int, 2>{}, ss);
-        step(std::integral_constant<int, 3>{}, ss);
+    // (the half period of a K that is no multiple of 256 stands behind the loop: a path from step 3 to step 0, with loads into wreg
+    // on their way, would make the compiler wait in every step)
+    const int np = nk >> 3;
+    const auto half = [&](auto FIRST, auto MORE, int p) __attribute__((always_inline)) {
+        constexpr int u = decltype(FIRST)::value;
+        step(std::integral_constant<int, u>{}, MORE, p);
+        step(std::integral_constant<int, u + 1>{}, MORE, p);
+        step(std::integral_constant<int, u + 2>{}, MORE, p);
+        step(std::integral_constant<int, u + 3>{}, MORE, p);
+    };
+    for (int p = 0; p < np; ++p) {
+        half(std::integral_constant<int, 0>{}, std::true_type{}, p);
+        half(std::integral_constant<int, 4>{}, std::true_type{}, p);
     }
+    if (nk & 4) half(std::integral_constant<int, 0>{}, std::false_type{}, np);
     // the last loads are for steps past K and never read; wait out the last MFMAs' latency
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15\n\ts_barrier" ::: "memory");
     pair_finish<MT, true>(P, smem, acc, 0, cw, lane, 64 * cw + 4 * i, row0, rows, n0, tk);

@@ -23,7 +23,8 @@ inline int ensure_dynamic_lds(const void* kernel, int bytes, std::atomic<uint64_
 
 int launch_dequant_fp4_bf16(const moe_dequant_args* a, hipStream_t stream);
 // The kernels of the two grouped ops.  TILES_PAIR_EXACT and TILES_PAIR_EXACT16 have the GEMV op's arithmetic (weights not
-// rounded to bf16), the other TILES that of the GEMM op; STRIPS and FP4_ROWS come with either.
+// rounded to bf16), the other TILES that of the GEMM op; STRIPS and FP4_ROWS come with either.  TILES_PAIR is the k-split kind
+// for the N-contiguous containers and GK_FP4_K, the only kind they have, for the K-contiguous fp4 ones.
 enum class GroupedKernel {
     VECTOR,               // K-contiguous containers without matrix cores (moe_gemv.hip)
     FP4_ROWS,             // K-contiguous fp4, 16 rows of an expert per pass (moe_gemv.hip)
