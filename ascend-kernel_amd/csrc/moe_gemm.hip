@@ -51,7 +51,8 @@ struct GemmParams {
     int epilogue;   // moe_epilogue
     int slot;       // this launch's counter in tile_queue; -1: none, every tile in the fixed order
     unsigned long long stamp;   // what this launch raises its counter to before it draws from it
-    // what the scheduler keeps in LDS: 2 the first tile of every expert and the experts' clamped row bounds; 1 the
+    // what the scheduler keeps in LDS: 3 the first tile of every expert, the experts' clamped row bounds and the order
+    // in which the experts are taken (see order_experts); 2 the first two; 1 the
     // first tiles only (the row bounds are read from group_list per tile); 0 neither fits: the first tile of every
     // thread's run of experts only, and a tile is found by walking its run (any number of experts)
     int table_mode;
@@ -1298,6 +1299,66 @@ __device__ __forceinline__ void expert_chunks(int m, int& chunks, int& bpc) {
     bpc = (nblk + chunks - 1) / chunks;
 }
 
+// The order in which a launch takes its experts: those with the largest tiles (most row blocks per chunk) first, those
+// without rows last, otherwise as they come.  A tile's time goes by its row blocks, and with the largest tiles up to half
+// of a launch long, one that starts among the last leaves most of the chip waiting for it.
+// us as they come / in this order, rows unevenly routed (skew: see moe_dispatch.cpp): fp4 SwiGLU, 1511 tokens x 8 on 256
+// experts of 7168 x 2048, skew 1: 592 / 565; bf16, 1021 x 8 on 64 of 7168 x 2048, skew 0.25: 488 / 476.  Orders given by group_list
+// to a kernel that took it as it was, skew 1: int4, 2000 x 4 on 64 of 7168 x 2048: 327 / 296; fp4_b32, 1500 x 8 on 128
+// of 4096 x 3072: 420 / 399; fp8 and int8 on 128 of 4096 x 2048: 325 / 308 and 310 / 297; evenly routed, the same time.
+// Every workgroup works the same order out: a counting sort, ranks from ballots; 64 experts of a wavefront at a
+// time leave one count per class in scratch (LDS of the tile routine, [rounds * WAVES][16]).
+template <int MTM, int BLOCK, int WAVES, typename Rows>
+__device__ __forceinline__ void order_experts(int G, int tid, int* scratch, uint16_t* order, Rows expert_rows) {
+    static_assert(MTM < 15, "classes 0 .. MTM, 15 for no expert");
+    const int lane = tid & 63, wave = tid >> 6, rounds = (G + 64 * WAVES - 1) / (64 * WAVES);
+    auto class_of = [&](int g) {
+        if (g >= G) return 15;
+        int first, chunks, bpc;
+        expert_chunks<MTM, BLOCK>(expert_rows(g, first), chunks, bpc);
+        return MTM - bpc;
+    };
+    for (int r = 0; r < rounds; ++r) {
+        const int c = class_of(r * 64 * WAVES + tid);
+        int n = 0;
+#pragma unroll
+        for (int k = 0; k <= MTM; ++k) {
+            const int in = __popcll(__ballot(c == k));
+            if (lane == k) n = in;
+        }
+        if (lane < 16) scratch[(r * WAVES + wave) * 16 + lane] = n;
+    }
+    __syncthreads();
+    // lane k (mod 16): where class k starts for the next 64 experts of this wavefront
+    const int col = lane & 15;
+    int all = 0, next = 0;
+    for (int j = 0; j < rounds * WAVES; ++j) {
+        const int n = scratch[j * 16 + col];
+        all += n;
+        next += j < wave ? n : 0;
+    }
+    int incl = all;
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) {
+        const int up = __shfl_up(incl, off, 16);
+        if (col >= off) incl += up;
+    }
+    next += incl - all;
+    for (int r = 0; r < rounds; ++r) {
+        const int g = r * 64 * WAVES + tid, c = class_of(g);
+        unsigned long long same = 0;
+#pragma unroll
+        for (int k = 0; k <= MTM; ++k) {
+            const unsigned long long in = __ballot(c == k);
+            if (c == k) same = in;
+        }
+        const int at = __shfl(next, c, 64) + __popcll(same & ((1ull << lane) - 1));
+        if (g < G) order[at] = (uint16_t)g;
+        for (int j = r * WAVES + wave; j < (r + 1) * WAVES + wave && j < rounds * WAVES; ++j) next += scratch[j * 16 + col];
+    }
+    __syncthreads();
+}
+
 template <int FMT, int KIND>
 struct KernelCfg {
     static constexpr bool PAIR = KIND == GK_PAIR || KIND == GK_PAIR_SMALL || KIND == GK_QUAD || pair_exact(KIND);
@@ -1312,6 +1373,8 @@ struct KernelCfg {
     static constexpr int WG_PER_CU = pair_wgs();
     static constexpr int WAVES_PER_SIMD = WG_PER_CU * WAVES / 4;
     static constexpr int MTM = PAIR ? pair_mt_max(KIND) : FP4_K ? FK_MT_MAX : KIND == GK_BF16_128 ? 4 : BF_MT_MAX;   // row blocks per tile
+    // tiles of up to 32 rows take the time of their weights, in any order
+    static constexpr bool ORDERED = MTM > PAIR_SMALL_MT_MAX;
     // 16-byte LDS units of the tile routine (the tile prefix array follows them)
     static constexpr int lds_units() {
         if constexpr (PAIR)
@@ -1349,6 +1412,8 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
     // [rowc[g], rowc[g + 1]) if that is not empty (same result as clamping start and end separately).  Kept in
     // LDS so that the scheduler does not wait for a global load per tile (2 to 4 us under a streaming kernel).
     int* rowc = prefix + (P.G + 1);
+    // [G] table_mode 3: the expert at each place of prefix[]
+    uint16_t* order = reinterpret_cast<uint16_t*>(rowc + (P.G + 1));
     const int tid = threadIdx.x;
     const int ntile_n = (P.N + C::BN - 1) / C::BN;
     // scan partials (one per wavefront); later part[0] carries the ticket drawn from the queue, part[1] the tile
@@ -1358,7 +1423,7 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
     auto clamp_row = [&](int64_t v) { return (int)min(max(v, (int64_t)0), P.M); };
     auto expert_rows = [&](int g, int& first) {
         int hi;
-        if (P.table_mode == 2) {
+        if (P.table_mode >= 2) {
             first = rowc[g];
             hi = rowc[g + 1];
         } else {
@@ -1368,6 +1433,8 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         return max(hi - first, 0);
     };
 
+    auto expert_at = [&](int e) { return C::ORDERED && P.table_mode == 3 ? (int)order[e] : e; };
+
     // the launch's counter is looked at, and raised to the launch's stamp, now: long before the first draw from it
     if (tid == 0) part[PART_FIXED] = P.slot >= 0 && queue_open(tile_queue + GM_QUEUE_STRIDE * max(P.slot, 0), P.stamp, blockIdx.x < 8);
 
@@ -1376,15 +1443,17 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
     const int entries = P.table_mode ? P.G : THREADS;   // the table has entries + 1 elements
     {
         const int g0 = min(P.G, tid * per), g1 = min(P.G, g0 + per);
-        if (P.table_mode == 2) {
+        if (P.table_mode >= 2) {
             for (int g = g0; g < g1; ++g) rowc[g + 1] = clamp_row(P.gl[g]);
             if (tid == 0) rowc[0] = 0;
             __syncthreads();
         }
+        if constexpr (C::ORDERED)
+            if (P.table_mode == 3) order_experts<MTM, C::BLOCK, WAVES>(P.G, tid, reinterpret_cast<int*>(smem), order, expert_rows);
         int sum = 0;
-        for (int g = g0; g < g1; ++g) {
+        for (int e = g0; e < g1; ++e) {
             int first, chunks, bpc;
-            expert_chunks<MTM, C::BLOCK>(expert_rows(g, first), chunks, bpc);
+            expert_chunks<MTM, C::BLOCK>(expert_rows(expert_at(e), first), chunks, bpc);
             sum += chunks * ntile_n;
         }
         // scan over the threads: within a wavefront by shuffles, across wavefronts through their totals in
@@ -1408,10 +1477,10 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         if (tid == 0) prefix[entries] = all;
         int run = before + incl - sum;
         if (P.table_mode) {
-            for (int g = g0; g < g1; ++g) {
+            for (int e = g0; e < g1; ++e) {
                 int first, chunks, bpc;
-                expert_chunks<MTM, C::BLOCK>(expert_rows(g, first), chunks, bpc);
-                prefix[g] = run;
+                expert_chunks<MTM, C::BLOCK>(expert_rows(expert_at(e), first), chunks, bpc);
+                prefix[e] = run;
                 run += chunks * ntile_n;
             }
         } else {
@@ -1490,7 +1559,9 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         // everything below is wave-uniform; readfirstlane lets the compiler keep it in SGPRs
         const int found = __builtin_amdgcn_readfirstlane(seg * stride + max(upto, 1) - 1);
         int g = found, local = __builtin_amdgcn_readfirstlane(T - prefix[found]);
-        if (P.table_mode == 0) {
+        if (C::ORDERED && P.table_mode == 3) {
+            g = __builtin_amdgcn_readfirstlane((int)order[found]);
+        } else if (P.table_mode == 0) {
             // found is a thread's run of experts: walk it 64 experts at a time (group_list from memory, the tile
             // counts summed across the wavefront) up to the expert that holds tile number `local` of the run
             const int e_end = min(P.G, (found + 1) * per);
@@ -1600,8 +1671,8 @@ static int launch_gemm_kind(const GemmParams& P, const moe_grouped_args* a, hipS
     // GemmParams::table_mode)
     constexpr size_t units = (size_t)C::lds_units() * 16, thread_table = (size_t)(64 * C::WAVES + 1) * sizeof(int);
     static_assert(units + thread_table <= lds_max, "any number of experts");
-    const int table_mode = units + 2 * table <= lds_max ? 2 : units + table <= lds_max ? 1 : 0;
-    const size_t lds = units + (table_mode ? table_mode * table : thread_table);
+    int table_mode = units + 2 * table <= lds_max ? 2 : units + table <= lds_max ? 1 : 0;
+    size_t lds = units + (table_mode ? table_mode * table : thread_table);
     static std::atomic<uint64_t> lds_set{0};
     if (const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&grouped_gemm_kernel<FMT, KIND>), (int)lds_max, lds_set))
         return rc;
@@ -1612,6 +1683,11 @@ static int launch_gemm_kind(const GemmParams& P, const moe_grouped_args* a, hipS
     const int64_t max_chunks = a->M / (C::BLOCK * C::MTM) + a->G;
     const int64_t max_tiles = max_chunks * ((a->N + C::BN - 1) / C::BN);
     const int64_t want = max_tiles < (int64_t)cus * C::WG_PER_CU ? max_tiles : (int64_t)cus * C::WG_PER_CU;
+    // where a workgroup may get more than one tile, the experts with the largest ones come first (as far as LDS has room)
+    if (C::ORDERED && table_mode == 2 && max_tiles > want && lds + (size_t)a->G * sizeof(uint16_t) <= lds_max) {
+        table_mode = 3;
+        lds += (size_t)a->G * sizeof(uint16_t);
+    }
     // a multiple of 8 so that the XCD-aware order covers every tile index
     const int64_t grid = want > 0 ? (want + 7) / 8 * 8 : 8;
     GemmParams Q = P;
