@@ -60,10 +60,22 @@ static bool fp4_rows_preferred(const moe_grouped_args* a) {
     return a->M <= (a->M <= 64 ? 8 : 5) * a->G;
 }
 
+// The same kernel where K is no multiple of 512 and its last iteration is not full.  us, the other kernel / this one, fp4_b32 and
+// fp4_b16.  GEMV op (vector): 8 rows, 1 to 8 experts, K = 1152: 8.0 / 5.5 and 8.8 / 6.7; 62 x 4 rows on 64 experts of 4736 x 768,
+// skew 1: 196 / 46 and 212 / 59; 32 x 8 on 256 of 1920 x 2000: 131 / 63 and 146 / 83; but a token on 8 of 6912 x 512: 29 / 29 and
+// 30 / 34.  GEMM op (tiles): 49 rows on 16 of 6912 x 512 60 / 32 and 63 / 34, 100 on 64 of 4480 x 1024 44 / 35 and 45 / 37, 512 on
+// 256 of 6912 x 2048 438 / 386 and 439 / 417; with many columns and a short K the tiles are level or ahead: 16 rows on 256 of
+// 1792 x 3584 (57344 columns) 22 / 25 and 24 / 26, 240 on 64 of 3328 x 2048 54 / 55 and 57 / 59.  Where K is an odd multiple of 128 the
+// rows of weights do not begin with lines.
+static bool fp4_rows_partial_preferred(const moe_grouped_args* a, bool gemv_op) {
+    if (gemv_op) return !(a->format == MOE_FMT_FP4_B16 && a->M <= 8 && columns(a) <= 8192 && a->K >= 4096);
+    return columns(a) <= 32768 || (a->K % 256 == 0 && a->K >= 4096);
+}
+
 static GroupedKernel fp4_kcontiguous_kernel(const moe_grouped_args* a, bool gemv_op) {
-    const bool whole = a->K % FP4_ROWS_K == 0;
-    if (gemv_op) return whole ? GroupedKernel::FP4_ROWS : GroupedKernel::VECTOR;
-    return whole && fp4_rows_preferred(a) ? GroupedKernel::FP4_ROWS : GroupedKernel::TILES_PAIR;
+    const bool rows = a->K % 512 == 0 || (a->K >= FP4_ROWS_K_MIN && a->K % FP4_ROWS_K == 0 && fp4_rows_partial_preferred(a, gemv_op));
+    if (gemv_op) return rows ? GroupedKernel::FP4_ROWS : GroupedKernel::VECTOR;
+    return rows && fp4_rows_preferred(a) ? GroupedKernel::FP4_ROWS : GroupedKernel::TILES_PAIR;
 }
 
 // Strips for launches of up to 128 tiles of 256 columns, i.e. half of the CUs, and decode-like batches: with 32768 columns (16

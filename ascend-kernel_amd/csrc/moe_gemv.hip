@@ -4,7 +4,7 @@
 // gemv_impl.h:201-398).  Unlike the reference, more than 4 rows per expert are accepted.
 //
 // Two kernels live here, both for the K-contiguous containers:
-//   gemv_kmajor_kernel    bf16 weights (and fp4 with K % 512 != 0): no matrix cores -- wide vector loads, packed-bf16
+//   gemv_kmajor_kernel    bf16 weights (and fp4 with K % 128 != 0): no matrix cores -- wide vector loads, packed-bf16
 //                         dot products (v_dot2c_f32_bf16), wavefront shuffles for the reductions, 4 rows per pass
 //   gemv_fp4_mfma_kernel  fp4 codes: one v_mfma_f32_16x16x32_bf16 per 32-k block and 16 weight rows (a vector kernel
 //                         needs (1 + rows) / 2 instructions per 4-bit weight, more than the chip can issue while HBM
@@ -257,8 +257,8 @@ constexpr int GF_ROWS = 16;               // activation rows per pass
 constexpr int GF_LDS_UNITS = 3584;        // 56 KiB of x per staged chunk
 constexpr int GF_SCALE_UNITS = 128;       // per wavefront: the 4 q lanes' 2 x 16 bytes of scales for 16 rows
 constexpr int GF_U = 4;                   // 128-k groups (one 16-byte load per lane each) per loop iteration
-constexpr int GF_KSTEP = 128 * GF_U;      // k per loop iteration; K must be a multiple
-static_assert(GF_KSTEP == FP4_ROWS_K, "what the dispatch goes by");
+constexpr int GF_KSTEP = 128 * GF_U;      // k per loop iteration
+static_assert(FP4_ROWS_K == 128 && FP4_ROWS_K_MIN == 256, "whole groups; fetch_s below reads 8 scales of a row at a time");
 
 __device__ __forceinline__ uint32_t e2m1_pair_bf16(uint32_t word, int sel) {
     switch (sel) {
@@ -273,6 +273,8 @@ __device__ __forceinline__ uint32_t e2m1_pair_bf16(uint32_t word, int sel) {
 // grouped GEMM op (grouped_matmul_antiquant.h:537-662: weights are RNE_bf16(e2m1 * scale), so the
 // scale has to be applied per element before the MFMA: ~2 VALU instructions per element) instead of
 // that of the GEMV op (fp32 weights: the scale is applied to the block's partial sum).
+// WHOLE: K is a multiple of 512.  Otherwise the last iteration has one to three groups: its loads past the row's end repeat the
+// last group (or the last scales), and the groups that are not there are not multiplied.
 // BLK = k per scale (32 or 16).  With 16, a 32-k block of a lane's row has two scales: the lanes
 // q < 2 of a column hold its first half, q >= 2 the second, so with the GEMM's rounding each lane
 // simply uses its half's scale, and with the GEMV's arithmetic the block takes two MFMAs, each on
@@ -281,7 +283,7 @@ __device__ __forceinline__ uint32_t e2m1_pair_bf16(uint32_t word, int sel) {
 // 16 k of x row r, row 8 + r only the last 16 k, so the product's rows < 8 (lanes q < 2) are the first
 // scale's partial sums and rows >= 8 (q >= 2) the second's; each lane applies its own half's scale and the
 // halves are added once at the end.
-template <int MB, bool ROUNDW, int BLK>
+template <int MB, bool ROUNDW, int BLK, bool WHOLE>
 __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ wg, const uint16_t* __restrict__ sg,
                                                    const uint16_t* __restrict__ x, uint16_t* __restrict__ y,
                                                    u32x4_t* xs, int64_t row0, int mg, int n0, int N, int K, int epilogue) {
@@ -307,7 +309,8 @@ __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ w
 
     for (int kc0 = 0; kc0 < K; kc0 += KC) {
         const int klen = min(KC, K - kc0);
-        const int niter = klen / GF_KSTEP;             // iterations of U groups
+        const int ngroups = klen / 128;
+        const int niter = (ngroups + U - 1) / U;       // iterations of U groups
         const int nblk = klen / BLK;                   // scales of the chunk (>= 16)
         const uint8_t* wp = wg + (kc0 >> 1);                                   // group c of the chunk: + 64 c bytes
         const uint8_t* sp = reinterpret_cast<const uint8_t*>(sg) + (kc0 / BLK) * 2;  // scale b of the chunk: + 2 b bytes
@@ -428,15 +431,28 @@ __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ w
                 // ordinary loads: an instruction covers 64 bytes of each of 16 rows, half a cache line; the other half
                 // comes with the next instruction and must still find the line (measured on this pattern alone:
                 // 6.3 TB/s with ordinary loads, 5.7 with nontemporal ones)
-                w[u] = *reinterpret_cast<const u32x4_t*>(wp + (woff + (uint32_t)((it * U + u) * 64)));
+                w[u] = *reinterpret_cast<const u32x4_t*>(wp + (woff + (uint32_t)((WHOLE ? it * U + u : min(it * U + u, ngroups - 1)) * 64)));
         };
         // scales 64 T + 16 q .. + 15 of this lane's row in the chunk: those of iteration 4 T + q (block 32)
         // or of half of iteration 2 T + (q >> 1) (block 16); clamped into the chunk (iterations past its
         // end do not exist)
         auto fetch_s = [&](u32x4_t (&sv)[2], int T) {
-            const int b0 = min(64 * T + 16 * q, nblk - 16);
-            sv[0] = *reinterpret_cast<const u32x4_t*>(sp + (soff + (uint32_t)(b0 * 2)));
-            sv[1] = *reinterpret_cast<const u32x4_t*>(sp + (soff + (uint32_t)(b0 * 2 + 16)));
+            if constexpr (WHOLE) {
+                const int b0 = min(64 * T + 16 * q, nblk - 16);
+                sv[0] = *reinterpret_cast<const u32x4_t*>(sp + (soff + (uint32_t)(b0 * 2)));
+                sv[1] = *reinterpret_cast<const u32x4_t*>(sp + (soff + (uint32_t)(b0 * 2 + 16)));
+            } else {
+                // 8 scales at a time, ending with the row at the latest; with block 32 the last group's 4 scales may be
+                // the second half of what is read then (a chunk of a single group begins behind others of its row)
+                typedef u32x4_t __attribute__((aligned(8))) u32x4_a8_t;   // scale rows of an odd number of groups
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const int b0 = 64 * T + 16 * q + 8 * e, at = min(b0, nblk - 8);
+                    u32x4_t v = *reinterpret_cast<const u32x4_a8_t*>(sp + (int64_t)soff + at * 2);
+                    if (BLK == 32 && b0 - at == 4) { v[0] = v[2]; v[1] = v[3]; }
+                    sv[e] = v;
+                }
+            }
         };
         u32x4_t sc[2], sn[2];
         // iteration `it` on the weights in w; rotates the scale registers every PER iterations
@@ -450,6 +466,7 @@ __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ w
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
+                if (!WHOLE && it * U + u >= ngroups) break;
                 if constexpr (BLK == 32) {
                     // this iteration's scales are those of lane (i, t): 2 dwords per group
                     if (u == 0) {
@@ -520,7 +537,7 @@ __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ w
     }
 }
 
-template <bool ROUNDW, int BLK>
+template <bool ROUNDW, int BLK, bool WHOLE>
 __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemv_fp4_mfma_kernel(const uint16_t* __restrict__ x,
                                                                          const uint8_t* __restrict__ w,
                                                                          const uint16_t* __restrict__ scale,
@@ -536,19 +553,19 @@ __global__ __launch_bounds__(64 * GF_WAVES, 4) void gemv_fp4_mfma_kernel(const u
     const uint16_t* sg = scale + (int64_t)g * N * (K / BLK);
     for (int64_t row0 = start; row0 < end; row0 += GF_ROWS) {
         const int mg = (int)min((int64_t)GF_ROWS, end - row0);
-        if (mg <= 4) gemv_fp4_mfma_rows<4, ROUNDW, BLK>(wg, sg, x, y, xs, row0, mg, n0, N, K, epilogue);
-        else if (mg <= 8) gemv_fp4_mfma_rows<8, ROUNDW, BLK>(wg, sg, x, y, xs, row0, mg, n0, N, K, epilogue);
-        else gemv_fp4_mfma_rows<16, ROUNDW, BLK>(wg, sg, x, y, xs, row0, mg, n0, N, K, epilogue);
+        if (mg <= 4) gemv_fp4_mfma_rows<4, ROUNDW, BLK, WHOLE>(wg, sg, x, y, xs, row0, mg, n0, N, K, epilogue);
+        else if (mg <= 8) gemv_fp4_mfma_rows<8, ROUNDW, BLK, WHOLE>(wg, sg, x, y, xs, row0, mg, n0, N, K, epilogue);
+        else gemv_fp4_mfma_rows<16, ROUNDW, BLK, WHOLE>(wg, sg, x, y, xs, row0, mg, n0, N, K, epilogue);
     }
 }
 
-template <bool ROUNDW, int BLK>
+template <bool ROUNDW, int BLK, bool WHOLE>
 static int launch_fp4_mfma(const moe_grouped_args* a, hipStream_t stream) {
     dim3 grid((unsigned)((a->N + GF_NR_WG - 1) / GF_NR_WG), (unsigned)a->G);
     constexpr size_t lds = (size_t)(GF_LDS_UNITS + GF_WAVES * GF_SCALE_UNITS) * 16;   // 72 KB: two workgroups per CU
     static std::atomic<uint64_t> lds_set{0};
-    if (const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemv_fp4_mfma_kernel<ROUNDW, BLK>), (int)lds, lds_set)) return rc;
-    hipLaunchKernelGGL((gemv_fp4_mfma_kernel<ROUNDW, BLK>), grid, dim3(64 * GF_WAVES), lds, stream,
+    if (const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemv_fp4_mfma_kernel<ROUNDW, BLK, WHOLE>), (int)lds, lds_set)) return rc;
+    hipLaunchKernelGGL((gemv_fp4_mfma_kernel<ROUNDW, BLK, WHOLE>), grid, dim3(64 * GF_WAVES), lds, stream,
                        static_cast<const uint16_t*>(a->x), static_cast<const uint8_t*>(a->weight),
                        static_cast<const uint16_t*>(a->scale), a->group_list, static_cast<uint16_t*>(a->y), a->M,
                        (int)a->K, (int)a->N, (int)a->epilogue);
@@ -574,6 +591,11 @@ int launch_vector(const moe_grouped_args* a, hipStream_t stream) {
         case MOE_FMT_FP4_B16: return launch_kmajor<MOE_FMT_FP4_B16>(a, stream);
         default: return MOE_ERR_BAD_FORMAT;
     }
+}
+
+template <bool ROUNDW, int BLK>
+static int launch_fp4_mfma(const moe_grouped_args* a, hipStream_t stream) {
+    return a->K % GF_KSTEP ? launch_fp4_mfma<ROUNDW, BLK, false>(a, stream) : launch_fp4_mfma<ROUNDW, BLK, true>(a, stream);
 }
 
 int launch_fp4_rows(const moe_grouped_args* a, bool gemm_rounding, hipStream_t stream) {

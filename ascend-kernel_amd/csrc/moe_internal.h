@@ -32,7 +32,7 @@ enum class GroupedKernel {
     TILES_PAIR, TILES_PAIR_EXACT, TILES_PAIR_SMALL, TILES_PAIR_EXACT16, TILES_QUAD,   // kinds of moe_gemm.hip
     TILES_BF16, TILES_BF16_128   // tiles of up to BF16_ROWS, of up to 128 rows
 };
-constexpr int FP4_ROWS_K = 512;   // K of an FP4_ROWS call is a multiple
+constexpr int FP4_ROWS_K = 128, FP4_ROWS_K_MIN = 256;   // K of an FP4_ROWS call is a multiple and not less
 constexpr int PAIR_ROWS = 160;    // rows of the largest tile of the quantized containers
 constexpr int BF16_ROWS = 224;    // rows of the largest bf16 tile
 // the kernel of a valid call, by its sizes, format and epilogue (moe_dispatch.cpp)

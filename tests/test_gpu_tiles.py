@@ -121,3 +121,22 @@ def test_order_of_experts(fmt, G, N, kernel):
     got = H.run_cabi(case, H.upload(case), "gemm")
     H.assert_close(got, H.oracle_out(case), rows=slice(0, used), what=f"order of experts {fmt} G={G}")
     assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
+
+
+@pytest.mark.parametrize("K", [256, 384, 640, 768, 896, 1152, 1664, 3712, 7296])
+@pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
+def test_fp4_rows_of_a_partly_filled_last_step(fmt, K):
+    """gemv_fp4_mfma_kernel where K is no multiple of 512: one to three groups of 128 k in the last step, the shortest K, chunks of
+    x that end with a single group (1664, 3712 and 7296 with 16, 8 and 4 rows staged); both roundings, a ragged N, SwiGLU."""
+    counts = [0, 1, 3, 4, 5, 8, 9, 16, 17]
+    _say(f"{fmt} partly filled last step K={K}")
+    for op, N in (("gemv", 141), ("gemm", 256), ("swiglu", 256)):
+        used = sum(counts) if op != "swiglu" else 30
+        case = H.make_case(fmt, 9, K, N, np.minimum(np.cumsum(counts), used), seed=K + N, extra_rows=2)
+        assert H.kernel_of(case, "gemv" if op == "gemv" else "gemm", swiglu=op == "swiglu") == "fp4_rows"
+        if op == "swiglu":
+            got, want = _swiglu(case)
+        else:
+            got, want = H.run_cabi(case, H.upload(case), op), H.oracle_out(case, gemv=op == "gemv")
+        H.assert_close(got, want, rows=slice(0, used), what=f"{fmt} {op} K={K}")
+        assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
