@@ -1303,9 +1303,14 @@ __device__ __forceinline__ void expert_chunks(int m, int& chunks, int& bpc) {
 // without rows last, otherwise as they come.  A tile's time goes by its row blocks, and with the largest tiles up to half
 // of a launch long, one that starts among the last leaves most of the chip waiting for it.
 // us as they come / in this order, rows unevenly routed (skew: see moe_dispatch.cpp): fp4 SwiGLU, 1511 tokens x 8 on 256
-// experts of 7168 x 2048, skew 1: 592 / 565; bf16, 1021 x 8 on 64 of 7168 x 2048, skew 0.25: 488 / 476.  Orders given by group_list
+// experts of 7168 x 2048, skew 1: 578 / 563, skew 0.25: 628 / 615; int4, 2000 x 4 on 64 of 7168 x 2048, skew 0.25: 307 / 282; fp8
+// and int8, 1500 x 8 on 128 of 4096 x 2048, skews 0 to 1: 0.99 to 1.02 times as fast.  Orders given by group_list
 // to a kernel that took it as it was, skew 1: int4, 2000 x 4 on 64 of 7168 x 2048: 327 / 296; fp4_b32, 1500 x 8 on 128
-// of 4096 x 3072: 420 / 399; fp8 and int8 on 128 of 4096 x 2048: 325 / 308 and 310 / 297; evenly routed, the same time.
+// of 4096 x 3072: 420 / 399; evenly routed, the same time.
+// Not for bf16, whose tiles wait for memory or for the matrix cores by their size: large and small ones side by side use both, and
+// that goes either way.  1021 x 8 on 64 of 7168 x 2048, three routings each of skew 0.25 and 0.5: 508 / 485, 457 / 472, 462 / 476
+// and 510 / 470, 496 / 474, 502 / 476; 1500 x 2 on 16 of 4096 x 8192, skew 1: 287 / 302; 700 x 8 on 64 of 7168 x 2048, skew 0:
+// 359 / 366.  (Largest and median ones in turn: 0.955 to 1.077 times as fast as unordered over the same calls.)
 // Every workgroup works the same order out: a counting sort, ranks from ballots; 64 experts of a wavefront at a
 // time leave one count per class in scratch (LDS of the tile routine, [rounds * WAVES][16]).
 template <int MTM, int BLOCK, int WAVES, typename Rows>
@@ -1373,8 +1378,8 @@ struct KernelCfg {
     static constexpr int WG_PER_CU = pair_wgs();
     static constexpr int WAVES_PER_SIMD = WG_PER_CU * WAVES / 4;
     static constexpr int MTM = PAIR ? pair_mt_max(KIND) : FP4_K ? FK_MT_MAX : KIND == GK_BF16_128 ? 4 : BF_MT_MAX;   // row blocks per tile
-    // tiles of up to 32 rows take the time of their weights, in any order
-    static constexpr bool ORDERED = MTM > PAIR_SMALL_MT_MAX;
+    // tiles of up to 32 rows take the time of their weights, in any order; bf16: see order_experts
+    static constexpr bool ORDERED = MTM > PAIR_SMALL_MT_MAX && FMT != MOE_FMT_BF16;
     // 16-byte LDS units of the tile routine (the tile prefix array follows them)
     static constexpr int lds_units() {
         if constexpr (PAIR)

@@ -107,11 +107,11 @@ def test_fp4_k_contiguous_row_blocks(fmt, K, epilogue):
 
 @pytest.mark.parametrize("fmt,G,N,kernel", [("int4", 600, 256, "tiles_quad"), ("fp4", 300, 512, "tiles_quad"), ("fp8", 300, 256, "tiles_pair"),
                                             ("int8", 511, 256, "tiles_pair"), ("fp4_b16", 300, 512, "tiles_pair"),
-                                            ("bf16", 300, 256, "tiles_bf16"), ("bf16", 400, 256, "tiles_bf16")])
+                                            ("fp4_b16", 450, 256, "tiles_pair"), ("bf16", 300, 256, "tiles_bf16")])
 def test_order_of_experts(fmt, G, N, kernel):
     """Launches of more tiles than workgroups take the experts with the largest tiles first: more experts than a workgroup has
     threads (two and three rounds of the sort, the last one partly filled), every number of 16-row blocks from 1 to 10, experts
-    without rows; 400 bf16 experts, for whose order LDS has no room."""
+    without rows; 450 fp4_b16 experts, for whose order LDS has no room, and bf16, which takes them as they come."""
     some = [rows for b in range(16, 161, 16) for rows in (b - 1, b, b + 1)] + [0, 0, 1, 0, 330]
     counts = [some[(g * 17 + g // 35) % 35] for g in range(G)]
     _say(f"order of experts {fmt} G={G} N={N}")
