@@ -72,10 +72,36 @@ static bool fp4_rows_partial_preferred(const moe_grouped_args* a, bool gemv_op) 
     return columns(a) <= 32768 || (a->K % 256 == 0 && a->K >= 4096);
 }
 
+// Tiles of K-contiguous fp4.  Two workgroups of 4 wavefronts per CU (TILES_FP4_K) are the better routine where a CU gets two tiles or
+// more; a tile alone on its CU has half of the wavefronts there, and the 8-wavefront k-split routine is ahead.  us, TILES_FP4_K /
+// TILES_PAIR, evenly routed, fp4_b32 and fp4_b16: 8 experts of 7168 x 2048 (64 tiles), 32 rows each 86 / 72 and 87 / 76, 64 rows 94 / 79
+// and 98 / 85; 16 of 7168 x 4096 (256 tiles), 48 rows 1.12 and 1.06 times; 8 of 4480 x 7168, 128 rows 88 / 78 and 90 / 84; one
+// expert of 7168 x 512, 128 rows 115 / 90 and 118 / 100; but 16 of 7168 x 4352 (272 tiles), 48 rows 0.88 and 0.88 times, and with 640 k 0.90
+// and 0.88 times at 256 tiles (level at 1024 k, fp4_b16 at 1536).  Routing that leaves some experts more rows than a tile takes makes a
+// few more tiles than CUs: 64 of 7168 x 1024 with 64 rows on average at a skew of 1, 159 / 167 and 162 / 183.  fp4_b16 with up to 16
+// rows per expert and K an odd multiple of 128, whose rows of scales do not begin with 32 bytes: 0.92 to 0.96 times.
+// TILES_FP4_K cuts an expert of 145 to 160 rows, one tile of TILES_PAIR, in two.  That is the faster way while the tiles do not fill
+// the CUs (8 of 2048 x 1024, 152 rows: fp4_b16 35 / 44).  Beyond, it depends on how many experts have just that many.  152 rows on
+// average, evenly routed, balanced top-k routing and at a skew of 0.25, TILES_FP4_K / TILES_PAIR: fp4_b32, 64 experts of 7168 x 4096 1.26,
+// 0.98 and 0.93 times, 128 of 4096 x 2048 1.20, 1.00 and 0.88, but 128 of 2048 x 2048 1.15, 0.96 and 0.84; fp4_b16 1.17, 0.94 and 0.87
+// on the first and 1.07, 0.92 and 0.81 on the last.
+static int64_t fp4_tiles(const moe_grouped_args* a, int64_t rows) {
+    const int64_t experts = std::max(std::min(a->M, a->G), (int64_t)1);
+    return experts * ((a->M + rows * experts - 1) / (rows * experts)) * ((a->N + 255) / 256);
+}
+
+static GroupedKernel fp4_kcontiguous_tiles(const moe_grouped_args* a) {
+    const bool b32 = a->format == MOE_FMT_FP4_B32;
+    const int64_t quad = fp4_tiles(a, FP4_K_ROWS), pair = fp4_tiles(a, PAIR_ROWS);
+    const bool pairs = quad == pair ? pair <= 256 && a->K >= (b32 ? 1024 : 1536) && (b32 || a->K % 256 == 0 || a->M > 16 * a->G)
+                                    : quad > 256 && a->M <= PAIR_ROWS * a->G && b32 && a->K >= 4096;
+    return pairs ? GroupedKernel::TILES_PAIR : GroupedKernel::TILES_FP4_K;
+}
+
 static GroupedKernel fp4_kcontiguous_kernel(const moe_grouped_args* a, bool gemv_op) {
     const bool rows = a->K % 512 == 0 || (a->K >= FP4_ROWS_K_MIN && a->K % FP4_ROWS_K == 0 && fp4_rows_partial_preferred(a, gemv_op));
     if (gemv_op) return rows ? GroupedKernel::FP4_ROWS : GroupedKernel::VECTOR;
-    return rows && fp4_rows_preferred(a) ? GroupedKernel::FP4_ROWS : GroupedKernel::TILES_PAIR;
+    return rows && fp4_rows_preferred(a) ? GroupedKernel::FP4_ROWS : fp4_kcontiguous_tiles(a);
 }
 
 // Strips for launches of up to 128 tiles of 256 columns, i.e. half of the CUs, and decode-like batches: with 32768 columns (16
@@ -137,6 +163,7 @@ const char* grouped_kernel_name(GroupedKernel k) {
         case GroupedKernel::TILES_PAIR_SMALL: return "tiles_pair_small";
         case GroupedKernel::TILES_PAIR_EXACT16: return "tiles_pair_exact16";
         case GroupedKernel::TILES_QUAD: return "tiles_quad";
+        case GroupedKernel::TILES_FP4_K: return "tiles_fp4_k";
         case GroupedKernel::TILES_BF16: return "tiles_bf16";
         case GroupedKernel::TILES_BF16_128: return "tiles_bf16_128";
     }

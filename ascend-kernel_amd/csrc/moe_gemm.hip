@@ -13,10 +13,11 @@
 // weight slices of the same experts in that XCD's L2, and takes the last two or three tiles of every
 // workgroup from a work counter (see tile_queue).  Every wavefront owns its columns for ALL
 // rows of the tile, so each weight element is dequantized exactly once per tile.  Three tile routines:
-//   gemm_tile_pair  the N-contiguous containers (int4, int8, the reference's fp4 and fp8); x, packed weights and
-//                   scales arrive by LDS-direct loads into a ring of stages walked by an unrolled k loop.  Either 8
-//                   wavefronts, the two of a SIMD splitting the k range (int8, fp8), or 4 wavefronts that each take
-//                   their 64 columns through all of k, two such workgroups per CU (int4 and fp4 prefill);
+//   gemm_tile_pair  every quantized container (int4, int8, the K-contiguous fp4 containers, the
+//                   reference's fp4 and fp8); x, packed weights and scales arrive by LDS-direct loads into a
+//                   ring of stages walked by an unrolled k loop.  Either 8 wavefronts, the two of a SIMD
+//                   splitting the k range (int8, fp8, K-contiguous fp4 in launches of few tiles), or 4 wavefronts
+//                   that each take their 64 columns through all of k, two such workgroups per CU (int4 and fp4 prefill);
 //                   tiles of up to 160 rows, or of up to 32 / 16 rows with small stages (decode batches,
 //                   and the GEMV op's arithmetic on the N-contiguous containers)
 //   gemm_tile_fp4_k the K-contiguous fp4 containers: 4 wavefronts, two workgroups per CU, tiles of up to 144 rows; x in a
@@ -189,7 +190,7 @@ __device__ __forceinline__ uint32_t here(uint32_t v) {
 }
 
 // ---------------------------------------------------------------------------------
-// Tile routine for the N-contiguous containers (int4, int8, reference fp4 / fp8) with two
+// Tile routine for the quantized containers (int4, int8, reference fp4 / fp8, K-contiguous fp4) with two
 // wavefronts per SIMD that split the k range.  Described for int4; what differs for the others follows.
 //
 // A single wavefront issues at most one instruction every ~5 cycles whatever its kind, and an
@@ -234,9 +235,13 @@ __device__ __forceinline__ uint32_t here(uint32_t v) {
 // the bits of the two rounded operations, see i8_one_rounding); fp8 decodes two codes at a time through
 // fp16 (see e4m3_ref_pair_over_256_fp16) and gets the fp32 scale of its 128 x 128 block through the ring,
 // 4 bytes per wavefront and step.
+//
+// K-contiguous fp4 (weight [N, K/2]): a step's tile is 256 weight rows x 32 bytes; MFMA t of a lane takes
+// weight row 64 cw + 16 t + i, whose 8 codes of the sub-step are one dword; the scales [N, K/block] are
+// fetched 16 bytes per row at a time into buffers of their own (see kc_issue_scale).
 // ---------------------------------------------------------------------------------
 // Kernel variants.
-//   GK_PAIR     N-contiguous containers: 8 wavefronts, k range split between the two wavefronts of a SIMD, tiles of
+//   GK_PAIR     quantized containers: 8 wavefronts, k range split between the two wavefronts of a SIMD, tiles of
 //               up to 160 rows
 //   GK_PAIR_SMALL  GK_PAIR with tiles of at most 32 rows: x stages of 4 KB leave LDS for a second workgroup per
 //               CU (decode-sized batches on the 4-bit containers)
@@ -247,7 +252,7 @@ __device__ __forceinline__ uint32_t here(uint32_t v) {
 //               64 columns through the whole k range in steps of 32 k, two workgroups per CU.  The two wavefronts
 //               of a SIMD belong to different workgroups and work on different tiles: no partial sums to
 //               exchange, a barrier spans 4 wavefronts instead of 8, and while one workgroup is between two tiles
-//               (stores, tile search, first loads) the other has the SIMDs to itself.
+//               (stores, tile search, first loads) the other has the SIMDs to itself.  (The N-contiguous containers.)
 //   GK_FP4_K    gemm_tile_fp4_k
 //   GK_BF16     gemm_tile_bf16
 //   GK_BF16_128 the same with tiles of at most 128 rows (a limit read at run time instead costs the small calls of either 1.5 %)
@@ -289,9 +294,13 @@ template <int FMT>
 constexpr int pair_sc_units(int kind) {
     return (FMT == MOE_FMT_FP4_REF ? 128 : FMT == MOE_FMT_INT4 ? 64 : FMT == MOE_FMT_FP8_REF ? 8 : 0) * pair_bk(kind) / 64;
 }
+// The K-contiguous fp4 containers keep their scales [N, K/block] outside the stages: 16 bytes (2 or 4 steps'
+// worth) per weight row at a time, three buffers of 256 rows
+template <int FMT>
+constexpr int pair_kc_scale_units() { return (FMT == MOE_FMT_FP4_B32 || FMT == MOE_FMT_FP4_B16) ? 3 * 256 : 0; }
 template <int FMT>
 constexpr int pair_lds_units(int kind) {
-    return pair_stages<FMT>(kind) * (pair_a_units(kind) + pair_b_units<FMT>(kind) + pair_sc_units<FMT>(kind));
+    return pair_stages<FMT>(kind) * (pair_a_units(kind) + pair_b_units<FMT>(kind) + pair_sc_units<FMT>(kind)) + pair_kc_scale_units<FMT>();
 }
 
 // End of a k-split tile.  The two wavefronts of a pair (same columns, the two k halves) hold partial sums of the
@@ -300,17 +309,17 @@ constexpr int pair_lds_units(int kind) {
 // wavefront, the second by h == 1, so both reduce and store at the same time.  Rounds of at most 4 row
 // blocks (8 wavefronts x 4 blocks x 4 KB fit the x stage area, free now).
 // WHOLE: the wavefront holds the whole sums (no k split): it stores all of its row blocks, nothing is exchanged.
-template <int MT, bool WHOLE = false>
+template <int MT, bool KC, bool WHOLE = false>
 __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, f32x4_t (&acc)[MT][4], int h, int cw, int lane,
                                             int col0, int64_t row0, int rows, int n0, const Ticket& tk) {
-    const int q = lane >> 4;
+    const int i = lane & 15, q = lane >> 4;
     const bool takes = tk.counter != nullptr && threadIdx.x == 0;
     unsigned next_tile = 0;
     if (takes) next_tile = queue_draw_raw(tk.counter);
     constexpr int MH = (MT + 1) / 2, RR = MH < 4 ? MH : 4, ROUNDS = (MH + RR - 1) / RR;
     // the last tile of an N that is not a multiple of 256 (the reference's fp8 container: multiples of 128)
     // computes columns past N from whatever follows in the slab: they are not stored
-    const bool live = n0 + col0 < P.N;
+    const bool live = KC || n0 + col0 < P.N;
     const bool swi = P.epilogue == MOE_EPILOGUE_SWIGLU;
     // stores go through a buffer resource that ends after the tile's last valid row: those to padded rows
     // fall outside it and are dropped
@@ -318,7 +327,18 @@ __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, 
     const rsrc_t ry = make_rsrc(P.y + row0 * (int64_t)NO, (int64_t)rows * NO * 2);
     auto store_block = [&](int mt) {
         if (!live) return;
-        if (swi) {
+        if (swi && KC) {
+            // K-contiguous containers: the weight rows come in blocks of 32 = (16 gate rows, 16 up rows), which are
+            // the MFMAs t = (0, 1) and (2, 3) of this lane; y has N / 2 columns
+            const int vo = (4 * q * NO + ((n0 + 64 * cw) >> 1) + i) * 2;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    __builtin_amdgcn_raw_buffer_store_b16(
+                        (uint16_t)(pack_bf16_rne(swiglu(acc[mt][2 * u][r], acc[mt][2 * u + 1][r]), 0.f) & 0xffffu), ry,
+                        vo + 32 * u, (16 * mt + r) * NO * 2, 0);
+        } else if (swi) {
             // this lane's 4 columns are (gate, gate, up, up) of 2 output columns; y has N / 2 columns
             const int vo = (4 * q * NO + ((n0 + col0) >> 1)) * 2;
 #pragma unroll
@@ -326,6 +346,15 @@ __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, 
                 __builtin_amdgcn_raw_buffer_store_b32(
                     pack_bf16_rne(swiglu(acc[mt][0][r], acc[mt][2][r]), swiglu(acc[mt][1][r], acc[mt][3][r])), ry, vo,
                     (16 * mt + r) * NO * 2, 0);
+        } else if (KC) {
+            // K-contiguous containers: MFMA t holds column 64 cw + 16 t + i, one 2-byte store each
+            const int vy = (4 * q * P.N + n0 + 64 * cw + i) * 2;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(pack_bf16_rne(acc[mt][t][r], 0.f) & 0xffffu), ry,
+                                                          vy + 32 * t, (16 * mt + r) * P.N * 2, 0);
         } else {
             const int vy = (4 * q * P.N + n0 + col0) * 2;
 #pragma unroll
@@ -392,15 +421,20 @@ __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, 
 // the multiplies of the general case, and no masking.
 template <int FMT, int MT, int KIND, bool STACK2 = false>
 __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk) {
-    static_assert(FMT == MOE_FMT_INT4 || FMT == MOE_FMT_INT8 || FMT == MOE_FMT_FP4_REF || FMT == MOE_FMT_FP8_REF, "the N-contiguous containers");
+    static_assert(FMT != MOE_FMT_BF16, "the k-split tile routine decodes quantized containers");
     constexpr bool EXACT = pair_exact(KIND);
     static_assert(!STACK2 || (EXACT && FMT == MOE_FMT_FP4_REF && MT == 1), "two scale groups stacked in one MFMA: fp4, at most 8 rows");
     static_assert(!EXACT || FMT == MOE_FMT_INT4 || FMT == MOE_FMT_FP4_REF || FMT == MOE_FMT_FP8_REF,
                   "un-rounded weights: the N-contiguous containers of the GEMV op");
     constexpr bool FP4 = FMT == MOE_FMT_FP4_REF, I8 = FMT == MOE_FMT_INT8, F8 = FMT == MOE_FMT_FP8_REF;
+    // K-contiguous fp4 (weight [N, K/2], scales [N, K/KBLK]): the step's tile is 256 weight rows x 32 bytes
+    constexpr bool KC = FMT == MOE_FMT_FP4_B32 || FMT == MOE_FMT_FP4_B16;
+    constexpr int KBLK = FMT == MOE_FMT_FP4_B32 ? 32 : 16;
     constexpr bool B8 = I8 || F8;   // one byte per weight: tiles of 64 rows x 256 bytes
     // Q4: the kind without the k split (GK_QUAD): 4 wavefronts, steps of 32 k, every wavefront in every step
     constexpr bool Q4 = KIND == GK_QUAD;
+    static_assert(!Q4 || FMT == MOE_FMT_INT4 || FMT == MOE_FMT_INT8 || FMT == MOE_FMT_FP4_REF || FMT == MOE_FMT_FP8_REF,
+                  "the 4-wavefront kind serves the N-contiguous containers");
     constexpr int NW = pair_waves(KIND);
     constexpr int BK = pair_bk(KIND), S = pair_stages<FMT>(KIND), PAIR_SC_UNITS = pair_sc_units<FMT>(KIND);
     constexpr int PAIR_B_UNITS = pair_b_units<FMT>(KIND);
@@ -433,7 +467,9 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
 
     const int64_t KN = (int64_t)P.K * P.N;
     const rsrc_t rw = B8 ? make_rsrc(P.w + g * KN, KN) : make_rsrc(P.w + g * (KN >> 1), KN >> 1);
-    const rsrc_t rs = make_rsrc(static_cast<const uint16_t*>(P.scale) + (int64_t)g * P.scale_rows * P.N, (int64_t)P.scale_rows * P.N * 2);
+    const rsrc_t rs = KC ? make_rsrc(static_cast<const uint16_t*>(P.scale) + g * (KN / KBLK), (KN / KBLK) * 2)
+                         : make_rsrc(static_cast<const uint16_t*>(P.scale) + (int64_t)g * P.scale_rows * P.N,
+                                     (int64_t)P.scale_rows * P.N * 2);
     // fp8: the expert's fp32 block scales [K/128, N/128]; this wavefront's 128-column block
     const rsrc_t rs8 = make_rsrc(static_cast<const float*>(P.scale) + (int64_t)g * (P.K >> 7) * (P.N >> 7),
                                  (int64_t)(P.K >> 7) * (P.N >> 7) * 4);
@@ -453,13 +489,17 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     // int8 / fp8 (rows of 256 bytes): instruction e of wavefront wv brings rows 8 wv + 4 e + (lane >> 4); the
     // 64-byte quarters of a row are permuted by (row >> 3) & 3 = wv & 3, so that the four q groups read
     // from different quarters of the banks
-    const int vb = B8 ? (lane >> 4) * P.N + (((lane & 15) ^ (4 * (wv & 3))) * 16)
-                      : (lane >> 3) * (P.N >> 1) + (((lane & 7) ^ (4 * (wv & 1))) * 16);
+    // K-contiguous fp4: LDS unit 64 wv + lane of the stage holds one 16-byte half of weight row
+    // n = 32 wv + (lane >> 1); the halves of the rows with odd (n >> 3) are swapped (bank spread)
+    const int kc_n = 32 * wv + (lane >> 1);
+    const int vb = KC   ? kc_n * (P.K >> 1) + 16 * ((lane & 1) ^ ((kc_n >> 3) & 1))
+                   : B8 ? (lane >> 4) * P.N + (((lane & 15) ^ (4 * (wv & 3))) * 16)
+                        : (lane >> 3) * (P.N >> 1) + (((lane & 7) ^ (4 * (wv & 1))) * 16);
     constexpr int XI = Q4 ? MT : 2 * MT;          // x load instructions per step (1 KB each: 16 or 8 rows)
     constexpr int XROWS = Q4 ? 16 : 8;
     constexpr int NA = (XI + NW - 1) / NW;        // ... per wavefront
     constexpr int NB = B8 ? 2 : 1;                // packed-tile instructions
-    constexpr int NI = NA + NB + (PAIR_SC_UNITS ? 1 : 0);   // + this wavefront's share of the step's scales
+    constexpr int NI = NA + NB + ((PAIR_SC_UNITS || KC) ? 1 : 0);   // + this wavefront's share of the step's scales
     int ja[NA], ca[NA];
 #pragma unroll
     for (int m = 0; m < NA; ++m) {
@@ -470,16 +510,31 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     }
     // (Q4 on the reference's fp4 container: the 32 k of a step are the rows [16 hp, +16) and [32 + 16 hp, +16) of the
     // container's 64-row tile, hp = step & 1: wavefront wv brings the 8 rows from 32 (wv >> 1) + 16 hp + 8 (wv & 1) on)
-    const int cb = B8            ? 8 * wv * P.N + n0
+    const int cb = KC            ? n0 * (P.K >> 1)
+                   : B8          ? 8 * wv * P.N + n0
                    : (Q4 && FP4) ? (32 * (wv >> 1) + 8 * (wv & 1)) * (P.N >> 1) + (n0 >> 1)
                                  : 8 * wv * (P.N >> 1) + (n0 >> 1);
-    const int kb_step = B8 ? BK * P.N : BK * (P.N >> 1);
+    const int kb_step = KC ? BK / 2 : B8 ? BK * P.N : BK * (P.N >> 1);
     // byte offset of step kp's packed rows in the expert's slab
     auto b_step_offset = [&](int kp) {
         if constexpr (Q4 && FP4)
             return ((kp >> 1) * 64 + (kp & 1) * 16) * (P.N >> 1);
         else
             return kp * kb_step;
+    };
+    // K-contiguous fp4 scales.  Fetching the 4 or 8 bytes a weight row needs per step costs a request per
+    // row and step (measured: 20 % of the kernel); instead 16 bytes of a row -- the scales of SUP steps --
+    // are fetched at a time: the load slot of step kt brings, for step index kp = kt + KC_D, the rows
+    // [RPS (kp % SUP), + RPS) of super-block kp / SUP (one lane per row, RPW rows per wavefront) into buffer
+    // (kp / SUP) % 3 of 256 rows x 16 bytes behind the stages.  KC_D = SUP + 3: a load issued in step t is
+    // visible after barrier t + 2, and the scales of step s are read during step s - 1.  Three buffers: the
+    // first load into a buffer comes after the last read of its previous occupant.
+    constexpr int SUP = KBLK == 32 ? 4 : 2, KC_D = SUP + 3, RPS = 256 / SUP, RPW = RPS / 8;
+    const int kc_vs = lane * (P.K / KBLK) * 2;
+    auto kc_issue_scale = [&](int kp) {
+        const int sb = kp / SUP, j = kp % SUP, row = RPS * j + RPW * wv;
+        if (lane < RPW)
+            lds_load16(rs, lds_s + (sb % 3) * 256 + row, kc_vs, (n0 + row) * (P.K / KBLK) * 2 + sb * 16);
     };
     // scales of a step: int4 2 rows of 512 bytes, 128 bytes (8 lanes) per wavefront: bytes [128 (wv & 3), +128) of
     // row wv >> 2; fp4 4 rows (one per 16 k), 256 bytes (16 lanes) per wavefront: bytes [256 (wv & 1), +256) of row wv >> 1
@@ -500,6 +555,8 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             const int e = m - NA;
             lds_load16_at(rw, here(b_at) + ST * (PAIR_B_UNITS * 16) + e * 1024, vb,
                           cb + (B8 ? 4 * e * P.N : 0) + b_step_offset(kt + AHEAD));
+        } else if constexpr (KC) {
+            kc_issue_scale(kt + KC_D);
         } else if constexpr (F8) {
             // the block scale of the stage's 128-k block, 4 bytes by lane 0 (past K: reads as 0, unused)
             if (lane == 0)
@@ -592,6 +649,11 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
                      "s_cbranch_scc1 2f\n\ts_sleep 1\n\ts_branch 1b\n2:"
                      : "=&v"(seen_v), "=&s"(seen_s) : "s"(arrivals_at), "s"((uint32_t)NW * steps), "v"(early) : "memory", "scc");
     };
+    if constexpr (KC) {
+        // the scale loads the groups below do not cover (older than all of them: landed by the first barrier)
+#pragma unroll
+        for (int kp = 0; kp < KC_D - AHEAD; ++kp) kc_issue_scale(kp);
+    }
 #pragma unroll
     for (int st0 = 0; st0 < AHEAD; ++st0) issue_group(st0 - AHEAD, st0);
 #pragma unroll
@@ -628,7 +690,8 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     // this lane's packed dwords and scales of its sub-step of LDS stage st
     uint32_t r[8];
     u32x2_t sc = {0u, 0u}, sc2 = {0u, 0u};   // sc2: with EXACT, the fp4 scales of the second 16 k of the sub-step
-    auto read_raw = [&](int st) {
+    // (s: the step the stage belongs to)
+    auto read_raw = [&](int st, int s) {
         const uint16_t* sc16 = reinterpret_cast<const uint16_t*>(lds_s + st * PAIR_SC_UNITS);
         if constexpr (FP4) {
             // Reference pre-shuffle (grouped_gemm/test/python/test_group_gemm_fp4.py:129-142): the tile row
@@ -649,6 +712,22 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             } else {
                 sc = *reinterpret_cast<const u32x2_t*>(sc16 + 256 * (2 * h + (q >> 1)) + col0);
             }
+        } else if constexpr (KC) {
+            // MFMA t takes weight row n = 64 cw + 16 t + i: its 8 codes k = 32 h + 8 q + [0, 8) are dword q of
+            // the row's half h; the scale of that block
+            const uint32_t* t32 = reinterpret_cast<const uint32_t*>(lds_b + st * PAIR_B_UNITS);
+            // the row's 8 scales of super-block s / SUP; this lane's block among them
+            const uint16_t* sup = reinterpret_cast<const uint16_t*>(lds_s + ((s / SUP) % 3) * 256) +
+                                  (KBLK == 16 ? 4 * (s % SUP) + 2 * h + (q >> 1) : 2 * (s % SUP) + h);
+            uint32_t s4[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int n = 64 * cw + 16 * t + i;
+                r[t] = t32[(2 * n + (h ^ ((i >> 3) & 1))) * 4 + q];
+                s4[t] = sup[8 * n];
+            }
+            sc[0] = s4[0] | (s4[1] << 16);
+            sc[1] = s4[2] | (s4[3] << 16);
         } else if constexpr (B8) {
             // dword 16 cw + i of each of this lane's 8 k rows; the quarter of the row it lies in is
             // permuted by (row >> 3) & 3 = q (see vb)
@@ -663,7 +742,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             sc = *reinterpret_cast<const u32x2_t*>(sc16 + 256 * h + col0);
         }
     };
-    read_raw(0);
+    read_raw(0, 0);
 
     // One data step; st = step mod S is its LDS stage, sn the next one, sl the stage this step's loads
     // go to (wave-uniform).
@@ -679,7 +758,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
         if constexpr (EXACT) {
             m[0] = m[1] = m[2] = m[3] = FP4 ? 1.f : 512.f;
             z[0] = z[1] = z[2] = z[3] = FP4 ? 0.f : -8.f;
-        } else if constexpr (FP4) {
+        } else if constexpr (FP4 || KC) {
             m[0] = s0; m[1] = s1; m[2] = s2; m[3] = s3;
             z[0] = z[1] = z[2] = z[3] = 0.f;
         } else {
@@ -702,6 +781,20 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
                 // first x fragments of the MFMA phase, read under the rest of the decode
 #pragma unroll
                 for (int f = 0; f < R; ++f) afr[f & 3] = la[x_unit(16 * f + xrow)];
+            }
+            if constexpr (KC) {
+                // dword r[t] = 8 consecutive k of MFMA t's weight row: byte p = the k pair p
+#pragma unroll
+                for (int t = p0; t < p0 + 2; ++t) {
+                    const f32x2_t f0 = e2m1_pair_to_f32<0>(r[t]), f1 = e2m1_pair_to_f32<1>(r[t]);
+                    const f32x2_t f2 = e2m1_pair_to_f32<2>(r[t]), f3 = e2m1_pair_to_f32<3>(r[t]);
+                    bf[t][0] = pack_bf16_rne(f0[0] * m[t], f0[1] * m[t]);
+                    bf[t][1] = pack_bf16_rne(f1[0] * m[t], f1[1] * m[t]);
+                    bf[t][2] = pack_bf16_rne(f2[0] * m[t], f2[1] * m[t]);
+                    bf[t][3] = pack_bf16_rne(f3[0] * m[t], f3[1] * m[t]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                continue;
             }
             if constexpr (F8) {
                 // byte t of the dwords of k rows 2p, 2p+1, decoded as a pair through fp16 (see
@@ -897,7 +990,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             }
 #pragma unroll
             for (int m = (mt * NI + MT - 1) / MT; m < ((mt + 1) * NI + MT - 1) / MT; ++m) issue(m, kt, sl);
-            if (mt == 0) read_raw(sn);
+            if (mt == 0) read_raw(sn, kt + 1);
             __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_s_setprio(0);
@@ -910,10 +1003,21 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     // unrolled over the ring, so that every stage number is a constant and the LDS addresses of a step are
     // immediate offsets (with run-time stage numbers a step spent 9 vector and about 25 scalar instructions on
     // them: measured 10 % of the kernel's time at K = 7168); a tile starts at stage 0
-    for (int kt0 = 0; kt0 < nk; kt0 += S) {
+    // (the K-contiguous containers keep run-time stage numbers: their routine has no registers left for the
+    // unrolled form)
+    if constexpr (!KC) {
+        for (int kt0 = 0; kt0 < nk; kt0 += S) {
 #pragma unroll
-        for (int u = 0; u < S; ++u)
-            if (kt0 + u < nk) step(kt0 + u, u, (u + 1) % S, (u + S - 1) % S);
+            for (int u = 0; u < S; ++u)
+                if (kt0 + u < nk) step(kt0 + u, u, (u + 1) % S, (u + S - 1) % S);
+        }
+    } else {
+        for (int kt = 0, st = 0, sl = S - 1; kt < nk; ++kt) {
+            const int sn = st == S - 1 ? 0 : st + 1;
+            step(kt, st, sn, sl);
+            st = sn;
+            sl = sl == S - 1 ? 0 : sl + 1;
+        }
     }
     if constexpr (!SPLIT_BARRIER)
         if (h == 1) ring_barrier();   // barrier nk-1
@@ -929,7 +1033,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[0][t][e] += __shfl_xor(acc[0][t][e], 32);
     }
-    pair_finish<MT, Q4>(P, smem, acc, h, cw, lane, col0, row0, rows, n0, tk);
+    pair_finish<MT, KC, Q4>(P, smem, acc, h, cw, lane, col0, row0, rows, n0, tk);
 }
 
 // ---------------------------------------------------------------------------------
@@ -938,8 +1042,8 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
 //
 // Bound by issue, as the N-contiguous kinds: 2 vector instructions per weight (exact convert, times its scale, rounded to
 // bf16) beside the MFMAs, and next to that by requests to L2.  Two workgroups per CU hide each other's barriers and the time
-// between tiles, which the 8-wavefront k-split routine that served these containers before did not.
-// us, that routine / this one: 128 experts of 2048 x 7168, 2047 tokens x 8 rows: fp4_b16 686 / 570 (843 TFLOP/s), fp4_b32
+// between tiles, which the 8 wavefronts of GK_PAIR do not; with a single tile per CU GK_PAIR is ahead (see moe_dispatch.cpp).
+// us, GK_PAIR / this one: 128 experts of 2048 x 7168, 2047 tokens x 8 rows: fp4_b16 686 / 570 (843 TFLOP/s), fp4_b32
 // 635 / 551; 7168 x 2048 the same rows, fp4_b32: 624 / 593; 4608 x 3072, 1245 tokens x 8, unevenly routed, fp4_b16: 490 / 436; 8 of
 // 3968 x 13568, 841 rows each, fp4_b32: 699 / 627.  (The reference's fp4 container on GK_QUAD: 522, 534 on the first and third.)
 //
@@ -959,6 +1063,7 @@ constexpr int FK_XS = 4;                             // x stages
 constexpr int FK_X_UNITS = 16 * FK_MT_MAX * 4;       // 32 k
 constexpr int FK_W_UNITS = GM_BN * 8;                // 256 weight rows x 256 k
 constexpr int FK_S_UNITS = GM_BN * 2;                // their scales: 32 bytes a row (fp4_b32: 16)
+static_assert(16 * FK_MT_MAX == FP4_K_ROWS, "what the dispatch goes by");
 constexpr int fk_lds_units() { return FK_XS * FK_X_UNITS + FK_W_UNITS + FK_S_UNITS; }
 template <int FMT, int MT>
 __device__ __forceinline__ void gemm_tile_fp4_k(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk) {
@@ -1122,7 +1227,7 @@ __device__ __forceinline__ void gemm_tile_fp4_k(const GemmParams& P, u32x4_t* sm
     if (nk & 4) half(std::integral_constant<int, 0>{}, std::false_type{}, np);
     // the last loads are for steps past K and never read; wait out the last MFMAs' latency
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15\n\ts_barrier" ::: "memory");
-    pair_finish<MT, true>(P, smem, acc, 0, cw, lane, 64 * cw + 4 * i, row0, rows, n0, tk);
+    pair_finish<MT, false, true>(P, smem, acc, 0, cw, lane, 64 * cw + 4 * i, row0, rows, n0, tk);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1277,7 +1382,7 @@ __device__ __forceinline__ void gemm_tile_bf16(const GemmParams& P, u32x4_t* sme
     }
     // the last loads are for pairs behind the last one and never read; wait out the last MFMAs' latency
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15\n\ts_barrier" ::: "memory");
-    pair_finish<MT, true>(P, smem, acc, 0, cw, lane, 64 * cw + 4 * i, row0 + 16 * MT * wr, max(rows - 16 * MT * wr, 0), n0, tk);
+    pair_finish<MT, false, true>(P, smem, acc, 0, cw, lane, 64 * cw + 4 * i, row0 + 16 * MT * wr, max(rows - 16 * MT * wr, 0), n0, tk);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1367,8 +1472,8 @@ __device__ __forceinline__ void order_experts(int G, int tid, int* scratch, uint
 template <int FMT, int KIND>
 struct KernelCfg {
     static constexpr bool PAIR = KIND == GK_PAIR || KIND == GK_PAIR_SMALL || KIND == GK_QUAD || pair_exact(KIND);
-    static constexpr bool FP4_K = FMT == MOE_FMT_FP4_B32 || FMT == MOE_FMT_FP4_B16;
-    static_assert(FP4_K == (KIND == GK_FP4_K) && PAIR == (FMT != MOE_FMT_BF16 && !FP4_K), "the routine of the container");
+    static constexpr bool FP4_K = KIND == GK_FP4_K;
+    static_assert(PAIR == (FMT != MOE_FMT_BF16 && !FP4_K) && (!FP4_K || FMT == MOE_FMT_FP4_B32 || FMT == MOE_FMT_FP4_B16), "the routine of the container");
     static constexpr int WAVES = PAIR ? pair_waves(KIND) : FP4_K ? 4 : 8;
     static constexpr int BLOCK = PAIR || FP4_K ? 16 : 32;   // rows per row block of a tile routine's template argument
     static constexpr int BN = GM_BN;                                             // columns per tile
@@ -1378,8 +1483,9 @@ struct KernelCfg {
     static constexpr int WG_PER_CU = pair_wgs();
     static constexpr int WAVES_PER_SIMD = WG_PER_CU * WAVES / 4;
     static constexpr int MTM = PAIR ? pair_mt_max(KIND) : FP4_K ? FK_MT_MAX : KIND == GK_BF16_128 ? 4 : BF_MT_MAX;   // row blocks per tile
-    // tiles of up to 32 rows take the time of their weights, in any order; bf16: see order_experts
-    static constexpr bool ORDERED = MTM > PAIR_SMALL_MT_MAX && FMT != MOE_FMT_BF16;
+    // tiles of up to 32 rows take the time of their weights, in any order; bf16: see order_experts; launches of K-contiguous fp4 on
+    // GK_PAIR have a tile per CU, mostly
+    static constexpr bool ORDERED = MTM > PAIR_SMALL_MT_MAX && FMT != MOE_FMT_BF16 && !(PAIR && (FMT == MOE_FMT_FP4_B32 || FMT == MOE_FMT_FP4_B16));
     // 16-byte LDS units of the tile routine (the tile prefix array follows them)
     static constexpr int lds_units() {
         if constexpr (PAIR)
@@ -1740,6 +1846,12 @@ int launch_tiles(const moe_grouped_args* a, GroupedKernel kind, hipStream_t stre
             switch (a->format) {
                 case MOE_FMT_FP8_REF: return launch_gemm_kind<MOE_FMT_FP8_REF, GK_PAIR>(P, a, stream);
                 case MOE_FMT_INT8: return launch_gemm_kind<MOE_FMT_INT8, GK_PAIR>(P, a, stream);
+                case MOE_FMT_FP4_B32: return launch_gemm_kind<MOE_FMT_FP4_B32, GK_PAIR>(P, a, stream);
+                case MOE_FMT_FP4_B16: return launch_gemm_kind<MOE_FMT_FP4_B16, GK_PAIR>(P, a, stream);
+                default: return MOE_ERR_BAD_FORMAT;
+            }
+        case GroupedKernel::TILES_FP4_K:
+            switch (a->format) {
                 case MOE_FMT_FP4_B32: return launch_gemm_kind<MOE_FMT_FP4_B32, GK_FP4_K>(P, a, stream);
                 case MOE_FMT_FP4_B16: return launch_gemm_kind<MOE_FMT_FP4_B16, GK_FP4_K>(P, a, stream);
                 default: return MOE_ERR_BAD_FORMAT;

@@ -23,17 +23,17 @@ inline int ensure_dynamic_lds(const void* kernel, int bytes, std::atomic<uint64_
 
 int launch_dequant_fp4_bf16(const moe_dequant_args* a, hipStream_t stream);
 // The kernels of the two grouped ops.  TILES_PAIR_EXACT and TILES_PAIR_EXACT16 have the GEMV op's arithmetic (weights not
-// rounded to bf16), the other TILES that of the GEMM op; STRIPS and FP4_ROWS come with either.  TILES_PAIR is the k-split kind
-// for the N-contiguous containers and GK_FP4_K, the only kind they have, for the K-contiguous fp4 ones.
+// rounded to bf16), the other TILES that of the GEMM op; STRIPS and FP4_ROWS come with either.
 enum class GroupedKernel {
     VECTOR,               // K-contiguous containers without matrix cores (moe_gemv.hip)
     FP4_ROWS,             // K-contiguous fp4, 16 rows of an expert per pass (moe_gemv.hip)
     STRIPS_32, STRIPS_64, STRIPS_128,   // N-contiguous containers in strips of that many columns (moe_stream.hip)
-    TILES_PAIR, TILES_PAIR_EXACT, TILES_PAIR_SMALL, TILES_PAIR_EXACT16, TILES_QUAD,   // kinds of moe_gemm.hip
+    TILES_PAIR, TILES_PAIR_EXACT, TILES_PAIR_SMALL, TILES_PAIR_EXACT16, TILES_QUAD, TILES_FP4_K,   // kinds of moe_gemm.hip
     TILES_BF16, TILES_BF16_128   // tiles of up to BF16_ROWS, of up to 128 rows
 };
 constexpr int FP4_ROWS_K = 128, FP4_ROWS_K_MIN = 256;   // K of an FP4_ROWS call is a multiple and not less
-constexpr int PAIR_ROWS = 160;    // rows of the largest tile of the quantized containers
+constexpr int PAIR_ROWS = 160;    // rows of the largest tile of TILES_PAIR and TILES_QUAD
+constexpr int FP4_K_ROWS = 144;   // of TILES_FP4_K
 constexpr int BF16_ROWS = 224;    // rows of the largest bf16 tile
 // the kernel of a valid call, by its sizes, format and epilogue (moe_dispatch.cpp)
 GroupedKernel grouped_kernel(const moe_grouped_args* a, bool gemv_op);

@@ -40,12 +40,31 @@ def test_tiles_of_the_n_contiguous_containers():
 def test_k_contiguous_fp4(fmt):
     at = lambda op, r, K, swiglu=False: kernel(fmt, op, r * 64, 64, K, 2048, swiglu)   # noqa: E731
     assert (at("gemv", 1, 7168), at("gemv", 100, 7168), at("gemv", 1, 7168 + 32)) == ("fp4_rows", "fp4_rows", "vector")
-    assert (at("gemm", 12, 7168), at("gemm", 13, 7168), at("gemm", 1, 7168 + 128)) == ("fp4_rows", "tiles_pair", "tiles_pair")
+    assert (at("gemm", 12, 7168), at("gemm", 13, 7168), at("gemm", 1, 7168 + 128)) == ("fp4_rows", "tiles_fp4_k", "tiles_fp4_k")
     # with SwiGLU, 5 rows per expert; 8 with up to 64 rows in all
-    assert (at("gemm", 5, 7168, True), at("gemm", 6, 7168, True)) == ("fp4_rows", "tiles_pair")
+    assert (at("gemm", 5, 7168, True), at("gemm", 6, 7168, True)) == ("fp4_rows", "tiles_fp4_k")
     few = lambda M, G: kernel(fmt, "gemm", M, G, 4096, 2048, True)   # noqa: E731
     assert (few(64, 8), few(65, 8)) == ("fp4_rows", "tiles_pair")
     assert (few(32, 4), few(33, 4)) == ("fp4_rows", "tiles_pair")
+
+
+@pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
+def test_k_contiguous_fp4_tiles(fmt):
+    tiles = lambda r, G, K, N: kernel(fmt, "gemm", r * G, G, K, N)   # noqa: E731
+    k_min = {"fp4_b32": 1024, "fp4_b16": 1536}[fmt]
+    # a tile per CU: 256 tiles, and from some length of K on
+    for r in (13, 144, 161, 288):
+        chunks = -(-r // 160)
+        assert (tiles(r, 16 // chunks, 7168, 4096), tiles(r, 16 // chunks, 7168, 4352)) == ("tiles_pair", "tiles_fp4_k")
+        assert (tiles(r, 8, k_min, 1024), tiles(r, 8, k_min - 128, 1024)) == ("tiles_pair", "tiles_fp4_k")
+    # fp4_b16, few rows, K an odd multiple of 128
+    assert (tiles(16, 8, 7168 - 128, 1024), tiles(17, 8, 7168 - 128, 1024), tiles(16, 8, 7168 - 256, 1024)) == (
+        "tiles_pair" if fmt == "fp4_b32" else "tiles_fp4_k", "tiles_pair", "tiles_pair")
+    # 145 to 160 rows per expert: in two while that does not fill the CUs, beyond, in one on fp4_b32 with a long K
+    assert (tiles(145, 8, 7168, 4096), tiles(160, 8, 7168, 4096)) == ("tiles_fp4_k", "tiles_fp4_k")
+    large = "tiles_pair" if fmt == "fp4_b32" else "tiles_fp4_k"
+    assert (tiles(145, 16, 4096, 4096), tiles(160, 64, 4096, 4096), tiles(160, 64, 4096 - 128, 4096)) == (large, large, "tiles_fp4_k")
+    assert (tiles(144, 64, 4096, 4096), tiles(161, 64, 4096, 4096), tiles(320, 64, 4096, 4096)) == ("tiles_fp4_k",) * 3
 
 
 def test_bf16():

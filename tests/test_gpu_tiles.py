@@ -95,6 +95,25 @@ def test_fp4_k_contiguous_row_blocks(fmt, K, epilogue):
     counts = [rows for b in range(16, 161, 16) for rows in (b - 1, b, b + 1)] + [1, 0, 321]
     _say(f"{fmt} row blocks K={K} epilogue={epilogue}")
     case = H.make_case(fmt, len(counts), K, 512, np.cumsum(counts), seed=K, extra_rows=3)
+    assert H.kernel_of(case, "gemm", swiglu=epilogue == "swiglu") == "tiles_fp4_k"
+    used = int(case["group_list"][-1])
+    if epilogue == "swiglu":
+        got, want = _swiglu(case)
+    else:
+        got, want = H.run_cabi(case, H.upload(case), "gemm"), H.oracle_out(case)
+    H.assert_close(got, want, rows=slice(0, used), what=f"{fmt} K={K} {epilogue}")
+    assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
+
+
+@pytest.mark.parametrize("epilogue", ["none", "swiglu"])
+@pytest.mark.parametrize("K", [1536, 1664, 1920])   # 6, 6.5 and 7.5 super-blocks of scales of fp4_b32; 12, 13 and 15 of fp4_b16
+@pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
+def test_fp4_k_contiguous_pair_row_blocks(fmt, K, epilogue):
+    """gemm_tile_pair on the K-contiguous fp4 containers (launches of few tiles): every number of 16-row blocks from 1 to 11, the
+    row before and after each, two and three chunks, over two column tiles."""
+    counts = [rows for b in range(16, 161, 16) for rows in (b - 1, b, b + 1)] + [1, 0, 321]
+    _say(f"{fmt} pair row blocks K={K} epilogue={epilogue}")
+    case = H.make_case(fmt, len(counts), K, 512, np.cumsum(counts), seed=K, extra_rows=3)
     assert H.kernel_of(case, "gemm", swiglu=epilogue == "swiglu") == "tiles_pair"
     used = int(case["group_list"][-1])
     if epilogue == "swiglu":
@@ -105,9 +124,22 @@ def test_fp4_k_contiguous_row_blocks(fmt, K, epilogue):
     assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
 
 
+@pytest.mark.parametrize("K,kernel", [(896, "tiles_fp4_k"), (1664, "tiles_pair")])
+@pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
+def test_fp4_k_contiguous_tiles_round_their_weights(fmt, K, kernel):
+    """Both tile routines multiply weights rounded to bf16: few outputs differ from the oracle with that rounding (where the order
+    of the sums moves one across a rounding boundary), a sizeable share from the oracle without it."""
+    _say(f"{fmt} {kernel} rounding")
+    case = H.make_case(fmt, 4, K, 512, [40, 90, 130, 200], seed=K)
+    assert H.kernel_of(case, "gemm") == kernel
+    got = H.run_cabi(case, H.upload(case), "gemm")
+    own, other = (float(np.mean(got != H.oracle_out(case, gemv=g))) for g in (False, True))
+    assert other > 0.03 and own < 0.25 * other, f"{own:.4f} of the outputs differ from rounded weights, {other:.4f} from un-rounded ones"
+
+
 @pytest.mark.parametrize("fmt,G,N,kernel", [("int4", 600, 256, "tiles_quad"), ("fp4", 300, 512, "tiles_quad"), ("fp8", 300, 256, "tiles_pair"),
-                                            ("int8", 511, 256, "tiles_pair"), ("fp4_b16", 300, 512, "tiles_pair"),
-                                            ("fp4_b16", 450, 256, "tiles_pair"), ("bf16", 300, 256, "tiles_bf16")])
+                                            ("int8", 511, 256, "tiles_pair"), ("fp4_b16", 300, 512, "tiles_fp4_k"),
+                                            ("fp4_b16", 450, 256, "tiles_fp4_k"), ("bf16", 300, 256, "tiles_bf16")])
 def test_order_of_experts(fmt, G, N, kernel):
     """Launches of more tiles than workgroups take the experts with the largest tiles first: more experts than a workgroup has
     threads (two and three rounds of the sort, the last one partly filled), every number of 16-row blocks from 1 to 10, experts
