@@ -1404,14 +1404,34 @@ __device__ __forceinline__ void expert_chunks(int m, int& chunks, int& bpc) {
     bpc = (nblk + chunks - 1) / chunks;
 }
 
+// Inclusive sums over the lanes of a row of 16, and of the wavefront: DPP shifts (a shuffle goes through LDS, about 100 cycles each,
+// one after the other, at the start of every workgroup)
+__device__ __forceinline__ int row_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    return v;
+}
+__device__ __forceinline__ int wave_scan(int v) {
+    v = row_scan(v);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15, rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31, rows 2 and 3
+    return v;
+}
+
 // The order in which a launch takes its experts: those with the largest tiles (most row blocks per chunk) first, those
 // without rows last, otherwise as they come.  A tile's time goes by its row blocks, and with the largest tiles up to half
 // of a launch long, one that starts among the last leaves most of the chip waiting for it.
 // us as they come / in this order, rows unevenly routed (skew: see moe_dispatch.cpp): fp4 SwiGLU, 1511 tokens x 8 on 256
-// experts of 7168 x 2048, skew 1: 578 / 563, skew 0.25: 628 / 615; int4, 2000 x 4 on 64 of 7168 x 2048, skew 0.25: 307 / 282; fp8
-// and int8, 1500 x 8 on 128 of 4096 x 2048, skews 0 to 1: 0.99 to 1.02 times as fast.  Orders given by group_list
-// to a kernel that took it as it was, skew 1: int4, 2000 x 4 on 64 of 7168 x 2048: 327 / 296; fp4_b32, 1500 x 8 on 128
-// of 4096 x 3072: 420 / 399; evenly routed, the same time.
+// experts of 7168 x 2048, skew 1: 578 / 563, skew 0.25: 628 / 615; int4, 2000 x 4 on 64 of 7168 x 2048, skew 0.25: 307 / 282.
+// It takes 0.3 us of every workgroup with 4 wavefronts, 0.6 with 8 (an earlier form with shuffles and a second pass over the experts
+// 1.1 and 1.3), which small launches and those that need no order lose: only launches of KernelCfg::ORDER_MIN_WORK do it.  Times as fast as
+// unordered, median (worst, best) evenly routed, by balanced top-k routing and at a skew of 1: int4 and fp4 on GK_QUAD, 0.25 to 0.5
+// million tiles times k (20 us) 0.978 (0.967), 0.977 (0.94), 1.06; 0.5 to 1 million 0.995 (0.98), 1.0 (0.97), 1.01; 1 to 3 million
+// (50 to 100 us) 0.99 (0.98), 1.0 (0.965), 1.06 (0.96, 1.27); more 0.995 (0.976), 1.005 (0.972), 1.065 (0.98, 1.3).  int8 and fp8 on
+// GK_PAIR, 0.5 to 3 million (40 to 110 us) 0.99 (0.974), 0.983 (0.93), 1.01 (0.94, 1.24); more 0.997 (0.98), 0.997 (0.967),
+// 1.035 (0.953, 1.16).
 // Not for bf16, whose tiles wait for memory or for the matrix cores by their size: large and small ones side by side use both, and
 // that goes either way.  1021 x 8 on 64 of 7168 x 2048, three routings each of skew 0.25 and 0.5: 508 / 485, 457 / 472, 462 / 476
 // and 510 / 470, 496 / 474, 502 / 476; 1500 x 2 on 16 of 4096 x 8192, skew 1: 287 / 302; 700 x 8 on 64 of 7168 x 2048, skew 0:
@@ -1419,17 +1439,21 @@ __device__ __forceinline__ void expert_chunks(int m, int& chunks, int& bpc) {
 // Every workgroup works the same order out: a counting sort, ranks from ballots; 64 experts of a wavefront at a
 // time leave one count per class in scratch (LDS of the tile routine, [rounds * WAVES][16]).
 template <int MTM, int BLOCK, int WAVES, typename Rows>
-__device__ __forceinline__ void order_experts(int G, int tid, int* scratch, uint16_t* order, Rows expert_rows) {
+__device__ __forceinline__ void order_experts(int G, int ntile_n, int tid, int* scratch, uint16_t* order, int* tiles, Rows expert_rows) {
     static_assert(MTM < 15, "classes 0 .. MTM, 15 for no expert");
-    const int lane = tid & 63, wave = tid >> 6, rounds = (G + 64 * WAVES - 1) / (64 * WAVES);
-    auto class_of = [&](int g) {
-        if (g >= G) return 15;
-        int first, chunks, bpc;
-        expert_chunks<MTM, BLOCK>(expert_rows(g, first), chunks, bpc);
-        return MTM - bpc;
+    const int lane = tid & 63, wave = tid >> 6, col = lane & 15, rounds = (G + 64 * WAVES - 1) / (64 * WAVES);
+    int c = 15, n_tiles = 0;   // of this thread's expert in the round
+    auto look = [&](int g) {
+        c = 15;
+        if (g < G) {
+            int first, chunks, bpc;
+            expert_chunks<MTM, BLOCK>(expert_rows(g, first), chunks, bpc);
+            c = MTM - bpc;
+            n_tiles = chunks * ntile_n;
+        }
     };
     for (int r = 0; r < rounds; ++r) {
-        const int c = class_of(r * 64 * WAVES + tid);
+        look(r * 64 * WAVES + tid);
         int n = 0;
 #pragma unroll
         for (int k = 0; k <= MTM; ++k) {
@@ -1440,22 +1464,18 @@ __device__ __forceinline__ void order_experts(int G, int tid, int* scratch, uint
     }
     __syncthreads();
     // lane k (mod 16): where class k starts for the next 64 experts of this wavefront
-    const int col = lane & 15;
     int all = 0, next = 0;
-    for (int j = 0; j < rounds * WAVES; ++j) {
-        const int n = scratch[j * 16 + col];
-        all += n;
-        next += j < wave ? n : 0;
-    }
-    int incl = all;
+    for (int r = 0; r < rounds; ++r)
 #pragma unroll
-    for (int off = 1; off < 16; off <<= 1) {
-        const int up = __shfl_up(incl, off, 16);
-        if (col >= off) incl += up;
-    }
-    next += incl - all;
-    for (int r = 0; r < rounds; ++r) {
-        const int g = r * 64 * WAVES + tid, c = class_of(g);
+        for (int w = 0; w < WAVES; ++w) {
+            const int n = scratch[(r * WAVES + w) * 16 + col];
+            all += n;
+            next += r == 0 && w < wave ? n : 0;
+        }
+    next += row_scan(all) - all;
+    for (int r = 0;;) {
+        const int g = r * 64 * WAVES + tid;
+        if (rounds > 1) look(g);
         unsigned long long same = 0;
 #pragma unroll
         for (int k = 0; k <= MTM; ++k) {
@@ -1463,8 +1483,14 @@ __device__ __forceinline__ void order_experts(int G, int tid, int* scratch, uint
             if (c == k) same = in;
         }
         const int at = __shfl(next, c, 64) + __popcll(same & ((1ull << lane) - 1));
-        if (g < G) order[at] = (uint16_t)g;
-        for (int j = r * WAVES + wave; j < (r + 1) * WAVES + wave && j < rounds * WAVES; ++j) next += scratch[j * 16 + col];
+        if (g < G) {
+            order[at] = (uint16_t)g;
+            tiles[at] = n_tiles;
+        }
+        if (++r == rounds) break;
+        // before the wavefront's next 64 experts come these, those of the wavefronts behind it and the next of those in front
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) next += scratch[((w < wave ? r : r - 1) * WAVES + w) * 16 + col];
     }
     __syncthreads();
 }
@@ -1483,9 +1509,11 @@ struct KernelCfg {
     static constexpr int WG_PER_CU = pair_wgs();
     static constexpr int WAVES_PER_SIMD = WG_PER_CU * WAVES / 4;
     static constexpr int MTM = PAIR ? pair_mt_max(KIND) : FP4_K ? FK_MT_MAX : KIND == GK_BF16_128 ? 4 : BF_MT_MAX;   // row blocks per tile
-    // tiles of up to 32 rows take the time of their weights, in any order; bf16: see order_experts; launches of K-contiguous fp4 on
-    // GK_PAIR have a tile per CU, mostly
-    static constexpr bool ORDERED = MTM > PAIR_SMALL_MT_MAX && FMT != MOE_FMT_BF16 && !(PAIR && (FMT == MOE_FMT_FP4_B32 || FMT == MOE_FMT_FP4_B16));
+    // tiles of up to 32 rows take the time of their weights, in any order; bf16: see order_experts; K-contiguous fp4 on GK_PAIR has
+    // a tile per CU or evenly filled ones (6 % slower in this order at 256 tiles, evenly routed)
+    static constexpr bool ORDERED = KIND == GK_QUAD || KIND == GK_FP4_K || (KIND == GK_PAIR && (FMT == MOE_FMT_INT8 || FMT == MOE_FMT_FP8_REF));
+    // ... in launches of at least that many tiles (an upper bound) times k
+    static constexpr int64_t ORDER_MIN_WORK = KIND == GK_PAIR ? 3 << 20 : 1 << 19;
     // 16-byte LDS units of the tile routine (the tile prefix array follows them)
     static constexpr int lds_units() {
         if constexpr (PAIR)
@@ -1544,8 +1572,6 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         return max(hi - first, 0);
     };
 
-    auto expert_at = [&](int e) { return C::ORDERED && P.table_mode == 3 ? (int)order[e] : e; };
-
     // the launch's counter is looked at, and raised to the launch's stamp, now: long before the first draw from it
     if (tid == 0) part[PART_FIXED] = P.slot >= 0 && queue_open(tile_queue + GM_QUEUE_STRIDE * max(P.slot, 0), P.stamp, blockIdx.x < 8);
 
@@ -1560,22 +1586,20 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
             __syncthreads();
         }
         if constexpr (C::ORDERED)
-            if (P.table_mode == 3) order_experts<MTM, C::BLOCK, WAVES>(P.G, tid, reinterpret_cast<int*>(smem), order, expert_rows);
-        int sum = 0;
-        for (int e = g0; e < g1; ++e) {
+            if (P.table_mode == 3) order_experts<MTM, C::BLOCK, WAVES>(P.G, ntile_n, tid, reinterpret_cast<int*>(smem), order, prefix, expert_rows);
+        // tiles of the expert at place e (order_experts has left them in the table)
+        auto tiles_at = [&](int e) {
+            if (C::ORDERED && P.table_mode == 3) return prefix[e];
             int first, chunks, bpc;
-            expert_chunks<MTM, C::BLOCK>(expert_rows(expert_at(e), first), chunks, bpc);
-            sum += chunks * ntile_n;
-        }
-        // scan over the threads: within a wavefront by shuffles, across wavefronts through their totals in
+            expert_chunks<MTM, C::BLOCK>(expert_rows(e, first), chunks, bpc);
+            return chunks * ntile_n;
+        };
+        int sum = 0;
+        for (int e = g0; e < g1; ++e) sum += tiles_at(e);
+        // scan over the threads: within a wavefront by DPP, across wavefronts through their totals in
         // LDS (a loop of one thread over all partial sums took 8 us at the start of every workgroup)
         const int lane = tid & 63, wave = tid >> 6;
-        int incl = sum;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int up = __shfl_up(incl, off, 64);
-            if (lane >= off) incl += up;
-        }
+        const int incl = wave_scan(sum);
         if (lane == 63) part[wave] = incl;
         __syncthreads();
         int before = 0, all = 0;
@@ -1589,10 +1613,9 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         int run = before + incl - sum;
         if (P.table_mode) {
             for (int e = g0; e < g1; ++e) {
-                int first, chunks, bpc;
-                expert_chunks<MTM, C::BLOCK>(expert_rows(expert_at(e), first), chunks, bpc);
+                const int n = tiles_at(e);
                 prefix[e] = run;
-                run += chunks * ntile_n;
+                run += n;
             }
         } else {
             prefix[tid] = run;
@@ -1794,8 +1817,9 @@ static int launch_gemm_kind(const GemmParams& P, const moe_grouped_args* a, hipS
     const int64_t max_chunks = a->M / (C::BLOCK * C::MTM) + a->G;
     const int64_t max_tiles = max_chunks * ((a->N + C::BN - 1) / C::BN);
     const int64_t want = max_tiles < (int64_t)cus * C::WG_PER_CU ? max_tiles : (int64_t)cus * C::WG_PER_CU;
-    // where a workgroup may get more than one tile, the experts with the largest ones come first (as far as LDS has room)
-    if (C::ORDERED && table_mode == 2 && max_tiles > want && lds + (size_t)a->G * sizeof(uint16_t) <= lds_max) {
+    // where a workgroup may get more than one tile, the experts with the largest ones come first (as far as LDS has room, and in
+    // launches long enough for it, see order_experts)
+    if (C::ORDERED && table_mode == 2 && max_tiles > want && max_tiles * a->K >= C::ORDER_MIN_WORK && lds + (size_t)a->G * sizeof(uint16_t) <= lds_max) {
         table_mode = 3;
         lds += (size_t)a->G * sizeof(uint16_t);
     }

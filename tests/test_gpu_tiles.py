@@ -141,9 +141,8 @@ def test_fp4_k_contiguous_tiles_round_their_weights(fmt, K, kernel):
                                             ("int8", 511, 256, "tiles_pair"), ("fp4_b16", 300, 512, "tiles_fp4_k"),
                                             ("fp4_b16", 450, 256, "tiles_fp4_k"), ("bf16", 300, 256, "tiles_bf16")])
 def test_order_of_experts(fmt, G, N, kernel):
-    """Launches of more tiles than workgroups take the experts with the largest tiles first: more experts than a workgroup has
-    threads (two and three rounds of the sort, the last one partly filled), every number of 16-row blocks from 1 to 10, experts
-    without rows; 450 fp4_b16 experts, for whose order LDS has no room, and bf16, which takes them as they come."""
+    """Launches of more tiles than workgroups, too short for an order of their own (see test_long_launches_order_their_experts): more
+    experts than a workgroup has threads, every number of 16-row blocks from 1 to 10, experts without rows."""
     some = [rows for b in range(16, 161, 16) for rows in (b - 1, b, b + 1)] + [0, 0, 1, 0, 330]
     counts = [some[(g * 17 + g // 35) % 35] for g in range(G)]
     _say(f"order of experts {fmt} G={G} N={N}")
@@ -172,3 +171,44 @@ def test_fp4_rows_of_a_partly_filled_last_step(fmt, K):
             got, want = H.run_cabi(case, H.upload(case), op), H.oracle_out(case, gemv=op == "gemv")
         H.assert_close(got, want, rows=slice(0, used), what=f"{fmt} {op} K={K}")
         assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
+
+
+@pytest.mark.parametrize("fmt,G,K,N,kernel", [("int4", 600, 1024, 256, "tiles_quad"), ("fp4", 300, 1024, 512, "tiles_quad"),
+                                              ("fp4_b32", 300, 1024, 512, "tiles_fp4_k"), ("fp4_b16", 300, 1024, 512, "tiles_fp4_k"),
+                                              ("fp4_b16", 450, 1024, 256, "tiles_fp4_k"), ("int8", 511, 4096, 256, "tiles_pair"),
+                                              ("fp8", 1100, 2048, 256, "tiles_pair")])
+def test_long_launches_order_their_experts(fmt, G, K, N, kernel):
+    """Launches of at least 1 << 19 tiles times k (tiles_pair: 3 << 20) take the experts with the largest tiles first: more experts than a
+    workgroup has threads (two and three rounds of the sort, the last one partly filled), every number of 16-row blocks from 1 to 10,
+    experts without rows; 450 fp4_b16 experts, for whose order LDS has no room.  No output depends on the order: the same bits as two
+    launches of half of the experts each, which are too short for one."""
+    import moe_gfx950 as mg
+
+    limit = 3 << 20 if kernel == "tiles_pair" else 1 << 19
+    some = [rows for b in range(16, 161, 16) for rows in (b - 1, b, b + 1)] + [0, 0, 1, 0, 330]
+    counts = [some[(g * 17 + g // 35) % 35] for g in range(G)]
+    _say(f"long launch {fmt} G={G} N={N}")
+    gen = torch.Generator(device="cuda").manual_seed(G)
+    weight = torch.randint(0, 64 if fmt == "fp8" else 256, (G, K * N // (1 if fmt in ("int8", "fp8") else 2)), dtype=torch.uint8, device="cuda", generator=gen)
+    scales = {"int4": K // 128 * N, "fp4": K // 16 * N, "fp4_b32": K // 32 * N, "fp4_b16": K // 16 * N, "int8": N, "fp8": (K // 128) * (N // 128)}[fmt]
+    scale = torch.rand(G, scales, device="cuda", generator=gen).mul_(0.05).to(torch.float32 if fmt == "fp8" else torch.bfloat16)
+    offset = torch.randn(G, N, device="cuda", generator=gen).to(torch.bfloat16) if fmt == "int8" else None
+    x = torch.randn(sum(counts), K, device="cuda", generator=gen).to(torch.bfloat16)
+
+    def launch(g0, g1):
+        """Experts [g0, g1) on their rows; tiles (at most) times k."""
+        first, rows = sum(counts[:g0]), sum(counts[g0:g1])
+        gl = torch.tensor(np.cumsum(counts[g0:g1]), device="cuda")
+        y = torch.full((rows, N), 0x7FC0, dtype=torch.int16, device="cuda")
+        args = mg.grouped_args(mg.format_from_compute_type(fmt), x[first:].data_ptr(), weight[g0:].data_ptr(), scale[g0:].data_ptr(),
+                               0 if offset is None else offset[g0:].data_ptr(), gl.data_ptr(), y.data_ptr(), rows, K, N, g1 - g0,
+                               {"int4": K // 128, "fp4": K // 16}.get(fmt, 1))
+        assert mg.grouped_kernel(args, "gemm") == kernel
+        mg.grouped_gemm(args, torch.cuda.current_stream().cuda_stream)
+        return y, (rows // (144 if kernel == "tiles_fp4_k" else 160) + g1 - g0) * (N // 256) * K
+
+    whole, work = launch(0, G)
+    halves, works = zip(launch(0, G // 2), launch(G // 2, G))
+    torch.cuda.synchronize()
+    assert max(works) < limit <= work
+    assert torch.equal(whole, torch.cat(halves)) and not bool((whole == 0x7FC0).any())
