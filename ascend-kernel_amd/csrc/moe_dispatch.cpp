@@ -60,16 +60,25 @@ static bool fp4_rows_preferred(const moe_grouped_args* a) {
     return a->M <= (a->M <= 64 ? 8 : 5) * a->G;
 }
 
-// The same kernel where K is no multiple of 512 and its last iteration is not full.  us, the other kernel / this one, fp4_b32 and
-// fp4_b16.  GEMV op (vector): 8 rows, 1 to 8 experts, K = 1152: 8.0 / 5.5 and 8.8 / 6.7; 62 x 4 rows on 64 experts of 4736 x 768,
-// skew 1: 196 / 46 and 212 / 59; 32 x 8 on 256 of 1920 x 2000: 131 / 63 and 146 / 83; but a token on 8 of 6912 x 512: 29 / 29 and
-// 30 / 34.  GEMM op (tiles): 49 rows on 16 of 6912 x 512 60 / 32 and 63 / 34, 100 on 64 of 4480 x 1024 44 / 35 and 45 / 37, 512 on
-// 256 of 6912 x 2048 438 / 386 and 439 / 417; with many columns and a short K the tiles are level or ahead: 16 rows on 256 of
-// 1792 x 3584 (57344 columns) 22 / 25 and 24 / 26, 240 on 64 of 3328 x 2048 54 / 55 and 57 / 59.  Where K is an odd multiple of 128 the
-// rows of weights do not begin with lines.
-static bool fp4_rows_partial_preferred(const moe_grouped_args* a, bool gemv_op) {
-    if (gemv_op) return !(a->format == MOE_FMT_FP4_B16 && a->M <= 8 && columns(a) <= 8192 && a->K >= 4096);
-    return columns(a) <= 32768 || (a->K % 256 == 0 && a->K >= 4096);
+// The same kernel where K is no multiple of 512 and its last iteration is not full, GEMV op (else the vector kernel).  us, the vector
+// kernel / this one, fp4_b32 and fp4_b16: 8 rows, 1 to 8 experts, K = 1152: 8.0 / 5.5 and 8.8 / 6.7; 62 x 4 rows on 64 experts of 4736 x
+// 768, skew 1: 196 / 46 and 212 / 59; 32 x 8 on 256 of 1920 x 2000: 131 / 63 and 146 / 83; but a token on 8 of 6912 x 512: 29 / 29 and
+// 30 / 34.
+static bool fp4_rows_partial_gemv(const moe_grouped_args* a) {
+    return !(a->format == MOE_FMT_FP4_B16 && a->M <= 8 && columns(a) <= 8192 && a->K >= 4096);
+}
+
+// GEMM op, K no multiple of 512: the tiles take such a K as any other, so that the bounds by rows per expert lie lower, and go by the
+// columns: few make a tile per CU at best, whose time hardly depends on its rows; with many, an expert of more than 16 rows is passes in
+// a row here.  Tiles / this kernel, balanced top-k routing and skews of 0.25 and 1, median over K = 1152 to 7040 (fp4_b16 differs by
+// 0.05): up to 32768 columns 12 rows per expert 1.8, 1.7 and 1.04; up to 65536 columns 4 rows 1.33, 1.31 and 1.21, 8 rows 1.25, 1.0 and
+// 0.86, 10 rows 1.22, 0.90 and 0.71; more columns 2 rows 1.22, 1.2 and 1.0, 4 rows 1.18, 1.16 and 0.84, 6 rows 1.12, 1.03 and 0.72,
+// 12 rows 0.9, 0.82 and 0.5.  With SwiGLU the same within 0.03.
+// Fewer rows than experts: the workgroups of experts without rows count beside a short K.  6 rows on 256 of 1280 x 7424 17.6 / 21.9, 12
+// on 256 of 1280 x 4608 16.9 / 19.6, but 100 on 64 of 4480 x 1024 44 / 35.
+static bool fp4_rows_partial_gemm(const moe_grouped_args* a) {
+    if (columns(a) <= 32768) return a->M <= 12 * a->G;
+    return (a->K >= 4096 || a->M >= a->G) && a->M <= (columns(a) <= 65536 ? 4 : 2) * a->G;
 }
 
 // Tiles of K-contiguous fp4.  Two workgroups of 4 wavefronts per CU (TILES_FP4_K) are the better routine where a CU gets two tiles or
@@ -99,9 +108,10 @@ static GroupedKernel fp4_kcontiguous_tiles(const moe_grouped_args* a) {
 }
 
 static GroupedKernel fp4_kcontiguous_kernel(const moe_grouped_args* a, bool gemv_op) {
-    const bool rows = a->K % 512 == 0 || (a->K >= FP4_ROWS_K_MIN && a->K % FP4_ROWS_K == 0 && fp4_rows_partial_preferred(a, gemv_op));
-    if (gemv_op) return rows ? GroupedKernel::FP4_ROWS : GroupedKernel::VECTOR;
-    return rows && fp4_rows_preferred(a) ? GroupedKernel::FP4_ROWS : fp4_kcontiguous_tiles(a);
+    const bool whole = a->K % 512 == 0, partial = a->K >= FP4_ROWS_K_MIN && a->K % FP4_ROWS_K == 0;
+    if (gemv_op) return whole || (partial && fp4_rows_partial_gemv(a)) ? GroupedKernel::FP4_ROWS : GroupedKernel::VECTOR;
+    const bool rows = fp4_rows_preferred(a) && (whole || (partial && fp4_rows_partial_gemm(a)));
+    return rows ? GroupedKernel::FP4_ROWS : fp4_kcontiguous_tiles(a);
 }
 
 // Strips for launches of up to 128 tiles of 256 columns, i.e. half of the CUs, and decode-like batches: with 32768 columns (16

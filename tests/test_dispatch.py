@@ -40,12 +40,34 @@ def test_tiles_of_the_n_contiguous_containers():
 def test_k_contiguous_fp4(fmt):
     at = lambda op, r, K, swiglu=False: kernel(fmt, op, r * 64, 64, K, 2048, swiglu)   # noqa: E731
     assert (at("gemv", 1, 7168), at("gemv", 100, 7168), at("gemv", 1, 7168 + 32)) == ("fp4_rows", "fp4_rows", "vector")
-    assert (at("gemm", 12, 7168), at("gemm", 13, 7168), at("gemm", 1, 7168 + 128)) == ("fp4_rows", "tiles_fp4_k", "tiles_fp4_k")
+    assert (at("gemm", 12, 7168), at("gemm", 13, 7168), at("gemm", 5, 7168 + 128)) == ("fp4_rows", "tiles_fp4_k", "tiles_fp4_k")
     # with SwiGLU, 5 rows per expert; 8 with up to 64 rows in all
     assert (at("gemm", 5, 7168, True), at("gemm", 6, 7168, True)) == ("fp4_rows", "tiles_fp4_k")
     few = lambda M, G: kernel(fmt, "gemm", M, G, 4096, 2048, True)   # noqa: E731
     assert (few(64, 8), few(65, 8)) == ("fp4_rows", "tiles_pair")
     assert (few(32, 4), few(33, 4)) == ("fp4_rows", "tiles_pair")
+
+
+@pytest.mark.parametrize("K", [640, 1152, 3328, 6912, 7040])
+@pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
+def test_k_contiguous_fp4_gemm_of_a_partly_filled_last_step(fmt, K):
+    rows = lambda M, G, N, swiglu=False: kernel(fmt, "gemm", M, G, K, N, swiglu) == "fp4_rows"   # noqa: E731
+    # rows per expert by the columns over all experts that own rows
+    for G, N, bound in ((16, 2048, 12), (16, 2304, 4), (32, 2048, 4), (32, 2304, 2), (256, 3584, 2)):
+        assert (rows(bound * G, G, N), rows(bound * G + 1, G, N)) == (True, False)
+    # fewer rows than experts
+    assert (rows(16, 256, 2048), rows(16, 256, 2304), rows(255, 256, 512)) == (True, K >= 4096, K >= 4096)
+    # with SwiGLU not more than elsewhere: 5, or 8 with up to 64 rows in all
+    assert (rows(5 * 16, 16, 2048, True), rows(5 * 16 + 1, 16, 2048, True)) == (True, False)
+    assert (rows(64, 8, 2048, True), rows(65, 8, 2048, True)) == (True, False)
+    assert (rows(2 * 32, 32, 2304, True), rows(2 * 32 + 1, 32, 2304, True)) == (True, False)
+
+
+def test_k_contiguous_fp4_shortest_k():
+    # the shortest K of the rows kernel is two groups of 128
+    for fmt in ("fp4_b32", "fp4_b16"):
+        assert (kernel(fmt, "gemm", 8, 8, 128, 512), kernel(fmt, "gemm", 8, 8, 256, 512)) == ("tiles_fp4_k", "fp4_rows")
+        assert (kernel(fmt, "gemv", 8, 8, 128, 512), kernel(fmt, "gemv", 8, 8, 256, 512)) == ("vector", "fp4_rows")
 
 
 @pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
