@@ -72,13 +72,13 @@ static bool fp4_rows_partial_gemv(const moe_grouped_args* a) {
 // columns: few make a tile per CU at best, whose time hardly depends on its rows; with many, an expert of more than 16 rows is passes in
 // a row here.  Tiles / this kernel, balanced top-k routing and skews of 0.25 and 1, median over K = 1152 to 7040 (fp4_b16 differs by
 // 0.05): up to 32768 columns 12 rows per expert 1.8, 1.7 and 1.04; up to 65536 columns 4 rows 1.33, 1.31 and 1.21, 8 rows 1.25, 1.0 and
-// 0.86, 10 rows 1.22, 0.90 and 0.71; more columns 2 rows 1.22, 1.2 and 1.0, 4 rows 1.18, 1.16 and 0.84, 6 rows 1.12, 1.03 and 0.72,
+// 0.86, 10 rows 1.22, 0.90 and 0.71; more columns 3 rows 1.2, 1.2 and 0.95, 4 rows 1.18, 1.16 and 0.84, 6 rows 1.12, 1.03 and 0.72,
 // 12 rows 0.9, 0.82 and 0.5.  With SwiGLU the same within 0.03.
 // Fewer rows than experts: the workgroups of experts without rows count beside a short K.  6 rows on 256 of 1280 x 7424 17.6 / 21.9, 12
 // on 256 of 1280 x 4608 16.9 / 19.6, but 100 on 64 of 4480 x 1024 44 / 35.
 static bool fp4_rows_partial_gemm(const moe_grouped_args* a) {
     if (columns(a) <= 32768) return a->M <= 12 * a->G;
-    return (a->K >= 4096 || a->M >= a->G) && a->M <= (columns(a) <= 65536 ? 4 : 2) * a->G;
+    return (a->K >= 4096 || a->M >= a->G) && a->M <= (columns(a) <= 65536 ? 4 : 3) * a->G;
 }
 
 // Tiles of K-contiguous fp4.  Two workgroups of 4 wavefronts per CU (TILES_FP4_K) are the better routine where a CU gets two tiles or
@@ -86,7 +86,8 @@ static bool fp4_rows_partial_gemm(const moe_grouped_args* a) {
 // TILES_PAIR, evenly routed, fp4_b32 and fp4_b16: 8 experts of 7168 x 2048 (64 tiles), 32 rows each 86 / 72 and 87 / 76, 64 rows 94 / 79
 // and 98 / 85; 16 of 7168 x 4096 (256 tiles), 48 rows 1.12 and 1.06 times; 8 of 4480 x 7168, 128 rows 88 / 78 and 90 / 84; one
 // expert of 7168 x 512, 128 rows 115 / 90 and 118 / 100; but 16 of 7168 x 4352 (272 tiles), 48 rows 0.88 and 0.88 times, and with 640 k 0.90
-// and 0.88 times at 256 tiles (level at 1024 k, fp4_b16 at 1536).  Routing that leaves some experts more rows than a tile takes makes a
+// and 0.88 times at 256 tiles (level at 1024 k; fp4_b16 0.94 at 1024, 1.01 at 1536 to 1792, 1.04 at 2048, but 0.90 to 0.94 with more
+// than 100 rows at 1664).  Routing that leaves some experts more rows than a tile takes makes a
 // few more tiles than CUs: 64 of 7168 x 1024 with 64 rows on average at a skew of 1, 159 / 167 and 162 / 183.  fp4_b16 with up to 16
 // rows per expert and K an odd multiple of 128, whose rows of scales do not begin with 32 bytes: 0.92 to 0.96 times.
 // TILES_FP4_K cuts an expert of 145 to 160 rows, one tile of TILES_PAIR, in two.  That is the faster way while the tiles do not fill
@@ -102,7 +103,7 @@ static int64_t fp4_tiles(const moe_grouped_args* a, int64_t rows) {
 static GroupedKernel fp4_kcontiguous_tiles(const moe_grouped_args* a) {
     const bool b32 = a->format == MOE_FMT_FP4_B32;
     const int64_t quad = fp4_tiles(a, FP4_K_ROWS), pair = fp4_tiles(a, PAIR_ROWS);
-    const bool pairs = quad == pair ? pair <= 256 && a->K >= (b32 ? 1024 : 1536) && (b32 || a->K % 256 == 0 || a->M > 16 * a->G)
+    const bool pairs = quad == pair ? pair <= 256 && a->K >= (b32 ? 1024 : 2048) && (b32 || a->K % 256 == 0 || a->M > 16 * a->G)
                                     : quad > 256 && a->M <= PAIR_ROWS * a->G && b32 && a->K >= 4096;
     return pairs ? GroupedKernel::TILES_PAIR : GroupedKernel::TILES_FP4_K;
 }

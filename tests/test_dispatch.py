@@ -53,14 +53,14 @@ def test_k_contiguous_fp4(fmt):
 def test_k_contiguous_fp4_gemm_of_a_partly_filled_last_step(fmt, K):
     rows = lambda M, G, N, swiglu=False: kernel(fmt, "gemm", M, G, K, N, swiglu) == "fp4_rows"   # noqa: E731
     # rows per expert by the columns over all experts that own rows
-    for G, N, bound in ((16, 2048, 12), (16, 2304, 4), (32, 2048, 4), (32, 2304, 2), (256, 3584, 2)):
+    for G, N, bound in ((16, 2048, 12), (16, 2304, 4), (32, 2048, 4), (32, 2304, 3), (256, 3584, 3)):
         assert (rows(bound * G, G, N), rows(bound * G + 1, G, N)) == (True, False)
     # fewer rows than experts
     assert (rows(16, 256, 2048), rows(16, 256, 2304), rows(255, 256, 512)) == (True, K >= 4096, K >= 4096)
     # with SwiGLU not more than elsewhere: 5, or 8 with up to 64 rows in all
     assert (rows(5 * 16, 16, 2048, True), rows(5 * 16 + 1, 16, 2048, True)) == (True, False)
     assert (rows(64, 8, 2048, True), rows(65, 8, 2048, True)) == (True, False)
-    assert (rows(2 * 32, 32, 2304, True), rows(2 * 32 + 1, 32, 2304, True)) == (True, False)
+    assert (rows(3 * 32, 32, 2304, True), rows(3 * 32 + 1, 32, 2304, True)) == (True, False)
 
 
 def test_k_contiguous_fp4_shortest_k():
@@ -73,7 +73,7 @@ def test_k_contiguous_fp4_shortest_k():
 @pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
 def test_k_contiguous_fp4_tiles(fmt):
     tiles = lambda r, G, K, N: kernel(fmt, "gemm", r * G, G, K, N)   # noqa: E731
-    k_min = {"fp4_b32": 1024, "fp4_b16": 1536}[fmt]
+    k_min = {"fp4_b32": 1024, "fp4_b16": 2048}[fmt]
     # a tile per CU: 256 tiles, and from some length of K on
     for r in (13, 144, 161, 288):
         chunks = -(-r // 160)

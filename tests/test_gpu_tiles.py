@@ -106,7 +106,7 @@ def test_fp4_k_contiguous_row_blocks(fmt, K, epilogue):
 
 
 @pytest.mark.parametrize("epilogue", ["none", "swiglu"])
-@pytest.mark.parametrize("K", [1536, 1664, 1920])   # 6, 6.5 and 7.5 super-blocks of scales of fp4_b32; 12, 13 and 15 of fp4_b16
+@pytest.mark.parametrize("K", [2048, 2176, 2432])   # 8, 8.5 and 9.5 super-blocks of scales of fp4_b32; 16, 17 and 19 of fp4_b16
 @pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
 def test_fp4_k_contiguous_pair_row_blocks(fmt, K, epilogue):
     """gemm_tile_pair on the K-contiguous fp4 containers (launches of few tiles): every number of 16-row blocks from 1 to 11, the
@@ -124,7 +124,7 @@ def test_fp4_k_contiguous_pair_row_blocks(fmt, K, epilogue):
     assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
 
 
-@pytest.mark.parametrize("K,kernel", [(896, "tiles_fp4_k"), (1664, "tiles_pair")])
+@pytest.mark.parametrize("K,kernel", [(896, "tiles_fp4_k"), (2176, "tiles_pair")])
 @pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
 def test_fp4_k_contiguous_tiles_round_their_weights(fmt, K, kernel):
     """Both tile routines multiply weights rounded to bf16: few outputs differ from the oracle with that rounding (where the order
