@@ -62,10 +62,17 @@ static bool fp4_rows_preferred(const moe_grouped_args* a) {
 
 // The same kernel where K is no multiple of 512 and its last iteration is not full, GEMV op (else the vector kernel).  us, the vector
 // kernel / this one, fp4_b32 and fp4_b16: 8 rows, 1 to 8 experts, K = 1152: 8.0 / 5.5 and 8.8 / 6.7; 62 x 4 rows on 64 experts of 4736 x
-// 768, skew 1: 196 / 46 and 212 / 59; 32 x 8 on 256 of 1920 x 2000: 131 / 63 and 146 / 83; but a token on 8 of 6912 x 512: 29 / 29 and
-// 30 / 34.
+// 768, skew 1: 196 / 46 and 212 / 59; 32 x 8 on 256 of 1920 x 2000: 131 / 63 and 146 / 83.  With 3 or 4 rows of an expert the vector kernel
+// takes 1.4 times as long as with 1 or 2, this one as long.  Single rows, weights from HBM: the vector kernel is level or ahead where its steps
+// of 2048 k are well filled against the 512 k of this one (K = 3456 to 4096, 5248 to 6144, 6784 to 8192, ...), and most with enough columns for
+// requests to count: 8 rows on 8 of 64 experts, K = 6912, 2048 columns 31 / 39 and 41 / 44, 4096 columns 35 / 43 and 46 / 47, 512
+// columns 26 / 25 and 36 / 30, one expert of 512 columns 20 / 24 and 27 / 29; K = 8064, 8193 to 32768 columns in all 0.73 and 0.88 times, K =
+// 4736, up to 8192 columns 1.06 and 1.23 times.  So while experts with several rows are rare (4 tokens on 128 experts), and fp4_b16
+// beyond 8192 columns only.
 static bool fp4_rows_partial_gemv(const moe_grouped_args* a) {
-    return !(a->format == MOE_FMT_FP4_B16 && a->M <= 8 && columns(a) <= 8192 && a->K >= 4096);
+    const int64_t steps = (a->K + 2047) / 2048, groups = (a->K + 511) / 512;
+    const bool filled = a->K >= 3456 && 7 * steps <= 2 * groups, single_rows = a->M == 1 || 4 * a->M <= a->G;
+    return !(filled && single_rows && columns(a) <= 32768 && (a->format == MOE_FMT_FP4_B32 || columns(a) > 8192));
 }
 
 // GEMM op, K no multiple of 512: the tiles take such a K as any other, so that the bounds by rows per expert lie lower, and go by the

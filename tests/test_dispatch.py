@@ -63,6 +63,20 @@ def test_k_contiguous_fp4_gemm_of_a_partly_filled_last_step(fmt, K):
     assert (rows(3 * 32, 32, 2304, True), rows(3 * 32 + 1, 32, 2304, True)) == (True, False)
 
 
+@pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
+def test_k_contiguous_fp4_gemv_of_a_partly_filled_last_step(fmt):
+    vector = lambda M, G, K, N: kernel(fmt, "gemv", M, G, K, N) == "vector"   # noqa: E731
+    b32 = fmt == "fp4_b32"
+    # well filled steps of the vector kernel
+    assert [K for K in range(2176, 8192, 128) if K % 512 and vector(8, 64, K, 2048)] == [
+        K for lo, hi in ((3456, 4096), (5248, 6144), (6784, 8192)) for K in range(lo, hi, 128) if K % 512]
+    # few rows for the number of experts
+    assert (vector(16, 64, 6912, 2048), vector(17, 64, 6912, 1024), vector(1, 1, 6912, 16384), vector(2, 2, 6912, 8192)) == (True, False, True, False)
+    # columns
+    assert (vector(16, 64, 6912, 512), vector(16, 64, 6912, 513)) == (b32, True)
+    assert (vector(16, 64, 6912, 2048), vector(16, 64, 6912, 2049)) == (True, False)
+
+
 def test_k_contiguous_fp4_shortest_k():
     # the shortest K of the rows kernel is two groups of 128
     for fmt in ("fp4_b32", "fp4_b16"):

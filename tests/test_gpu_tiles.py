@@ -173,6 +173,18 @@ def test_fp4_rows_of_a_partly_filled_last_step(fmt, K):
         assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
 
 
+@pytest.mark.parametrize("K", [3456, 6912])
+@pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
+def test_fp4_vector_kernel_on_single_rows(fmt, K):
+    """gemv_kmajor_kernel on fp4 where gemv_fp4_mfma_kernel's last step would be partly filled: the last of its own steps and, beyond
+    4096 k, the last chunk of x partly filled; experts with one and with five rows, a ragged N."""
+    counts = [0, 1, 0, 0, 5, 0, 0, 1] + [0] * 24 + [1]
+    _say(f"{fmt} vector kernel K={K}")
+    case = H.make_case(fmt, len(counts), K, 1205, np.cumsum(counts), seed=K)
+    assert H.kernel_of(case, "gemv") == "vector"
+    H.assert_close(H.run_cabi(case, H.upload(case), "gemv"), H.oracle_out(case, gemv=True), what=f"{fmt} vector K={K}")
+
+
 @pytest.mark.parametrize("fmt,G,K,N,kernel", [("int4", 600, 1024, 256, "tiles_quad"), ("fp4", 300, 1024, 512, "tiles_quad"),
                                               ("fp4_b32", 300, 1024, 512, "tiles_fp4_k"), ("fp4_b16", 300, 1024, 512, "tiles_fp4_k"),
                                               ("fp4_b16", 450, 1024, 256, "tiles_fp4_k"), ("int8", 511, 4096, 256, "tiles_pair"),
