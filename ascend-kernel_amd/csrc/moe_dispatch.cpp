@@ -49,14 +49,18 @@ static GroupedKernel bf16_kernel(const moe_grouped_args* a, bool gemv_op) {
 }
 
 // fp4 [N, K/2].  The matrix-core GEMV kernel reads every weight row as contiguous runs, takes 16 rows of an expert per pass and
-// has a variant with the GEMM's weight rounding; the bound for the GEMM op is where the k-split tiles overtake it (256 experts
-// of 7168 x 2048: 8 rows per expert 496 vs 631 us, 16 rows 754 vs 651 us).  With the SwiGLU epilogue, fp4_b32, routing skew
-// 0.25 / 1 (see bf16), this kernel against tiles, us: 256 experts of 2048 x 1024, 4 rows per expert on average 63 / 62 against
-// 84 / 59, 5 rows 66 / 77 against 87 / 59, 8 rows 83 / 102 against 91 / 67 (an expert of 109 rows is 7 passes in a row); 256 of
-// 7168 x 4096, 4 rows 809 / 568 against 1145 / 663; 128 of 4096 x 1536, 8 rows 120 / 144 against 132 / 88.  Up to 64 rows in all,
-// four passes at most: 8 of 4096 x 2048, 8 rows 23 / 39 against 36 / 36.
+// has a variant with the GEMM's weight rounding.  An expert of more than 16 rows is passes in a row, so that the bound for the GEMM op,
+// where tiles overtake it with balanced top-k routing, depends on the routing.  us, this kernel / tiles, fp4_b32, evenly routed,
+// balanced top-k routing, skews of 0.25 and 1 (see bf16): 256 experts of 7168 x 2048, 4 rows per expert 394 / 534, 409 / 532, 402 / 527, 296 /
+// 251, 8 rows 447 / 545, 466 / 542, 504 / 541, 485 / 310, 10 rows 479 / 547, 505 / 546, 553 / 547, 566 / 322, 12 rows 486 / 546, 566 / 542, 612
+// / 545, 691 / 347; 64 of the same 8 rows 120 / 137, 125 / 133, 147 / 133, 188 / 127, 10 rows 130 / 137, 146 / 135, 152 / 139, 234 / 131.  Up to
+// 65536 columns the tiles are one per CU, at best, and take longer: 8 of 4096 x 2048, 12 rows 25 / 40, 25 / 40, 26 / 40, 41 / 41.
+// fp4_b16 the same within 0.07.
+// With the SwiGLU epilogue the line lies lower (skews 0.25 and 1): 256 of 2048 x 1024, 4 rows 66 / 81 and 68 / 43, 5 rows 74 / 81 and
+// 81 / 47, 8 rows 84 / 83 and 121 / 60 (an expert of 109 rows is 7 passes in a row); 256 of 7168 x 2048, 4 rows 387 / 520 and 291 / 249, 8 rows
+// 496 / 537 and 496 / 308.  Up to 64 rows in all, four passes at most: 8 of 4096 x 2048, 8 rows 23 / 39 against 36 / 36.
 static bool fp4_rows_preferred(const moe_grouped_args* a) {
-    if (a->epilogue != MOE_EPILOGUE_SWIGLU) return a->M <= 12 * a->G;
+    if (a->epilogue != MOE_EPILOGUE_SWIGLU) return a->M <= (columns(a) <= 65536 ? 12 : 9) * a->G;
     return a->M <= (a->M <= 64 ? 8 : 5) * a->G;
 }
 

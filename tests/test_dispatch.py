@@ -40,7 +40,10 @@ def test_tiles_of_the_n_contiguous_containers():
 def test_k_contiguous_fp4(fmt):
     at = lambda op, r, K, swiglu=False: kernel(fmt, op, r * 64, 64, K, 2048, swiglu)   # noqa: E731
     assert (at("gemv", 1, 7168), at("gemv", 100, 7168), at("gemv", 1, 7168 + 32)) == ("fp4_rows", "fp4_rows", "vector")
-    assert (at("gemm", 12, 7168), at("gemm", 13, 7168), at("gemm", 5, 7168 + 128)) == ("fp4_rows", "tiles_fp4_k", "tiles_fp4_k")
+    assert (at("gemm", 9, 7168), at("gemm", 10, 7168), at("gemm", 5, 7168 + 128)) == ("fp4_rows", "tiles_fp4_k", "tiles_fp4_k")
+    # up to 65536 columns, 12 rows per expert
+    wide = lambda r, G, N: kernel(fmt, "gemm", r * G, G, 7168, N)   # noqa: E731
+    assert (wide(12, 32, 2048), wide(13, 32, 2048), wide(12, 32, 2304), wide(9, 32, 2304)) == ("fp4_rows", "tiles_pair", "tiles_fp4_k", "fp4_rows")
     # with SwiGLU, 5 rows per expert; 8 with up to 64 rows in all
     assert (at("gemm", 5, 7168, True), at("gemm", 6, 7168, True)) == ("fp4_rows", "tiles_fp4_k")
     few = lambda M, G: kernel(fmt, "gemm", M, G, 4096, 2048, True)   # noqa: E731
