@@ -1404,19 +1404,12 @@ __device__ __forceinline__ void expert_chunks(int m, int& chunks, int& bpc) {
     bpc = (nblk + chunks - 1) / chunks;
 }
 
-// Inclusive sums over the lanes of a row of 16, and of the wavefront: DPP shifts (a shuffle goes through LDS, about 100 cycles each,
-// one after the other, at the start of every workgroup)
+// Inclusive sums over the lanes of a row of 16: DPP shifts (a shuffle goes through LDS, about 100 cycles)
 __device__ __forceinline__ int row_scan(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
     v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
     v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
     v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-    return v;
-}
-__device__ __forceinline__ int wave_scan(int v) {
-    v = row_scan(v);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15, rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31, rows 2 and 3
     return v;
 }
 
@@ -1425,13 +1418,14 @@ __device__ __forceinline__ int wave_scan(int v) {
 // of a launch long, one that starts among the last leaves most of the chip waiting for it.
 // us as they come / in this order, rows unevenly routed (skew: see moe_dispatch.cpp): fp4 SwiGLU, 1511 tokens x 8 on 256
 // experts of 7168 x 2048, skew 1: 578 / 563, skew 0.25: 628 / 615; int4, 2000 x 4 on 64 of 7168 x 2048, skew 0.25: 307 / 282.
-// It takes 0.3 us of every workgroup with 4 wavefronts, 0.6 with 8 (an earlier form with shuffles and a second pass over the experts
+// It takes 0.55 us of every workgroup with 4 wavefronts, 0.8 with 8 (an earlier form with shuffles and a second pass over the experts
 // 1.1 and 1.3), which small launches and those that need no order lose: only launches of KernelCfg::ORDER_MIN_WORK do it.  Times as fast as
 // unordered, median (worst, best) evenly routed, by balanced top-k routing and at a skew of 1: int4 and fp4 on GK_QUAD, 0.25 to 0.5
-// million tiles times k (20 us) 0.978 (0.967), 0.977 (0.94), 1.06; 0.5 to 1 million 0.995 (0.98), 1.0 (0.97), 1.01; 1 to 3 million
-// (50 to 100 us) 0.99 (0.98), 1.0 (0.965), 1.06 (0.96, 1.27); more 0.995 (0.976), 1.005 (0.972), 1.065 (0.98, 1.3).  int8 and fp8 on
-// GK_PAIR, 0.5 to 3 million (40 to 110 us) 0.99 (0.974), 0.983 (0.93), 1.01 (0.94, 1.24); more 0.997 (0.98), 0.997 (0.967),
-// 1.035 (0.953, 1.16).
+// million tiles times k (20 us) 0.966 (0.93), 0.968 (0.94), 1.05; 0.5 to 1 million 0.99 (0.967), 0.995 (0.95), 1.0; 1 to 3 million
+// (50 to 100 us) 0.99 (0.95), 0.995 (0.965), 1.06 (0.95, 1.26); more 0.995 (0.973), 1.0 (0.96), 1.07 (0.966, 1.3).  int8 and fp8 on
+// GK_PAIR, 0.5 to 3 million (40 to 110 us) 0.987 (0.97), 0.975 (0.9), 1.01 (0.92, 1.22); more 0.997 (0.973), 0.995 (0.966),
+// 1.035 (0.955, 1.15).  (The scan that follows stays on shuffles: with DPP it saves 0.25 us more, but the k loops of int8 on GK_QUAD, laid out
+// a little differently around it, came out 1 to 4 % slower at K = 7168.)
 // Not for bf16, whose tiles wait for memory or for the matrix cores by their size: large and small ones side by side use both, and
 // that goes either way.  1021 x 8 on 64 of 7168 x 2048, three routings each of skew 0.25 and 0.5: 508 / 485, 457 / 472, 462 / 476
 // and 510 / 470, 496 / 474, 502 / 476; 1500 x 2 on 16 of 4096 x 8192, skew 1: 287 / 302; 700 x 8 on 64 of 7168 x 2048, skew 0:
@@ -1596,10 +1590,15 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         };
         int sum = 0;
         for (int e = g0; e < g1; ++e) sum += tiles_at(e);
-        // scan over the threads: within a wavefront by DPP, across wavefronts through their totals in
+        // scan over the threads: within a wavefront by shuffles, across wavefronts through their totals in
         // LDS (a loop of one thread over all partial sums took 8 us at the start of every workgroup)
         const int lane = tid & 63, wave = tid >> 6;
-        const int incl = wave_scan(sum);
+        int incl = sum;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int up = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += up;
+        }
         if (lane == 63) part[wave] = incl;
         __syncthreads();
         int before = 0, all = 0;
