@@ -1048,8 +1048,10 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
 // 3968 x 13568, 841 rows each, fp4_b32: 699 / 627.  (The reference's fp4 container on GK_QUAD: 522, 534 on the first and third.)
 //
 // The weight rows of a wavefront's columns are read by that wavefront alone, so its weights and scales are its own business:
-// it loads them for 256 k at a time, whole 128-byte lines of 64 rows, into registers, a period of 8 steps ahead, puts them into
-// its own LDS when the last of the previous period is read, and waits for nobody.  (64 bytes of a row at a time, straight to
+// it loads them for 256 k at a time, whole 128-byte lines of 64 rows, into registers during the first steps of the period before, puts
+// them into its own LDS when the last of that period is read, and shares no barrier for them.  (Loads are counted in order: the wait for x at
+// the end of a step also waits for the weights requested two steps earlier, so they have 2 to 3 steps to land, not the 4 to 8 until
+// they are needed.)  (64 bytes of a row at a time, straight to
 // LDS: the other half of a line was gone from L2 when its turn came, 64 workgroups of 256 lines each on an XCD; 1.6 GB fetched
 // instead of 1.2, by counters, and 635 us instead of 593 at K = 7168.  Both halves back to back but in instructions of 16 rows x
 // 64 bytes: 615 us, twice the requests.)  Only x is shared: a ring of four 32-k stages, three steps ahead, one barrier per step.

@@ -4,7 +4,8 @@
 // gemv_impl.h:201-398).  Unlike the reference, more than 4 rows per expert are accepted.
 //
 // Two kernels live here, both for the K-contiguous containers:
-//   gemv_kmajor_kernel    bf16 weights (and fp4 with K % 128 != 0): no matrix cores -- wide vector loads, packed-bf16
+//   gemv_kmajor_kernel    bf16 weights (and the fp4 calls of the GEMV op that moe_dispatch.cpp leaves to it: K % 128 != 0, K = 128, few
+//                         single rows): no matrix cores -- wide vector loads, packed-bf16
 //                         dot products (v_dot2c_f32_bf16), wavefront shuffles for the reductions, 4 rows per pass
 //   gemv_fp4_mfma_kernel  fp4 codes: one v_mfma_f32_16x16x32_bf16 per 32-k block and 16 weight rows (a vector kernel
 //                         needs (1 + rows) / 2 instructions per 4-bit weight, more than the chip can issue while HBM
@@ -311,7 +312,7 @@ __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ w
         const int klen = min(KC, K - kc0);
         const int ngroups = klen / 128;
         const int niter = (ngroups + U - 1) / U;       // iterations of U groups
-        const int nblk = klen / BLK;                   // scales of the chunk (>= 16)
+        const int nblk = klen / BLK;                   // scales of the chunk (WHOLE: >= 16; otherwise >= 8, block 32: >= 4)
         const uint8_t* wp = wg + (kc0 >> 1);                                   // group c of the chunk: + 64 c bytes
         const uint8_t* sp = reinterpret_cast<const uint8_t*>(sg) + (kc0 / BLK) * 2;  // scale b of the chunk: + 2 b bytes
         // x fragment of block 4 c + j: unit (16 c + 4 j + q) ^ r of row r = xj[j][16 c].  MFMA rows
@@ -434,8 +435,8 @@ __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ w
                 w[u] = *reinterpret_cast<const u32x4_t*>(wp + (woff + (uint32_t)((WHOLE ? it * U + u : min(it * U + u, ngroups - 1)) * 64)));
         };
         // scales 64 T + 16 q .. + 15 of this lane's row in the chunk: those of iteration 4 T + q (block 32)
-        // or of half of iteration 2 T + (q >> 1) (block 16); clamped into the chunk (iterations past its
-        // end do not exist)
+        // or of half of iteration 2 T + (q >> 1) (block 16); not beyond the chunk's end (iterations past it
+        // do not exist), where WHOLE is not set from up to 4 scales before its start
         auto fetch_s = [&](u32x4_t (&sv)[2], int T) {
             if constexpr (WHOLE) {
                 const int b0 = min(64 * T + 16 * q, nblk - 16);

@@ -54,8 +54,9 @@ extern "C" {
 typedef void *moe_stream_t;
 
 /* Experts per call of either grouped op.  (moe_grouped_gemm keeps a table of G + 1 tile counts in LDS next to its
- * tile buffers while that fits -- about 900 experts for bf16, 1900 to 5500 for most other kernels -- and beyond that one
- * entry per thread, walking group_list for the rest: any count works, small ones are faster.) */
+ * tile buffers while that fits -- about 900 experts for bf16 and for prefill on the K-contiguous fp4 containers, 1900 to
+ * 5500 for most other kernels -- and beyond that one entry per thread, walking group_list for the rest: any count works, small
+ * ones are faster.) */
 #define MOE_GEMM_MAX_EXPERTS 65535
 
 typedef enum moe_status {
