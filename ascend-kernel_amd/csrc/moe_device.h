@@ -71,6 +71,18 @@ __device__ __forceinline__ float fp16_hi_times(uint32_t h2, float s, float neg_z
     return r;
 }
 
+// fp32(low / high fp16 of h2) * m + z in one instruction, rounded once.
+__device__ __forceinline__ float fp16_lo_fma(uint32_t h2, float m, float z) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h2), "v"(m), "v"(z));
+    return r;
+}
+__device__ __forceinline__ float fp16_hi_fma(uint32_t h2, float m, float z) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h2), "v"(m), "v"(z));
+    return r;
+}
+
 __device__ __forceinline__ float wave_reduce_sum(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);

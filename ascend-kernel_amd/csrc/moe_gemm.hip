@@ -200,7 +200,7 @@ __device__ __forceinline__ uint32_t here(uint32_t v) {
 // all rows of the tile (4 MFMAs per x fragment), but only one of the two 32-k sub-steps of
 // every 64-k step: the pair (wv, wv + 4) shares a SIMD and accumulates two partial sums that
 // are added once per tile through LDS.  Every weight element is still decoded exactly once
-// per tile, a lane decodes 4 nibbles of a dword at a time (2.5 VALU instructions per
+// per tile, a lane decodes 4 nibbles of a dword at a time (2.25 VALU instructions per
 // element), and each wavefront reads half of the x fragments.
 //
 // Each wavefront alternates a decode phase (its sub-step of the packed stage -> 4 bf16 B
@@ -218,11 +218,13 @@ __device__ __forceinline__ uint32_t here(uint32_t v) {
 // own repeat one: measured, the repeated loads cost nothing, a branch around them does), so "at most
 // (S - 3) NI outstanding" means exactly that.
 //
-// Decode of a k-row pair (a, b) of one dword column: v_perm gathers the two bytes of each row
-// this lane owns, the low nibbles (& 0x0f0f0f0f) and high nibbles (>> 4 & 0x0f0f0f0f) are bytes
-// 0x00..0x0f, which read as OCP e4m3 are exactly q / 512 -- v_cvt_pk_f32_fp8 converts two at
-// once -- and one fma per element applies 512 * scale and the zero point:
-// q s - 8 s = (q - 8) s exactly.
+// Decode of a k-row pair (a, b) of one dword column: v_perm gathers the two bytes of each row this lane owns, row a's
+// into the low, row b's into the high half of a dword.  Masked with 0x000f and put under 0x6400 a half is the fp16
+// 1024 + q (0x00f0: 1024 + 16 q), so v_fma_mix_f32 converts a weight and takes its scale and the zero point in one
+// instruction: (1024 + q) s - 1032 s, or (1024 + 16 q) s / 16 - 72 s, is (q - 8) s exactly (12 bits; scales below 2^117).
+// 2.25 instructions per weight; masks, conversions from e4m3 and fmas took 2.5.  us, before / now: a prefill layer of 4096
+// tokens x 8 on 256 experts of 7168 x 2048 2883 / 2842, decode layers of 64 x 8 and 16 x 8 1059 / 998 and 413 / 391, 512 rows
+// on 64 experts of 2048 x 4096 122 / 117.
 //
 // The same routine serves the reference's pre-shuffled fp4 container: its 64 x 128-byte tile is
 // brought in by the same loads, a lane's 8 k rows of its 2 bytes are two 16-byte LDS reads, each
@@ -446,6 +448,10 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     // 395 us (fp4) with the plain barrier; one per CU, fp8, 555 against 580 us with the split one).
     constexpr bool SPLIT_BARRIER = pair_wg_per_cu<FMT>(KIND) == 1;
     constexpr int PAIR_A_UNITS = pair_a_units(KIND);
+    // The next step's packed dwords are read ahead of the MFMAs instead of behind the first ones: with 4 or 8 MFMAs a step their
+    // latency otherwise ends in the next decode (int4, a tile per CU, 2 rows: 64 experts of 2048 x 1024 22.6 / 21.3 us).
+    // fp4 gains nothing from it, the GEMV op's kinds lose 0.5 to 4 %: they still need the scales of the step being multiplied.
+    constexpr bool EARLY_RAW = FMT == MOE_FMT_INT4 && KIND == GK_PAIR_SMALL;
     static_assert(16 * MT * (BK / 8) <= PAIR_A_UNITS, "tile rows beyond the x stage");
     u32x4_t* lds_a = smem;
     u32x4_t* lds_b = lds_a + S * PAIR_A_UNITS;
@@ -581,8 +587,9 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     constexpr bool I4X = EXACT && FMT == MOE_FMT_INT4;
     uint32_t sel = I4X ? h2 | ((4u + h2) << 8) | ((h2 + 1u) << 16) | ((5u + h2) << 24)
                        : h2 | ((h2 + 1u) << 8) | ((4u + h2) << 16) | ((5u + h2) << 24);
-    uint32_t mask = 0x0f0f0f0fu;
+    uint32_t mask = FMT == MOE_FMT_INT4 && !EXACT ? 0x000f000fu : 0x0f0f0f0fu, mask_hi = 0x00f000f0u, magic = 0x64006400u;
     asm volatile("" : "+s"(mask), "+s"(sel));   // kept opaque so that each stays one SGPR operand
+    if constexpr (FMT == MOE_FMT_INT4 && !EXACT) asm volatile("" : "+s"(mask_hi), "+v"(magic));
     const int d = 16 * (cw >> 1) + i;            // dword column of this lane
     const int unit = (d >> 2) ^ (4 * (q & 1));
     // row of the x stage this lane's fragment row i comes from (STACK2: see above)
@@ -762,8 +769,8 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             m[0] = s0; m[1] = s1; m[2] = s2; m[3] = s3;
             z[0] = z[1] = z[2] = z[3] = 0.f;
         } else {
-            m[0] = s0 * 512.f; m[1] = s1 * 512.f; m[2] = s2 * 512.f; m[3] = s3 * 512.f;
-            z[0] = -8.f * s0; z[1] = -8.f * s1; z[2] = -8.f * s2; z[3] = -8.f * s3;
+            m[0] = s0; m[1] = s1 * 0.0625f; m[2] = s2; m[3] = s3 * 0.0625f;
+            z[0] = -1032.f * s0; z[1] = -72.f * s1; z[2] = -1032.f * s2; z[3] = -72.f * s3;
         }
         // Written stage by stage over two row pairs at a time so that consecutive instructions are
         // independent (a VALU result is not available to the very next instruction); the fences
@@ -850,8 +857,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
                 __builtin_amdgcn_sched_barrier(0);
                 continue;
             }
-            uint32_t pr[2], lo[2], hi[2];
-            f32x2_t a02[2], b02[2], a13[2], b13[2];
+            uint32_t pr[2];
             float wa[2][4], wb[2][4];
 #pragma unroll
             for (int p = 0; p < 2; ++p) pr[p] = __builtin_amdgcn_perm(r[2 * (p0 + p) + 1], r[2 * (p0 + p)], sel);   // a.b0 a.b1 b.b0 b.b1
@@ -877,58 +883,47 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
                 __builtin_amdgcn_sched_barrier(0);
                 continue;
             }
-#pragma unroll
-            for (int p = 0; p < 2; ++p) { lo[p] = pr[p] & mask; hi[p] = pr[p] >> 4; }
             if constexpr (I4X) {
                 // The codes themselves as bf16, two at a time: a nibble read as e4m3 is q / 512, and the scaled
                 // convert (scale 2^9: only the exponent of that operand counts) yields the bf16 pair (q_a, q_b) of
                 // one column.  The zero point is taken off in the MFMA phase.
 #pragma unroll
                 for (int p = 0; p < 2; ++p) {
-                    hi[p] &= mask;
-                    bf[0][p0 + p] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo[p], 512.f, false));
-                    bf[2][p0 + p] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo[p], 512.f, true));
-                    bf[1][p0 + p] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi[p], 512.f, false));
-                    bf[3][p0 + p] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi[p], 512.f, true));
+                    const uint32_t lo = pr[p] & mask, hi = (pr[p] >> 4) & mask;
+                    bf[0][p0 + p] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.f, false));
+                    bf[2][p0 + p] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.f, true));
+                    bf[1][p0 + p] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.f, false));
+                    bf[3][p0 + p] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.f, true));
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 continue;
             }
-            __builtin_amdgcn_sched_barrier(0);
+            // int4: halves (a, b) as fp16, one fma each (see the head of this routine)
+            uint32_t h4[2][4];
 #pragma unroll
             for (int p = 0; p < 2; ++p) {
-                hi[p] &= mask;
-                a02[p] = __builtin_amdgcn_cvt_pk_f32_fp8(lo[p], false);
-                b02[p] = __builtin_amdgcn_cvt_pk_f32_fp8(lo[p], true);
+                const uint32_t up = pr[p] >> 8;
+                h4[p][0] = (pr[p] & mask) | magic;
+                h4[p][1] = (pr[p] & mask_hi) | magic;
+                h4[p][2] = (up & mask) | magic;
+                h4[p][3] = (up & mask_hi) | magic;
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                a13[p] = __builtin_amdgcn_cvt_pk_f32_fp8(hi[p], false);
-                b13[p] = __builtin_amdgcn_cvt_pk_f32_fp8(hi[p], true);
+            for (int t = 0; t < 4; t += 2) {
+#pragma unroll
+                for (int p = 0; p < 2; ++p)
+#pragma unroll
+                    for (int u = t; u < t + 2; ++u) {
+                        wa[p][u] = fp16_lo_fma(h4[p][u], m[u], z[u]);
+                        wb[p][u] = fp16_hi_fma(h4[p][u], m[u], z[u]);
+                    }
+                __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                wa[p][0] = fmaf(a02[p][0], m[0], z[0]); wb[p][0] = fmaf(b02[p][0], m[0], z[0]);
-                wa[p][2] = fmaf(a02[p][1], m[2], z[2]); wb[p][2] = fmaf(b02[p][1], m[2], z[2]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
+            for (int p = 0; p < 2; ++p)
 #pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                wa[p][1] = fmaf(a13[p][0], m[1], z[1]); wb[p][1] = fmaf(b13[p][0], m[1], z[1]);
-                wa[p][3] = fmaf(a13[p][1], m[3], z[3]); wb[p][3] = fmaf(b13[p][1], m[3], z[3]);
-            }
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                bf[0][p0 + p] = pack_bf16_rne(wa[p][0], wb[p][0]);
-                bf[2][p0 + p] = pack_bf16_rne(wa[p][2], wb[p][2]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                bf[1][p0 + p] = pack_bf16_rne(wa[p][1], wb[p][1]);
-                bf[3][p0 + p] = pack_bf16_rne(wa[p][3], wb[p][3]);
-            }
+                for (int t = 0; t < 4; ++t) bf[t][p0 + p] = pack_bf16_rne(wa[p][t], wb[p][t]);
             __builtin_amdgcn_sched_barrier(0);
         }
         // ---- MFMA phase, at raised issue priority: the other wavefront of the SIMD is decoding
@@ -938,6 +933,10 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
         if constexpr (SPLIT_BARRIER) ring_wait((uint32_t)kt, arrivals_seen);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(3);
+        if constexpr (EARLY_RAW) {
+            read_raw(sn, kt + 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         // Everybody is done with stage kt-1 and has its part of stage kt+1 in LDS: this step's loads (stage kt+4
         // replaces stage kt-1) and the packed dwords of the next step (stage kt+1) are fetched between the MFMAs.
 #pragma unroll
@@ -990,7 +989,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             }
 #pragma unroll
             for (int m = (mt * NI + MT - 1) / MT; m < ((mt + 1) * NI + MT - 1) / MT; ++m) issue(m, kt, sl);
-            if (mt == 0) read_raw(sn, kt + 1);
+            if (mt == 0 && !EARLY_RAW) read_raw(sn, kt + 1);
             __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_s_setprio(0);

@@ -1,0 +1,58 @@
+"""The weights that the GEMM op multiplies by, bit for bit: rows of x with a single 1 make y the rounded weights themselves, over
+every code and the whole range of scales, on every kernel that decodes the container."""
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+import helpers as H
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+def _scales(rng, shape, lo, hi):
+    """bf16 bits of both signs, magnitudes from 2^lo to 2^hi."""
+    e = rng.integers(lo + 127, hi + 127, shape)
+    return ((rng.integers(0, 2, shape) << 15) | (e << 7) | rng.integers(0, 128, shape)).astype(np.uint16)
+
+
+def _unit_rows(case, rng):
+    """x of zeros with a 1 per row, in turn over k, starting anywhere."""
+    M, K = case["M"], case["K"]
+    at = (np.arange(M) + rng.integers(0, K)) % K
+    x = np.zeros((M, K), np.uint16)
+    x[np.arange(M), at] = 0x3F80
+    case["x"] = x
+    return at
+
+
+def _check(case, at, kernel):
+    assert H.kernel_of(case, "gemm") == kernel
+    got = oracle.bf16_bits_to_f32(H.run_cabi(case, H.upload(case), "gemm"))
+    lo = 0
+    for g, hi in enumerate(case["group_list"]):
+        w = oracle.expand_weight(oracle.FMT_BY_NAME[case["fmt"]], case["weight"], case["scale"], case["offset"], g, True)
+        want = w.reshape(case["K"], case["N"])[at[lo:hi]]
+        assert np.array_equal(got[lo:hi], want), f"{case['fmt']} {kernel} expert {g}"
+        lo = hi
+
+
+# kernel, experts, K, N, rows per expert
+INT4 = [("strips_32", 4, 256, 512, 16), ("strips_64", 6, 256, 2048, 16), ("strips_128", 10, 256, 2048, 12),
+        ("tiles_pair_small", 20, 256, 2048, 12), ("tiles_quad", 2, 256, 256, 256), ("tiles_quad", 20, 256, 2048, 145)]
+
+
+@pytest.mark.parametrize("kernel,G,K,N,rows", INT4)
+def test_int4(kernel, G, K, N, rows):
+    _say(f"int4 weight bits {kernel}")
+    rng = np.random.default_rng(G + N)
+    case = H.make_case("int4", G, K, N, np.arange(1, G + 1) * rows, seed=G, group=32)
+    case["scale"] = _scales(rng, case["scale"].shape, -110, 117)
+    _check(case, _unit_rows(case, rng), kernel)
