@@ -240,13 +240,18 @@ __global__ __launch_bounds__(256) void gemv_kmajor_kernel(const uint16_t* __rest
 // The MFMA wants the 4 q lanes of a column to hold the 4 dwords of ONE block (a block has
 // one scale, and the MFMA sums over q): a 4x4 transpose of the dwords across the q lanes,
 // two v_permlane32_swap and two v_permlane16_swap per 16 bytes.
+// With the GEMM's rounding (ROUNDW below) the scale is in the weights when the MFMA sums over q, so its 32 k may come from four
+// blocks: MFMA j takes dword j of every lane's own block, x is read at those k (unit 16 c + 4 q + j), and a lane needs its own
+// block's scale only, one per 16 bytes.  No transpose, 2.14 instead of 2.45 vector instructions per weight, which is what bounds
+// that variant; us, before / now: 256 experts of 7168 x 2048, 512 rows, fp4_b32 370 / 346, fp4_b16 399 / 369; 480 rows on 64 of
+// 4096 x 1536 74 / 69 and 80 / 73; 8 single rows of 7168 x 512, fp4_b16 31 / 27.
 //
 // Scales: every lane of a column needs the same 4 scales per load, 8 bytes of a row -- read
 // that way, each 64-byte piece of a scale row is fetched from HBM several times.  Instead the
 // 4 q lanes of a row read 128 contiguous bytes of it once per 4 loop iterations (lane q: the
 // 16 scales of iteration 4 T + q) and the iteration's scales are picked up from the lane that
-// holds them through a wavefront's own 2 KB of LDS (written once per 4 iterations, read with 16-byte loads that
-// the 4 q lanes share: ds_bpermute, which this replaced, serves 4 lanes that ask for one lane's register one after
+// holds them through a wavefront's own 2 KB of LDS (written once per 4 iterations, ROUNDW: in the order in which the lanes
+// read them, 8 bytes each; otherwise read with 16-byte loads that the 4 q lanes share: ds_bpermute, which this replaced, serves 4 lanes that ask for one lane's register one after
 // the other -- the counters showed it as bank conflicts in 39 % of the LDS cycles).
 //
 // x (<= 16 rows of a chunk of K) is staged in LDS; the 16-byte units of row r are XOR-swizzled
@@ -320,11 +325,34 @@ __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ w
         // (lanes that read the same unit are served together: timed alone, this pattern reads as fast as
         // 64 consecutive units, and sending the repeated rows to other units was slower).
         const int r = i % MB;
+        // ROUNDW: dword j of the lane's own block 4 c + q, unit (16 c + 4 q + j) ^ r
         const u32x4_t* xj[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) xj[j] = xs + r * RS + ((4 * j + q) ^ r);
+        for (int j = 0; j < 4; ++j) xj[j] = xs + r * RS + ((ROUNDW ? 4 * q + j : 4 * j + q) ^ r);
 
-        // one 128-k group: w = this lane's 16 bytes (block 4 c + q of its row), s0/s1 = the 4 scales of
+        // one 128-k group with rounded weights: the codes stay with the lane that loaded them (see above); s[0], s[1] = the scales
+        // of the two halves of its block (block 32: the same)
+        auto group_rounded = [&](const u32x4_t& w, const float (&s)[2], int c) {
+#pragma unroll
+            for (int j0 = 0; j0 < 4; j0 += 2) {
+                u32x4_t aw[2], bw[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) aw[j] = xj[j0 + j][16 * c];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    bw[j][0] = e2m1_pair_scaled_bf16<0>(w[j0 + j], s[j0 >> 1]);
+                    bw[j][1] = e2m1_pair_scaled_bf16<1>(w[j0 + j], s[j0 >> 1]);
+                    bw[j][2] = e2m1_pair_scaled_bf16<2>(w[j0 + j], s[j0 >> 1]);
+                    bw[j][3] = e2m1_pair_scaled_bf16<3>(w[j0 + j], s[j0 >> 1]);
+                }
+                // two accumulators, so that consecutive MFMAs do not depend on each other
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, aw[0]),
+                                                              __builtin_bit_cast(bf16x8_t, bw[0]), acc, 0, 0, 0);
+                acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, aw[1]),
+                                                               __builtin_bit_cast(bf16x8_t, bw[1]), acc2, 0, 0, 0);
+            }
+        };
+        // the same with weights that are not rounded: w = this lane's 16 bytes (block 4 c + q of its row), s0/s1 = the 4 scales of
         // blocks 4 c .. 4 c + 3 as two bf16 pairs
         auto group = [&](const u32x4_t& w, const uint32_t (&sd)[BLK == 32 ? 2 : 4], int c) {
             // 4x4 transpose of the dwords over the q lanes: b[j] = this lane's 8 codes of block 4 c + j
@@ -333,15 +361,15 @@ __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ w
             const u32x2_t b01 = __builtin_amdgcn_permlane16_swap(t02[0], t13[0], false, false);
             const u32x2_t b23 = __builtin_amdgcn_permlane16_swap(t02[1], t13[1], false, false);
             const uint32_t b[4] = {b01[0], b01[1], b23[0], b23[1]};
-            // s[j]: block 32: the scale of block j; block 16: the scale of this lane's half of block j
-            // (ROUNDW) / of the first half (else), s2[j] that of the second half
+            // s[j]: block 32: the scale of block j; block 16: the scale of the half of block j whose sums this lane holds
+            // (STACK) / of the first half (else), s2[j] that of the second half
             float s[4], s2[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 if constexpr (BLK == 32) {
                     s[j] = (j & 1) ? bf16_hi(sd[j >> 1]) : bf16_lo(sd[j >> 1]);
                     s2[j] = 0.f;
-                } else if constexpr (ROUNDW || STACK) {
+                } else if constexpr (STACK) {
                     s[j] = hi_half ? bf16_hi(sd[j]) : bf16_lo(sd[j]);
                     s2[j] = 0.f;
                 } else {
@@ -356,20 +384,7 @@ __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ w
                 u32x4_t aw[2], bw[2];
 #pragma unroll
                 for (int j = 0; j < 2; ++j) aw[j] = xj[j0 + j][16 * c];
-                if constexpr (ROUNDW) {
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        bw[j][0] = e2m1_pair_scaled_bf16<0>(b[j0 + j], s[j0 + j]);
-                        bw[j][1] = e2m1_pair_scaled_bf16<1>(b[j0 + j], s[j0 + j]);
-                        bw[j][2] = e2m1_pair_scaled_bf16<2>(b[j0 + j], s[j0 + j]);
-                        bw[j][3] = e2m1_pair_scaled_bf16<3>(b[j0 + j], s[j0 + j]);
-                    }
-                    // two accumulators, so that consecutive MFMAs do not depend on each other
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, aw[0]),
-                                                                  __builtin_bit_cast(bf16x8_t, bw[0]), acc, 0, 0, 0);
-                    acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, aw[1]),
-                                                                   __builtin_bit_cast(bf16x8_t, bw[1]), acc2, 0, 0, 0);
-                } else if constexpr (STACK) {
+                if constexpr (STACK) {
                     f32x4_t part[2];
 #pragma unroll
                     for (int j = 0; j < 2; ++j)
@@ -456,14 +471,48 @@ __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ w
             }
         };
         u32x4_t sc[2], sn[2];
+        u32x2_t sc2;
         // iteration `it` on the weights in w; rotates the scale registers every PER iterations
         auto iteration = [&](const u32x4_t (&w)[U], int it) {
             const int t = it & (PER - 1);
             if (t == 0) {
                 // (a wavefront's LDS accesses complete in order: the reads of the previous scales are done)
-                ss[(2 * q) * 16 + i] = sn[0];
-                ss[(2 * q + 1) * 16 + i] = sn[1];
+                if constexpr (ROUNDW) {
+                    // unit 64 q' + 16 k + i of 8 bytes: of the 16 scales of lane (i, q'), those that lane (i, k) multiplies by
+                    u32x2_t* const sx = reinterpret_cast<u32x2_t*>(ss) + 64 * q + i;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        // block 32: block k of the iteration's four groups; block 16: both halves of block k of two groups
+                        const uint32_t sel = k & 1 ? 0x07060302u : 0x05040100u;
+                        if constexpr (BLK == 32)
+                            sx[16 * k] = u32x2_t{__builtin_amdgcn_perm(sn[0][2 + (k >> 1)], sn[0][k >> 1], sel),
+                                                 __builtin_amdgcn_perm(sn[1][2 + (k >> 1)], sn[1][k >> 1], sel)};
+                        else
+                            sx[16 * k] = u32x2_t{sn[0][k], sn[1][k]};
+                    }
+                } else {
+                    ss[(2 * q) * 16 + i] = sn[0];
+                    ss[(2 * q + 1) * 16 + i] = sn[1];
+                }
                 if (it + PER < niter) fetch_s(sn, it / PER + 1);
+            }
+            if constexpr (ROUNDW) {
+                const u32x2_t* const sx = reinterpret_cast<const u32x2_t*>(ss) + lane;   // unit 16 q + i of an iteration's 64
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (!WHOLE && it * U + u >= ngroups) break;
+                    float s[2];
+                    if constexpr (BLK == 32) {
+                        if (u == 0) sc2 = sx[64 * t];
+                        s[0] = s[1] = u & 1 ? bf16_hi(sc2[u >> 1]) : bf16_lo(sc2[u >> 1]);
+                    } else {
+                        if (!(u & 1)) sc2 = sx[64 * (2 * t + (u >> 1))];
+                        s[0] = bf16_lo(sc2[u & 1]);
+                        s[1] = bf16_hi(sc2[u & 1]);
+                    }
+                    group_rounded(w[u], s, it * U + u);
+                }
+                return;
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {

@@ -24,9 +24,9 @@ def _scales(rng, shape, lo, hi):
 
 
 def _unit_rows(case, rng):
-    """x of zeros with a 1 per row, in turn over k, starting anywhere."""
+    """x of zeros with a 1 per row: every k in turn, in any order."""
     M, K = case["M"], case["K"]
-    at = (np.arange(M) + rng.integers(0, K)) % K
+    at = np.resize(rng.permutation(K), M)
     x = np.zeros((M, K), np.uint16)
     x[np.arange(M), at] = 0x3F80
     case["x"] = x
@@ -56,3 +56,16 @@ def test_int4(kernel, G, K, N, rows):
     case = H.make_case("int4", G, K, N, np.arange(1, G + 1) * rows, seed=G, group=32)
     case["scale"] = _scales(rng, case["scale"].shape, -110, 117)
     _check(case, _unit_rows(case, rng), kernel)
+
+
+# experts, K, rows per expert: 4, 8 and 16 staged rows, whole iterations of 512 k and one to three groups of 128 behind them, K on
+# both sides of what is staged at a time (7168, 3584 and 1536)
+@pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
+@pytest.mark.parametrize("G,K,rows", [(64, 512, 4), (64, 640, 8), (64, 896, 12), (64, 1152, 3), (48, 1536, 12), (48, 1664, 12),
+                                      (32, 2048, 12), (32, 3712, 8), (32, 4096, 7), (24, 7168, 4), (24, 7296, 4), (24, 7680, 4)])
+def test_fp4_rows(fmt, G, K, rows):
+    _say(f"{fmt} weight bits K={K}, {rows} rows")
+    rng = np.random.default_rng(K)
+    case = H.make_case(fmt, G, K, 256, np.arange(1, G + 1) * rows, seed=K)
+    case["scale"] = _scales(rng, case["scale"].shape, -110, 117)
+    _check(case, _unit_rows(case, rng), "fp4_rows")
