@@ -69,3 +69,45 @@ def test_fp4_rows(fmt, G, K, rows):
     case = H.make_case(fmt, G, K, 256, np.arange(1, G + 1) * rows, seed=K)
     case["scale"] = _scales(rng, case["scale"].shape, -110, 117)
     _check(case, _unit_rows(case, rng), "fp4_rows")
+
+
+# kernel, experts, K, N, rows per expert
+FP8 = [("strips_32", 4, 256, 512, 16), ("strips_128", 10, 256, 2048, 12), ("tiles_pair", 20, 256, 2048, 40), ("tiles_pair", 4, 384, 384, 160),
+       ("tiles_quad", 2, 256, 256, 256)]
+
+
+@pytest.mark.parametrize("codes", ["without", "some", "all"])
+@pytest.mark.parametrize("kernel,G,K,N,rows", FP8)
+def test_fp8(kernel, G, K, N, rows, codes):
+    """0x7F and 0xFF are +-480 here and NaN to the hardware's conversions: none of them, one in the middle of some experts, any."""
+    _say(f"fp8 weight bits {kernel} 0x7F: {codes}")
+    rng = np.random.default_rng(G + N)
+    case = H.make_case("fp8", G, K, N, np.arange(1, G + 1) * rows, seed=G)
+    if codes != "all":
+        case["weight"][(case["weight"] & 0x7F) == 0x7F] ^= 1
+    if codes == "some":
+        for g in range(0, G, 2):
+            case["weight"][g, rng.integers(0, K), rng.integers(0, N)] |= 0x7F
+    e = rng.integers(-60, 40, case["scale"].shape)
+    case["scale"] = (case["scale"] * np.exp2(e)).astype(np.float32)
+    _check(case, _unit_rows(case, rng), kernel)
+
+
+@pytest.mark.parametrize("codes", ["without", "some", "all"])
+@pytest.mark.parametrize("rows", [3, 16, 17, 40])
+def test_fp8_gemv(rows, codes):
+    """The same of the GEMV op, whose weights are not rounded: with scales of powers of two bf16 holds them."""
+    _say(f"fp8 gemv weight bits, {rows} rows, 0x7F: {codes}")
+    rng = np.random.default_rng(rows)
+    G, K, N = 24, 256, 2048
+    case = H.make_case("fp8", G, K, N, np.arange(1, G + 1) * rows, seed=rows)
+    if codes != "all":
+        case["weight"][(case["weight"] & 0x7F) == 0x7F] ^= 1
+    if codes == "some":
+        for g in range(0, G, 2):
+            case["weight"][g, rng.integers(0, K), rng.integers(0, N)] |= 0x7F
+    case["scale"] = np.exp2(rng.integers(-60, 40, case["scale"].shape)).astype(np.float32)
+    at = _unit_rows(case, rng)
+    assert H.kernel_of(case, "gemv") == "tiles_pair_exact"
+    got, want = H.run_cabi(case, H.upload(case), "gemv"), H.oracle_out(case, gemv=True)
+    assert np.array_equal(oracle.bf16_bits_to_f32(got), oracle.bf16_bits_to_f32(want)), at
