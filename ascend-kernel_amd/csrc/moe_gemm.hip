@@ -300,6 +300,13 @@ constexpr int pair_sc_units(int kind) {
 // worth) per weight row at a time, three buffers of 256 rows
 template <int FMT>
 constexpr int pair_kc_scale_units() { return (FMT == MOE_FMT_FP4_B32 || FMT == MOE_FMT_FP4_B16) ? 3 * 256 : 0; }
+// GK_QUAD, tiles of up to 3 row blocks: they wait for their weights, of which 3 stages ahead of two workgroups are 30 KB on their way
+// per CU, enough for about 4 TB/s; their x needs little of the LDS, so they get 6 stages.  us, 4 / 6 stages: 16 rows each on 256
+// experts of 7168 x 2048, fp4 514 / 459, int4 519 / 476; 1511 tokens x 8 unevenly routed over the same, fp4 SwiGLU 568 / 540, int4
+// (skew 1) 584 / 551; 5600 rows on 64 of 2048 x 4096, fp4 131 / 124.  8 stages are no faster, and with 4 or 5 row blocks fp4 loses (64 rows
+// each on 128 experts 327 / 331).  A launch with a tile per workgroup at most keeps 4: it gains nothing from more and pays for fetching
+// the code of the longer ring (416 rows on 16 of 3328 x 2048: 42.0 / 43.2).  The one-byte containers are here for experts of many rows.
+constexpr int QUAD_DEEP_MT = 3, QUAD_DEEP_STAGES = 6;
 template <int FMT>
 constexpr int pair_lds_units(int kind) {
     return pair_stages<FMT>(kind) * (pair_a_units(kind) + pair_b_units<FMT>(kind) + pair_sc_units<FMT>(kind)) + pair_kc_scale_units<FMT>();
@@ -421,7 +428,9 @@ __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, 
 // leaves the first group's sums in the lanes q < 2 and the second group's in q >= 2, each lane applies the
 // scale of its own group, and the two halves are added once at the end of the tile: half the MFMAs and half
 // the multiplies of the general case, and no masking.
-template <int FMT, int MT, int KIND, bool STACK2 = false>
+//
+// DEEP (GK_QUAD, small tiles): the longer ring, see QUAD_DEEP_STAGES.
+template <int FMT, int MT, int KIND, bool STACK2 = false, bool DEEP = false>
 __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk) {
     static_assert(FMT != MOE_FMT_BF16, "the k-split tile routine decodes quantized containers");
     constexpr bool EXACT = pair_exact(KIND);
@@ -438,7 +447,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     static_assert(!Q4 || FMT == MOE_FMT_INT4 || FMT == MOE_FMT_INT8 || FMT == MOE_FMT_FP4_REF || FMT == MOE_FMT_FP8_REF,
                   "the 4-wavefront kind serves the N-contiguous containers");
     constexpr int NW = pair_waves(KIND);
-    constexpr int BK = pair_bk(KIND), S = pair_stages<FMT>(KIND), PAIR_SC_UNITS = pair_sc_units<FMT>(KIND);
+    constexpr int BK = pair_bk(KIND), S = DEEP ? QUAD_DEEP_STAGES : pair_stages<FMT>(KIND), PAIR_SC_UNITS = pair_sc_units<FMT>(KIND);
     constexpr int PAIR_B_UNITS = pair_b_units<FMT>(KIND);
     constexpr int AHEAD = S - 1;   // a step's loads fill the stage of step kt + AHEAD
     // Kinds of which two workgroups share a CU (decode batches, HBM bound) keep one s_barrier per step, placed so
@@ -447,11 +456,12 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     // faster (measured on 512 rows over 256 experts of 7168 x 2048: two per CU 335 against 340 us (int4), 390 against
     // 395 us (fp4) with the plain barrier; one per CU, fp8, 555 against 580 us with the split one).
     constexpr bool SPLIT_BARRIER = pair_wg_per_cu<FMT>(KIND) == 1;
-    constexpr int PAIR_A_UNITS = pair_a_units(KIND);
+    constexpr int PAIR_A_UNITS = DEEP ? 64 * MT : pair_a_units(KIND);
     // The next step's packed dwords are read ahead of the MFMAs instead of behind the first ones: with 4 or 8 MFMAs a step their
     // latency otherwise ends in the next decode (int4, a tile per CU, 2 rows: 64 experts of 2048 x 1024 22.6 / 21.3 us).
     // fp4 gains nothing from it, the GEMV op's kinds lose 0.5 to 4 %: they still need the scales of the step being multiplied.
     constexpr bool EARLY_RAW = FMT == MOE_FMT_INT4 && KIND == GK_PAIR_SMALL;
+    static_assert(S * (PAIR_A_UNITS + PAIR_B_UNITS + PAIR_SC_UNITS) <= pair_lds_units<FMT>(KIND), "stages beyond the LDS of the kernel");
     static_assert(16 * MT * (BK / 8) <= PAIR_A_UNITS, "tile rows beyond the x stage");
     u32x4_t* lds_a = smem;
     u32x4_t* lds_b = lds_a + S * PAIR_A_UNITS;
@@ -1583,9 +1593,12 @@ struct KernelCfg {
 };
 
 template <int FMT, int MT, int KIND>
-__device__ __forceinline__ void run_tile(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk) {
+__device__ __forceinline__ void run_tile(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk, bool deep) {
     using C = KernelCfg<FMT, KIND>;
     if constexpr (C::PAIR) {
+        if constexpr (KIND == GK_QUAD && MT <= QUAD_DEEP_MT && (FMT == MOE_FMT_INT4 || FMT == MOE_FMT_FP4_REF)) {
+            if (deep) return gemm_tile_pair<FMT, MT, KIND, false, true>(P, smem, g, row0, rows, n0, tk);
+        }
         if constexpr (FMT == MOE_FMT_FP4_REF && pair_exact(KIND) && MT == 1) {
             if (rows <= 8) return gemm_tile_pair<FMT, MT, KIND, true>(P, smem, g, row0, rows, n0, tk);
         }
@@ -1687,6 +1700,9 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         __syncthreads();
     }
     const int total = __builtin_amdgcn_readfirstlane(prefix[entries]);
+
+    // more than one tile per workgroup (see QUAD_DEEP_STAGES)
+    const bool deep = total > (int)gridDim.x;
 
     // XCD-aware order: workgroup b runs on XCD b % 8; give each XCD a contiguous run of
     // tiles in every sweep so that its workgroups share x rows in its own L2.
@@ -1808,34 +1824,34 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         const int n0 = nt * C::BN;
         switch (mt) {
             case 1:
-                if constexpr (MTM >= 1) run_tile<FMT, 1, KIND>(P, smem, g, row0, rows, n0, tk);
+                if constexpr (MTM >= 1) run_tile<FMT, 1, KIND>(P, smem, g, row0, rows, n0, tk, deep);
                 break;
             case 2:
-                if constexpr (MTM >= 2) run_tile<FMT, 2, KIND>(P, smem, g, row0, rows, n0, tk);
+                if constexpr (MTM >= 2) run_tile<FMT, 2, KIND>(P, smem, g, row0, rows, n0, tk, deep);
                 break;
             case 3:
-                if constexpr (MTM >= 3) run_tile<FMT, 3, KIND>(P, smem, g, row0, rows, n0, tk);
+                if constexpr (MTM >= 3) run_tile<FMT, 3, KIND>(P, smem, g, row0, rows, n0, tk, deep);
                 break;
             case 4:
-                if constexpr (MTM >= 4) run_tile<FMT, 4, KIND>(P, smem, g, row0, rows, n0, tk);
+                if constexpr (MTM >= 4) run_tile<FMT, 4, KIND>(P, smem, g, row0, rows, n0, tk, deep);
                 break;
             case 5:
-                if constexpr (MTM >= 5) run_tile<FMT, 5, KIND>(P, smem, g, row0, rows, n0, tk);
+                if constexpr (MTM >= 5) run_tile<FMT, 5, KIND>(P, smem, g, row0, rows, n0, tk, deep);
                 break;
             case 6:
-                if constexpr (MTM >= 6) run_tile<FMT, 6, KIND>(P, smem, g, row0, rows, n0, tk);
+                if constexpr (MTM >= 6) run_tile<FMT, 6, KIND>(P, smem, g, row0, rows, n0, tk, deep);
                 break;
             case 7:
-                if constexpr (MTM >= 7) run_tile<FMT, 7, KIND>(P, smem, g, row0, rows, n0, tk);
+                if constexpr (MTM >= 7) run_tile<FMT, 7, KIND>(P, smem, g, row0, rows, n0, tk, deep);
                 break;
             case 8:
-                if constexpr (MTM >= 8) run_tile<FMT, 8, KIND>(P, smem, g, row0, rows, n0, tk);
+                if constexpr (MTM >= 8) run_tile<FMT, 8, KIND>(P, smem, g, row0, rows, n0, tk, deep);
                 break;
             case 9:
-                if constexpr (MTM >= 9) run_tile<FMT, 9, KIND>(P, smem, g, row0, rows, n0, tk);
+                if constexpr (MTM >= 9) run_tile<FMT, 9, KIND>(P, smem, g, row0, rows, n0, tk, deep);
                 break;
             case 10:
-                if constexpr (MTM >= 10) run_tile<FMT, 10, KIND>(P, smem, g, row0, rows, n0, tk);
+                if constexpr (MTM >= 10) run_tile<FMT, 10, KIND>(P, smem, g, row0, rows, n0, tk, deep);
                 break;
             default: have_ticket = false; break;
         }

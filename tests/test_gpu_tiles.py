@@ -224,3 +224,19 @@ def test_long_launches_order_their_experts(fmt, G, K, N, kernel):
     torch.cuda.synchronize()
     assert max(works) < limit <= work
     assert torch.equal(whole, torch.cat(halves)) and not bool((whole == 0x7FC0).any())
+
+
+@pytest.mark.parametrize("K", [128, 256, 384, 512, 640, 896])   # 4, 8, 12, 16, 20 and 28 steps of 32 k
+@pytest.mark.parametrize("fmt", ["int4", "fp4"])
+def test_small_tiles_in_the_longer_ring(fmt, K):
+    """GK_QUAD gives tiles of up to 48 rows six stages where a workgroup gets more than one tile: every row count up to two beyond."""
+    counts = list(range(1, 51)) + [0, 48, 33, 16] + [17] * 12
+    N = 2048
+    _say(f"small tiles in the longer ring {fmt} K={K}")
+    case = H.make_case(fmt, len(counts), K, N, np.cumsum(counts), seed=K, extra_rows=3)
+    assert H.kernel_of(case, "gemm") == "tiles_quad"
+    assert sum(c > 0 for c in counts) * (N // 256) > 512, "more tiles than workgroups"
+    used = int(case["group_list"][-1])
+    got = H.run_cabi(case, H.upload(case), "gemm")
+    H.assert_close(got, H.oracle_out(case), rows=slice(0, used), what=f"{fmt} K={K}")
+    assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
