@@ -30,6 +30,7 @@
 // column i and rows 4q..4q+3.  The contraction index may be permuted freely as long
 // as A and B agree, and so may the column <-> (MFMA, lane) assignment; each weight
 // container picks the assignment that makes its global loads wide and contiguous.
+#include <algorithm>
 #include <type_traits>
 
 #include "moe_device.h"
@@ -59,6 +60,7 @@ struct GemmParams {
     int table_mode;
     // N-contiguous 4-bit containers: turns a 32-k sub-step index into its scale row
     ScaleRowDivider scale_div;
+    int nt;   // nontemporal weight loads, see NT_MIN_BYTES
 };
 
 // Work queue of the persistent grid.  Workgroups do not run at one speed (of two that share a CU the one
@@ -179,8 +181,11 @@ __device__ __forceinline__ void lds_load16(rsrc_t r, const u32x4_t* dst, int vof
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)MOE_LDS_PTR(p));
 }
+// AUX: LOAD_NT, or 0.
+constexpr int LOAD_NT = 2;   // nontemporal
+template <int AUX = 0>
 __device__ __forceinline__ void lds_load16_at(rsrc_t r, uint32_t dst, int voff, int soff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(uintptr_t)dst, 16, voff, soff, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(uintptr_t)dst, 16, voff, soff, 0, AUX);
 }
 // A wave-uniform value the compiler must take as it finds it: whatever is derived from the result is computed
 // where it is used instead of once per variant ahead of an unrolled loop (where it would occupy an SGPR each).
@@ -307,6 +312,17 @@ constexpr int pair_kc_scale_units() { return (FMT == MOE_FMT_FP4_B32 || FMT == M
 // each on 128 experts 327 / 331).  A launch with a tile per workgroup at most keeps 4: it gains nothing from more and pays for fetching
 // the code of the longer ring (416 rows on 16 of 3328 x 2048: 42.0 / 43.2).  The one-byte containers are here for experts of many rows.
 constexpr int QUAD_DEEP_MT = 3, QUAD_DEEP_STAGES = 6;
+// Nontemporal weight loads.  A weight line that is read once in a launch, whole, only pushes others out of L2 and the 256 MB behind
+// it.  So: the N-contiguous containers on GK_PAIR and the small-stage kinds, in tiles that hold all rows of their expert (GK_PAIR: 4 row
+// blocks, an expert in several chunks has 5 or more in each; small stages: one row block, nearly always), in launches that read more
+// weights than those caches can keep for the next launch that reads them.  us, without / with: GEMV op, 512 rows on 128 experts of 7168 x
+// 2048, fp8 307 / 270, on 256, int4 311 / 292, fp4 359 / 331; GEMM op, 512 rows on 256, fp4 374 / 355, int4 350 / 336; fp8, 128 rows on
+// 64 of 2048 x 1024 28.0 / 25.5, 1024 on 256 of 7168 x 2048 599 / 562; int8, 800 on 64 of 4096 x 4096 191 / 182.  Weights that
+// the caches still hold from the last time are faster read as usual: 84 MB of fp8 18.6 / 22.0, 67 MB of int4 21.3 / 21.6; 134 MB of
+// int4 39.3 / 37.2, 126 MB of fp4 33.3 / 31.2.  With row chunks that share their weights 256 rows of 8 experts, int8: 456 / 501; bf16, whose lines are
+// read in halves: 485 / 586; GK_QUAD gains nothing (int4, 16 rows each on 256 experts 476 / 470, fp4 unevenly routed 540 / 540).
+constexpr int64_t NT_MIN_BYTES = 96 << 20;
+constexpr int nt_mt_max(int kind) { return kind == GK_PAIR ? 4 : kind == GK_QUAD ? 0 : 1; }
 template <int FMT>
 constexpr int pair_lds_units(int kind) {
     return pair_stages<FMT>(kind) * (pair_a_units(kind) + pair_b_units<FMT>(kind) + pair_sc_units<FMT>(kind)) + pair_kc_scale_units<FMT>();
@@ -429,8 +445,8 @@ __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, 
 // scale of its own group, and the two halves are added once at the end of the tile: half the MFMAs and half
 // the multiplies of the general case, and no masking.
 //
-// DEEP (GK_QUAD, small tiles): the longer ring, see QUAD_DEEP_STAGES.
-template <int FMT, int MT, int KIND, bool STACK2 = false, bool DEEP = false>
+// DEEP (GK_QUAD, small tiles): the longer ring, see QUAD_DEEP_STAGES.  NT: nontemporal loads of the weights, see NT_MIN_BYTES.
+template <int FMT, int MT, int KIND, bool STACK2 = false, bool DEEP = false, bool NT = false>
 __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk) {
     static_assert(FMT != MOE_FMT_BF16, "the k-split tile routine decodes quantized containers");
     constexpr bool EXACT = pair_exact(KIND);
@@ -460,6 +476,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     // The next step's packed dwords are read ahead of the MFMAs instead of behind the first ones: with 4 or 8 MFMAs a step their
     // latency otherwise ends in the next decode (int4, a tile per CU, 2 rows: 64 experts of 2048 x 1024 22.6 / 21.3 us).
     // fp4 gains nothing from it, the GEMV op's kinds lose 0.5 to 4 %: they still need the scales of the step being multiplied.
+    constexpr int W_AUX = NT ? LOAD_NT : 0;   // (fp4: of the scales too, whose rows are read once; those of int4 serve four steps)
     constexpr bool EARLY_RAW = FMT == MOE_FMT_INT4 && KIND == GK_PAIR_SMALL;
     static_assert(S * (PAIR_A_UNITS + PAIR_B_UNITS + PAIR_SC_UNITS) <= pair_lds_units<FMT>(KIND), "stages beyond the LDS of the kernel");
     static_assert(16 * MT * (BK / 8) <= PAIR_A_UNITS, "tile rows beyond the x stage");
@@ -569,7 +586,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             lds_load16_at(rx, here(a_at[m]) + ST * (PAIR_A_UNITS * 16), va, ca[m] + (kt + AHEAD) * (BK * 2));
         } else if (m < NA + NB) {
             const int e = m - NA;
-            lds_load16_at(rw, here(b_at) + ST * (PAIR_B_UNITS * 16) + e * 1024, vb,
+            lds_load16_at<W_AUX>(rw, here(b_at) + ST * (PAIR_B_UNITS * 16) + e * 1024, vb,
                           cb + (B8 ? 4 * e * P.N : 0) + b_step_offset(kt + AHEAD));
         } else if constexpr (KC) {
             kc_issue_scale(kt + KC_D);
@@ -583,7 +600,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             const int grow = FP4  ? (kt + AHEAD) * (Q4 ? 2 : 4) + (wv >> 1)
                              : Q4 ? scale_row((uint32_t)(kt + AHEAD))
                                   : scale_row((uint32_t)((kt + AHEAD) * 2 + (wv >> 2)));
-            if (s_lane) lds_load16_at(rs, here(s_at) + ST * (PAIR_SC_UNITS * 16), lane16, grow * (P.N * 2) + cs);
+            if (s_lane) lds_load16_at<FP4 ? W_AUX : 0>(rs, here(s_at) + ST * (PAIR_SC_UNITS * 16), lane16, grow * (P.N * 2) + cs);
         }
     };
     auto issue_group = [&](int kt, int ST) {
@@ -1583,6 +1600,8 @@ struct KernelCfg {
     static constexpr bool ORDERED = KIND == GK_QUAD || KIND == GK_FP4_K || (KIND == GK_PAIR && (FMT == MOE_FMT_INT8 || FMT == MOE_FMT_FP8_REF));
     // ... in launches of at least that many tiles (an upper bound) times k
     static constexpr int64_t ORDER_MIN_WORK = KIND == GK_PAIR ? 3 << 20 : 1 << 19;
+    // tiles of mt row blocks have a form with nontemporal weight loads
+    static constexpr bool nontemporal(int mt) { return PAIR && FMT != MOE_FMT_FP4_B32 && FMT != MOE_FMT_FP4_B16 && mt <= nt_mt_max(KIND); }
     // 16-byte LDS units of the tile routine (the tile prefix array follows them)
     static constexpr int lds_units() {
         if constexpr (PAIR)
@@ -1596,6 +1615,14 @@ template <int FMT, int MT, int KIND>
 __device__ __forceinline__ void run_tile(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk, bool deep) {
     using C = KernelCfg<FMT, KIND>;
     if constexpr (C::PAIR) {
+        if constexpr (C::nontemporal(MT)) {
+            if (P.nt) {
+                if constexpr (FMT == MOE_FMT_FP4_REF && pair_exact(KIND)) {
+                    if (rows <= 8) return gemm_tile_pair<FMT, MT, KIND, true, false, true>(P, smem, g, row0, rows, n0, tk);
+                }
+                return gemm_tile_pair<FMT, MT, KIND, false, false, true>(P, smem, g, row0, rows, n0, tk);
+            }
+        }
         if constexpr (KIND == GK_QUAD && MT <= QUAD_DEEP_MT && (FMT == MOE_FMT_INT4 || FMT == MOE_FMT_FP4_REF)) {
             if (deep) return gemm_tile_pair<FMT, MT, KIND, false, true>(P, smem, g, row0, rows, n0, tk);
         }
@@ -1936,6 +1963,8 @@ static GemmParams gemm_params(const moe_grouped_args* a) {
     P.y = static_cast<uint16_t*>(a->y);
     P.M = a->M; P.K = (int)a->K; P.N = (int)a->N; P.G = (int)a->G; P.scale_rows = (int)a->scale_rows;
     P.epilogue = a->epilogue;
+    const bool byte = a->format == MOE_FMT_INT8 || a->format == MOE_FMT_FP8_REF;
+    P.nt = std::min(a->M, a->G) * (a->K * a->N >> (byte ? 0 : 1)) >= NT_MIN_BYTES;
     P.slot = -1;
     P.stamp = 0;
     P.table_mode = 0;
