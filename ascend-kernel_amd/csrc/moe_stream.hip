@@ -142,6 +142,15 @@ static __device__ __forceinline__ void stream_rows(const StreamParams& P, float*
     for (int t = 0; t < T; ++t) acc[t] = zero;
 
     auto consume = [&](const StreamStep<FMT, T>& d) {
+        // the two codes of byte `byte` of word
+        auto fp4_pair = [](uint32_t word, int byte, float s) {
+            switch (byte) {
+                case 0: return ROUNDW ? e2m1_pair_scaled_bf16<0>(word, s) : __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, 1.f, 0));
+                case 1: return ROUNDW ? e2m1_pair_scaled_bf16<1>(word, s) : __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, 1.f, 1));
+                case 2: return ROUNDW ? e2m1_pair_scaled_bf16<2>(word, s) : __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, 1.f, 2));
+                default: return ROUNDW ? e2m1_pair_scaled_bf16<3>(word, s) : __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, 1.f, 3));
+            }
+        };
         auto scale_of = [](const uint32_t (&s)[T / 2], int t) { return (t & 1) ? bf16_hi(s[t >> 1]) : bf16_lo(s[t >> 1]); };
         f32x4_t start = zero;
         if constexpr (I4 && !ROUNDW) {   // the fragments hold q: every product starts from -8 sum_k x
@@ -163,6 +172,24 @@ static __device__ __forceinline__ void stream_rows(const StreamParams& P, float*
 #pragma unroll
             for (int t = 0; t < TH; ++t) sc[t] = F8 ? f8s : I8 ? 1.f : scale_of(d.s, t0 + t);
             const uint32_t b0 = T == 8 ? (B8 ? 0u : t0 >> 1) : byte0;
+            // fp4, two or four columns: the lane's bytes of even and of odd k rows are gathered first, two or four row pairs to a dword,
+            // and only they are paired up, the nibbles of two rows in a byte: 10 and 12 instructions for 16 and 32 weights where
+            // pairing whole dwords and shifting took 28
+            uint32_t even_col[2] = {0u, 0u}, odd_col[2] = {0u, 0u};   // T == 4: of row pairs 0 and 1, 2 and 3
+            if constexpr (FP4 && T < 8) {
+                auto pair_up = [&](uint32_t even, uint32_t odd, int e) {
+                    const uint32_t m = 0x0f0f0f0fu;
+                    even_col[e] = (even & m) | ((odd << 4) & ~m);
+                    odd_col[e] = ((even >> 4) & m) | (odd & ~m);
+                };
+                auto gather = [&](int hi, int lo) { return __builtin_amdgcn_perm(d.r[hi], d.r[lo], T == 2 ? b0 | ((4u + b0) << 8) | 0x0c0c0000u : b0 | ((b0 + 1u) << 8) | ((4u + b0) << 16) | ((b0 + 5u) << 24)); };
+                if constexpr (T == 2) {
+                    pair_up(__builtin_amdgcn_perm(gather(6, 4), gather(2, 0), 0x05040100u), __builtin_amdgcn_perm(gather(7, 5), gather(3, 1), 0x05040100u), 0);
+                } else {
+                    pair_up(gather(2, 0), gather(3, 1), 0);
+                    pair_up(gather(6, 4), gather(7, 5), 1);
+                }
+            }
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
                 // the dwords of k rows 2 p and 2 p + 1
@@ -182,18 +209,18 @@ static __device__ __forceinline__ void stream_rows(const StreamParams& P, float*
                                                                           : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h[t & 1], 512.f, true));
                         }
                     }
+                } else if constexpr (FP4 && T == 2) {
+                    bf[0][p] = fp4_pair(even_col[0], p, sc[0]);
+                    bf[1][p] = fp4_pair(odd_col[0], p, sc[1]);
+                } else if constexpr (FP4 && T == 4) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) bf[t][p] = fp4_pair(t & 1 ? odd_col[p >> 1] : even_col[p >> 1], 2 * (p & 1) + (t >> 1), sc[t]);
                 } else if constexpr (FP4) {
                     // nibbles of the two rows paired in a byte: even, odd columns
                     const uint32_t m = 0x0f0f0f0fu;
                     const uint32_t h[2] = {((a & m) | ((b << 4) & ~m)) >> (8 * b0), (((a >> 4) & m) | (b & ~m)) >> (8 * b0)};
 #pragma unroll
-                    for (int t = 0; t < TH; ++t) {
-                        if constexpr (ROUNDW)
-                            bf[t][p] = t < 2 ? e2m1_pair_scaled_bf16<0>(h[t & 1], sc[t]) : e2m1_pair_scaled_bf16<1>(h[t & 1], sc[t]);
-                        else
-                            bf[t][p] = __builtin_bit_cast(uint32_t, t < 2 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(h[t & 1], 1.f, 0)
-                                                                          : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(h[t & 1], 1.f, 1));
-                    }
+                    for (int t = 0; t < TH; ++t) bf[t][p] = fp4_pair(h[t & 1], t >> 1, sc[t]);
                 } else {
 #pragma unroll
                     for (int t = 0; t < TH; ++t) {

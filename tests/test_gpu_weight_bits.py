@@ -111,3 +111,34 @@ def test_fp8_gemv(rows, codes):
     assert H.kernel_of(case, "gemv") == "tiles_pair_exact"
     got, want = H.run_cabi(case, H.upload(case), "gemv"), H.oracle_out(case, gemv=True)
     assert np.array_equal(oracle.bf16_bits_to_f32(got), oracle.bf16_bits_to_f32(want)), at
+
+
+# kernel, experts, K, N, rows per expert
+FP4 = [("strips_32", 4, 256, 512, 16), ("strips_32", 2, 1088, 256, 5), ("strips_64", 6, 256, 2048, 16), ("strips_128", 10, 256, 2048, 12),
+       ("tiles_pair_small", 20, 256, 2048, 12), ("tiles_quad", 2, 256, 256, 256)]
+
+
+@pytest.mark.parametrize("kernel,G,K,N,rows", FP4)
+def test_fp4(kernel, G, K, N, rows):
+    _say(f"fp4 weight bits {kernel}")
+    rng = np.random.default_rng(G + N)
+    case = H.make_case("fp4", G, K, N, np.arange(1, G + 1) * rows, seed=G)
+    case["scale"] = _scales(rng, case["scale"].shape, -110, 117)
+    _check(case, _unit_rows(case, rng), kernel)
+
+
+@pytest.mark.parametrize("rows", [1, 8, 9, 16])
+@pytest.mark.parametrize("kernel,G,N", [("strips_32", 4, 512), ("strips_64", 6, 2048), ("strips_128", 10, 2048)])
+def test_fp4_gemv_strips(kernel, G, N, rows):
+    """The GEMV op's weights are not rounded: with scales of powers of two bf16 holds them."""
+    _say(f"fp4 gemv weight bits {kernel}, {rows} rows")
+    if rows > 12 and kernel == "strips_128":
+        rows = 12
+    rng = np.random.default_rng(G + rows)
+    K = 256
+    case = H.make_case("fp4", G, K, N, np.arange(1, G + 1) * rows, seed=rows)
+    case["scale"] = ((rng.integers(-60, 60, case["scale"].shape) + 127) << 7).astype(np.uint16)
+    at = _unit_rows(case, rng)
+    assert H.kernel_of(case, "gemv") == kernel
+    got, want = H.run_cabi(case, H.upload(case), "gemv"), H.oracle_out(case, gemv=True)
+    assert np.array_equal(oracle.bf16_bits_to_f32(got), oracle.bf16_bits_to_f32(want)), at
