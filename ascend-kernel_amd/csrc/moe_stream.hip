@@ -5,10 +5,9 @@
 // (a barrier each), and 8 rows of 8 experts with N = 512 make 16 of those tiles for 256 CUs.  Here a workgroup takes 16 T
 // columns (32, 64 or 128) of one expert and its wavefronts split K between them: each streams its own range into registers,
 // a few 32-k steps ahead, without LDS or barriers, and the partial sums meet once in LDS.  That case (18 MB of fp4 weights and
-// scales): 47.6 -> 11.2 us, int4 48 -> 15, fp8 70 -> 16; two tokens on 256 experts of 7168 x 2048: int4 49 -> 33 us.
+// scales): 47.6 -> 9.6 us, int4 48 -> 12.6, fp8 70 -> 16; two tokens on 256 experts of 7168 x 2048: int4 49 -> 33 us.
 // What bounds it now: the launch, group_list and one step's latency are about 6 us; then what a few wavefronts per SIMD
-// issue (about 1.5 vector instructions per weight, 3.2 in 32-column strips, where four lanes load a dword of 8 codes
-// and use two of them; half of a wavefront's time there is waiting for its loads).
+// issue (about 1.5 vector instructions per weight, 1.75 in 32-column strips of fp4) and the CU's vector memory path.
 //
 // MFMA: v_mfma_f32_16x16x32_bf16, x rows in A, weights in B.  Lane (i, q) = (lane & 15, lane >> 4) loads, of each of the 8 k
 // rows 8 q + [0, 8) of a step, the dword (T = 8 and bytes: two) with its columns T i + [0, T): the 8 values of one column are
@@ -49,10 +48,20 @@ static __device__ __forceinline__ f32x4_t mfma(const u32x4_t& a, const u32x4_t& 
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
+// 4-bit codes, two columns a lane: the four lanes of a quad use a byte each of the same dwords.  A lane that loads all 8 rows of its
+// dword loads four times what it uses, and the CU's vector memory path (64 bytes a cycle) is what such a launch then waits for as much
+// as for instruction issue.  So each lane of a quad loads two rows, and a 4 x 4 byte transpose over the quad (two DPP moves and two
+// v_perm per dword) gives every lane its byte of all eight.  us, without / with: 8 single rows of 7168 x 512, fp4 GEMV op 10.5 / 9.6,
+// GEMM op 11.2 / 10.5, int4 14.5 / 12.9; 192 rows on 8 experts of 4096 x 1024, fp4 15.1 / 13.4.  (Six or eight steps in flight instead of
+// four in the registers that this frees: 0 to 2 % faster with fp4 and K = 7168, 2 to 11 % slower otherwise.  16 wavefronts: 0.88 to 1.02 times.)
+template <int FMT, int T>
+constexpr bool stream_quad() { return T == 2 && (FMT == MOE_FMT_FP4_REF || FMT == MOE_FMT_INT4); }
+
 template <int FMT, int T>
 struct StreamStep {   // what a wavefront holds of one 32-k step
-    // k row j: the dword that holds this lane's columns; 8 columns of bytes: r[2 j] and r[2 j + 1]
-    uint32_t r[T == 8 && (FMT == MOE_FMT_INT8 || FMT == MOE_FMT_FP8_REF) ? 16 : 8];
+    // k row j: the dword that holds this lane's columns; 8 columns of bytes: r[2 j] and r[2 j + 1]; stream_quad: lane l of a quad
+    // holds the quad's dwords of rows 2 l and 2 l + 1
+    uint32_t r[stream_quad<FMT, T>() ? 2 : T == 8 && (FMT == MOE_FMT_INT8 || FMT == MOE_FMT_FP8_REF) ? 16 : 8];
     u32x4_t x;
     uint32_t s[T / 2], s2[T / 2];   // scales of the T columns (fp8: s[0]); s2: fp4 without rounding, the second 16 k's
 };
@@ -64,6 +73,7 @@ static __device__ __forceinline__ void stream_rows(const StreamParams& P, float*
     constexpr bool FP4 = FMT == MOE_FMT_FP4_REF, F8 = FMT == MOE_FMT_FP8_REF, I8 = FMT == MOE_FMT_INT8, I4 = FMT == MOE_FMT_INT4;
     constexpr bool B8 = F8 || I8;
     constexpr int ST_COLS = 16 * T;
+    constexpr bool QUAD = stream_quad<FMT, T>();
     constexpr bool TWO = FP4 && !ROUNDW && !STACK;   // two MFMAs per 32 k and column, one per scale
     // steps in flight (6, or 3 for 128 columns, change nothing; three where a fourth does not fit 128 registers)
     constexpr int D = FP4 && !ROUNDW && T == 4 ? 3 : 4;
@@ -81,9 +91,16 @@ static __device__ __forceinline__ void stream_rows(const StreamParams& P, float*
     const int vx = STACK ? ((i >> 3) == (q >> 1) ? (i & 7) * P.K * 2 + q * 16 : 0x40000000) : i * P.K * 2 + q * 16;
     const int row_bytes = B8 ? P.N : P.N >> 1;
     const int col = n0 + T * i;   // this lane's first column
-    const int vw = FP4  ? (32 * (q & 1) + 8 * (q >> 1) + ((col >> 5) & 7)) * row_bytes + ((col >> 8) << 7) + 32 * ((col >> 3) & 3)
+    const int ql = lane & 3;   // QUAD: which two of the 8 k rows this lane loads
+    const int vw = FP4  ? (QUAD ? 8 * ql : 0) + (32 * (q & 1) + 8 * (q >> 1) + ((col >> 5) & 7)) * row_bytes + ((col >> 8) << 7) + 32 * ((col >> 3) & 3)
                    : B8 ? 8 * q * row_bytes + (col & ~3)
-                        : 8 * q * row_bytes + ((col >> 3) << 2);
+                        : (8 * q + (QUAD ? 2 * ql : 0)) * row_bytes + ((col >> 3) << 2);
+    // QUAD: byte l of the dwords v of the quad's four lanes, in lane l
+    const uint32_t quad_sel1 = ql & 1 ? 0x03070105u : 0x06020400u, quad_sel2 = ql & 2 ? 0x03020706u : 0x05040100u;
+    auto quad_transpose = [&](uint32_t v) {
+        const uint32_t h = __builtin_amdgcn_perm((uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, true), v, quad_sel1);      // lane l ^ 1
+        return __builtin_amdgcn_perm((uint32_t)__builtin_amdgcn_mov_dpp((int)h, 0x4e, 0xf, 0xf, true), h, quad_sel2);   // lane l ^ 2
+    };
     const int vs = FP4 && !TWO ? (q >> 1) * (P.N * 2) + col * 2 : col * 2;
     const uint32_t byte0 = B8 ? col & 3 : (col & 7) >> 1;   // the byte of a dword this lane's columns start at
 
@@ -113,15 +130,21 @@ static __device__ __forceinline__ void stream_rows(const StreamParams& P, float*
         d.x = __builtin_amdgcn_raw_buffer_load_b128(rx, vx, s * 64, 0);
         if constexpr (FP4) {
             const int so = ((s >> 1) * 64 + (s & 1) * 16) * row_bytes;
-            const u32x4_t lo = __builtin_amdgcn_raw_buffer_load_b128(rw, vw, so, 0);
-            const u32x4_t hi = __builtin_amdgcn_raw_buffer_load_b128(rw, vw + 16, so, 0);
+            if constexpr (QUAD) {
+                const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(rw, vw, so, 0);
+                d.r[0] = v[0];
+                d.r[1] = v[1];
+            } else {
+                const u32x4_t lo = __builtin_amdgcn_raw_buffer_load_b128(rw, vw, so, 0);
+                const u32x4_t hi = __builtin_amdgcn_raw_buffer_load_b128(rw, vw + 16, so, 0);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) { d.r[j] = lo[j]; d.r[4 + j] = hi[j]; }
+                for (int j = 0; j < 4; ++j) { d.r[j] = lo[j]; d.r[4 + j] = hi[j]; }
+            }
             load_scales(d.s, 2 * s * (P.N * 2));
             if constexpr (TWO) load_scales(d.s2, (2 * s + 1) * (P.N * 2));
         } else {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
+            for (int j = 0; j < (QUAD ? 2 : 8); ++j) {
                 if constexpr (B8 && T == 8) {
                     const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(rw, vw, (32 * s + j) * row_bytes, 0);
                     d.r[2 * j] = v[0];
@@ -172,29 +195,56 @@ static __device__ __forceinline__ void stream_rows(const StreamParams& P, float*
 #pragma unroll
             for (int t = 0; t < TH; ++t) sc[t] = F8 ? f8s : I8 ? 1.f : scale_of(d.s, t0 + t);
             const uint32_t b0 = T == 8 ? (B8 ? 0u : t0 >> 1) : byte0;
-            // fp4, two or four columns: the lane's bytes of even and of odd k rows are gathered first, two or four row pairs to a dword,
-            // and only they are paired up, the nibbles of two rows in a byte: 10 and 12 instructions for 16 and 32 weights where
-            // pairing whole dwords and shifting took 28
+            // fp4, two or four columns: the lane's bytes of even and of odd k rows are gathered first, two or four row pairs to a dword
+            // (QUAD: from the quad's lanes), and only they are paired up, the nibbles of two rows in a byte.  (Pairing whole dwords and
+            // shifting took 28 instructions for 16 or 32 weights, this takes 12.)
             uint32_t even_col[2] = {0u, 0u}, odd_col[2] = {0u, 0u};   // T == 4: of row pairs 0 and 1, 2 and 3
+            uint32_t even_rows = 0u, odd_rows = 0u;                   // QUAD: the lane's bytes of rows 0, 2, 4, 6 and 1, 3, 5, 7
+            if constexpr (QUAD) {
+                even_rows = quad_transpose(d.r[0]);
+                odd_rows = quad_transpose(d.r[1]);
+            }
             if constexpr (FP4 && T < 8) {
                 auto pair_up = [&](uint32_t even, uint32_t odd, int e) {
                     const uint32_t m = 0x0f0f0f0fu;
                     even_col[e] = (even & m) | ((odd << 4) & ~m);
                     odd_col[e] = ((even >> 4) & m) | (odd & ~m);
                 };
-                auto gather = [&](int hi, int lo) { return __builtin_amdgcn_perm(d.r[hi], d.r[lo], T == 2 ? b0 | ((4u + b0) << 8) | 0x0c0c0000u : b0 | ((b0 + 1u) << 8) | ((4u + b0) << 16) | ((b0 + 5u) << 24)); };
-                if constexpr (T == 2) {
-                    pair_up(__builtin_amdgcn_perm(gather(6, 4), gather(2, 0), 0x05040100u), __builtin_amdgcn_perm(gather(7, 5), gather(3, 1), 0x05040100u), 0);
+                if constexpr (QUAD) {
+                    pair_up(even_rows, odd_rows, 0);
                 } else {
-                    pair_up(gather(2, 0), gather(3, 1), 0);
-                    pair_up(gather(6, 4), gather(7, 5), 1);
+                    const uint32_t sel = b0 | ((b0 + 1u) << 8) | ((4u + b0) << 16) | ((b0 + 5u) << 24);
+                    pair_up(__builtin_amdgcn_perm(d.r[2], d.r[0], sel), __builtin_amdgcn_perm(d.r[3], d.r[1], sel), 0);
+                    pair_up(__builtin_amdgcn_perm(d.r[6], d.r[4], sel), __builtin_amdgcn_perm(d.r[7], d.r[5], sel), 1);
+                }
+            }
+            // int4, two columns: (even row, odd row) per byte, row pairs 0 and 1, 2 and 3; a nibble read as e4m3 is q / 512
+            uint32_t quad_q[2][2] = {{0u, 0u}, {0u, 0u}};   // [even, odd column][row pairs]
+            if constexpr (I4 && QUAD) {
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const uint32_t u = __builtin_amdgcn_perm(odd_rows, even_rows, e ? 0x07030602u : 0x05010400u);
+                    quad_q[0][e] = u & 0x0f0f0f0fu;
+                    quad_q[1][e] = (u >> 4) & 0x0f0f0f0fu;
                 }
             }
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
                 // the dwords of k rows 2 p and 2 p + 1
-                const uint32_t a = B8 && T == 8 ? d.r[4 * p + (t0 >> 2)] : d.r[2 * p], b = B8 && T == 8 ? d.r[4 * p + 2 + (t0 >> 2)] : d.r[2 * p + 1];
-                if constexpr (I4) {
+                const uint32_t a = QUAD ? 0u : B8 && T == 8 ? d.r[4 * p + (t0 >> 2)] : d.r[2 * p], b = QUAD ? 0u : B8 && T == 8 ? d.r[4 * p + 2 + (t0 >> 2)] : d.r[2 * p + 1];
+                if constexpr (I4 && QUAD) {
+#pragma unroll
+                    for (int t = 0; t < TH; ++t) {
+                        const uint32_t h = quad_q[t][p >> 1];
+                        if constexpr (ROUNDW) {
+                            const f32x2_t f = p & 1 ? __builtin_amdgcn_cvt_pk_f32_fp8(h, true) : __builtin_amdgcn_cvt_pk_f32_fp8(h, false);
+                            bf[t][p] = pack_bf16_rne(fmaf(f[0], 512.f * sc[t], -8.f * sc[t]), fmaf(f[1], 512.f * sc[t], -8.f * sc[t]));
+                        } else {
+                            bf[t][p] = __builtin_bit_cast(uint32_t, p & 1 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h, 512.f, true)
+                                                                          : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h, 512.f, false));
+                        }
+                    }
+                } else if constexpr (I4) {
                     // the lane's bytes of the two rows side by side, (a, b) per byte; a nibble read as e4m3 is q / 512
                     const uint32_t sel = b0 | ((4u + b0) << 8) | (T >= 4 ? ((b0 + 1u) << 16) | ((b0 + 5u) << 24) : 0x0c0c0000u);
                     const uint32_t u = __builtin_amdgcn_perm(b, a, sel);
