@@ -72,7 +72,7 @@ def test_fp4_rows(fmt, G, K, rows):
 
 
 # kernel, experts, K, N, rows per expert
-FP8 = [("strips_32", 4, 256, 512, 16), ("strips_128", 10, 256, 2048, 12), ("tiles_pair", 20, 256, 2048, 40), ("tiles_pair", 4, 384, 384, 160),
+FP8 = [("strips_32", 4, 256, 512, 16), ("strips_64", 6, 256, 2048, 16), ("strips_128", 10, 256, 2048, 12), ("tiles_pair", 20, 256, 2048, 40), ("tiles_pair", 4, 384, 384, 160),
        ("tiles_quad", 2, 256, 256, 256)]
 
 
@@ -94,12 +94,13 @@ def test_fp8(kernel, G, K, N, rows, codes):
 
 
 @pytest.mark.parametrize("codes", ["without", "some", "all"])
-@pytest.mark.parametrize("rows", [3, 16, 17, 40])
-def test_fp8_gemv(rows, codes):
+@pytest.mark.parametrize("kernel,G,N,rows", [("tiles_pair_exact", 24, 2048, r) for r in (3, 16, 17, 40)]
+                         + [("strips_32", 4, 512, 5), ("strips_64", 6, 2048, 16), ("strips_128", 10, 2048, 12)])
+def test_fp8_gemv(kernel, G, N, rows, codes):
     """The same of the GEMV op, whose weights are not rounded: with scales of powers of two bf16 holds them."""
-    _say(f"fp8 gemv weight bits, {rows} rows, 0x7F: {codes}")
+    _say(f"fp8 gemv weight bits {kernel}, {rows} rows, 0x7F: {codes}")
     rng = np.random.default_rng(rows)
-    G, K, N = 24, 256, 2048
+    K = 256
     case = H.make_case("fp8", G, K, N, np.arange(1, G + 1) * rows, seed=rows)
     if codes != "all":
         case["weight"][(case["weight"] & 0x7F) == 0x7F] ^= 1
@@ -108,7 +109,7 @@ def test_fp8_gemv(rows, codes):
             case["weight"][g, rng.integers(0, K), rng.integers(0, N)] |= 0x7F
     case["scale"] = np.exp2(rng.integers(-60, 40, case["scale"].shape)).astype(np.float32)
     at = _unit_rows(case, rng)
-    assert H.kernel_of(case, "gemv") == "tiles_pair_exact"
+    assert H.kernel_of(case, "gemv") == kernel
     got, want = H.run_cabi(case, H.upload(case), "gemv"), H.oracle_out(case, gemv=True)
     assert np.array_equal(oracle.bf16_bits_to_f32(got), oracle.bf16_bits_to_f32(want)), at
 
