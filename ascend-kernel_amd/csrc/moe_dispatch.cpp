@@ -144,16 +144,27 @@ static GroupedKernel strip_width(const moe_grouped_args* a) {
     return columns(a) <= 8192 ? GroupedKernel::STRIPS_32 : columns(a) <= 16384 ? GroupedKernel::STRIPS_64 : GroupedKernel::STRIPS_128;
 }
 
+// GEMM op on the 4-bit containers: the small-stage kind (tiles of up to 32 rows, 8 wavefronts that split K, two workgroups per CU)
+// against the prefill kind (up to 160 rows, 4 wavefronts).  Times as fast, evenly and unevenly routed (skew 0.5; see bf16):
+//   12 rows per expert and fewer, always: 256 experts of 7168 x 2048, 4 rows int4 445 / 382 us, fp4 427 / 404, 12 rows 476 / 422 and 461 /
+//   441.  Beyond, it depends on the routing, as an expert of many rows is many passes over its weights: 16 rows, balanced top-k routing
+//   int4 483 / 425, fp4 464 / 451, skew 0.5 473 / 470 and 459 / 485, skew 1 354 / 401 and 359 / 418.
+//   Launches in which the prefill kind has a tile per CU at most: its 4 wavefronts are then alone there, and small tiles are
+//   more and fill it.  K = 4096, int4 and fp4.  Up to 128 tiles (8 experts of N = 2048 and 4096): 32 rows 1.4 - 1.5, 48 rows 1.3 - 1.9, 64
+//   and 96 rows 1.02 - 2.0 (not used: the bound stays where the gain is 1.3 and more).  192 and 256 tiles (12 and 16 experts of N =
+//   4096): 16 rows 1.2 - 1.7, 24 rows 1.17 - 1.7, 32 rows 0.97 - 1.7, 40 rows 0.91 - 1.19, 64 rows 0.83 - 1.18, 96 rows 0.61 - 1.05.
+static bool small_tiles_preferred(const moe_grouped_args* a) {
+    const int64_t tiles = std::min(a->M, a->G) * ((a->N + 255) / 256);
+    return a->M <= (tiles <= 128 ? 48 : tiles <= 256 ? 24 : 12) * a->G;
+}
+
 static GroupedKernel n_contiguous_kernel(const moe_grouped_args* a, bool gemv_op) {
     if (strips_preferred(a)) return strip_width(a);
-    // decode-like batches (on average at most 12 rows per expert) on the 4-bit containers: the small-stage kind (at 8 rows per
-    // expert int4 409 vs 506 us, fp4 448 vs 474 us; at 24 the large tiles win, 531 vs 549 us and 512 vs 609 us).  The
-    // one-byte containers gain nothing from it.  GEMV op, fp4: 16-row tiles, two workgroups per CU; an expert with more rows
-    // than that costs a pass over its weights per 16 rows.
-    const bool decode = a->M <= 12 * a->G;
-    if (gemv_op) return decode && a->format == MOE_FMT_FP4_REF ? GroupedKernel::TILES_PAIR_EXACT16 : GroupedKernel::TILES_PAIR_EXACT;
+    // GEMV op, fp4: 16-row tiles, two workgroups per CU, in decode-like batches (on average at most 12 rows per expert); an expert with
+    // more rows than that costs a pass over its weights per 16 rows.
+    if (gemv_op) return a->M <= 12 * a->G && a->format == MOE_FMT_FP4_REF ? GroupedKernel::TILES_PAIR_EXACT16 : GroupedKernel::TILES_PAIR_EXACT;
     const bool four_bit = a->format == MOE_FMT_INT4 || a->format == MOE_FMT_FP4_REF;
-    if (four_bit && decode) return GroupedKernel::TILES_PAIR_SMALL;
+    if (four_bit && small_tiles_preferred(a)) return GroupedKernel::TILES_PAIR_SMALL;
     // prefill: workgroups of 4 wavefronts without the k split, two per CU.  The 4-bit
     // ones always (256 experts of 128 rows, K = 7168, N = 4096: int4 1792 against 1905 us, fp4 1724 against 1867 us
     // with the k-split kind).  The one-byte ones, whose tiles move twice the bytes, when an expert has more rows than

@@ -264,3 +264,23 @@ def test_nontemporal_weights(op, fmt, G, K, N, spare):
     got = H.run_cabi(case, H.upload(case), op)
     H.assert_close(got, H.oracle_out(case, gemv=op == "gemv"), rows=slice(0, used), what=f"{op} {fmt}")
     assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
+
+
+@pytest.mark.parametrize("epilogue", ["none", "swiglu"])
+@pytest.mark.parametrize("fmt", ["int4", "fp4"])
+@pytest.mark.parametrize("G,N,rows,kernel", [(8, 4096, 48, "tiles_pair_small"), (8, 4096, 49, "tiles_quad"), (16, 4096, 24, "tiles_pair_small"),
+                                             (16, 4096, 25, "tiles_quad"), (17, 4096, 13, "tiles_quad"), (1, 256, 48, "tiles_pair_small")])
+def test_small_tiles_of_few_tile_launches(G, N, rows, kernel, fmt, epilogue):
+    """The bounds by rows per expert and tiles between the small-stage and the prefill kind, unevenly owned: experts of many chunks."""
+    K = 320
+    counts = [rows] * G
+    if G > 2:
+        counts[0], counts[1] = 0, 2 * rows
+    _say(f"{fmt} {kernel} {rows} rows on {G} experts {epilogue}")
+    case = H.make_case(fmt, G, K, N, np.cumsum(counts), seed=rows, group=32)
+    assert H.kernel_of(case, "gemm", swiglu=epilogue == "swiglu") == kernel
+    if epilogue == "swiglu":
+        got, want = _swiglu(case)
+    else:
+        got, want = H.run_cabi(case, H.upload(case), "gemm"), H.oracle_out(case)
+    H.assert_close(got, want, what=f"{fmt} {kernel} {epilogue}")
