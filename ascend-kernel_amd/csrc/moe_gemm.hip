@@ -127,6 +127,7 @@ struct Ticket {
     queue_word_t* counter;   // null: the caller draws the ticket itself
     int* out;
     int* arrivals;           // a word of LDS for the tile routine's arrival counter (see gemm_tile_pair)
+    int* wide;               // 5 words of LDS: not 0 if the tile is to be looked at again (see wide_scales), and its g, row0, rows, n0
 };
 
 // Buffer resources keep the addressing compact: one 128-bit descriptor in SGPRs per
@@ -226,7 +227,8 @@ __device__ __forceinline__ uint32_t here(uint32_t v) {
 // Decode of a k-row pair (a, b) of one dword column: v_perm gathers the two bytes of each row this lane owns, row a's
 // into the low, row b's into the high half of a dword.  Masked with 0x000f and put under 0x6400 a half is the fp16
 // 1024 + q (0x00f0: 1024 + 16 q), so v_fma_mix_f32 converts a weight and takes its scale and the zero point in one
-// instruction: (1024 + q) s - 1032 s, or (1024 + 16 q) s / 16 - 72 s, is (q - 8) s exactly (12 bits; scales below 2^117).
+// instruction: (1024 + q) s - 1032 s, or (1024 + 16 q) s / 16 - 72 s, is (q - 8) s exactly (12 bits).
+// From scales of 2^117.98 on 1032 s is beyond fp32 and the weight no number: see wide_scales.
 // 2.25 instructions per weight; masks, conversions from e4m3 and fmas took 2.5.  us, before / now: a prefill layer of 4096
 // tokens x 8 on 256 experts of 7168 x 2048 2883 / 2842, decode layers of 64 x 8 and 16 x 8 1059 / 998 and 413 / 391, 512 rows
 // on 64 experts of 2048 x 4096 122 / 117.
@@ -323,6 +325,12 @@ constexpr int QUAD_DEEP_MT = 3, QUAD_DEEP_STAGES = 6;
 // read in halves: 485 / 586; GK_QUAD gains nothing (int4, 16 rows each on 256 experts 476 / 470, fp4 unevenly routed 540 / 540).
 constexpr int64_t NT_MIN_BYTES = 96 << 20;
 constexpr int nt_mt_max(int kind) { return kind == GK_PAIR ? 4 : kind == GK_QUAD ? 0 : 1; }
+// int4 with rounded weights: the usual decode takes scales below 2^117.98.  A tile with a larger one has columns that are no number;
+// a wavefront that finds one in its sums says so in LDS (Ticket::wide), and the workgroup then looks whether such a scale is the
+// reason and if so computes the tile once more, 16 rows at a time, with a decode that takes all scales (redo_wide).  A check of the scales
+// in every step instead, three vector instructions and a branch, made decode-like launches 1.3 to 2.5 % slower, others 0.6 to 1.2 %.
+template <int FMT>
+constexpr bool wide_scales(int kind) { return FMT == MOE_FMT_INT4 && !pair_exact(kind); }
 template <int FMT>
 constexpr int pair_lds_units(int kind) {
     return pair_stages<FMT>(kind) * (pair_a_units(kind) + pair_b_units<FMT>(kind) + pair_sc_units<FMT>(kind)) + pair_kc_scale_units<FMT>();
@@ -446,7 +454,8 @@ __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, 
 // the multiplies of the general case, and no masking.
 //
 // DEEP (GK_QUAD, small tiles): the longer ring, see QUAD_DEEP_STAGES.  NT: nontemporal loads of the weights, see NT_MIN_BYTES.
-template <int FMT, int MT, int KIND, bool STACK2 = false, bool DEEP = false, bool NT = false>
+// WIDE: int4 with any scale, see wide_scales.
+template <int FMT, int MT, int KIND, bool STACK2 = false, bool DEEP = false, bool NT = false, bool WIDE = false>
 __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk) {
     static_assert(FMT != MOE_FMT_BF16, "the k-split tile routine decodes quantized containers");
     constexpr bool EXACT = pair_exact(KIND);
@@ -778,6 +787,20 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     };
     read_raw(0, 0);
 
+    // WIDE, k rows 2 p0 .. 2 p0 + 3 of the sub-step: q - 8 first (exact), then its product with the scale
+    auto decode_i4_wide = [&](int p0) __attribute__((always_inline)) {
+        const float s[4] = {bf16_lo(sc[0]), bf16_hi(sc[0]), bf16_lo(sc[1]), bf16_hi(sc[1])};
+#pragma unroll
+        for (int p = p0; p < p0 + 2; ++p) {
+            const uint32_t pr = __builtin_amdgcn_perm(r[2 * p + 1], r[2 * p], sel);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const uint32_t h4 = ((t < 2 ? pr : pr >> 8) & (t & 1 ? mask_hi : mask)) | magic;
+                const float one = t & 1 ? 0.0625f : 1.f, zero_point = t & 1 ? -72.f : -1032.f;
+                bf[t][p] = pack_bf16_rne(fp16_lo_fma(h4, one, zero_point) * s[t], fp16_hi_fma(h4, one, zero_point) * s[t]);
+            }
+        }
+    };
     // fp8, k rows 2 p0 .. 2 p0 + 3 of the sub-step.  decode_f8: byte t of the dwords of two k rows as a pair through fp16 (see
     // e4m3_ref_pair_over_256), where 0x7F and 0xFF are the reference's +-480; the 2^8 goes into the block scale.
     auto decode_f8 = [&](int p0) __attribute__((always_inline)) {
@@ -921,6 +944,11 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
                         }
                     }
                 }
+                __builtin_amdgcn_sched_barrier(0);
+                continue;
+            }
+            if constexpr (WIDE) {
+                decode_i4_wide(p0);
                 __builtin_amdgcn_sched_barrier(0);
                 continue;
             }
@@ -1122,6 +1150,21 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
         for (int t = 0; t < 4; ++t)
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[0][t][e] += __shfl_xor(acc[0][t][e], 32);
+    }
+    if constexpr (wide_scales<FMT>(KIND) && !WIDE) {
+        // a weight that is no number leaves none in its column, in any row: row block 0 tells (see redo_wide)
+        float bad[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(acc[0][t]));   // not read ahead of the wait above
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bad[e] = fmaf(acc[0][t][e], 0.f, bad[e]);
+        if (__any(__builtin_isnan((bad[0] + bad[1]) + (bad[2] + bad[3])))) [[unlikely]] {
+            if (lane == 0) {
+                tk.wide[0] = 1; tk.wide[1] = g; tk.wide[2] = (int)row0; tk.wide[3] = rows; tk.wide[4] = n0;
+            }
+        }
     }
     pair_finish<MT, KC, Q4>(P, smem, acc, h, cw, lane, col0, row0, rows, n0, tk);
 }
@@ -1637,6 +1680,32 @@ __device__ __forceinline__ void run_tile(const GemmParams& P, u32x4_t* smem, int
     }
 }
 
+// The tile that a wavefront has found columns in that are no number: if one of its scales is beyond what the usual decode takes, once
+// more with the decode that takes all (see wide_scales); else x is the reason.  The whole workgroup comes here together; tk draws no
+// ticket (the tile has drawn the next one).
+template <int FMT, int KIND>
+__device__ __forceinline__ void redo_wide(const GemmParams& P, u32x4_t* smem, const Ticket& tk) {
+    const int tid = threadIdx.x;
+    auto word = [&](int e) { return __builtin_amdgcn_readfirstlane(tk.wide[e]); };
+    const int g = word(1), row0 = word(2), rows = word(3), n0 = word(4);
+    __syncthreads();   // everybody has read them
+    if (tid == 0) tk.wide[0] = 0;
+    __syncthreads();
+    const uint16_t* scale = static_cast<const uint16_t*>(P.scale) + (int64_t)g * P.scale_rows * P.N + n0;
+    const int columns = min(P.N - n0, KernelCfg<FMT, KIND>::BN);
+    bool found = false;
+    for (int64_t e = tid; e < (int64_t)P.scale_rows * columns; e += blockDim.x)
+        found = found || (scale[e / columns * P.N + e % columns] & 0x7fffu) >= 0x7a00u;   // 2^117
+    if (found) tk.wide[0] = 1;
+    __syncthreads();
+    const int wide = word(0);
+    __syncthreads();
+    if (tid == 0) tk.wide[0] = 0;
+    if (!wide) return;
+    for (int r = 0; r < rows; r += 16)
+        gemm_tile_pair<FMT, 1, KIND, false, false, false, true>(P, smem, g, row0 + r, min(rows - r, 16), n0, tk);
+}
+
 template <int FMT, int KIND>
 __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT, KIND>::WAVES_PER_SIMD)) void grouped_gemm_kernel(GemmParams P) {
     using C = KernelCfg<FMT, KIND>;
@@ -1657,6 +1726,7 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
     // scan partials (one per wavefront); later part[0] carries the ticket drawn from the queue, part[1] the tile
     // resolved from it, part[2] the tile routine's arrival counter
     __shared__ int part[32];
+    constexpr int PART_WIDE = 20;    // Ticket::wide
     constexpr int PART_FIXED = 16;   // first whether this workgroup uses the launch's counter, then its number of fixed sweeps
     auto clamp_row = [&](int64_t v) { return (int)min(max(v, (int64_t)0), P.M); };
     auto expert_rows = [&](int g, int& first) {
@@ -1673,6 +1743,8 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
 
     // the launch's counter is looked at, and raised to the launch's stamp, now: long before the first draw from it
     if (tid == 0) part[PART_FIXED] = P.slot >= 0 && queue_open(tile_queue + GM_QUEUE_STRIDE * max(P.slot, 0), P.stamp, blockIdx.x < 8);
+
+    if (wide_scales<FMT>(KIND) && tid == 0) part[PART_WIDE] = 0;   // (set by the tile routine, cleared by redo_wide)
 
     // exclusive scan of tiles per expert: each thread takes a contiguous run of experts
     const int per = (P.G + THREADS - 1) / THREADS;
@@ -1748,9 +1820,16 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
 
     bool have_ticket = false;   // the previous tile routine left its ticket in part[0]
     queue_word_t* const q_own = tile_queue + GM_QUEUE_STRIDE * max(P.slot, 0);
+    auto ticket_from = [&](queue_word_t* counter) { return Ticket{counter, part, part + 2, part + PART_WIDE}; };
     for (int sw = 0;; ++sw) {
         int T;
+        const int look_again = wide_scales<FMT>(KIND) ? part[PART_WIDE] : 0;
         int fixed = __builtin_amdgcn_readfirstlane(part[PART_FIXED]);
+        if constexpr (wide_scales<FMT>(KIND)) {
+            // the previous tile's (set ahead of the barrier that ends the tile routine, and not again before one that every wavefront
+            // reaches after this; read here, beside the other word: behind the tile routine it cost 1 % of decode-like launches)
+            if (__builtin_amdgcn_readfirstlane(look_again)) [[unlikely]] redo_wide<FMT, KIND>(P, smem, ticket_from(nullptr));
+        }
         if (sw >= fixed) {
             if (fixed == GM_NO_QUEUE) break;
             if (!have_ticket) {
@@ -1779,7 +1858,7 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         }
         // from the last tile of the fixed order on, the tile routines draw the next ticket themselves
         const bool take = fixed != GM_NO_QUEUE && sw + 1 >= fixed;
-        const Ticket tk = {take ? q_own : nullptr, part, part + 2};
+        const Ticket tk = ticket_from(take ? q_own : nullptr);
         have_ticket = take;
         // largest e with prefix[e] <= T (empty experts have prefix[e] == prefix[e+1]): every wavefront looks at 64
         // evenly spaced entries at once, then at the entries between two of them -- two LDS round trips

@@ -57,6 +57,14 @@ static __device__ __forceinline__ f32x4_t mfma(const u32x4_t& a, const u32x4_t& 
 template <int FMT, int T>
 constexpr bool stream_quad() { return T == 2 && (FMT == MOE_FMT_FP4_REF || FMT == MOE_FMT_INT4); }
 
+// Two int4 codes, the low or the high bytes of h, as fp32: a nibble read as e4m3 is q / 512, and the scaled conversion takes that back.
+// (With 512 in the weight's scale instead, scales of 2^119 and more would leave the range of fp32; with -8 times the scale only those do for
+// which the weight of code 0 does.)
+template <bool HIGH>
+static __device__ __forceinline__ f32x2_t int4_codes(uint32_t h) {
+    return __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(h, 512.f, HIGH);
+}
+
 template <int FMT, int T>
 struct StreamStep {   // what a wavefront holds of one 32-k step
     // k row j: the dword that holds this lane's columns; 8 columns of bytes: r[2 j] and r[2 j + 1]; stream_quad: lane l of a quad
@@ -265,8 +273,8 @@ static __device__ __forceinline__ void stream_rows(const StreamParams& P, float*
                     for (int t = 0; t < TH; ++t) {
                         const uint32_t h = quad_q[t][p >> 1];
                         if constexpr (ROUNDW) {
-                            const f32x2_t f = p & 1 ? __builtin_amdgcn_cvt_pk_f32_fp8(h, true) : __builtin_amdgcn_cvt_pk_f32_fp8(h, false);
-                            bf[t][p] = pack_bf16_rne(fmaf(f[0], 512.f * sc[t], -8.f * sc[t]), fmaf(f[1], 512.f * sc[t], -8.f * sc[t]));
+                            const f32x2_t f = p & 1 ? int4_codes<true>(h) : int4_codes<false>(h);
+                            bf[t][p] = pack_bf16_rne(fmaf(f[0], sc[t], -8.f * sc[t]), fmaf(f[1], sc[t], -8.f * sc[t]));
                         } else {
                             bf[t][p] = __builtin_bit_cast(uint32_t, p & 1 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h, 512.f, true)
                                                                           : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h, 512.f, false));
@@ -280,8 +288,8 @@ static __device__ __forceinline__ void stream_rows(const StreamParams& P, float*
 #pragma unroll
                     for (int t = 0; t < TH; ++t) {
                         if constexpr (ROUNDW) {
-                            const f32x2_t f = t < 2 ? __builtin_amdgcn_cvt_pk_f32_fp8(h[t & 1], false) : __builtin_amdgcn_cvt_pk_f32_fp8(h[t & 1], true);
-                            bf[t][p] = pack_bf16_rne(fmaf(f[0], 512.f * sc[t], -8.f * sc[t]), fmaf(f[1], 512.f * sc[t], -8.f * sc[t]));
+                            const f32x2_t f = t < 2 ? int4_codes<false>(h[t & 1]) : int4_codes<true>(h[t & 1]);
+                            bf[t][p] = pack_bf16_rne(fmaf(f[0], sc[t], -8.f * sc[t]), fmaf(f[1], sc[t], -8.f * sc[t]));
                         } else {
                             bf[t][p] = __builtin_bit_cast(uint32_t, t < 2 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h[t & 1], 512.f, false)
                                                                           : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h[t & 1], 512.f, true));

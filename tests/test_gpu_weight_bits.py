@@ -8,6 +8,7 @@ import torch
 
 import helpers as H
 import oracle
+from test_gpu_tiles import _swiglu
 
 pytestmark = pytest.mark.gpu
 
@@ -56,6 +57,50 @@ def test_int4(kernel, G, K, N, rows):
     case = H.make_case("int4", G, K, N, np.arange(1, G + 1) * rows, seed=G, group=32)
     case["scale"] = _scales(rng, case["scale"].shape, -110, 117)
     _check(case, _unit_rows(case, rng), kernel)
+
+
+# ... and the longer ring of tiles_quad (more than 512 tiles, up to 48 rows), nontemporal loads of tiles_pair_small (96 MiB of weights)
+INT4_EXTREME = INT4 + [("tiles_quad", 128, 256, 2048, 13), ("tiles_quad", 70, 256, 2048, 40), ("tiles_pair_small", 96, 1024, 2048, 12)]
+
+
+@pytest.mark.parametrize("kernel,G,K,N,rows", INT4_EXTREME)
+def test_int4_extreme_scales(kernel, G, K, N, rows):
+    """Scales up to 2^125, beyond which code 0 itself is out of range, and down to the least subnormal: in all columns of some experts, in
+    a few groups of others (the tiles decode a step with a scale of 2^117 and more in another way), among ordinary ones."""
+    _say(f"int4 weight bits, extreme scales, {kernel}")
+    rng = np.random.default_rng(G + N + 1)
+    case = H.make_case("int4", G, K, N, np.arange(1, G + 1) * rows, seed=G, group=32)
+    case["scale"] = _scales(rng, case["scale"].shape, -10, 10)
+    large, small = _scales(rng, case["scale"].shape, 115, 125), _scales(rng, case["scale"].shape, -127, -110)
+    for g in range(G):
+        pick = [1.0, 0.002, 0.5, 1.0][g % 4]
+        at = rng.random(case["scale"].shape[1:]) < pick
+        case["scale"][g][at] = (small if g % 4 == 3 else large)[g][at]
+    _check(case, _unit_rows(case, rng), kernel)
+
+
+@pytest.mark.parametrize("epilogue", ["none", "swiglu"])
+@pytest.mark.parametrize("kernel,G,N,rows", [("tiles_pair_small", 20, 2048, 12), ("tiles_quad", 4, 512, 170), ("tiles_quad", 80, 2048, 20)])
+def test_int4_rows_that_are_no_number(kernel, G, N, rows, epilogue):
+    """NaN and infinities in rows of x look to the tiles like scales out of the usual decode's range; without such a scale, and beside one,
+    they stay in their rows."""
+    _say(f"int4 {kernel} {epilogue}, x with NaN")
+    rng = np.random.default_rng(rows)
+    K = 256
+    case = H.make_case("int4", G, K, N, np.arange(1, G + 1) * rows, seed=G)
+    bad = rng.random(case["M"]) < 0.1
+    case["x"][bad, rng.integers(0, K, bad.sum())] = rng.choice(np.array([0x7FC0, 0x7F80, 0xFF80], np.uint16), bad.sum())
+    for g in range(0, G, 3):   # one column of a large scale, on zeros of x
+        case["scale"][g, 0, int(rng.integers(0, N))] = (127 + 119) << 7
+        case["x"][g * rows:(g + 1) * rows, :128] &= 0x8000
+    case["x"][bad, 200] |= 0x7FC0
+    assert H.kernel_of(case, "gemm", swiglu=epilogue == "swiglu") == kernel
+    if epilogue == "swiglu":
+        got, want = _swiglu(case)
+    else:
+        got, want = H.run_cabi(case, H.upload(case), "gemm"), H.oracle_out(case)
+    H.assert_close(got, want, rows=~bad, what=f"{kernel} {epilogue}")
+    assert not np.isfinite(oracle.bf16_bits_to_f32(got)[bad]).any()
 
 
 # experts, K, rows per expert: 4, 8 and 16 staged rows, whole iterations of 512 k and one to three groups of 128 behind them, K on
