@@ -57,6 +57,12 @@ __device__ __forceinline__ f32x2_t e4m3_ref_pair_over_256(uint32_t pair) {
     return f32x2_t{(float)v[0], (float)v[1]};
 }
 
+// Two fp16 times 2^8 (exact for what e4m3_ref_pair_over_256_fp16 returns).
+__device__ __forceinline__ uint32_t fp16_pair_times_256(uint32_t h2) {
+    typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, h2) * half2_t{256.f, 256.f});
+}
+
 // fp32(low / high fp16 of h2) * s in one instruction (v_fma_mix_f32 converts the fp16 operand on the way
 // in; the product is rounded to fp32 once, exactly as a conversion followed by a multiply).  The addend
 // is -0.0 so that the sign of a zero product survives.

@@ -325,12 +325,13 @@ constexpr int QUAD_DEEP_MT = 3, QUAD_DEEP_STAGES = 6;
 // read in halves: 485 / 586; GK_QUAD gains nothing (int4, 16 rows each on 256 experts 476 / 470, fp4 unevenly routed 540 / 540).
 constexpr int64_t NT_MIN_BYTES = 96 << 20;
 constexpr int nt_mt_max(int kind) { return kind == GK_PAIR ? 4 : kind == GK_QUAD ? 0 : 1; }
-// int4 with rounded weights: the usual decode takes scales below 2^117.98.  A tile with a larger one has columns that are no number;
-// a wavefront that finds one in its sums says so in LDS (Ticket::wide), and the workgroup then looks whether such a scale is the
-// reason and if so computes the tile once more, 16 rows at a time, with a decode that takes all scales (redo_wide).  A check of the scales
-// in every step instead, three vector instructions and a branch, made decode-like launches 1.3 to 2.5 % slower, others 0.6 to 1.2 %.
+// Rounded weights of int4 and fp8: the usual decodes take scales below 2^117.98 (int4) and 2^120 (fp8, columns with a 0x7F or 0xFF among
+// the wavefront's codes).  A tile with a larger one has columns that are no number; a wavefront that finds one in its sums says so in LDS
+// (Ticket::wide), and the workgroup then looks whether such a scale is the reason and if so computes the tile once more, 16 rows at a
+// time, with a decode that takes all scales (redo_wide).  A check of the scales in every step instead, with a branch: int4 1.3 to 2.5 % slower in
+// decode-like launches, 0.6 to 1.2 % in others; fp8 with random codes 2 to 3 %.
 template <int FMT>
-constexpr bool wide_scales(int kind) { return FMT == MOE_FMT_INT4 && !pair_exact(kind); }
+constexpr bool wide_scales(int kind) { return (FMT == MOE_FMT_INT4 || FMT == MOE_FMT_FP8_REF) && !pair_exact(kind); }
 template <int FMT>
 constexpr int pair_lds_units(int kind) {
     return pair_stages<FMT>(kind) * (pair_a_units(kind) + pair_b_units<FMT>(kind) + pair_sc_units<FMT>(kind)) + pair_kc_scale_units<FMT>();
@@ -454,7 +455,7 @@ __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, 
 // the multiplies of the general case, and no masking.
 //
 // DEEP (GK_QUAD, small tiles): the longer ring, see QUAD_DEEP_STAGES.  NT: nontemporal loads of the weights, see NT_MIN_BYTES.
-// WIDE: int4 with any scale, see wide_scales.
+// WIDE: int4 and fp8 with any scale, see wide_scales.
 template <int FMT, int MT, int KIND, bool STACK2 = false, bool DEEP = false, bool NT = false, bool WIDE = false>
 __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk) {
     static_assert(FMT != MOE_FMT_BF16, "the k-split tile routine decodes quantized containers");
@@ -787,7 +788,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     };
     read_raw(0, 0);
 
-    // WIDE, k rows 2 p0 .. 2 p0 + 3 of the sub-step: q - 8 first (exact), then its product with the scale
+    // int4, WIDE: k rows 2 p0 .. 2 p0 + 3 of the sub-step: q - 8 first (exact), then its product with the scale
     auto decode_i4_wide = [&](int p0) __attribute__((always_inline)) {
         const float s[4] = {bf16_lo(sc[0]), bf16_hi(sc[0]), bf16_lo(sc[1]), bf16_hi(sc[1])};
 #pragma unroll
@@ -802,9 +803,10 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
         }
     };
     // fp8, k rows 2 p0 .. 2 p0 + 3 of the sub-step.  decode_f8: byte t of the dwords of two k rows as a pair through fp16 (see
-    // e4m3_ref_pair_over_256), where 0x7F and 0xFF are the reference's +-480; the 2^8 goes into the block scale.
+    // e4m3_ref_pair_over_256), where 0x7F and 0xFF are the reference's +-480; the 2^8 goes into the block scale (WIDE: into the
+    // fp16 pair, half an instruction per weight more).
     auto decode_f8 = [&](int p0) __attribute__((always_inline)) {
-        const float scl = __uint_as_float(sc[0]) * 256.f;
+        const float scl = __uint_as_float(sc[0]) * (WIDE ? 1.f : 256.f);
         float nz = -0.0f;
         asm volatile("" : "+v"(nz));   // kept in a register: not an inline constant
 #pragma unroll
@@ -813,7 +815,8 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const uint32_t sel8 = (uint32_t)t | 0x0c00u | ((uint32_t)(4 + t) << 16) | 0x0c000000u;   // [a.byte t, 0, b.byte t, 0]
-                const uint32_t h2 = e4m3_ref_pair_over_256_fp16(__builtin_amdgcn_perm(b, a, sel8));
+                uint32_t h2 = e4m3_ref_pair_over_256_fp16(__builtin_amdgcn_perm(b, a, sel8));
+                if constexpr (WIDE) h2 = fp16_pair_times_256(h2);
                 if constexpr (EXACT) {
                     // the e4m3 values themselves (worth 2^-8): exact in bf16
                     typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
@@ -947,7 +950,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
                 __builtin_amdgcn_sched_barrier(0);
                 continue;
             }
-            if constexpr (WIDE) {
+            if constexpr (FMT == MOE_FMT_INT4 && WIDE) {
                 decode_i4_wide(p0);
                 __builtin_amdgcn_sched_barrier(0);
                 continue;
@@ -1112,7 +1115,7 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
         if constexpr (F8) {
             // fragments with a NaN among them are decoded again, and from the next turn of the ring on the tile goes through decode_f8
             int kt0 = 0;
-            for (; kt0 < nk && f8_plain; kt0 += S) {
+            for (; kt0 < nk && f8_plain && !WIDE; kt0 += S) {
 #pragma unroll
                 for (int u = 0; u < S; ++u)
                     if (kt0 + u < nk) step(kt0 + u, u, (u + 1) % S, (u + S - 1) % S, std::true_type{});
@@ -1691,11 +1694,18 @@ __device__ __forceinline__ void redo_wide(const GemmParams& P, u32x4_t* smem, co
     __syncthreads();   // everybody has read them
     if (tid == 0) tk.wide[0] = 0;
     __syncthreads();
-    const uint16_t* scale = static_cast<const uint16_t*>(P.scale) + (int64_t)g * P.scale_rows * P.N + n0;
-    const int columns = min(P.N - n0, KernelCfg<FMT, KIND>::BN);
+    constexpr bool F8 = FMT == MOE_FMT_FP8_REF;
+    // the tile's scales: [rows of scales][columns] out of rows of `stride`
+    const int per = F8 ? 128 : 1, stride = P.N / per, columns = (min(P.N - n0, KernelCfg<FMT, KIND>::BN) + per - 1) / per;
+    const int64_t scale_rows = F8 ? P.K / 128 : P.scale_rows, first = g * scale_rows * stride + n0 / per;
     bool found = false;
-    for (int64_t e = tid; e < (int64_t)P.scale_rows * columns; e += blockDim.x)
-        found = found || (scale[e / columns * P.N + e % columns] & 0x7fffu) >= 0x7a00u;   // 2^117
+    for (int64_t e = tid; e < scale_rows * columns; e += blockDim.x) {
+        const int64_t at = first + e / columns * stride + e % columns;
+        if constexpr (F8)
+            found = found || fabsf(static_cast<const float*>(P.scale)[at]) >= 0x1p120f;
+        else
+            found = found || (static_cast<const uint16_t*>(P.scale)[at] & 0x7fffu) >= 0x7a00u;   // 2^117
+    }
     if (found) tk.wide[0] = 1;
     __syncthreads();
     const int wide = word(0);

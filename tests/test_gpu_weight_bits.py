@@ -138,6 +138,41 @@ def test_fp8(kernel, G, K, N, rows, codes):
     _check(case, _unit_rows(case, rng), kernel)
 
 
+@pytest.mark.parametrize("kernel,G,K,N,rows", [("strips_32", 4, 2048, 512, 16), ("strips_64", 6, 2048, 2048, 16), ("strips_128", 10, 2048, 2048, 12),
+                                               ("tiles_pair", 20, 1024, 2048, 40), ("tiles_pair", 48, 1024, 2048, 17), ("tiles_quad", 2, 1024, 256, 256)])
+def test_fp8_extreme_scales(kernel, G, K, N, rows):
+    """Block scales up to 2^127 beside codes 0x7F: a weight does not depend on its neighbours' codes.  0x7F stands in blocks with ordinary
+    scales in front of the large ones (even experts) and in the blocks with the large scales (their columns overflow and are left out)."""
+    _say(f"fp8 weight bits, extreme scales, {kernel}")
+    rng = np.random.default_rng(G + N + 1)
+    case = H.make_case("fp8", G, K, N, np.arange(1, G + 1) * rows, seed=G)
+    w = case["weight"]
+    w[(w & 0x7F) == 0x7F] ^= 1
+    case["scale"][:] = np.exp2(rng.integers(-20, 20, case["scale"].shape)) * np.where(rng.random(case["scale"].shape) < 0.5, 1, -1)
+    for kb in range(1, K // 128, 2):   # odd blocks of k: weights up to 1, scales up to 2^127
+        at = slice(128 * kb, 128 * kb + 128)
+        w[:, at] = (w[:, at] & 0x80) | (w[:, at] & 0x7F) % 0x39
+        case["scale"][:, kb] = case["scale"][:, kb] * np.exp2(107.0)
+    finite = np.ones((G, N), bool)
+    for g in range(G):
+        for n in range(int(rng.integers(0, 64)), N, 64):
+            k = int(rng.integers(0, K // 256)) * 256
+            if g % 2 == 0:
+                w[g, k + int(rng.integers(0, 128)), n] |= 0x7F
+            else:
+                w[g, k + 128 + int(rng.integers(0, 128)), n] |= 0x7F
+                finite[g, n] = False
+    at = _unit_rows(case, rng)
+    assert H.kernel_of(case, "gemm") == kernel
+    got = oracle.bf16_bits_to_f32(H.run_cabi(case, H.upload(case), "gemm"))
+    lo = 0
+    for g, hi in enumerate(case["group_list"]):
+        want = oracle.expand_weight(oracle.FMT_BY_NAME["fp8"], w, case["scale"], None, g, True).reshape(K, N)[at[lo:hi]]
+        assert np.isfinite(want[:, finite[g]]).all()
+        assert np.array_equal(got[lo:hi][:, finite[g]], want[:, finite[g]]), f"{kernel} expert {g}"
+        lo = hi
+
+
 @pytest.mark.parametrize("codes", ["without", "some", "all"])
 @pytest.mark.parametrize("kernel,G,N,rows", [("tiles_pair_exact", 24, 2048, r) for r in (3, 16, 17, 40)]
                          + [("strips_32", 4, 512, 5), ("strips_64", 6, 2048, 16), ("strips_128", 10, 2048, 12)])
