@@ -229,6 +229,11 @@ const char* moe_test_grouped_kernel(const moe_grouped_args* a, int gemv_op) {
     return moe::grouped_kernel_name(moe::grouped_kernel(a, gemv_op != 0));
 }
 
+int moe_test_nontemporal_rows(const moe_grouped_args* a, int gemv_op) {
+    if ((gemv_op ? moe_grouped_gemv_validate(a) : moe_grouped_gemm_validate(a)) != MOE_OK) return -1;
+    return moe::nontemporal_rows(a, moe::grouped_kernel(a, gemv_op != 0));
+}
+
 int64_t moe_test_shift_launch_number(int64_t delta) { return moe::gemm_shift_launch_number(delta); }
 
 }  // extern "C"

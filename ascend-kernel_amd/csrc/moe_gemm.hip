@@ -60,7 +60,7 @@ struct GemmParams {
     int table_mode;
     // N-contiguous 4-bit containers: turns a 32-k sub-step index into its scale row
     ScaleRowDivider scale_div;
-    int nt;   // nontemporal weight loads, see NT_MIN_BYTES
+    int nt_rows;   // experts of up to so many rows: nontemporal weight loads, see nontemporal_rows
 };
 
 // Work queue of the persistent grid.  Workgroups do not run at one speed (of two that share a CU the one
@@ -314,16 +314,7 @@ constexpr int pair_kc_scale_units() { return (FMT == MOE_FMT_FP4_B32 || FMT == M
 // each on 128 experts 327 / 331).  A launch with a tile per workgroup at most keeps 4: it gains nothing from more and pays for fetching
 // the code of the longer ring (416 rows on 16 of 3328 x 2048: 42.0 / 43.2).  The one-byte containers are here for experts of many rows.
 constexpr int QUAD_DEEP_MT = 3, QUAD_DEEP_STAGES = 6;
-// Nontemporal weight loads.  A weight line that is read once in a launch, whole, only pushes others out of L2 and the 256 MB behind
-// it.  So: the N-contiguous containers on GK_PAIR and the small-stage kinds, in tiles that hold all rows of their expert (GK_PAIR: 4 row
-// blocks, an expert in several chunks has 5 or more in each; small stages: one row block, nearly always), in launches that read more
-// weights than those caches can keep for the next launch that reads them.  us, without / with: GEMV op, 512 rows on 128 experts of 7168 x
-// 2048, fp8 307 / 270, on 256, int4 311 / 292, fp4 359 / 331; GEMM op, 512 rows on 256, fp4 374 / 355, int4 350 / 336; fp8, 128 rows on
-// 64 of 2048 x 1024 28.0 / 25.5, 1024 on 256 of 7168 x 2048 599 / 562; int8, 800 on 64 of 4096 x 4096 191 / 182.  Weights that
-// the caches still hold from the last time are faster read as usual: 84 MB of fp8 18.6 / 22.0, 67 MB of int4 21.3 / 21.6; 134 MB of
-// int4 39.3 / 37.2, 126 MB of fp4 33.3 / 31.2.  With row chunks that share their weights 256 rows of 8 experts, int8: 456 / 501; bf16, whose lines are
-// read in halves: 485 / 586; GK_QUAD gains nothing (int4, 16 rows each on 256 experts 476 / 470, fp4 unevenly routed 540 / 540).
-constexpr int64_t NT_MIN_BYTES = 96 << 20;
+// Row blocks of the largest tiles that have a form with nontemporal weight loads (see nontemporal_rows)
 constexpr int nt_mt_max(int kind) { return kind == GK_PAIR ? 4 : kind == GK_QUAD ? 0 : 1; }
 // Rounded weights of int4 and fp8: the usual decodes take scales below 2^117.98 (int4) and 2^120 (fp8, columns with a 0x7F or 0xFF among
 // the wavefront's codes).  A tile with a larger one has columns that are no number; a wavefront that finds one in its sums says so in LDS
@@ -454,7 +445,7 @@ __device__ __forceinline__ void pair_finish(const GemmParams& P, u32x4_t* smem, 
 // scale of its own group, and the two halves are added once at the end of the tile: half the MFMAs and half
 // the multiplies of the general case, and no masking.
 //
-// DEEP (GK_QUAD, small tiles): the longer ring, see QUAD_DEEP_STAGES.  NT: nontemporal loads of the weights, see NT_MIN_BYTES.
+// DEEP (GK_QUAD, small tiles): the longer ring, see QUAD_DEEP_STAGES.  NT: nontemporal loads of the weights, see nontemporal_rows.
 // WIDE: int4 and fp8 with any scale, see wide_scales.
 template <int FMT, int MT, int KIND, bool STACK2 = false, bool DEEP = false, bool NT = false, bool WIDE = false>
 __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk) {
@@ -486,8 +477,8 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
     // The next step's packed dwords are read ahead of the MFMAs instead of behind the first ones: with 4 or 8 MFMAs a step their
     // latency otherwise ends in the next decode (int4, a tile per CU, 2 rows: 64 experts of 2048 x 1024 22.6 / 21.3 us).
     // fp4 gains nothing from it, the GEMV op's kinds lose 0.5 to 4 %: they still need the scales of the step being multiplied.
-    constexpr int W_AUX = NT ? LOAD_NT : 0;   // (fp4: of the scales too, whose rows are read once; those of int4 serve four steps)
     constexpr bool EARLY_RAW = FMT == MOE_FMT_INT4 && KIND == GK_PAIR_SMALL;
+    constexpr int W_AUX = NT ? LOAD_NT : 0;   // (fp4: of the scales too, whose rows are read once; those of int4 serve four steps)
     static_assert(S * (PAIR_A_UNITS + PAIR_B_UNITS + PAIR_SC_UNITS) <= pair_lds_units<FMT>(KIND), "stages beyond the LDS of the kernel");
     static_assert(16 * MT * (BK / 8) <= PAIR_A_UNITS, "tile rows beyond the x stage");
     u32x4_t* lds_a = smem;
@@ -1658,11 +1649,11 @@ struct KernelCfg {
 };
 
 template <int FMT, int MT, int KIND>
-__device__ __forceinline__ void run_tile(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk, bool deep) {
+__device__ __forceinline__ void run_tile(const GemmParams& P, u32x4_t* smem, int g, int64_t row0, int rows, int n0, const Ticket& tk, bool deep, bool nt) {
     using C = KernelCfg<FMT, KIND>;
     if constexpr (C::PAIR) {
         if constexpr (C::nontemporal(MT)) {
-            if (P.nt) {
+            if (nt) {
                 if constexpr (FMT == MOE_FMT_FP4_REF && pair_exact(KIND)) {
                     if (rows <= 8) return gemm_tile_pair<FMT, MT, KIND, true, false, true>(P, smem, g, row0, rows, n0, tk);
                 }
@@ -1938,36 +1929,37 @@ __global__ __launch_bounds__((64 * KernelCfg<FMT, KIND>::WAVES), (KernelCfg<FMT,
         const int rhi = __builtin_amdgcn_readfirstlane((int)(gbeg >> 32));
         const int64_t row0 = (((int64_t)rhi << 32) | (uint32_t)rlo) + rbeg;
         const int n0 = nt * C::BN;
+        const bool nontemporal = m <= P.nt_rows;   // the expert's only tile of these columns
         switch (mt) {
             case 1:
-                if constexpr (MTM >= 1) run_tile<FMT, 1, KIND>(P, smem, g, row0, rows, n0, tk, deep);
+                if constexpr (MTM >= 1) run_tile<FMT, 1, KIND>(P, smem, g, row0, rows, n0, tk, deep, nontemporal);
                 break;
             case 2:
-                if constexpr (MTM >= 2) run_tile<FMT, 2, KIND>(P, smem, g, row0, rows, n0, tk, deep);
+                if constexpr (MTM >= 2) run_tile<FMT, 2, KIND>(P, smem, g, row0, rows, n0, tk, deep, nontemporal);
                 break;
             case 3:
-                if constexpr (MTM >= 3) run_tile<FMT, 3, KIND>(P, smem, g, row0, rows, n0, tk, deep);
+                if constexpr (MTM >= 3) run_tile<FMT, 3, KIND>(P, smem, g, row0, rows, n0, tk, deep, nontemporal);
                 break;
             case 4:
-                if constexpr (MTM >= 4) run_tile<FMT, 4, KIND>(P, smem, g, row0, rows, n0, tk, deep);
+                if constexpr (MTM >= 4) run_tile<FMT, 4, KIND>(P, smem, g, row0, rows, n0, tk, deep, nontemporal);
                 break;
             case 5:
-                if constexpr (MTM >= 5) run_tile<FMT, 5, KIND>(P, smem, g, row0, rows, n0, tk, deep);
+                if constexpr (MTM >= 5) run_tile<FMT, 5, KIND>(P, smem, g, row0, rows, n0, tk, deep, nontemporal);
                 break;
             case 6:
-                if constexpr (MTM >= 6) run_tile<FMT, 6, KIND>(P, smem, g, row0, rows, n0, tk, deep);
+                if constexpr (MTM >= 6) run_tile<FMT, 6, KIND>(P, smem, g, row0, rows, n0, tk, deep, nontemporal);
                 break;
             case 7:
-                if constexpr (MTM >= 7) run_tile<FMT, 7, KIND>(P, smem, g, row0, rows, n0, tk, deep);
+                if constexpr (MTM >= 7) run_tile<FMT, 7, KIND>(P, smem, g, row0, rows, n0, tk, deep, nontemporal);
                 break;
             case 8:
-                if constexpr (MTM >= 8) run_tile<FMT, 8, KIND>(P, smem, g, row0, rows, n0, tk, deep);
+                if constexpr (MTM >= 8) run_tile<FMT, 8, KIND>(P, smem, g, row0, rows, n0, tk, deep, nontemporal);
                 break;
             case 9:
-                if constexpr (MTM >= 9) run_tile<FMT, 9, KIND>(P, smem, g, row0, rows, n0, tk, deep);
+                if constexpr (MTM >= 9) run_tile<FMT, 9, KIND>(P, smem, g, row0, rows, n0, tk, deep, nontemporal);
                 break;
             case 10:
-                if constexpr (MTM >= 10) run_tile<FMT, 10, KIND>(P, smem, g, row0, rows, n0, tk, deep);
+                if constexpr (MTM >= 10) run_tile<FMT, 10, KIND>(P, smem, g, row0, rows, n0, tk, deep, nontemporal);
                 break;
             default: have_ticket = false; break;
         }
@@ -2042,7 +2034,27 @@ static int launch_gemm_kind(const GemmParams& P, const moe_grouped_args* a, hipS
     return hipGetLastError() == hipSuccess ? MOE_OK : MOE_ERR_LAUNCH;
 }
 
-static GemmParams gemm_params(const moe_grouped_args* a) {
+// Nontemporal weight loads.  A weight line that is read once in a launch, whole, only pushes others out of L2 and the 256 MB behind
+// it.  So: the N-contiguous containers on GK_PAIR and the small-stage kinds, for experts whose rows are one tile (GK_PAIR: of up to 4 row
+// blocks, small stages: of one), in launches that may read more weights (min(M, G) experts, if each has rows) than those caches
+// can keep for the next launch that reads them.  us, without / with: GEMV op, 512 rows on 128 experts of 7168 x
+// 2048, fp8 307 / 270, on 256, int4 311 / 292, fp4 359 / 331; GEMM op, 512 rows on 256, fp4 374 / 355, int4 350 / 336; fp8, 128 rows on
+// 64 of 2048 x 1024 28.0 / 25.5, 1024 on 256 of 7168 x 2048 599 / 562; int8, 800 on 64 of 4096 x 4096 191 / 182.  Weights that
+// the caches still hold from the last time are faster read as usual: 84 MB of fp8 18.6 / 22.0, 67 MB of int4 21.3 / 21.6; 134 MB of
+// int4 39.3 / 37.2, 126 MB of fp4 33.3 / 31.2.  With row chunks that share their weights 256 rows of 8 experts, int8: 456 / 501; fp4,
+// 512 rows on 64 of 7168 x 2048 at a skew of 1, without / with in every tile of one row block / with for experts of one tile: GEMV op 105 / 111 /
+// 102, GEMM op 105 / 112 / 99.  bf16, whose lines are read in halves: 485 / 586; GK_QUAD gains nothing (int4, 16 rows each on 256 experts 476 / 470, fp4 unevenly routed 540 / 540).
+constexpr int64_t NT_MIN_BYTES = 96 << 20;
+int nontemporal_rows(const moe_grouped_args* a, GroupedKernel k) {
+    const bool pair = k == GroupedKernel::TILES_PAIR;
+    const bool small = k == GroupedKernel::TILES_PAIR_SMALL || k == GroupedKernel::TILES_PAIR_EXACT || k == GroupedKernel::TILES_PAIR_EXACT16;
+    const bool byte = a->format == MOE_FMT_INT8 || a->format == MOE_FMT_FP8_REF, four_bit = a->format == MOE_FMT_INT4 || a->format == MOE_FMT_FP4_REF;
+    if (!(pair || small) || !(byte || four_bit)) return 0;
+    if (std::min(a->M, a->G) * (a->K * a->N >> (byte ? 0 : 1)) < NT_MIN_BYTES) return 0;
+    return 16 * nt_mt_max(pair ? GK_PAIR : GK_PAIR_SMALL);
+}
+
+static GemmParams gemm_params(const moe_grouped_args* a, GroupedKernel kind) {
     GemmParams P;
     P.x = static_cast<const uint16_t*>(a->x);
     P.w = static_cast<const uint8_t*>(a->weight);
@@ -2052,8 +2064,7 @@ static GemmParams gemm_params(const moe_grouped_args* a) {
     P.y = static_cast<uint16_t*>(a->y);
     P.M = a->M; P.K = (int)a->K; P.N = (int)a->N; P.G = (int)a->G; P.scale_rows = (int)a->scale_rows;
     P.epilogue = a->epilogue;
-    const bool byte = a->format == MOE_FMT_INT8 || a->format == MOE_FMT_FP8_REF;
-    P.nt = std::min(a->M, a->G) * (a->K * a->N >> (byte ? 0 : 1)) >= NT_MIN_BYTES;
+    P.nt_rows = nontemporal_rows(a, kind);
     P.slot = -1;
     P.stamp = 0;
     P.table_mode = 0;
@@ -2062,7 +2073,7 @@ static GemmParams gemm_params(const moe_grouped_args* a) {
 }
 
 int launch_tiles(const moe_grouped_args* a, GroupedKernel kind, hipStream_t stream) {
-    const GemmParams P = gemm_params(a);
+    const GemmParams P = gemm_params(a, kind);
     switch (kind) {
         case GroupedKernel::TILES_PAIR:
             switch (a->format) {

@@ -44,6 +44,8 @@ int launch_vector(const moe_grouped_args* a, hipStream_t stream);
 int launch_fp4_rows(const moe_grouped_args* a, bool gemm_rounding, hipStream_t stream);
 int launch_strips(const moe_grouped_args* a, GroupedKernel width, bool gemm_rounding, hipStream_t stream);
 int launch_tiles(const moe_grouped_args* a, GroupedKernel kind, hipStream_t stream);
+// rows of the largest experts whose weights launch_tiles loads nontemporally, 0: of none
+int nontemporal_rows(const moe_grouped_args* a, GroupedKernel kind);
 // moves the grouped GEMM's launch number (which picks a launch's tile counter and stamp) by delta; returns the new number
 int64_t gemm_shift_launch_number(int64_t delta);
 int launch_prepack_fp4_ref(const moe_prepack_fp4_args* a, hipStream_t stream);

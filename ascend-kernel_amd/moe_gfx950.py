@@ -27,7 +27,7 @@ SYMBOLS = (
     "moe_dequant_fp4_bf16", "moe_grouped_gemm", "moe_grouped_gemv",
     "moe_prepack_fp4_ref_validate", "moe_prepack_fp4_ref_workspace_bytes", "moe_prepack_fp4_ref",
     "moe_route_validate", "moe_route_workspace_bytes", "moe_route", "moe_route_static", "moe_test_shift_launch_number",
-    "moe_test_grouped_kernel",
+    "moe_test_grouped_kernel", "moe_test_nontemporal_rows",
 )
 
 
@@ -84,6 +84,8 @@ lib.moe_test_shift_launch_number.restype = ctypes.c_int64
 lib.moe_test_shift_launch_number.argtypes = [ctypes.c_int64]
 lib.moe_test_grouped_kernel.restype = ctypes.c_char_p
 lib.moe_test_grouped_kernel.argtypes = [ctypes.POINTER(GroupedArgs), ctypes.c_int]
+lib.moe_test_nontemporal_rows.restype = ctypes.c_int
+lib.moe_test_nontemporal_rows.argtypes = [ctypes.POINTER(GroupedArgs), ctypes.c_int]
 lib.moe_route_static.argtypes = [ctypes.POINTER(RouteArgs), ctypes.c_void_p]
 ROUTE_STATIC_SCRATCH_BYTES = 2 << 20
 
@@ -129,6 +131,14 @@ def grouped_kernel(args: GroupedArgs, op: str) -> str:
     if name is None:
         raise ValueError(f"not a valid {op} call")
     return name.decode()
+
+
+def nontemporal_rows(args: GroupedArgs, op: str) -> int:
+    """Rows of the largest experts whose weights that kernel loads nontemporally, 0: of none (test support, host only)."""
+    rows = lib.moe_test_nontemporal_rows(ctypes.byref(args), int(op == "gemv"))
+    if rows < 0:
+        raise ValueError(f"not a valid {op} call")
+    return rows
 
 
 def grouped_gemv(args: GroupedArgs, stream: int = 0) -> None:

@@ -264,6 +264,9 @@ int64_t moe_test_shift_launch_number(int64_t delta);
  * arguments, NULL if they are not valid.  Host only; the pointers are not followed.  The names may change. */
 const char *moe_test_grouped_kernel(const moe_grouped_args *args, int gemv_op);
 
+/* Test support: experts of up to so many rows have their weights loaded nontemporally by that kernel (0: none, -1: not valid). */
+int moe_test_nontemporal_rows(const moe_grouped_args *args, int gemv_op);
+
 #ifdef __cplusplus
 }
 #endif

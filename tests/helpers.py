@@ -94,13 +94,27 @@ def oracle_out(case, gemv: bool = False, row_mask=None) -> np.ndarray:
                                case["offset"], case["group_list"], round_bf16=not gemv, row_mask=row_mask)
 
 
-def kernel_of(case, op: str, swiglu: bool = False) -> str:
-    """Name of the kernel that a call of these sizes runs (host only: the pointers stand for any aligned ones)."""
+def _sizes(case, swiglu: bool):
+    """Arguments of a call of these sizes (the pointers stand for any aligned ones)."""
     import moe_gfx950 as mg
 
     p = 0x1000
-    return mg.grouped_kernel(mg.grouped_args(mg.format_from_compute_type(case["fmt"]), p, p, p, p, p, p, case["M"], case["K"], case["N"],
-                                             case["G"], case["scale_rows"], epilogue=mg.EPILOGUE_SWIGLU if swiglu else mg.EPILOGUE_NONE), op)
+    return mg.grouped_args(mg.format_from_compute_type(case["fmt"]), p, p, p, p, p, p, case["M"], case["K"], case["N"],
+                           case["G"], case["scale_rows"], epilogue=mg.EPILOGUE_SWIGLU if swiglu else mg.EPILOGUE_NONE)
+
+
+def kernel_of(case, op: str, swiglu: bool = False) -> str:
+    """Name of the kernel that a call of these sizes runs (host only)."""
+    import moe_gfx950 as mg
+
+    return mg.grouped_kernel(_sizes(case, swiglu), op)
+
+
+def nontemporal_rows(case, op: str) -> int:
+    """Rows of the largest experts whose weights that kernel loads nontemporally (host only)."""
+    import moe_gfx950 as mg
+
+    return mg.nontemporal_rows(_sizes(case, False), op)
 
 
 # ----------------------------------------------------------------------------- GPU side

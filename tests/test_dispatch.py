@@ -36,6 +36,25 @@ def test_tiles_of_the_n_contiguous_containers():
     assert rows[13] == dict.fromkeys(("fp4", "int4", "fp8"), "tiles_pair_exact")
 
 
+def test_nontemporal_weights():
+    """Experts of one tile (of 4 row blocks on GK_PAIR, of one on the small-stage kinds) where the experts that may own rows have 96 MiB."""
+    def rows(fmt, op, M, G, K, N):
+        case = dict(fmt=fmt, M=M, K=K, N=N, G=G, scale_rows={"fp4": K // 16, "int4": K // 32}.get(fmt, 1))
+        return H.kernel_of(case, op), H.nontemporal_rows(case, op)
+
+    for fmt, op, M, kernel, most in (("fp8", "gemm", 1600, "tiles_pair", 64), ("int8", "gemm", 1600, "tiles_pair", 64), ("int4", "gemm", 600, "tiles_pair_small", 16),
+                                     ("fp4", "gemm", 600, "tiles_pair_small", 16), ("fp8", "gemv", 600, "tiles_pair_exact", 16), ("int4", "gemv", 600, "tiles_pair_exact", 16),
+                                     ("fp4", "gemv", 1600, "tiles_pair_exact", 16), ("fp4", "gemv", 600, "tiles_pair_exact16", 16),
+                                     ("int4", "gemm", 1600, "tiles_quad", 0), ("fp4", "gemm", 1600, "tiles_quad", 0)):
+        N = 2048 if fmt in ("fp8", "int8") else 4096   # 1.5 MiB an expert
+        assert rows(fmt, op, M, 64, 768, N) == (kernel, most)
+        assert rows(fmt, op, M, 64, 704 if fmt != "fp8" else 640, N) == (kernel, 0)
+        assert (rows(fmt, op, 64, 256, 768, N)[1], rows(fmt, op, 63, 256, 768, N)[1]) == (rows(fmt, op, 64, 64, 768, N)[1], 0)   # 64 or 63 experts own rows
+    assert rows("int8", "gemm", 161 * 64, 64, 7168, 4096) == ("tiles_quad", 0)
+    for fmt in ("fp4_b32", "fp4_b16", "bf16"):
+        assert rows(fmt, "gemm", 1600, 64, 7168, 4096)[1] == 0
+
+
 @pytest.mark.parametrize("fmt", ["fp4_b32", "fp4_b16"])
 def test_k_contiguous_fp4(fmt):
     at = lambda op, r, K, swiglu=False: kernel(fmt, op, r * 64, 64, K, 2048, swiglu)   # noqa: E731

@@ -242,24 +242,26 @@ def test_small_tiles_in_the_longer_ring(fmt, K):
     assert (got[used:] == 0x7FC0).all(), "rows beyond group_list[-1] were written"
 
 
-# op, container, experts, K, N; the weights of all experts are 96 MiB or just under
-NONTEMPORAL = [("gemm", "fp8", 48, 1024, 2048), ("gemm", "int8", 48, 1024, 2048), ("gemm", "int4", 96, 1024, 2048), ("gemm", "fp4", 96, 1024, 2048),
-               ("gemv", "fp8", 48, 1024, 2048), ("gemv", "int4", 96, 1024, 2048), ("gemv", "fp4", 96, 1024, 2048), ("gemv", "fp4", 100, 1024, 2048)]
+# op, container, experts, K, N, kernel; the weights of all experts are 96 MiB or just under
+NONTEMPORAL = [("gemm", "fp8", 48, 1024, 2048, "tiles_pair"), ("gemm", "int8", 48, 1024, 2048, "tiles_pair"), ("gemm", "int4", 96, 1024, 2048, "tiles_pair_small"),
+               ("gemm", "fp4", 96, 1024, 2048, "tiles_pair_small"), ("gemv", "fp8", 48, 1024, 2048, "tiles_pair_exact"),
+               ("gemv", "int4", 96, 1024, 2048, "tiles_pair_exact"), ("gemv", "fp4", 96, 1024, 2048, "tiles_pair_exact"),
+               ("gemv", "fp4", 96, 1024, 2048, "tiles_pair_exact16")]
 
 
 @pytest.mark.parametrize("spare", [0, 1])
-@pytest.mark.parametrize("op,fmt,G,K,N", NONTEMPORAL)
-def test_nontemporal_weights(op, fmt, G, K, N, spare):
-    """Launches that read 96 MiB of weights load those of small tiles nontemporally, smaller ones (here by an expert) do not: the row
-    counts around each tile size, experts of several chunks."""
-    _say(f"nontemporal weights {op} {fmt} spare={spare}")
+@pytest.mark.parametrize("op,fmt,G,K,N,kernel", NONTEMPORAL)
+def test_nontemporal_weights(op, fmt, G, K, N, kernel, spare):
+    """Launches that read 96 MiB of weights load those of experts of one small tile nontemporally, smaller ones (here by an expert) do not: the
+    row counts around each tile size, experts of several chunks."""
+    _say(f"nontemporal weights {op} {fmt} {kernel} spare={spare}")
     counts = ([1, 8, 9, 15, 16, 17, 0, 31, 32, 33] if op == "gemv" or fmt in ("int4", "fp4") else [1, 16, 17, 33, 63, 64, 65, 161, 0, 80]) * G
     counts = counts[:G - spare]
-    if (fmt in ("int4", "fp4") and op == "gemm") or G == 100:   # 12 rows per expert at most, on average
+    if kernel in ("tiles_pair_small", "tiles_pair_exact16"):   # 12 rows per expert at most, on average
         counts = [c if g % 3 else min(c, 1) for g, c in enumerate(counts)]
     case = H.make_case(fmt, len(counts), K, N, np.cumsum(counts), seed=G + spare, extra_rows=3)
-    kernel = H.kernel_of(case, op)
-    assert kernel in {"gemm": ("tiles_pair", "tiles_pair_small"), "gemv": ("tiles_pair_exact", "tiles_pair_exact16")}[op], kernel
+    assert H.kernel_of(case, op) == kernel
+    assert H.nontemporal_rows(case, op) == (0 if spare else 64 if kernel == "tiles_pair" else 16)
     used = int(case["group_list"][-1])
     got = H.run_cabi(case, H.upload(case), op)
     H.assert_close(got, H.oracle_out(case, gemv=op == "gemv"), rows=slice(0, used), what=f"{op} {fmt}")
