@@ -149,13 +149,27 @@ static GroupedKernel strip_width(const moe_grouped_args* a) {
 //   12 rows per expert and fewer, always: 256 experts of 7168 x 2048, 4 rows int4 445 / 382 us, fp4 427 / 404, 12 rows 476 / 422 and 461 /
 //   441.  Beyond, it depends on the routing, as an expert of many rows is many passes over its weights: 16 rows, balanced top-k routing
 //   int4 483 / 425, fp4 464 / 451, skew 0.5 473 / 470 and 459 / 485, skew 1 354 / 401 and 359 / 418.
-//   Launches in which the prefill kind has a tile per CU at most: its 4 wavefronts are then alone there, and small tiles are
-//   more and fill it.  K = 4096, int4 and fp4.  Up to 128 tiles (8 experts of N = 2048 and 4096): 32 rows 1.4 - 1.5, 48 rows 1.3 - 1.9, 64
-//   and 96 rows 1.02 - 2.0 (not used: the bound stays where the gain is 1.3 and more).  192 and 256 tiles (12 and 16 experts of N =
-//   4096): 16 rows 1.2 - 1.7, 24 rows 1.17 - 1.7, 32 rows 0.97 - 1.7, 40 rows 0.91 - 1.19, 64 rows 0.83 - 1.18, 96 rows 0.61 - 1.05.
+//   Launches in which the prefill kind has a tile per CU at most, evenly routed: its 4 wavefronts are then alone there, and small tiles
+//   are more and fill it, until they too are more than the CUs, which a short K does not make up for.  Smallest / mean / largest over 8 to
+//   256 experts, K from 512, skews of 0 to 1.  Up to 128 tiles, int4: 32 rows 1.1 / 1.4 / 2.1, 40 rows 1.1 / 1.5 / 2.1, 48 rows 1.0 / 1.5 / 2.0
+//   from K = 1024 on, but 0.9 at K = 512; fp4: 32 rows 1.1 / 1.4 / 2.1, 40 rows 1.0 / 1.4 / 2.1, 48 rows 0.96 / 1.4 / 2.0 from K = 1536 on, 0.9 and 0.8 at
+//   K = 1024 and 512;
+//   64 rows as low as 0.9 up to K = 2048.  129 to 192 tiles: 20 rows 1.0 / 1.3 / 1.9, 24 rows from K = 1536 on 1.15 / 1.4 / 1.95, at K = 1024 as low
+//   as 0.9.  Up to 256 tiles, 24 rows: K = 3072 1.0 / 1.2 / 1.6, 7168 1.1 / 1.3 / 1.9; K = 2560 int4 1.0 / 1.2 / 1.5, fp4 as low as 0.92,
+//   K = 1024 int4 0.94, fp4 0.85, K = 256 0.8 and 0.75.  K = 256 with fewer tiles: 0.95 to 1.2.
 static bool small_tiles_preferred(const moe_grouped_args* a) {
     const int64_t tiles = std::min(a->M, a->G) * ((a->N + 255) / 256);
-    return a->M <= (tiles <= 128 ? 48 : tiles <= 256 ? 24 : 12) * a->G;
+    const bool int4 = a->format == MOE_FMT_INT4;
+    int rows = 12;
+    if (a->K >= 512) {
+        if (tiles <= 128)
+            rows = a->K >= (int4 ? 1024 : 1536) ? 48 : 40;
+        else if (tiles <= 192)
+            rows = a->K >= 1536 ? 24 : 20;
+        else if (tiles <= 256 && a->K >= (int4 ? 2560 : 3072))
+            rows = 24;
+    }
+    return a->M <= rows * a->G;
 }
 
 static GroupedKernel n_contiguous_kernel(const moe_grouped_args* a, bool gemv_op) {

@@ -36,6 +36,27 @@ def test_tiles_of_the_n_contiguous_containers():
     assert rows[13] == dict.fromkeys(("fp4", "int4", "fp8"), "tiles_pair_exact")
 
 
+@pytest.mark.parametrize("fmt", ["int4", "fp4"])
+def test_small_tiles_of_few_tile_launches(fmt):
+    """Rows per expert up to which the small-stage kind is taken: no more than are ahead of the prefill kind at that K and number of tiles."""
+    def bound(G, N, K):
+        names = [kernel(fmt, "gemm", r * G, G, K, N) for r in range(13, 50)]
+        assert names == sorted(names) and set(names) <= {"tiles_pair_small", "tiles_quad"}
+        return 12 + names.count("tiles_pair_small")
+
+    for G, N in ((8, 4096), (128, 256), (33, 768)):     # up to 128 tiles
+        K = {"int4": 1024, "fp4": 1536}[fmt]
+        assert [bound(G, N, k) for k in (448, 512, K - 64, K, 7168)] == [12, 40, 40, 48, 48]
+    for G, N in ((12, 4096), (129, 256), (64, 768)):    # up to 192
+        assert [bound(G, N, K) for K in (448, 512, 1472, 1536, 7168)] == [12, 20, 20, 24, 24]
+    K = {"int4": 2560, "fp4": 3072}[fmt]
+    for G, N in ((16, 4096), (256, 256), (193, 256)):   # up to 256
+        assert [bound(G, N, k) for k in (512, 1024, K - 64, K, 7168)] == [12, 12, 12, 24, 24]
+    assert [bound(257, 256, k) for k in (512, 7168)] == [12, 12]
+    # fewer rows than experts: 12 per expert at least
+    assert kernel(fmt, "gemm", 1000, 2000, 1024, 4096) == "tiles_pair_small"
+
+
 def test_nontemporal_weights():
     """Experts of one tile (of 4 row blocks on GK_PAIR, of one on the small-stage kinds) where the experts that may own rows have 96 MiB."""
     def rows(fmt, op, M, G, K, N):

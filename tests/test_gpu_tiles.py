@@ -270,11 +270,12 @@ def test_nontemporal_weights(op, fmt, G, K, N, kernel, spare):
 
 @pytest.mark.parametrize("epilogue", ["none", "swiglu"])
 @pytest.mark.parametrize("fmt", ["int4", "fp4"])
-@pytest.mark.parametrize("G,N,rows,kernel", [(8, 4096, 48, "tiles_pair_small"), (8, 4096, 49, "tiles_quad"), (16, 4096, 24, "tiles_pair_small"),
-                                             (16, 4096, 25, "tiles_quad"), (17, 4096, 13, "tiles_quad"), (1, 256, 48, "tiles_pair_small")])
-def test_small_tiles_of_few_tile_launches(G, N, rows, kernel, fmt, epilogue):
-    """The bounds by rows per expert and tiles between the small-stage and the prefill kind, unevenly owned: experts of many chunks."""
-    K = 320
+@pytest.mark.parametrize("G,K,N,rows,kernel", [(8, 1600, 4096, 48, "tiles_pair_small"), (8, 1600, 4096, 49, "tiles_quad"), (8, 960, 4096, 40, "tiles_pair_small"),
+                                               (8, 960, 4096, 48, "tiles_quad"), (12, 1600, 4096, 24, "tiles_pair_small"), (16, 1600, 4096, 24, "tiles_quad"),
+                                               (8, 3136, 8192, 24, "tiles_pair_small"), (8, 3136, 8192, 25, "tiles_quad"), (17, 320, 4096, 13, "tiles_quad"),
+                                               (8, 448, 4096, 13, "tiles_quad"), (1, 1600, 256, 48, "tiles_pair_small")])
+def test_small_tiles_of_few_tile_launches(G, K, N, rows, kernel, fmt, epilogue):
+    """The bounds by rows per expert, tiles and K between the small-stage and the prefill kind, unevenly owned: experts of many chunks."""
     counts = [rows] * G
     if G > 2:
         counts[0], counts[1] = 0, 2 * rows
