@@ -51,14 +51,13 @@ static GroupedKernel bf16_kernel(const moe_grouped_args* a, bool gemv_op) {
 // fp4 [N, K/2].  The matrix-core GEMV kernel reads every weight row as contiguous runs, takes 16 rows of an expert per pass and
 // has a variant with the GEMM's weight rounding.  An expert of more than 16 rows is passes in a row, so that the bound for the GEMM op,
 // where tiles overtake it with balanced top-k routing, depends on the routing.  us, this kernel / tiles, fp4_b32, evenly routed,
-// balanced top-k routing, skews of 0.25 and 1 (see bf16): 256 experts of 7168 x 2048, 4 rows per expert 394 / 534, 409 / 532, 402 / 527, 296 /
-// 251, 8 rows 447 / 545, 466 / 542, 504 / 541, 485 / 310, 10 rows 479 / 547, 505 / 546, 553 / 547, 566 / 322, 12 rows 486 / 546, 566 / 542, 612
-// / 545, 691 / 347; 64 of the same 8 rows 120 / 137, 125 / 133, 147 / 133, 188 / 127, 10 rows 130 / 137, 146 / 135, 152 / 139, 234 / 131.  Up to
-// 65536 columns the tiles are one per CU, at best, and take longer: 8 of 4096 x 2048, 12 rows 25 / 40, 25 / 40, 26 / 40, 41 / 41.
-// fp4_b16 the same within 0.07.
-// With the SwiGLU epilogue the line lies lower (skews 0.25 and 1): 256 of 2048 x 1024, 4 rows 66 / 81 and 68 / 43, 5 rows 74 / 81 and
-// 81 / 47, 8 rows 84 / 83 and 121 / 60 (an expert of 109 rows is 7 passes in a row); 256 of 7168 x 2048, 4 rows 387 / 520 and 291 / 249, 8 rows
-// 496 / 537 and 496 / 308.  Up to 64 rows in all, four passes at most: 8 of 4096 x 2048, 8 rows 23 / 39 against 36 / 36.
+// balanced top-k routing, skews of 0.25 and 1 (see bf16): 256 experts of 7168 x 2048, 4 rows per expert 389 / 519, 403 / 515, 386 / 508, 300 /
+// 263, 8 rows 434 / 532, 467 / 533, 479 / 531, 590 / 321, 10 rows 470 / 534, 478 / 535, 537 / 539, 646 / 373, 12 rows 479 / 543, 532 / 543, 580
+// / 542, 727 / 382; 64 of the same 8 rows 113 / 131, 127 / 131, 136 / 132, 158 / 126, 10 rows 120 / 132, 133 / 133, 145 / 137, 186 / 127.  Up to
+// 65536 columns the tiles are one per CU, at best, and take longer: 8 of 4096 x 2048, 12 rows 22 / 37, 23 / 37, 34 / 38, 52 / 40.
+// With the SwiGLU epilogue the line lies lower (skews 0.25 and 1): 256 of 2048 x 1024, 4 rows 61 / 78 and 74 / 47, 5 rows 71 / 79 and
+// 88 / 48, 8 rows 79 / 81 and 131 / 60 (an expert of 109 rows is 7 passes in a row); 256 of 7168 x 2048, 4 rows 402 / 506 and 292 / 263, 8 rows
+// 481 / 527 and 462 / 319.  Up to 64 rows in all, four passes at most: 8 of 4096 x 2048, 8 rows 22 / 37 against 37 / 37.
 static bool fp4_rows_preferred(const moe_grouped_args* a) {
     if (a->epilogue != MOE_EPILOGUE_SWIGLU) return a->M <= (columns(a) <= 65536 ? 12 : 9) * a->G;
     return a->M <= (a->M <= 64 ? 8 : 5) * a->G;
@@ -82,11 +81,12 @@ static bool fp4_rows_partial_gemv(const moe_grouped_args* a) {
 // GEMM op, K no multiple of 512: the tiles take such a K as any other, so that the bounds by rows per expert lie lower, and go by the
 // columns: few make a tile per CU at best, whose time hardly depends on its rows; with many, an expert of more than 16 rows is passes in
 // a row here.  Tiles / this kernel, balanced top-k routing and skews of 0.25 and 1, median over K = 1152 to 7040 (fp4_b16 differs by
-// 0.05): up to 32768 columns 12 rows per expert 1.8, 1.7 and 1.04; up to 65536 columns 4 rows 1.33, 1.31 and 1.21, 8 rows 1.25, 1.0 and
-// 0.86, 10 rows 1.22, 0.90 and 0.71; more columns 3 rows 1.2, 1.2 and 0.95, 4 rows 1.18, 1.16 and 0.84, 6 rows 1.12, 1.03 and 0.72,
-// 12 rows 0.9, 0.82 and 0.5.  With SwiGLU the same within 0.03.
-// Fewer rows than experts: the workgroups of experts without rows count beside a short K.  6 rows on 256 of 1280 x 7424 17.6 / 21.9, 12
-// on 256 of 1280 x 4608 16.9 / 19.6, but 100 on 64 of 4480 x 1024 44 / 35.
+// 0.1): 32768 columns 12 rows per expert 1.2, 1.2 and 0.7; 65536 columns 4 rows 1.37, 1.39 and 1.41, 8 rows 1.32, 1.30 and
+// 0.99, 10 rows 1.3, 1.0 and 0.8; 262144 columns 3 rows 1.39, 1.39 and 1.27, 4 rows 1.36, 1.34 and 1.11, 6 rows 1.30, 1.27 and 0.86,
+// 12 rows 1.07, 0.99 and 0.52.
+// Fewer rows than experts: the workgroups of experts without rows count beside a short K.  6 rows on 256 of 1280 x 7424 16.0 / 15.0, 12
+// on 256 of 1280 x 4608 16.8 / 15.5, but 100 on 64 of 4480 x 1024 53 / 38.  (With the transposes that the GEMM op's form of this kernel had
+// when the line was drawn: 17.6 / 21.9, 16.9 / 19.6 and 44 / 35.)
 static bool fp4_rows_partial_gemm(const moe_grouped_args* a) {
     if (columns(a) <= 32768) return a->M <= 12 * a->G;
     return (a->K >= 4096 || a->M >= a->G) && a->M <= (columns(a) <= 65536 ? 4 : 3) * a->G;
@@ -126,32 +126,34 @@ static GroupedKernel fp4_kcontiguous_kernel(const moe_grouped_args* a, bool gemv
     return rows ? GroupedKernel::FP4_ROWS : fp4_kcontiguous_tiles(a);
 }
 
-// Strips for launches of up to 128 tiles of 256 columns, i.e. half of the CUs, and decode-like batches: with 32768 columns (16
-// experts of 7168 x 2048) int4 34 - 36 us in strips against 49 - 60 in tiles, fp4 33 / 50, fp8 49 / 72; with 49152 columns
-// tiles are ahead (int4 63 / 53, fp8 90 / 82), with 65536 by a factor of 1.3.  With up to 16384 columns twice as many rows:
-// 192 rows unevenly owned by 8 experts of 4096 x 2048, tiles / strips: int4 65 / 25 us, fp4 58 / 21, fp8 49 / 28, int8 44 / 25;
-// all 192 owned by one expert: int4 66 / 22, int8 45 / 21.  The passes are found by looking through group_list, 256 experts
-// at a time.
+// Strips for launches of up to 128 tiles of 256 columns, i.e. half of the CUs, and decode-like batches.  us, strips / tiles, 7168 x 2048,
+// 1 and 4 rows per expert (skew 0.25): 16 experts (32768 columns) int4 34 / 58 and 36 / 59, fp4 29 / 52 and 31 / 52, fp8 46 / 64 and 48 / 64; 24
+// (49152) int4 62 / 58 and 64 / 58, fp4 52 / 52 and 54 / 52, fp8 79 / 67 and 82 / 67; 32 (65536) int4 65 / 59, fp4 57 / 54, fp8 89 / 73.
+// With 12 rows an expert of more than 16 is a second pass: 16 experts int4 63 / 61, fp4 53 / 55, fp8 77 / 65.  With up to 16384 columns
+// twice as many rows: 192 rows on 8 experts of 4096 x 2048 at a skew of 0.5 int4 29 / 39, fp4 19 / 35, fp8 35 / 42, int8 34 / 43;
+// all 192 owned by one expert int4 20 / 38, fp4 18 / 35, fp8 20 / 45, int8 21 / 45.  The passes are found by looking through group_list, 256
+// experts at a time.
 static bool strips_preferred(const moe_grouped_args* a) {
     return a->G <= 1024 && columns(a) <= 32768 && a->M <= (columns(a) <= 16384 ? 24 : 12) * a->G;
 }
 
 // The narrowest strips whose first passes leave every CU at most one workgroup (an expert with more rows than one pass takes
 // has a workgroup per pass and strip, so there may be more).  Measured, 8 experts of K = 7168, 32 / 64 / 128 columns
-// a strip: N = 512 (4096 columns in all) int4 15 / 18 / 27 us, fp8 16 / 21 / 34; N = 2048 (16384) int4 28 / 20 / 28, fp8
-// 46 / 32 / 39; 16 experts of N = 2048 (32768) int4 75 / 49 / 34, fp8 89 / 60 / 49.
+// a strip: N = 512 (4096 columns in all) int4 12 / 16 / 25 us, fp4 10 / 13 / 23, fp8 15 / 16 / 24; N = 2048 (16384) int4 37 / 27 / 31, fp4 18 /
+// 17 / 26, fp8 47 / 32 / 36; 16 experts of N = 2048 (32768) int4 68 / 49 / 34, fp4 31 / 30 / 29, fp8 88 / 59 / 46.
 static GroupedKernel strip_width(const moe_grouped_args* a) {
     return columns(a) <= 8192 ? GroupedKernel::STRIPS_32 : columns(a) <= 16384 ? GroupedKernel::STRIPS_64 : GroupedKernel::STRIPS_128;
 }
 
 // GEMM op on the 4-bit containers: the small-stage kind (tiles of up to 32 rows, 8 wavefronts that split K, two workgroups per CU)
-// against the prefill kind (up to 160 rows, 4 wavefronts).  Times as fast, evenly and unevenly routed (skew 0.5; see bf16):
-//   12 rows per expert and fewer, always: 256 experts of 7168 x 2048, 4 rows int4 445 / 382 us, fp4 427 / 404, 12 rows 476 / 422 and 461 /
-//   441.  Beyond, it depends on the routing, as an expert of many rows is many passes over its weights: 16 rows, balanced top-k routing
-//   int4 483 / 425, fp4 464 / 451, skew 0.5 473 / 470 and 459 / 485, skew 1 354 / 401 and 359 / 418.
+// against the prefill kind (up to 160 rows, 4 wavefronts).  us, prefill / small-stage kind:
+//   12 rows per expert and fewer, always: 256 experts of 7168 x 2048, balanced top-k routing, 4 rows int4 428 / 369, fp4 409 / 380, 12 rows
+//   455 / 393 and 452 / 410, at a skew of 0.5 (see bf16) 454 / 410 and 423 / 425.  Beyond, it depends on the routing, as an expert of many rows
+//   is many passes over its weights: 16 rows, balanced int4 478 / 414, fp4 455 / 444, skew 0.5 473 / 446 and 446 / 450, skew 1 347 / 380 and
+//   352 / 391 (12 rows at a skew of 1: 330 / 351 and 337 / 340).
 //   Launches in which the prefill kind has a tile per CU at most, evenly routed: its 4 wavefronts are then alone there, and small tiles
-//   are more and fill it, until they too are more than the CUs, which a short K does not make up for.  Smallest / mean / largest over 8 to
-//   256 experts, K from 512, skews of 0 to 1.  Up to 128 tiles, int4: 32 rows 1.1 / 1.4 / 2.1, 40 rows 1.1 / 1.5 / 2.1, 48 rows 1.0 / 1.5 / 2.0
+//   are more and fill it, until they too are more than the CUs, which a short K does not make up for.  Times as fast, smallest / mean / largest
+//   over 8 to 256 experts, K from 512, skews of 0 to 1.  Up to 128 tiles, int4: 32 rows 1.1 / 1.4 / 2.1, 40 rows 1.1 / 1.5 / 2.1, 48 rows 1.0 / 1.5 / 2.0
 //   from K = 1024 on, but 0.9 at K = 512; fp4: 32 rows 1.1 / 1.4 / 2.1, 40 rows 1.0 / 1.4 / 2.1, 48 rows 0.96 / 1.4 / 2.0 from K = 1536 on, 0.9 and 0.8 at
 //   K = 1024 and 512;
 //   64 rows as low as 0.9 up to K = 2048.  129 to 192 tiles: 20 rows 1.0 / 1.3 / 1.9, 24 rows from K = 1536 on 1.15 / 1.4 / 1.95, at K = 1024 as low
