@@ -242,8 +242,8 @@ __global__ __launch_bounds__(256) void gemv_kmajor_kernel(const uint16_t* __rest
 // two v_permlane32_swap and two v_permlane16_swap per 16 bytes.
 // With the GEMM's rounding (ROUNDW below) the scale is in the weights when the MFMA sums over q, so its 32 k may come from four
 // blocks: MFMA j takes dword j of every lane's own block, x is read at those k (unit 16 c + 4 q + j), and a lane needs its own
-// block's scale only, one per 16 bytes.  No transpose, 2.14 instead of 2.45 vector instructions per weight, which is what bounds
-// that variant; us, before / now: 256 experts of 7168 x 2048, 512 rows, fp4_b32 370 / 346, fp4_b16 399 / 369; 480 rows on 64 of
+// block's scale only, one per 16 bytes.  No transpose, 2.15 instead of 2.43 vector instructions per weight (by counters, MFMAs
+// included; a wavefront now issues in 26 % of its cycles, waits for a slot in 33 %, for its loads in 41 %); us, before / now: 256 experts of 7168 x 2048, 512 rows, fp4_b32 370 / 346, fp4_b16 399 / 369; 480 rows on 64 of
 // 4096 x 1536 74 / 69 and 80 / 73; 8 single rows of 7168 x 512, fp4_b16 31 / 27.
 //
 // Scales: every lane of a column needs the same 4 scales per load, 8 bytes of a row -- read
@@ -282,9 +282,9 @@ __device__ __forceinline__ uint32_t e2m1_pair_bf16(uint32_t word, int sel) {
 // WHOLE: K is a multiple of 512.  Otherwise the last iteration has one to three groups: its loads past the row's end repeat the
 // last group (or the last scales), and the groups that are not there are not multiplied.
 // BLK = k per scale (32 or 16).  With 16, a 32-k block of a lane's row has two scales: the lanes
-// q < 2 of a column hold its first half, q >= 2 the second, so with the GEMM's rounding each lane
-// simply uses its half's scale, and with the GEMV's arithmetic the block takes two MFMAs, each on
-// one half of the lanes' codes (the other half zeroed), each partial sum scaled by its own scale.
+// q < 2 of a column hold its first half, q >= 2 the second, behind the transpose; the block takes two MFMAs, each on
+// one half of the lanes' codes (the other half zeroed), each partial sum scaled by its own scale.  (With the GEMM's rounding
+// there is no transpose: a lane has all 32 codes of its block and uses both scales.)
 // With at most 8 activation rows (STACK below) one MFMA does: fragment row r < 8 of x keeps only the first
 // 16 k of x row r, row 8 + r only the last 16 k, so the product's rows < 8 (lanes q < 2) are the first
 // scale's partial sums and rows >= 8 (q >= 2) the second's; each lane applies its own half's scale and the
@@ -298,7 +298,8 @@ __device__ __forceinline__ void gemv_fp4_mfma_rows(const uint8_t* __restrict__ w
     constexpr int U = GF_U;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i = lane & 15, q = lane >> 4;
-    // this wavefront's scale exchange: unit (2 q' + e) * 16 + i holds register e of lane (i, q')
+    // this wavefront's scale exchange: unit (2 q' + e) * 16 + i holds register e of lane (i, q'); ROUNDW: 8-byte units 64 q' + 16 k + i,
+    // what lane (i, k) needs of it
     u32x4_t* ss = xs + GF_LDS_UNITS + wave * GF_SCALE_UNITS;
     const int n = n0 + wave * 16 + i;
     const int nn = min(n, N - 1);

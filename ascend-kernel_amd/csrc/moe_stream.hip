@@ -6,8 +6,9 @@
 // columns (32, 64 or 128) of one expert and its wavefronts split K between them: each streams its own range into registers,
 // a few 32-k steps ahead, without LDS or barriers, and the partial sums meet once in LDS.  That case (18 MB of fp4 weights and
 // scales): 47.6 -> 9.6 us, int4 48 -> 12.6, fp8 70 -> 16; two tokens on 256 experts of 7168 x 2048: int4 49 -> 33 us.
-// What bounds it now: the launch, group_list and one step's latency are about 6 us; then what a few wavefronts per SIMD
-// issue (about 1.5 vector instructions per weight, 1.75 in 32-column strips of fp4) and the CU's vector memory path.
+// What bounds it now: the launch, group_list and one step's latency are about 6 us; then the wait for the loads of a few wavefronts per
+// SIMD (by counters 57 % of their cycles in that case, 33 % issuing: about 1.5 vector instructions per weight, 1.75 in 32-column strips of
+// fp4, 2.5 with what a wavefront does before and after its 28 steps).
 //
 // MFMA: v_mfma_f32_16x16x32_bf16, x rows in A, weights in B.  Lane (i, q) = (lane & 15, lane >> 4) loads, of each of the 8 k
 // rows 8 q + [0, 8) of a step, the dword (T = 8 and bytes: two) with its columns T i + [0, T): the 8 values of one column are
@@ -49,8 +50,9 @@ static __device__ __forceinline__ f32x4_t mfma(const u32x4_t& a, const u32x4_t& 
 }
 
 // 4-bit codes, two columns a lane: the four lanes of a quad use a byte each of the same dwords.  A lane that loads all 8 rows of its
-// dword loads four times what it uses, and the CU's vector memory path (64 bytes a cycle) is what such a launch then waits for as much
-// as for instruction issue.  So each lane of a quad loads two rows, and a 4 x 4 byte transpose over the quad (two DPP moves and two
+// dword loads four times what it uses, which takes the CU's vector memory path (64 bytes a cycle) four times as long (counters, together
+// with the gathering of bytes below: lookups in the vector cache 1.29 / 0.83 M, address unit busy 6.6 / 5.4 k cycles, 3.2 / 2.5 vector
+// instructions per weight).  So each lane of a quad loads two rows, and a 4 x 4 byte transpose over the quad (two DPP moves and two
 // v_perm per dword) gives every lane its byte of all eight.  us, without / with: 8 single rows of 7168 x 512, fp4 GEMV op 10.5 / 9.6,
 // GEMM op 11.2 / 10.5, int4 14.5 / 12.9; 192 rows on 8 experts of 4096 x 1024, fp4 15.1 / 13.4.  (Six or eight steps in flight instead of
 // four in the registers that this frees: 0 to 2 % faster with fp4 and K = 7168, 2 to 11 % slower otherwise.  16 wavefronts: 0.88 to 1.02 times.)

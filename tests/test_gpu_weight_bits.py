@@ -1,5 +1,5 @@
 """The weights that the GEMM op multiplies by, bit for bit: rows of x with a single 1 make y the rounded weights themselves, over
-every code and the whole range of scales, on every kernel that decodes the container."""
+every code and scales of most of the range (int4 and fp8: up to its ends), on every kernel that decodes the container."""
 import sys
 
 import numpy as np
@@ -66,7 +66,7 @@ INT4_EXTREME = INT4 + [("tiles_quad", 128, 256, 2048, 13), ("tiles_quad", 70, 25
 @pytest.mark.parametrize("kernel,G,K,N,rows", INT4_EXTREME)
 def test_int4_extreme_scales(kernel, G, K, N, rows):
     """Scales up to 2^125, beyond which code 0 itself is out of range, and down to the least subnormal: in all columns of some experts, in
-    a few groups of others (the tiles decode a step with a scale of 2^117 and more in another way), among ordinary ones."""
+    a few groups of others, among ordinary ones (the tiles compute a tile with a scale of 2^117.98 and more twice)."""
     _say(f"int4 weight bits, extreme scales, {kernel}")
     rng = np.random.default_rng(G + N + 1)
     case = H.make_case("int4", G, K, N, np.arange(1, G + 1) * rows, seed=G, group=32)
