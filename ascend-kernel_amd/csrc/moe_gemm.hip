@@ -1146,17 +1146,20 @@ __device__ __forceinline__ void gemm_tile_pair(const GemmParams& P, u32x4_t* sme
             for (int e = 0; e < 4; ++e) acc[0][t][e] += __shfl_xor(acc[0][t][e], 32);
     }
     if constexpr (wide_scales<FMT>(KIND) && !WIDE) {
-        // a weight that is no number leaves none in its column, in any row: row block 0 tells (see redo_wide)
-        float bad[4] = {0.f, 0.f, 0.f, 0.f};
+        // a weight that is no number leaves none in its column, in any row: row block 0 tells (see redo_wide); fp8: the hardware's
+        // conversions take any scale
+        if (!F8 || !f8_plain) {
+            float bad[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(acc[0][t]));   // not read ahead of the wait above
+            for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(acc[0][t]));   // not read ahead of the wait above
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+            for (int t = 0; t < 4; ++t)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) bad[e] = fmaf(acc[0][t][e], 0.f, bad[e]);
-        if (__any(__builtin_isnan((bad[0] + bad[1]) + (bad[2] + bad[3])))) [[unlikely]] {
-            if (lane == 0) {
-                tk.wide[0] = 1; tk.wide[1] = g; tk.wide[2] = (int)row0; tk.wide[3] = rows; tk.wide[4] = n0;
+                for (int e = 0; e < 4; ++e) bad[e] = fmaf(acc[0][t][e], 0.f, bad[e]);
+            if (__any(__builtin_isnan((bad[0] + bad[1]) + (bad[2] + bad[3])))) [[unlikely]] {
+                if (lane == 0) {
+                    tk.wide[0] = 1; tk.wide[1] = g; tk.wide[2] = (int)row0; tk.wide[3] = rows; tk.wide[4] = n0;
+                }
             }
         }
     }

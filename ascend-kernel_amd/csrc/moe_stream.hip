@@ -265,91 +265,96 @@ static __device__ __forceinline__ void stream_rows(const StreamParams& P, float*
                     decoded = f8_plain;
                 }
             }
-            // PAIR (fp8, rounded weights): the 2^8 that the decode through fp16 leaves out goes into the fp16 pairs, not into the block scale,
-            // which from 2^120 on it would take out of the range of fp32
-            auto decode = [&](auto PAIR) __attribute__((always_inline)) {
+            if constexpr (F8 && ROUNDW) {
+                // Through fp16 (see e4m3_ref_pair_over_256).  PAIR: the 2^8 that this leaves out goes into the fp16 pairs, not into the block scale, which
+                // from 2^120 on it would take out of the range of fp32.  32-column strips, which wait for their loads, pay nothing for
+                // the half instruction per weight (8 single rows of 7168 x 512 15.7 / 15.6 us); the others 2 % with random codes, so they
+                // look at the scale.
+                auto through_fp16 = [&](auto PAIR) __attribute__((always_inline)) {
 #pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    // the dwords of k rows 2 p and 2 p + 1
-                    const uint32_t a = QUAD ? 0u : B8 && T == 8 ? d.r[4 * p + (t0 >> 2)] : d.r[2 * p], b = QUAD ? 0u : B8 && T == 8 ? d.r[4 * p + 2 + (t0 >> 2)] : d.r[2 * p + 1];
-                    if constexpr (I4 && QUAD) {
-#pragma unroll
-                        for (int t = 0; t < TH; ++t) {
-                            const uint32_t h = quad_q[t][p >> 1];
-                            if constexpr (ROUNDW) {
-                                const f32x2_t f = p & 1 ? int4_codes<true>(h) : int4_codes<false>(h);
-                                bf[t][p] = pack_bf16_rne(fmaf(f[0], sc[t], -8.f * sc[t]), fmaf(f[1], sc[t], -8.f * sc[t]));
-                            } else {
-                                bf[t][p] = __builtin_bit_cast(uint32_t, p & 1 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h, 512.f, true)
-                                                                              : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h, 512.f, false));
-                            }
-                        }
-                    } else if constexpr (I4) {
-                        // the lane's bytes of the two rows side by side, (a, b) per byte; a nibble read as e4m3 is q / 512
-                        const uint32_t sel = b0 | ((4u + b0) << 8) | (T >= 4 ? ((b0 + 1u) << 16) | ((b0 + 5u) << 24) : 0x0c0c0000u);
-                        const uint32_t u = __builtin_amdgcn_perm(b, a, sel);
-                        const uint32_t h[2] = {u & 0x0f0f0f0fu, (u >> 4) & 0x0f0f0f0fu};   // even, odd columns
-#pragma unroll
-                        for (int t = 0; t < TH; ++t) {
-                            if constexpr (ROUNDW) {
-                                const f32x2_t f = t < 2 ? int4_codes<false>(h[t & 1]) : int4_codes<true>(h[t & 1]);
-                                bf[t][p] = pack_bf16_rne(fmaf(f[0], sc[t], -8.f * sc[t]), fmaf(f[1], sc[t], -8.f * sc[t]));
-                            } else {
-                                bf[t][p] = __builtin_bit_cast(uint32_t, t < 2 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h[t & 1], 512.f, false)
-                                                                              : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h[t & 1], 512.f, true));
-                            }
-                        }
-                    } else if constexpr (FP4 && T == 2) {
-                        bf[0][p] = fp4_pair(even_col[0], p, sc[0]);
-                        bf[1][p] = fp4_pair(odd_col[0], p, sc[1]);
-                    } else if constexpr (FP4 && T == 4) {
-#pragma unroll
-                        for (int t = 0; t < 4; ++t) bf[t][p] = fp4_pair(t & 1 ? odd_col[p >> 1] : even_col[p >> 1], 2 * (p & 1) + (t >> 1), sc[t]);
-                    } else if constexpr (FP4) {
-                        // nibbles of the two rows paired in a byte: even, odd columns
-                        const uint32_t m = 0x0f0f0f0fu;
-                        const uint32_t h[2] = {((a & m) | ((b << 4) & ~m)) >> (8 * b0), (((a >> 4) & m) | (b & ~m)) >> (8 * b0)};
-#pragma unroll
-                        for (int t = 0; t < TH; ++t) bf[t][p] = fp4_pair(h[t & 1], t >> 1, sc[t]);
-                    } else {
+                    for (int p = 0; p < 4; ++p) {
+                        const uint32_t a = T == 8 ? d.r[4 * p + (t0 >> 2)] : d.r[2 * p], b = T == 8 ? d.r[4 * p + 2 + (t0 >> 2)] : d.r[2 * p + 1];
 #pragma unroll
                         for (int t = 0; t < TH; ++t) {
                             const uint32_t at = T >= 4 ? (uint32_t)t : b0 + t;
-                            if constexpr (F8) {
-                                const uint32_t sel8 = at | 0x0c00u | ((4u + at) << 16) | 0x0c000000u;   // [a.byte, 0, b.byte, 0]
-                                uint32_t h2 = e4m3_ref_pair_over_256_fp16(__builtin_amdgcn_perm(b, a, sel8));
-                                if constexpr (PAIR) h2 = fp16_pair_times_256(h2);
-                                if constexpr (ROUNDW) {
-                                    const float s = PAIR ? __uint_as_float(d.s[0]) : f8s;
-                                    float nz = -0.0f;
-                                    asm volatile("" : "+v"(nz));   // kept in a register: not an inline constant
-                                    bf[t][p] = pack_bf16_rne(fp16_lo_times(h2, s, nz), fp16_hi_times(h2, s, nz));
-                                } else {
-                                    typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-                                    const half2_t hv = __builtin_bit_cast(half2_t, h2);
-                                    bf[t][p] = pack_bf16_rne((float)hv[0], (float)hv[1]);
-                                }
-                            } else {
-                                const float qa = (float)(int)(int8_t)(a >> (8 * at)), qb = (float)(int)(int8_t)(b >> (8 * at));
-                                bf[t][p] = pack_bf16_rne(__fmul_rn(__fadd_rn(qa, ch_o[t0 + t]), ch_s[t0 + t]), __fmul_rn(__fadd_rn(qb, ch_o[t0 + t]), ch_s[t0 + t]));
-                            }
+                            const uint32_t sel8 = at | 0x0c00u | ((4u + at) << 16) | 0x0c000000u;   // [a.byte, 0, b.byte, 0]
+                            uint32_t h2 = e4m3_ref_pair_over_256_fp16(__builtin_amdgcn_perm(b, a, sel8));
+                            if constexpr (PAIR) h2 = fp16_pair_times_256(h2);
+                            const float s = PAIR ? __uint_as_float(d.s[0]) : f8s;
+                            float nz = -0.0f;
+                            asm volatile("" : "+v"(nz));   // kept in a register: not an inline constant
+                            bf[t][p] = pack_bf16_rne(fp16_lo_times(h2, s, nz), fp16_hi_times(h2, s, nz));
+                        }
+                    }
+                };
+                if (T < 4)
+                    through_fp16(std::true_type{});
+                else if (!decoded) {
+                    if (((uint32_t)__builtin_amdgcn_readfirstlane((int)d.s[0]) & 0x7fffffffu) >= 0x7b800000u) [[unlikely]]   // 2^120
+                        through_fp16(std::true_type{});
+                    else
+                        through_fp16(std::false_type{});
+                }
+            } else
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                // the dwords of k rows 2 p and 2 p + 1
+                const uint32_t a = QUAD ? 0u : B8 && T == 8 ? d.r[4 * p + (t0 >> 2)] : d.r[2 * p], b = QUAD ? 0u : B8 && T == 8 ? d.r[4 * p + 2 + (t0 >> 2)] : d.r[2 * p + 1];
+                if constexpr (I4 && QUAD) {
+#pragma unroll
+                    for (int t = 0; t < TH; ++t) {
+                        const uint32_t h = quad_q[t][p >> 1];
+                        if constexpr (ROUNDW) {
+                            const f32x2_t f = p & 1 ? int4_codes<true>(h) : int4_codes<false>(h);
+                            bf[t][p] = pack_bf16_rne(fmaf(f[0], sc[t], -8.f * sc[t]), fmaf(f[1], sc[t], -8.f * sc[t]));
+                        } else {
+                            bf[t][p] = __builtin_bit_cast(uint32_t, p & 1 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h, 512.f, true)
+                                                                          : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h, 512.f, false));
+                        }
+                    }
+                } else if constexpr (I4) {
+                    // the lane's bytes of the two rows side by side, (a, b) per byte; a nibble read as e4m3 is q / 512
+                    const uint32_t sel = b0 | ((4u + b0) << 8) | (T >= 4 ? ((b0 + 1u) << 16) | ((b0 + 5u) << 24) : 0x0c0c0000u);
+                    const uint32_t u = __builtin_amdgcn_perm(b, a, sel);
+                    const uint32_t h[2] = {u & 0x0f0f0f0fu, (u >> 4) & 0x0f0f0f0fu};   // even, odd columns
+#pragma unroll
+                    for (int t = 0; t < TH; ++t) {
+                        if constexpr (ROUNDW) {
+                            const f32x2_t f = t < 2 ? int4_codes<false>(h[t & 1]) : int4_codes<true>(h[t & 1]);
+                            bf[t][p] = pack_bf16_rne(fmaf(f[0], sc[t], -8.f * sc[t]), fmaf(f[1], sc[t], -8.f * sc[t]));
+                        } else {
+                            bf[t][p] = __builtin_bit_cast(uint32_t, t < 2 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h[t & 1], 512.f, false)
+                                                                          : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h[t & 1], 512.f, true));
+                        }
+                    }
+                } else if constexpr (FP4 && T == 2) {
+                    bf[0][p] = fp4_pair(even_col[0], p, sc[0]);
+                    bf[1][p] = fp4_pair(odd_col[0], p, sc[1]);
+                } else if constexpr (FP4 && T == 4) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) bf[t][p] = fp4_pair(t & 1 ? odd_col[p >> 1] : even_col[p >> 1], 2 * (p & 1) + (t >> 1), sc[t]);
+                } else if constexpr (FP4) {
+                    // nibbles of the two rows paired in a byte: even, odd columns
+                    const uint32_t m = 0x0f0f0f0fu;
+                    const uint32_t h[2] = {((a & m) | ((b << 4) & ~m)) >> (8 * b0), (((a >> 4) & m) | (b & ~m)) >> (8 * b0)};
+#pragma unroll
+                    for (int t = 0; t < TH; ++t) bf[t][p] = fp4_pair(h[t & 1], t >> 1, sc[t]);
+                } else {
+#pragma unroll
+                    for (int t = 0; t < TH; ++t) {
+                        const uint32_t at = T >= 4 ? (uint32_t)t : b0 + t;
+                        if constexpr (F8) {
+                            const uint32_t sel8 = at | 0x0c00u | ((4u + at) << 16) | 0x0c000000u;   // [a.byte, 0, b.byte, 0]
+                            const uint32_t h2 = e4m3_ref_pair_over_256_fp16(__builtin_amdgcn_perm(b, a, sel8));
+                            typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+                            const half2_t hv = __builtin_bit_cast(half2_t, h2);
+                            bf[t][p] = pack_bf16_rne((float)hv[0], (float)hv[1]);
+                        } else {
+                            const float qa = (float)(int)(int8_t)(a >> (8 * at)), qb = (float)(int)(int8_t)(b >> (8 * at));
+                            bf[t][p] = pack_bf16_rne(__fmul_rn(__fadd_rn(qa, ch_o[t0 + t]), ch_s[t0 + t]), __fmul_rn(__fadd_rn(qb, ch_o[t0 + t]), ch_s[t0 + t]));
                         }
                     }
                 }
-            };
-            // (32-column strips, which wait for their loads, pay nothing for the half instruction per weight: 8 single rows of 7168 x
-            // 512 15.7 / 15.6 us; the others 2 % with random codes, so they look at the scale)
-            if constexpr (F8 && ROUNDW) {
-                if (T < 4)
-                    decode(std::true_type{});
-                else if (!decoded) {
-                    if (((uint32_t)__builtin_amdgcn_readfirstlane((int)d.s[0]) & 0x7fffffffu) >= 0x7b800000u) [[unlikely]]   // 2^120
-                        decode(std::true_type{});
-                    else
-                        decode(std::false_type{});
-                }
-            } else {
-                decode(std::false_type{});
             }
 #pragma unroll
             for (int t = 0; t < TH; ++t) {
