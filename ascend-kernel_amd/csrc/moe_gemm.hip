@@ -1685,7 +1685,9 @@ __device__ __forceinline__ void redo_wide(const GemmParams& P, u32x4_t* smem, co
     const int tid = threadIdx.x;
     auto word = [&](int e) { return __builtin_amdgcn_readfirstlane(tk.wide[e]); };
     const int g = word(1), row0 = word(2), rows = word(3), n0 = word(4);
-    __syncthreads();   // everybody has read them
+    // everybody has read them, and the tile's stores have ended: the second time another wavefront may store a row block
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
     if (tid == 0) tk.wide[0] = 0;
     __syncthreads();
     constexpr bool F8 = FMT == MOE_FMT_FP8_REF;
