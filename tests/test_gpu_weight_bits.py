@@ -139,7 +139,8 @@ def test_fp8(kernel, G, K, N, rows, codes):
 
 
 @pytest.mark.parametrize("kernel,G,K,N,rows", [("strips_32", 4, 2048, 512, 16), ("strips_64", 6, 2048, 2048, 16), ("strips_128", 10, 2048, 2048, 12),
-                                               ("tiles_pair", 20, 1024, 2048, 40), ("tiles_pair", 48, 1024, 2048, 17), ("tiles_quad", 2, 1024, 256, 256)])
+                                               ("tiles_pair", 20, 1024, 2048, 40), ("tiles_pair", 48, 1024, 2048, 17), ("tiles_quad", 2, 1024, 256, 256),
+                                               ("tiles_pair", 4, 512, 384, 160), ("tiles_quad", 4, 512, 384, 161)])
 def test_fp8_extreme_scales(kernel, G, K, N, rows):
     """Block scales up to 2^127 beside codes 0x7F: a weight does not depend on its neighbours' codes.  0x7F stands in blocks with ordinary
     scales in front of the large ones (even experts) and in the blocks with the large scales (their columns overflow and are left out)."""
